@@ -930,8 +930,8 @@ int sbslpm_direct_sum_inv_lap(sbslpm_ctx* c, int64_t n, const double* x, const d
   if (nt == 0) return SBSLPM_OK;
   int rc = ensure_scratch(c, direct_partials_size(nt, n, 1));
   if (rc) return rc;
-  launch_direct_inv_lap(nt, x + lb, y + lb, z + lb, n, x, y, z, area, pots, lb, false, c->scratch, soln + lb,
-                        c->stream);
+  launch_direct_inv_lap(nt, x + lb, y + lb, z + lb, n, x, y, z, area, pots, lb, false, c->dt.logtab, c->scratch,
+                        soln + lb, c->stream);
   return launched(c);
 }
 
@@ -951,7 +951,8 @@ int sbslpm_direct_sum_inv_lap_noalloc(sbslpm_ctx* c, int64_t n, const double* x,
                     "; split [lb, ub) into smaller slices");
   double* buf = direct_noalloc_scratch(c->device);
   if (!buf) return fail(c, SBSLPM_E_HIP, "direct_sum_inv_lap_noalloc: fixed scratch not set up on this device");
-  launch_direct_inv_lap(nt, x + lb, y + lb, z + lb, n, x, y, z, area, pots, lb, false, buf, soln + lb, c->stream);
+  launch_direct_inv_lap(nt, x + lb, y + lb, z + lb, n, x, y, z, area, pots, lb, false, c->dt.logtab, buf, soln + lb,
+                        c->stream);
   return launched(c);
 }
 
@@ -963,7 +964,8 @@ int sbslpm_direct_sum_inv_lap_targets(sbslpm_ctx* c, int64_t nt, const double* t
   if (nt == 0) return SBSLPM_OK;
   int rc = ensure_scratch(c, direct_partials_size(nt, ns, 1));
   if (rc) return rc;
-  launch_direct_inv_lap(nt, tx, ty, tz, ns, sx, sy, sz, area, pots, 0, true, c->scratch, soln, c->stream);
+  launch_direct_inv_lap(nt, tx, ty, tz, ns, sx, sy, sz, area, pots, 0, true, c->dt.logtab, c->scratch, soln,
+                        c->stream);
   return launched(c);
 }
 

@@ -197,6 +197,42 @@ __device__ inline double rcp64_pair(double d) {
   return fma(r, fma(-d, r, 1.0), r);
 }
 
+// 1/d_k of four denominators from one reciprocal of their product: the
+// estimate and its two Newton steps are shared, nine multiplies hand each
+// quotient out (19 vector-issue slots for four, a quarter-rate estimate counting
+// four, against 32 with rcp64 each).  Each product adds half an ulp, about 1.5
+// ulp in all; a zero denominator makes the whole batch NaN, as it makes the
+// sum that the batch belongs to without sharing.  The product of four must stay
+// in range, which d in [1e-16, 4] does by a wide margin.
+__device__ inline void rcp4(const double (&d)[4], double (&g)[4]) {
+  const double p01 = d[0] * d[1], p23 = d[2] * d[3];
+  const double r = rcp64(p01 * p23);
+  const double r01 = r * p23, r23 = r * p01;
+  g[0] = r01 * d[1];
+  g[1] = r01 * d[0];
+  g[2] = r23 * d[3];
+  g[3] = r23 * d[2];
+}
+
+// 1 - x.y in three fused multiply-adds from 1: the partial results shrink
+// towards the result, so the rounding is no larger than that of x.y formed
+// first and subtracted.
+__device__ inline double one_minus_dot(double x, double y, double z, double a, double b, double c) {
+  return fma(-z, c, fma(-y, b, fma(-x, a, 1.0)));
+}
+
+// A uniform constant moved into a vector register: the first step of a Horner
+// scheme whose multiplier is such a register is one three-operand fma (with
+// two constants in scalar registers the instruction set needs a copy).
+__device__ inline double in_vgpr(double v) {
+  __asm__ volatile("" : "+v"(v));
+  return v;
+}
+__device__ inline float in_vgpr_f(float v) {
+  __asm__ volatile("" : "+v"(v));
+  return v;
+}
+
 // interp_funcs_impl.hpp:114-142: leaf containing (x,y,z) or -1; xe gets the
 // label coordinates on the located face (locate_uniform: no panel reads).
 __device__ inline int locate_leaf(const DevTree& t, double x, double y, double z, double* xe) {
@@ -598,8 +634,8 @@ int direct_noalloc_init(int device);
 double* direct_noalloc_scratch(int device);
 void launch_direct_inv_lap(int64_t nt, const double* tx, const double* ty, const double* tz, int64_t ns,
                            const double* sx, const double* sy, const double* sz, const double* area,
-                           const double* pots, int64_t self_offset, bool guard_coincident, double* partials,
-                           double* soln, hipStream_t s);
+                           const double* pots, int64_t self_offset, bool guard_coincident,
+                           const LogTabEntry* logtab, double* partials, double* soln, hipStream_t s);
 void launch_direct_bve_vel(int64_t nt, const double* tx, const double* ty, const double* tz, int64_t ns,
                            const double* sx, const double* sy, const double* sz, const double* area,
                            const double* vor, const double* const* disp, double eps, double* partials,

@@ -2,8 +2,10 @@
 // and the Biot-Savart direct sum the reference lacks (same pair kernel as
 // bve_vel_impl.hpp:54-66).
 //
-// One wave64 per 64 targets and one source chunk per grid row; sources are
-// read as wave-uniform loads.  Each (target tile, chunk) writes a partial sum
+// A workgroup of four waves owns 64 NT targets (NT per lane) and one source
+// chunk per grid row; each wave takes a quarter of the chunk, sources are
+// wave-uniform loads taken four at a time, and the four waves' sums are added
+// in wave order through LDS.  Each (target tile, chunk) writes a partial sum
 // and a second kernel adds the chunks in a fixed order, so the result is
 // deterministic and needs no atomics (the reference does one atomic per pair).
 #include <algorithm>
@@ -18,51 +20,146 @@ constexpr int kWaves = 4;
 
 struct Plan {
   int64_t tiles, chunks, chunk_len;
+  int nt_lane;
 };
 
+// chunks is bounded by the waves of 64 targets it takes to fill the chip (4096)
+// and by 256 sources per chunk; it alone sets the scratch the sums need.
+// Two targets per lane halve the source loads and the uniform work per pair:
+// taken unless the second target would idle in a list of a few 64-target rows
+// (one row of 64 against 400,000 sources: 2x the pairs for nothing).
 Plan plan(int64_t nt, int64_t ns) {
   Plan p;
-  p.tiles = (nt + 63) / 64;
-  int64_t want = (4096 + p.tiles - 1) / p.tiles;  // aim for >= 4096 waves
+  const int64_t rows = (nt + 63) / 64;
+  int64_t want = (4096 + rows - 1) / rows;
   int64_t maxc = (ns + 255) / 256;
   p.chunks = std::max<int64_t>(1, std::min(want, maxc));
   p.chunk_len = (ns + p.chunks - 1) / p.chunks;
-  p.chunks = (ns + p.chunk_len - 1) / p.chunk_len;
+  p.chunks = p.chunk_len > 0 ? (ns + p.chunk_len - 1) / p.chunk_len : 1;
   if (p.chunks < 1) p.chunks = 1;
+  p.nt_lane = (rows & 1) && rows < 8 ? 1 : 2;
+  p.tiles = (rows + p.nt_lane - 1) / p.nt_lane;
   return p;
+}
+
+// This wave's part [a, b) of the workgroup's source chunk: quarters rounded up
+// to whole batches of four.
+__device__ inline void wave_sources(int64_t ns, int64_t chunk_len, int wave, int64_t& a, int64_t& b) {
+  const int64_t j0 = (int64_t)blockIdx.y * chunk_len, j1 = std::min<int64_t>(ns, j0 + chunk_len);
+  const int64_t q = ((j1 - j0 + 4 * kWaves - 1) / (4 * kWaves)) * 4;
+  a = std::min<int64_t>(j1, j0 + wave * q);
+  b = std::min<int64_t>(j1, a + q);
+}
+
+// Sum of v over the workgroup's waves in wave order, valid in wave 0.
+template <int K>
+__device__ inline void wave_sum(double (&v)[K], int wave, int lane) {
+  __shared__ double red[kWaves - 1][K][64];
+  if (wave > 0)
+#pragma unroll
+    for (int k = 0; k < K; ++k) red[wave - 1][k][lane] = v[k];
+  __syncthreads();
+  if (wave == 0)
+#pragma unroll
+    for (int w = 0; w < kWaves - 1; ++w)
+#pragma unroll
+      for (int k = 0; k < K; ++k) v[k] += red[w][k][lane];
 }
 
 // guard 0: skip j == self_offset + i (the reference's i != j);
 // guard 1: skip x.y >= 1 - 1e-15 (the FMM kernel's coincidence guard).
+// The logarithm is log_tab (fasttab.hpp, within 1.14 ulp) where 1 - x.y is a
+// normal number below 4; a batch of sources that holds the targets themselves,
+// a coincident or (guard 1) a skipped pair, or an argument outside that range
+// takes the library's logarithm with the guards, in the whole wave (one
+// unsigned maximum per pair and a ballot per batch).
+// Bound: FP64 vector issue, 27 instructions per pair (the library logarithm
+// on every pair took about 90).  24,576 x 24,576 points: 2.13 -> 0.57 ms.
+template <int NT>
 __global__ __launch_bounds__(256) void k_direct_log(int64_t nt, const double* __restrict__ tx,
                                                     const double* __restrict__ ty, const double* __restrict__ tz,
                                                     int64_t ns, const double* __restrict__ sx,
                                                     const double* __restrict__ sy, const double* __restrict__ sz,
                                                     const double* __restrict__ area, const double* __restrict__ pots,
                                                     int64_t self_offset, int guard, int64_t chunk_len,
+                                                    const LogTabEntry* __restrict__ logtab,
                                                     double* __restrict__ partials) {
   // x.y rounded exactly as written in direct_sum_impl.hpp:23 (no fused
   // multiply-add): for nearly coincident points log(1 - x.y) amplifies a
   // one-ulp change of x.y by 1/(1 - x.y).
 #pragma clang fp contract(off)
+  __shared__ LogTabEntry ltab[kLogTabSize];
+  for (int i = threadIdx.x; i < kLogTabSize; i += blockDim.x) ltab[i] = logtab[i];
+  __syncthreads();
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int lane = threadIdx.x & 63;
-  const int64_t tile = (int64_t)blockIdx.x * kWaves + wave;
-  if (tile * 64 >= nt) return;
-  const int64_t i = std::min<int64_t>(tile * 64 + lane, nt - 1);
-  const int64_t self = self_offset + i;
-  const double x = tx[i], y = ty[i], z = tz[i];
-  const int64_t j0 = (int64_t)blockIdx.y * chunk_len, j1 = std::min<int64_t>(ns, j0 + chunk_len);
-  double acc = 0;
-  for (int64_t j = j0; j < j1; ++j) {
-    const double dp = x * sx[j] + y * sy[j] + z * sz[j];
-    const double l = log(fmax(1.0 - dp, 1e-300)) * (area[j] * pots[j]);
-    const bool skip = guard ? !(dp < 1.0 - 1e-15) : (j == self);
-    acc += skip ? 0.0 : l;
+  const int64_t i0 = (int64_t)blockIdx.x * (64 * NT);
+  double x[NT], y[NT], z[NT], acc[NT];
+#pragma unroll
+  for (int t = 0; t < NT; ++t) {
+    const int64_t i = std::min<int64_t>(i0 + t * 64 + lane, nt - 1);
+    x[t] = tx[i]; y[t] = ty[i]; z[t] = tz[i];
+    acc[t] = 0;
   }
-  if (tile * 64 + lane < nt) partials[(int64_t)blockIdx.y * nt + i] = kNegInv4Pi * acc;
+  int64_t a, b;
+  wave_sources(ns, chunk_len, wave, a, b);
+  const int64_t self_lo = self_offset + i0, self_hi = self_lo + 64 * NT;
+  // high words of the fast form's range: [2^-48, 4) or (1e-300, 4)
+  const uint32_t lo = guard ? 0x3cf00000u : 0x01a56e20u;
+  const uint32_t span = 0x40100000u - lo;
+  const double c6 = in_vgpr(-1.0 / 6.0);
+  auto guarded = [&](int t, int64_t j) {
+    const int64_t i = std::min<int64_t>(i0 + t * 64 + lane, nt - 1);
+    const double dp = x[t] * sx[j] + y[t] * sy[j] + z[t] * sz[j];
+    const double l = log(fmax(1.0 - dp, 1e-300)) * (area[j] * pots[j]);
+    const bool skip = guard ? !(dp < 1.0 - 1e-15) : (j == self_offset + i);
+    acc[t] += skip ? 0.0 : l;
+  };
+  int64_t j = a;
+  for (; j + 4 <= b; j += 4) {
+    double d[NT][4];
+    uint32_t far = 0;
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+      const double s0 = sx[j + k], s1 = sy[j + k], s2 = sz[j + k];
+#pragma unroll
+      for (int t = 0; t < NT; ++t) {
+        d[t][k] = 1.0 - (x[t] * s0 + y[t] * s1 + z[t] * s2);
+        const uint32_t h = (uint32_t)__double2hiint(d[t][k]) - lo;
+        far = h > far ? h : far;
+      }
+    }
+    const bool own = !guard && j < self_hi && j + 4 > self_lo;
+    if (own || __builtin_amdgcn_ballot_w64(far >= span) != 0) {
+      for (int k = 0; k < 4; ++k)
+#pragma unroll
+        for (int t = 0; t < NT; ++t) guarded(t, j + k);
+      continue;
+    }
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+      const double q = area[j + k] * pots[j + k];
+#pragma unroll
+      for (int t = 0; t < NT; ++t) acc[t] = fma(log_tab(d[t][k], ltab, c6), q, acc[t]);
+    }
+  }
+  for (; j < b; ++j)
+#pragma unroll
+    for (int t = 0; t < NT; ++t) guarded(t, j);
+  wave_sum(acc, wave, lane);
+  if (wave == 0)
+#pragma unroll
+    for (int t = 0; t < NT; ++t)
+      if (i0 + t * 64 + lane < nt) partials[(int64_t)blockIdx.y * nt + i0 + t * 64 + lane] = kNegInv4Pi * acc[t];
 }
 
+// Bound: FP64 vector issue.  The four denominators of a batch share one
+// reciprocal (rcp4: 12.5 instruction slots per pair with the loads' share
+// against 17 with a reciprocal each), and 1 - x.y is one chain of fused
+// multiply-adds from 1.  4,096 targets x 393,216 sources: 4.09 -> 0.78 ms (one
+// target per lane and one source per step waited on each source's scalar loads;
+// now vector issue is busy 83% of the time, at 2.1 GHz under this load).
+template <int NT>
 __global__ __launch_bounds__(256) void k_direct_bs(int64_t nt, const double* __restrict__ tx,
                                                    const double* __restrict__ ty, const double* __restrict__ tz,
                                                    int64_t ns, const double* __restrict__ sx,
@@ -71,25 +168,60 @@ __global__ __launch_bounds__(256) void k_direct_bs(int64_t nt, const double* __r
                                                    double eps, int64_t chunk_len, double* __restrict__ partials) {
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int lane = threadIdx.x & 63;
-  const int64_t tile = (int64_t)blockIdx.x * kWaves + wave;
-  if (tile * 64 >= nt) return;
-  const int64_t i = std::min<int64_t>(tile * 64 + lane, nt - 1);
-  const double x = tx[i], y = ty[i], z = tz[i];
-  const int64_t j0 = (int64_t)blockIdx.y * chunk_len, j1 = std::min<int64_t>(ns, j0 + chunk_len);
-  double w0 = 0, w1 = 0, w2 = 0;
-  for (int64_t j = j0; j < j1; ++j) {
-    const double a = sx[j], b = sy[j], c = sz[j];
-    const double dp = x * a + y * b + z * c;
-    const double g = rcp64((1.0 - dp) + eps) * (area[j] * vor[j]);
-    w0 = fma(g, a, w0);
-    w1 = fma(g, b, w1);
-    w2 = fma(g, c, w2);
+  const int64_t i0 = (int64_t)blockIdx.x * (64 * NT);
+  double x[NT], y[NT], z[NT], w[3 * NT];
+#pragma unroll
+  for (int t = 0; t < NT; ++t) {
+    const int64_t i = std::min<int64_t>(i0 + t * 64 + lane, nt - 1);
+    x[t] = tx[i]; y[t] = ty[i]; z[t] = tz[i];
+    w[3 * t] = w[3 * t + 1] = w[3 * t + 2] = 0;
   }
-  if (tile * 64 + lane < nt) {
+  int64_t a, b;
+  wave_sources(ns, chunk_len, wave, a, b);
+  int64_t j = a;
+  for (; j + 4 <= b; j += 4) {
+    double s0[4], s1[4], s2[4], q[4];
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+      s0[k] = sx[j + k]; s1[k] = sy[j + k]; s2[k] = sz[j + k];
+      q[k] = area[j + k] * vor[j + k];
+    }
+#pragma unroll
+    for (int t = 0; t < NT; ++t) {
+      double d[4], g[4];
+#pragma unroll
+      for (int k = 0; k < 4; ++k) d[k] = one_minus_dot(x[t], y[t], z[t], s0[k], s1[k], s2[k]) + eps;
+      rcp4(d, g);
+#pragma unroll
+      for (int k = 0; k < 4; ++k) {
+        const double gq = g[k] * q[k];
+        w[3 * t] = fma(gq, s0[k], w[3 * t]);
+        w[3 * t + 1] = fma(gq, s1[k], w[3 * t + 1]);
+        w[3 * t + 2] = fma(gq, s2[k], w[3 * t + 2]);
+      }
+    }
+  }
+  for (; j < b; ++j) {
+    const double s0 = sx[j], s1 = sy[j], s2 = sz[j], q = area[j] * vor[j];
+#pragma unroll
+    for (int t = 0; t < NT; ++t) {
+      const double g = rcp64(one_minus_dot(x[t], y[t], z[t], s0, s1, s2) + eps) * q;
+      w[3 * t] = fma(g, s0, w[3 * t]);
+      w[3 * t + 1] = fma(g, s1, w[3 * t + 1]);
+      w[3 * t + 2] = fma(g, s2, w[3 * t + 2]);
+    }
+  }
+  wave_sum(w, wave, lane);
+  if (wave > 0) return;
+#pragma unroll
+  for (int t = 0; t < NT; ++t) {
+    const int64_t i = i0 + t * 64 + lane;
+    if (i >= nt) continue;
+    const double *u = w + 3 * t;
     double* p = partials + (int64_t)blockIdx.y * 3 * nt;
-    p[i] = kNegInv4Pi * (y * w2 - z * w1);
-    p[nt + i] = kNegInv4Pi * (z * w0 - x * w2);
-    p[2 * nt + i] = kNegInv4Pi * (x * w1 - y * w0);
+    p[i] = kNegInv4Pi * (y[t] * u[2] - z[t] * u[1]);
+    p[nt + i] = kNegInv4Pi * (z[t] * u[0] - x[t] * u[2]);
+    p[2 * nt + i] = kNegInv4Pi * (x[t] * u[1] - y[t] * u[0]);
   }
 }
 
@@ -97,14 +229,21 @@ struct Ptr3 {
   double* p[3];
 };
 
-__global__ void k_reduce(int64_t nt, int ncomp, int64_t chunks, const double* __restrict__ partials, Ptr3 out) {
-  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= nt) return;
-  for (int f = 0; f < ncomp; ++f) {
-    double s = 0;
-    for (int64_t c = 0; c < chunks; ++c) s += partials[(c * ncomp + f) * nt + i];
-    out.p[f][i] += s;
-  }
+// out[blockIdx.y] += the chunks' partial sums: 64 targets per workgroup, wave w
+// adds chunks w, w + 4, ..., the waves' sums are added in wave order.  (With one
+// thread per target walking every chunk of three components, the 64 chunks of
+// 4,096 targets took 52 us, a chain of loads in 64 waves; now 4.9 us.)
+__global__ __launch_bounds__(256) void k_reduce(int64_t nt, int ncomp, int64_t chunks,
+                                                const double* __restrict__ partials, Ptr3 out) {
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int lane = threadIdx.x & 63;
+  const int f = (int)blockIdx.y;
+  const int64_t i = (int64_t)blockIdx.x * 64 + lane, ic = std::min<int64_t>(i, nt - 1);
+  double s[1] = {0};
+#pragma unroll 4
+  for (int64_t c = wave; c < chunks; c += kWaves) s[0] += partials[(c * ncomp + f) * nt + ic];
+  wave_sum(s, wave, lane);
+  if (wave == 0 && i < nt) out.p[f][i] += s[0];
 }
 
 // Displaced, re-projected source positions (bve_vel_impl.hpp:57-60).
@@ -158,15 +297,16 @@ int64_t direct_partials_size(int64_t nt, int64_t ns, int ncomp) {
 
 void launch_direct_inv_lap(int64_t nt, const double* tx, const double* ty, const double* tz, int64_t ns,
                            const double* sx, const double* sy, const double* sz, const double* area,
-                           const double* pots, int64_t self_offset, bool guard_coincident, double* partials,
-                           double* soln, hipStream_t s) {
+                           const double* pots, int64_t self_offset, bool guard_coincident,
+                           const LogTabEntry* logtab, double* partials, double* soln, hipStream_t s) {
   if (nt <= 0) return;
-  Plan p = plan(nt, ns);
-  dim3 grid((unsigned)((p.tiles + kWaves - 1) / kWaves), (unsigned)p.chunks);
-  hipLaunchKernelGGL(k_direct_log, grid, dim3(64 * kWaves), 0, s, nt, tx, ty, tz, ns, sx, sy, sz, area, pots,
-                     self_offset, guard_coincident ? 1 : 0, p.chunk_len, partials);
+  const Plan p = plan(nt, ns);
+  const dim3 grid((unsigned)p.tiles, (unsigned)p.chunks);
+  auto kernel = p.nt_lane == 2 ? k_direct_log<2> : k_direct_log<1>;
+  hipLaunchKernelGGL(kernel, grid, dim3(64 * kWaves), 0, s, nt, tx, ty, tz, ns, sx, sy, sz, area, pots, self_offset,
+                     guard_coincident ? 1 : 0, p.chunk_len, logtab, partials);
   Ptr3 out{{soln, nullptr, nullptr}};
-  hipLaunchKernelGGL(k_reduce, dim3((unsigned)((nt + 255) / 256)), dim3(256), 0, s, nt, 1, p.chunks,
+  hipLaunchKernelGGL(k_reduce, dim3((unsigned)((nt + 63) / 64), 1), dim3(64 * kWaves), 0, s, nt, 1, p.chunks,
                      (const double*)partials, out);
 }
 
@@ -175,7 +315,7 @@ void launch_direct_bve_vel(int64_t nt, const double* tx, const double* ty, const
                            const double* vor, const double* const* disp, double eps, double* partials,
                            double* const* vel, hipStream_t s) {
   if (nt <= 0) return;
-  Plan p = plan(nt, ns);
+  const Plan p = plan(nt, ns);
   const double *ax = sx, *ay = sy, *az = sz;
   if (disp && disp[0]) {
     double* moved = partials + p.chunks * 3 * nt;
@@ -183,11 +323,12 @@ void launch_direct_bve_vel(int64_t nt, const double* tx, const double* ty, const
                        disp[1], disp[2], moved);
     ax = moved; ay = moved + ns; az = moved + 2 * ns;
   }
-  dim3 grid((unsigned)((p.tiles + kWaves - 1) / kWaves), (unsigned)p.chunks);
-  hipLaunchKernelGGL(k_direct_bs, grid, dim3(64 * kWaves), 0, s, nt, tx, ty, tz, ns, ax, ay, az, area, vor, eps,
+  const dim3 grid((unsigned)p.tiles, (unsigned)p.chunks);
+  auto kernel = p.nt_lane == 2 ? k_direct_bs<2> : k_direct_bs<1>;
+  hipLaunchKernelGGL(kernel, grid, dim3(64 * kWaves), 0, s, nt, tx, ty, tz, ns, ax, ay, az, area, vor, eps,
                      p.chunk_len, partials);
   Ptr3 out{{vel[0], vel[1], vel[2]}};
-  hipLaunchKernelGGL(k_reduce, dim3((unsigned)((nt + 255) / 256)), dim3(256), 0, s, nt, 3, p.chunks,
+  hipLaunchKernelGGL(k_reduce, dim3((unsigned)((nt + 63) / 64), 3), dim3(64 * kWaves), 0, s, nt, 3, p.chunks,
                      (const double*)partials, out);
 }
 

@@ -31,19 +31,6 @@ struct CPtr3 {
   const double* p[3];
 };
 
-// A uniform constant moved into a vector register: the first step of a Horner
-// scheme whose multiplier is such a register is one three-operand fma (with
-// two constants in scalar registers the instruction set needs a copy).
-__device__ inline double in_vgpr(double v) {
-  __asm__ volatile("" : "+v"(v));
-  return v;
-}
-__device__ inline float in_vgpr_f(float v) {
-  __asm__ volatile("" : "+v"(v));
-  return v;
-}
-
-
 // Member slices of a batched launch (gridDim.y members): charges and
 // displacements of the sources, outputs of the targets.
 __device__ inline void member_sources(const DevTree& t, const double* __restrict__& q_part,

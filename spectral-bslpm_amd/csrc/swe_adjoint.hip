@@ -272,17 +272,6 @@ __global__ void k_lap_tgt(DevTree t, const double* __restrict__ psi_part, const 
   rec[u] = LapTgt{t.px[u], t.py[u], t.pz[u], p};
 }
 
-// Horner multipliers of the FP64 transposed Laplacian in vector registers (the
-// first step of each Horner scheme is then one three-operand fma).
-__device__ inline double in_vgpr(double v) {
-  __asm__ volatile("" : "+v"(v));
-  return v;
-}
-__device__ inline float in_vgpr_f(float v) {
-  __asm__ volatile("" : "+v"(v));
-  return v;
-}
-
 // K(t) and K'(t) eps^{5/2} in the folded form of lapkernel.hpp.  fast: t >= 6 eps
 // (K = A + E B, K' = A' + E D); otherwise the erf factor f and the e^{-s^2}
 // term g, and zero at or below the cut.
