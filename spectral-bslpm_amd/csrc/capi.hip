@@ -231,12 +231,16 @@ int upload(sbslpm_ctx* c, void* dst, const void* src, size_t bytes) {
 // workgroups of `waves` tiles, for the ranges of the matrix-core kernels
 // (mfma) or of the vector-unit ones.
 static PairShape full_list_shape(const Tree& t, int waves, int xcd, bool mfma) {
-  PairShape sh{waves, xcd, 0};
+  PairShape sh{waves, xcd, 0, 0};
   if (xcd == 2) {
     const int* xs = t.xcd_start.data() + (mfma ? 0 : 9);
-    int most = 0;
-    for (int x = 0; x < 8; ++x) most = std::max(most, (xs[x + 1] - xs[x] + waves - 1) / waves);
+    int most = 0, tiles = 0;
+    for (int x = 0; x < 8; ++x) {
+      most = std::max(most, (xs[x + 1] - xs[x] + waves - 1) / waves);
+      tiles = std::max(tiles, xs[x + 1] - xs[x]);
+    }
     sh.grid = 8 * most;
+    sh.grid1 = 8 * tiles;
   }
   return sh;
 }

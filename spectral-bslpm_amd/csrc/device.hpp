@@ -70,11 +70,13 @@ constexpr int kWavesPerBlock = 4;
 //          only; `grid` is then the launch's workgroup count, 8 x the largest
 //          range in workgroups.
 // The default (four waves, mapping 0) needs no ranges; at 6 x 512^2 the
-// autotuner picks mapping 2.
+// autotuner picks mapping 2.  The FP64 kernel gives a whole workgroup to each
+// tile (pairwalk.hpp): there only the mapping counts, with grid1 workgroups.
 struct PairShape {
   int waves = kWavesPerBlock;
   int xcd = 0;
   int grid = 0;
+  int grid1 = 0;
 };
 
 // Hardware dispatches workgroup b to XCD b % 8.  Give each XCD a contiguous

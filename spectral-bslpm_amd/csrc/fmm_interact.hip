@@ -20,6 +20,7 @@
 
 #include "device.hpp"
 #include "lapkernel.hpp"
+#include "pairwalk.hpp"
 
 namespace sbslpm {
 namespace {
@@ -123,36 +124,56 @@ __global__ void k_src32(DevTree t, const double* __restrict__ q_part, const doub
   rec[u] = SrcRec32{(float)(x - P.cx), (float)(y - P.cy), (float)(z - P.cz), (float)(kNegInv4Pi * q)};
 }
 
-// FP64 Biot-Savart pair kernel, the reference's arithmetic:
-// g = -q/(4 pi (1 - x.y + eps)).
-__global__ __launch_bounds__(256) void k_bve64(DevTree t, const TargetTile* __restrict__ tiles, int ntiles,
-                                               const SourceSet* __restrict__ sets,
-                                               const SrcRec64* __restrict__ rec, double eps, Ptr3 part,
-                                               Ptr3 proxy, int assign, int xcd) {
+// FP64 Biot-Savart pair kernel: g = -q/(4 pi (1 - x.y + eps)).  S waves share a
+// tile (pairwalk.hpp) and take the sources in batches of four with one shared
+// reciprocal (rcp4).
+// Bound: FP64 vector issue, 12.25 slots per pair against 15 with a reciprocal
+// each, at the 2.1 GHz the chip holds under this load.  Microseconds per launch
+// before (one wave per tile, one source at a time) and now: 6 x 28^2 180 -> 20,
+// 6 x 64^2 303 -> 58, 6 x 224^2 642 -> 407, 6 x 512^2 2945 -> 2358 (2326 is the
+// issue time of its pairs alone).
+template <int S>
+__global__ __launch_bounds__(64 * S) void k_bve64(DevTree t, const TargetTile* __restrict__ tiles, int ntiles,
+                                                  const SourceSet* __restrict__ sets,
+                                                  const SrcRec64* __restrict__ rec, double eps, Ptr3 part, Ptr3 proxy,
+                                                  int assign, int xcd) {
   member_targets(t, part, proxy);
   rec += (int64_t)blockIdx.y * t.U;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int lane = threadIdx.x & 63;
-  const int tile = shaped_tile(t.xcd_start ? t.xcd_start + 9 : nullptr, wave, xcd);
-  if (tile >= ntiles) return;
+  const int tile = walk_tile(t.xcd_start ? t.xcd_start + 9 : nullptr, xcd);
+  if (tile >= ntiles) return;  // the whole workgroup
   const TargetTile T = tiles[tile];
   const int64_t u = (int64_t)T.first + (lane < T.count ? lane : T.count - 1);
   const double x = t.px[u], y = t.py[u], z = t.pz[u];
-  double w0 = 0, w1 = 0, w2 = 0;
-  for (int e = T.src_begin; e < T.src_end; ++e) {
-    const SourceSet S = sets[e];
-    const SrcRec64* __restrict__ r = rec + S.first;
-#pragma unroll 3
-    for (int k = 0; k < S.count; ++k) {
-      const SrcRec64 s = r[k];
-      const double dp = x * s.x + y * s.y + z * s.z;
-      const double g = rcp64_pair((1.0 - dp) + eps) * s.q;
-      w0 = fma(g, s.x, w0);
-      w1 = fma(g, s.y, w1);
-      w2 = fma(g, s.z, w2);
+  double w[3] = {0, 0, 0};
+  walk_sets<S>(T, sets, wave, [&](const SourceSet& set, int a, int b) {
+    const SrcRec64* __restrict__ r = rec + set.first;
+    int k = a;
+    for (; k + 4 <= b; k += 4) {
+      double d[4], g[4];
+#pragma unroll
+      for (int i = 0; i < 4; ++i) d[i] = one_minus_dot(x, y, z, r[k + i].x, r[k + i].y, r[k + i].z) + eps;
+      rcp4(d, g);
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const double gq = g[i] * r[k + i].q;
+        w[0] = fma(gq, r[k + i].x, w[0]);
+        w[1] = fma(gq, r[k + i].y, w[1]);
+        w[2] = fma(gq, r[k + i].z, w[2]);
+      }
     }
-  }
-  if (lane < T.count) store_u(t, u, part, proxy, y * w2 - z * w1, z * w0 - x * w2, x * w1 - y * w0, assign);
+    for (; k < b; ++k) {
+      const SrcRec64 s = r[k];
+      const double g = rcp64_pair(one_minus_dot(x, y, z, s.x, s.y, s.z) + eps) * s.q;
+      w[0] = fma(g, s.x, w[0]);
+      w[1] = fma(g, s.y, w[1]);
+      w[2] = fma(g, s.z, w[2]);
+    }
+  });
+  tile_sum<S>(w, wave, lane);
+  if (wave == 0 && lane < T.count)
+    store_u(t, u, part, proxy, y * w[2] - z * w[1], z * w[0] - x * w[2], x * w[1] - y * w[0], assign);
 }
 
 // FP64 log pair kernel: psi += -1/(4 pi) log(1 - x.y) q, pairs with
@@ -1014,8 +1035,10 @@ void launch_bve_interact64(const DevTree& t, const TargetTile* tiles, int ntiles
                            hipStream_t s, bool assign, int nmem, PairShape shape) {
   if (ntiles == 0) return;
   shape = checked_shape(t, shape);
-  hipLaunchKernelGGL(k_bve64, dim3(pair_grid(ntiles, shape), nmem), dim3(64 * shape.waves), 0, s, t, tiles,
-                     ntiles, sets, rec, eps, ptr3(out_part), ptr3(out_proxy), assign ? 1 : 0, shape.xcd);
+  const int S = tile_waves(ntiles);
+  auto kernel = S == 16 ? k_bve64<16> : S == 8 ? k_bve64<8> : k_bve64<4>;
+  hipLaunchKernelGGL(kernel, dim3(walk_grid(ntiles, shape), nmem), dim3(64 * S), 0, s, t, tiles, ntiles, sets, rec, eps,
+                     ptr3(out_part), ptr3(out_proxy), assign ? 1 : 0, shape.xcd);
 }
 
 void launch_poisson_interact64(const DevTree& t, const TargetTile* tiles, int ntiles, const SourceSet* sets,

@@ -1,0 +1,60 @@
+"""FP64 pair kernels whose workgroups share a target tile (csrc/pairwalk.hpp) against the
+oracle: 16, 8 and 4 waves per tile, source sets that batches of four and parts of a set divide
+unevenly (25, 36, 49, 81 and 121 points), one to three tiles per panel, accumulating and
+displaced.  Both sides sum the same pairs: 1e-12 leaves room for the rounding of 1 - x.y
+(a few units of 1e-16 over eps = 1e-4) at the nearest pairs."""
+import numpy as np
+import pytest
+
+from conftest import to_gpu, to_np
+
+pytestmark = pytest.mark.gpu
+
+EPS = 1e-4
+# levels, proxy degree, leaf grid side: tile lists of 30 to 8,190
+TREES = [(2, 4, 5), (3, 6, 7), (3, 8, 9), (4, 10, 11), (5, 8, 6), (6, 5, 6)]
+
+
+@pytest.fixture(scope="module", params=TREES, ids=lambda p: "L%d-d%d-m%d" % p)
+def case(request, sb, orc, torch_gpu):
+    levels, d, m = request.param
+    print(f"\n[case L{levels} d{d} m{m}]", flush=True)
+    ctx = sb.Context(sb.RunConfig(levels=levels, interp_degree=d, leaf_degree=m - 1, kernel_eps=EPS,
+                                  weights="clenshaw_curtis"))
+    o = orc.OracleFMM(levels, d, m - 1, 0.7, 1)
+    x, y, z, a = o.spec_points()
+    rng = np.random.default_rng(levels + d)
+    qp, qx = rng.normal(size=x.shape), rng.normal(size=(ctx.sizes.P, ctx.sizes.n))
+    dp = [1e-3 * rng.normal(size=x.shape) for _ in range(3)]
+    dx = [1e-3 * rng.normal(size=qx.shape) for _ in range(3)]
+    return dict(ctx=ctx, o=o, t=torch_gpu, W=sb.workloads, qp=qp, qx=qx, dp=dp, dx=dx, a=a, shape=x.shape)
+
+
+def up(case, arrays):
+    return [to_gpu(case["t"], v) for v in arrays]
+
+
+def close(case, got_part, got_proxy, part, proxy, start=0.0):
+    """Particle rows and the rows of non-leaf panels (leaf proxy rows are not targets)."""
+    case["ctx"].synchronize()
+    off = case["o"].offset
+    for g, e in zip(got_part, part):
+        e = np.asarray(e).reshape(case["shape"]) + start
+        assert np.linalg.norm(to_np(g) - e) <= 1e-12 * np.linalg.norm(e)
+    for g, e in zip(got_proxy, proxy):
+        e = np.asarray(e)[:off] + start
+        if np.any(np.asarray(e) != start):
+            assert np.linalg.norm(to_np(g)[:off] - e) <= 1e-12 * np.linalg.norm(e)
+
+
+@pytest.mark.parametrize("displaced", [False, True])
+def test_vortex_pairs(case, displaced):
+    ctx, o = case["ctx"], case["o"]
+    dp, dx = (case["dp"], case["dx"]) if displaced else (None, None)
+    ep, ex = o.bve_vel_interactions(case["qp"], case["qx"], EPS, dp, dx)
+    phi_part, phi_proxy = ctx.zeros_part(3), ctx.zeros_proxy(3)
+    for v in phi_part + phi_proxy:
+        v.fill_(0.5)
+    gp, gx = ctx.bve_vel_interactions(*up(case, [case["qp"], case["qx"]]), up(case, dp) if dp else None,
+                                      up(case, dx) if dx else None, phi_part=phi_part, phi_proxy=phi_proxy)
+    close(case, gp, gx, ep, ex, 0.5)
