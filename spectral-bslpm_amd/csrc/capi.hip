@@ -249,10 +249,12 @@ static PairShape full_list_shape(const Tree& t, int waves, int xcd, bool mfma) {
 // per process.
 struct HostTables {
   std::vector<LogTabEntry> log = std::vector<LogTabEntry>(kLogTabSize);
+  std::vector<LogTabEntry> log_wide = std::vector<LogTabEntry>(kLogWideSize);
   std::vector<double> exp = std::vector<double>(kExpTabSize);
   std::vector<double> exp_neg = std::vector<double>(kExpNegTabSize);
   HostTables() {
     build_log_table(log.data());
+    build_log_wide_table(log_wide.data());
     build_exp_table(exp.data());
     build_exp_neg_table(exp_neg.data());
   }
@@ -361,7 +363,7 @@ int sbslpm_ctx_create(const sbslpm_params* p, sbslpm_ctx** out) {
   size_t o_disppart = A.take<double>(3 * NP), o_dispproxy = A.take<double>(3 * Pn);
   size_t o_vstage = A.take<double>(9 * NP), o_newvor = A.take<double>(NP), o_dep = A.take<double>(3 * NP);
   size_t o_vnext = A.take<double>(NP), o_trnext = A.take<double>(NP * ntr);
-  size_t o_ltab = A.take<LogTabEntry>(kLogTabSize), o_etab = A.take<double>(kExpTabSize),
+  size_t o_ltab = A.take<LogTabEntry>(kLogTabSize), o_lwide = A.take<LogTabEntry>(kLogWideSize), o_etab = A.take<double>(kExpTabSize),
          o_entab = A.take<double>(kExpNegTabSize), o_xcd = A.take<int>(18);
   size_t total = A.take<char>(256);
   if (hipMalloc(&c->arena, total) != hipSuccess) {
@@ -397,6 +399,7 @@ int sbslpm_ctx_create(const sbslpm_params* p, sbslpm_ctx** out) {
   {
     const HostTables& ht = host_tables();
     rc |= upload(c, b + o_ltab, ht.log.data(), kLogTabSize * sizeof(LogTabEntry));
+    rc |= upload(c, b + o_lwide, ht.log_wide.data(), kLogWideSize * sizeof(LogTabEntry));
     rc |= upload(c, b + o_etab, ht.exp.data(), kExpTabSize * sizeof(double));
     rc |= upload(c, b + o_entab, ht.exp_neg.data(), kExpNegTabSize * sizeof(double));
   }
@@ -421,6 +424,7 @@ int sbslpm_ctx_create(const sbslpm_params* p, sbslpm_ctx** out) {
   d.proxy_leaf = (const int*)(b + o_pl); d.proxy_xieta = (const double*)(b + o_pxe);
   d.proxy_order = (const int*)(b + o_po);
   d.logtab = (const LogTabEntry*)(b + o_ltab);
+  d.logwide = (const LogTabEntry*)(b + o_lwide);
   d.exptab = (const double*)(b + o_etab);
   d.expnegtab = (const double*)(b + o_entab);
   d.xcd_start = (const int*)(b + o_xcd);
@@ -934,7 +938,7 @@ int sbslpm_direct_sum_inv_lap(sbslpm_ctx* c, int64_t n, const double* x, const d
   if (nt == 0) return SBSLPM_OK;
   int rc = ensure_scratch(c, direct_partials_size(nt, n, 1));
   if (rc) return rc;
-  launch_direct_inv_lap(nt, x + lb, y + lb, z + lb, n, x, y, z, area, pots, lb, false, c->dt.logtab, c->scratch,
+  launch_direct_inv_lap(nt, x + lb, y + lb, z + lb, n, x, y, z, area, pots, lb, false, c->dt.logwide, c->scratch,
                         soln + lb, c->stream);
   return launched(c);
 }
@@ -955,7 +959,7 @@ int sbslpm_direct_sum_inv_lap_noalloc(sbslpm_ctx* c, int64_t n, const double* x,
                     "; split [lb, ub) into smaller slices");
   double* buf = direct_noalloc_scratch(c->device);
   if (!buf) return fail(c, SBSLPM_E_HIP, "direct_sum_inv_lap_noalloc: fixed scratch not set up on this device");
-  launch_direct_inv_lap(nt, x + lb, y + lb, z + lb, n, x, y, z, area, pots, lb, false, c->dt.logtab, buf, soln + lb,
+  launch_direct_inv_lap(nt, x + lb, y + lb, z + lb, n, x, y, z, area, pots, lb, false, c->dt.logwide, buf, soln + lb,
                         c->stream);
   return launched(c);
 }
@@ -968,7 +972,7 @@ int sbslpm_direct_sum_inv_lap_targets(sbslpm_ctx* c, int64_t nt, const double* t
   if (nt == 0) return SBSLPM_OK;
   int rc = ensure_scratch(c, direct_partials_size(nt, ns, 1));
   if (rc) return rc;
-  launch_direct_inv_lap(nt, tx, ty, tz, ns, sx, sy, sz, area, pots, 0, true, c->dt.logtab, c->scratch, soln,
+  launch_direct_inv_lap(nt, tx, ty, tz, ns, sx, sy, sz, area, pots, 0, true, c->dt.logwide, c->scratch, soln,
                         c->stream);
   return launched(c);
 }

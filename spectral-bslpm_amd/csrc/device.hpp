@@ -38,7 +38,8 @@ struct DevTree {
   const int* proxy_leaf;      // [offset*n]
   const double* proxy_xieta;  // [offset*n][2]
   const int* proxy_order;     // [offset*n] proxy nodes sorted by leaf
-  const LogTabEntry* logtab;  // [kLogTabSize] table of log_tab (fasttab.hpp)
+  const LogTabEntry* logtab;   // [kLogTabSize] table of log_tab (fasttab.hpp)
+  const LogTabEntry* logwide;  // [kLogWideSize] table of log_wide
   const double* exptab;       // [kExpTabSize] table of exp_tab
   const double* expnegtab;    // [kExpNegTabSize] table of exp_neg
   const int* xcd_start;       // [2][9] cost-balanced XCD ranges of the target-major tile list (or null)
@@ -233,6 +234,12 @@ __device__ inline double in_vgpr(double v) {
 __device__ inline float in_vgpr_f(float v) {
   __asm__ volatile("" : "+v"(v));
   return v;
+}
+
+// Keeps uniform loads where they stand: without a use before a branch the
+// compiler moves them behind it, where their latency is waited for again.
+__device__ inline void loaded(double a, double b, double c, double d) {
+  __asm__ volatile("" ::"s"(a), "s"(b), "s"(c), "s"(d));
 }
 
 // interp_funcs_impl.hpp:114-142: leaf containing (x,y,z) or -1; xe gets the
@@ -637,7 +644,7 @@ double* direct_noalloc_scratch(int device);
 void launch_direct_inv_lap(int64_t nt, const double* tx, const double* ty, const double* tz, int64_t ns,
                            const double* sx, const double* sy, const double* sz, const double* area,
                            const double* pots, int64_t self_offset, bool guard_coincident,
-                           const LogTabEntry* logtab, double* partials, double* soln, hipStream_t s);
+                           const LogTabEntry* logwide, double* partials, double* soln, hipStream_t s);
 void launch_direct_bve_vel(int64_t nt, const double* tx, const double* ty, const double* tz, int64_t ns,
                            const double* sx, const double* sy, const double* sz, const double* area,
                            const double* vor, const double* const* disp, double eps, double* partials,

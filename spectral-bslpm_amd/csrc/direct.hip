@@ -2,9 +2,9 @@
 // and the Biot-Savart direct sum the reference lacks (same pair kernel as
 // bve_vel_impl.hpp:54-66).
 //
-// A workgroup of four waves owns 64 NT targets (NT per lane) and one source
-// chunk per grid row; each wave takes a quarter of the chunk, sources are
-// wave-uniform loads taken four at a time, and the four waves' sums are added
+// A workgroup of eight waves owns 64 NT targets (NT per lane) and one source
+// chunk per grid row; each wave takes an eighth of the chunk, sources are
+// wave-uniform loads taken four at a time, and the waves' sums are added
 // in wave order through LDS.  Each (target tile, chunk) writes a partial sum
 // and a second kernel adds the chunks in a fixed order, so the result is
 // deterministic and needs no atomics (the reference does one atomic per pair).
@@ -16,7 +16,7 @@
 namespace sbslpm {
 namespace {
 
-constexpr int kWaves = 4;
+constexpr int kWaves = 8;
 
 struct Plan {
   int64_t tiles, chunks, chunk_len;
@@ -42,7 +42,7 @@ Plan plan(int64_t nt, int64_t ns) {
   return p;
 }
 
-// This wave's part [a, b) of the workgroup's source chunk: quarters rounded up
+// This wave's part [a, b) of the workgroup's source chunk: eighths rounded up
 // to whole batches of four.
 __device__ inline void wave_sources(int64_t ns, int64_t chunk_len, int wave, int64_t& a, int64_t& b) {
   const int64_t j0 = (int64_t)blockIdx.y * chunk_len, j1 = std::min<int64_t>(ns, j0 + chunk_len);
@@ -68,28 +68,28 @@ __device__ inline void wave_sum(double (&v)[K], int wave, int lane) {
 
 // guard 0: skip j == self_offset + i (the reference's i != j);
 // guard 1: skip x.y >= 1 - 1e-15 (the FMM kernel's coincidence guard).
-// The logarithm is log_tab (fasttab.hpp, within 1.14 ulp) where 1 - x.y is a
-// normal number below 4; a batch of sources that holds the targets themselves,
-// a coincident or (guard 1) a skipped pair, or an argument outside that range
-// takes the library's logarithm with the guards, in the whole wave (one
-// unsigned maximum per pair and a ballot per batch).
-// Bound: FP64 vector issue, 27 instructions per pair (the library logarithm
-// on every pair took about 90).  24,576 x 24,576 points: 2.13 -> 0.57 ms.
+// The logarithm is log_wide (fasttab.hpp) where 1 - x.y is in its range; a batch
+// of sources that holds the targets themselves or a pair outside (closer than
+// 4e-5 rad, or skipped) takes the guarded form, with the library's logarithm for
+// the close ones (one unsigned maximum per pair and a ballot per batch).
+// Bound: FP64 vector issue, 20 instructions per pair (about 90 with the library's
+// logarithm on every pair).  24,576 x 24,576 points: 2.13 -> 0.44 ms
+// (0.57 with log_tab), vector issue busy 70% of the time.
 template <int NT>
-__global__ __launch_bounds__(256) void k_direct_log(int64_t nt, const double* __restrict__ tx,
+__global__ __launch_bounds__(64 * kWaves) void k_direct_log(int64_t nt, const double* __restrict__ tx,
                                                     const double* __restrict__ ty, const double* __restrict__ tz,
                                                     int64_t ns, const double* __restrict__ sx,
                                                     const double* __restrict__ sy, const double* __restrict__ sz,
                                                     const double* __restrict__ area, const double* __restrict__ pots,
                                                     int64_t self_offset, int guard, int64_t chunk_len,
-                                                    const LogTabEntry* __restrict__ logtab,
+                                                    const LogTabEntry* __restrict__ logwide,
                                                     double* __restrict__ partials) {
   // x.y rounded exactly as written in direct_sum_impl.hpp:23 (no fused
   // multiply-add): for nearly coincident points log(1 - x.y) amplifies a
   // one-ulp change of x.y by 1/(1 - x.y).
 #pragma clang fp contract(off)
-  __shared__ LogTabEntry ltab[kLogTabSize];
-  for (int i = threadIdx.x; i < kLogTabSize; i += blockDim.x) ltab[i] = logtab[i];
+  __shared__ LogTabEntry wide[kLogWideSize];
+  for (int i = threadIdx.x; i < kLogWideSize; i += blockDim.x) wide[i] = logwide[i];
   __syncthreads();
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int lane = threadIdx.x & 63;
@@ -104,33 +104,38 @@ __global__ __launch_bounds__(256) void k_direct_log(int64_t nt, const double* __
   int64_t a, b;
   wave_sources(ns, chunk_len, wave, a, b);
   const int64_t self_lo = self_offset + i0, self_hi = self_lo + 64 * NT;
-  // high words of the fast form's range: [2^-48, 4) or (1e-300, 4)
-  const uint32_t lo = guard ? 0x3cf00000u : 0x01a56e20u;
-  const uint32_t span = 0x40100000u - lo;
-  const double c6 = in_vgpr(-1.0 / 6.0);
+  const double c7 = in_vgpr(1.0 / 7.0);
   auto guarded = [&](int t, int64_t j) {
     const int64_t i = std::min<int64_t>(i0 + t * 64 + lane, nt - 1);
-    const double dp = x[t] * sx[j] + y[t] * sy[j] + z[t] * sz[j];
-    const double l = log(fmax(1.0 - dp, 1e-300)) * (area[j] * pots[j]);
-    const bool skip = guard ? !(dp < 1.0 - 1e-15) : (j == self_offset + i);
-    acc[t] += skip ? 0.0 : l;
+    const double d = 1.0 - (x[t] * sx[j] + y[t] * sy[j] + z[t] * sz[j]);
+    const bool skip = guard ? !(d > 1.0 - (1.0 - 1e-15)) : (j == self_offset + i);
+    const double v = skip ? 1.0 : d;
+    const uint32_t h = log_wide_cell(v);
+    const bool close = h >= kLogWideSpan;
+    double l = log_wide(v, close ? 0u : h, wide, c7);
+    if (__builtin_amdgcn_ballot_w64(close) != 0) l = close ? log(fmax(v, 1e-300)) : l;
+    const double q = area[j] * pots[j];
+    acc[t] = skip ? acc[t] : fma(l, q, acc[t]);
   };
   int64_t j = a;
   for (; j + 4 <= b; j += 4) {
     double d[NT][4];
-    uint32_t far = 0;
+    uint32_t h[NT][4], far = 0;
 #pragma unroll
     for (int k = 0; k < 4; ++k) {
       const double s0 = sx[j + k], s1 = sy[j + k], s2 = sz[j + k];
 #pragma unroll
       for (int t = 0; t < NT; ++t) {
         d[t][k] = 1.0 - (x[t] * s0 + y[t] * s1 + z[t] * s2);
-        const uint32_t h = (uint32_t)__double2hiint(d[t][k]) - lo;
-        far = h > far ? h : far;
+        h[t][k] = log_wide_cell(d[t][k]);
+        far = h[t][k] > far ? h[t][k] : far;
       }
     }
+    loaded(area[j], area[j + 1], area[j + 2], area[j + 3]);
+    loaded(pots[j], pots[j + 1], pots[j + 2], pots[j + 3]);
     const bool own = !guard && j < self_hi && j + 4 > self_lo;
-    if (own || __builtin_amdgcn_ballot_w64(far >= span) != 0) {
+    if (own || __builtin_amdgcn_ballot_w64(far >= kLogWideSpan) != 0) {
+#pragma unroll 1
       for (int k = 0; k < 4; ++k)
 #pragma unroll
         for (int t = 0; t < NT; ++t) guarded(t, j + k);
@@ -140,7 +145,7 @@ __global__ __launch_bounds__(256) void k_direct_log(int64_t nt, const double* __
     for (int k = 0; k < 4; ++k) {
       const double q = area[j + k] * pots[j + k];
 #pragma unroll
-      for (int t = 0; t < NT; ++t) acc[t] = fma(log_tab(d[t][k], ltab, c6), q, acc[t]);
+      for (int t = 0; t < NT; ++t) acc[t] = fma(log_wide(d[t][k], h[t][k], wide, c7), q, acc[t]);
     }
   }
   for (; j < b; ++j)
@@ -156,11 +161,11 @@ __global__ __launch_bounds__(256) void k_direct_log(int64_t nt, const double* __
 // Bound: FP64 vector issue.  The four denominators of a batch share one
 // reciprocal (rcp4: 12.5 instruction slots per pair with the loads' share
 // against 17 with a reciprocal each), and 1 - x.y is one chain of fused
-// multiply-adds from 1.  4,096 targets x 393,216 sources: 4.09 -> 0.78 ms (one
+// multiply-adds from 1.  4,096 targets x 393,216 sources: 4.09 -> 0.77 ms (one
 // target per lane and one source per step waited on each source's scalar loads;
 // now vector issue is busy 83% of the time, at 2.1 GHz under this load).
 template <int NT>
-__global__ __launch_bounds__(256) void k_direct_bs(int64_t nt, const double* __restrict__ tx,
+__global__ __launch_bounds__(64 * kWaves) void k_direct_bs(int64_t nt, const double* __restrict__ tx,
                                                    const double* __restrict__ ty, const double* __restrict__ tz,
                                                    int64_t ns, const double* __restrict__ sx,
                                                    const double* __restrict__ sy, const double* __restrict__ sz,
@@ -233,7 +238,7 @@ struct Ptr3 {
 // adds chunks w, w + 4, ..., the waves' sums are added in wave order.  (With one
 // thread per target walking every chunk of three components, the 64 chunks of
 // 4,096 targets took 52 us, a chain of loads in 64 waves; now 4.9 us.)
-__global__ __launch_bounds__(256) void k_reduce(int64_t nt, int ncomp, int64_t chunks,
+__global__ __launch_bounds__(64 * kWaves) void k_reduce(int64_t nt, int ncomp, int64_t chunks,
                                                 const double* __restrict__ partials, Ptr3 out) {
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int lane = threadIdx.x & 63;
@@ -298,13 +303,13 @@ int64_t direct_partials_size(int64_t nt, int64_t ns, int ncomp) {
 void launch_direct_inv_lap(int64_t nt, const double* tx, const double* ty, const double* tz, int64_t ns,
                            const double* sx, const double* sy, const double* sz, const double* area,
                            const double* pots, int64_t self_offset, bool guard_coincident,
-                           const LogTabEntry* logtab, double* partials, double* soln, hipStream_t s) {
+                           const LogTabEntry* logwide, double* partials, double* soln, hipStream_t s) {
   if (nt <= 0) return;
   const Plan p = plan(nt, ns);
   const dim3 grid((unsigned)p.tiles, (unsigned)p.chunks);
   auto kernel = p.nt_lane == 2 ? k_direct_log<2> : k_direct_log<1>;
   hipLaunchKernelGGL(kernel, grid, dim3(64 * kWaves), 0, s, nt, tx, ty, tz, ns, sx, sy, sz, area, pots, self_offset,
-                     guard_coincident ? 1 : 0, p.chunk_len, logtab, partials);
+                     guard_coincident ? 1 : 0, p.chunk_len, logwide, partials);
   Ptr3 out{{soln, nullptr, nullptr}};
   hipLaunchKernelGGL(k_reduce, dim3((unsigned)((nt + 63) / 64), 1), dim3(64 * kWaves), 0, s, nt, 1, p.chunks,
                      (const double*)partials, out);

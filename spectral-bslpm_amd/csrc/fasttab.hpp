@@ -16,6 +16,15 @@
 // k ln2 split as k ln2_hi (exact) + k ln2_lo, and k converted to a double by
 // placing it in the low bits of 2^52 (one subtraction).
 //
+// Logarithm over [2^-30, 2 + 2^-5) (log_wide): 64 cells per binade picked by the
+// exponent and six mantissa bits together, so one subtraction and a shift of
+// the high word index the table and no exponent term is left:
+//   r = x c_inv - 1 (one fma, |r| < 2^-7),  log x = logc + r (1 + r p(r)),
+// p the degree-5 Taylor polynomial (first omitted term r^8/8 < 2^-59), 11
+// vector instructions against log_tab's 17.  c_inv and logc as above, without
+// the special cells at 1: the error there is below 2^-59, which is small against
+// any sum of logarithms but not in relative terms.
+//
 // Exponential (general, exp_tab): n = rint(t 128/ln2), t = n ln2/128 + r with
 // |r| <= ln2/256 (Cody-Waite split of ln2/128),
 // exp t = 2^(n>>7) 2^((n&127)/128) (1 + p(r)), p(r) = r + r^2 (1/2 + r/6 +
@@ -45,6 +54,9 @@
 namespace sbslpm {
 
 constexpr int kLogTabSize = 1024;
+constexpr uint32_t kLogWideLo = 0x3e100000u;     // high word of 2^-30
+constexpr int kLogWideSize = 31 * 64 + 1;        // 31 binades and the first cell of [2, 4)
+constexpr uint32_t kLogWideSpan = (uint32_t)kLogWideSize << 14;  // range of (high word - kLogWideLo)
 constexpr int kExpTabSize = 128;
 constexpr int kExpNegTabSize = 3840;  // 2^(n/256), n = -3839..0
 constexpr double kExpNegMin = -10.375;  // exp_neg clamps its argument here (n >= -3832)
@@ -97,6 +109,21 @@ SBSLPM_HD inline double log_tab(double x, const LogTabEntry* __restrict__ tab, d
   return fma(kd, kTabLn2Hi, e.logc) + fma(kd, kTabLn2Lo, y);
 }
 
+// log x for 2^-30 <= x < 2 + 2^-5; h is x's high word minus kLogWideLo (below
+// kLogWideSpan), c7 is 1/7 (from a vector register, as c6 above).
+SBSLPM_HD inline double log_wide(double x, uint32_t h, const LogTabEntry* __restrict__ tab, double c7) {
+  const LogTabEntry e = tab[h >> 14];
+  const double r = fma(x, e.inv_c, -1.0);
+  double p = fma(r, c7, -1.0 / 6.0);
+  p = fma(p, r, 1.0 / 5.0);
+  p = fma(p, r, -1.0 / 4.0);
+  p = fma(p, r, 1.0 / 3.0);
+  p = fma(p, r, -1.0 / 2.0);
+  p = fma(p, r, 1.0);
+  return fma(p, r, e.logc);
+}
+SBSLPM_HD inline uint32_t log_wide_cell(double x) { return (uint32_t)(double_to_bits(x) >> 32) - kLogWideLo; }
+
 // exp t for |t| < 700.
 SBSLPM_HD inline double exp_tab(double t, const double* __restrict__ tab) {
   const double n = rint(t * kExpInvL);
@@ -129,34 +156,40 @@ SBSLPM_HD inline double exp_neg(double t, const double* __restrict__ tab, double
 }
 
 // Host: the tables.
+
+// A cell's entry: c_inv near 1/centre with -log(c_inv) close to a double.
+inline LogTabEntry log_cell(long double centre) {
+  const double base = (double)(1.0L / centre);
+  double best = base, best_err = 1e300;
+  uint64_t bb = double_to_bits(base);
+  for (int j = 0; j < 4096; ++j) {
+    const int64_t off = (j & 1) ? -(int64_t)((j + 1) / 2) : (int64_t)(j / 2);
+    const double c = bits_to_double(bb + (uint64_t)off);
+    const long double L = -logl((long double)c);
+    const double d = (double)L;
+    const long double ulp = (long double)(std::nextafter(std::fabs(d), INFINITY) - std::fabs(d));
+    const long double err = fabsl(L - (long double)d) / ulp;
+    if (err < best_err) {
+      best_err = (double)err;
+      best = c;
+    }
+    if (err < 1.0L / 64) break;
+  }
+  return LogTabEntry{best, (double)(-logl((long double)best))};
+}
+
 inline void build_log_table(LogTabEntry* tab) {
   constexpr int half = kLogTabSize / 2;
   for (int i = 0; i < kLogTabSize; ++i) {
     // the cell's range of m: exponent 0x3fe (i < half, m in [0.5, 1)) or 0x3ff
     const long double w = i < half ? 0.5L / half : 1.0L / half;
     const long double lo = i < half ? 0.5L + (i % half) * w : 1.0L + (i % half) * w;
-    if (i == half - 1 || i == half) {
-      tab[i] = LogTabEntry{1.0, 0.0};
-      continue;
-    }
-    const double base = (double)(1.0L / (lo + 0.5L * w));
-    double best = base, best_err = 1e300;
-    uint64_t bb = double_to_bits(base);
-    for (int j = 0; j < 4096; ++j) {
-      const int64_t off = (j & 1) ? -(int64_t)((j + 1) / 2) : (int64_t)(j / 2);
-      const double c = bits_to_double(bb + (uint64_t)off);
-      const long double L = -logl((long double)c);
-      const double d = (double)L;
-      const long double ulp = (long double)(std::nextafter(std::fabs(d), INFINITY) - std::fabs(d));
-      const long double err = fabsl(L - (long double)d) / ulp;
-      if (err < best_err) {
-        best_err = (double)err;
-        best = c;
-      }
-      if (err < 1.0L / 64) break;
-    }
-    tab[i] = LogTabEntry{best, (double)(-logl((long double)best))};
+    tab[i] = i == half - 1 || i == half ? LogTabEntry{1.0, 0.0} : log_cell(lo + 0.5L * w);
   }
+}
+
+inline void build_log_wide_table(LogTabEntry* tab) {
+  for (int i = 0; i < kLogWideSize; ++i) tab[i] = log_cell(ldexpl(1.0L + (i % 64 + 0.5L) / 64, i / 64 - 30));
 }
 
 inline void build_exp_table(double* tab) {

@@ -177,58 +177,98 @@ __global__ __launch_bounds__(64 * S) void k_bve64(DevTree t, const TargetTile* _
 }
 
 // FP64 log pair kernel: psi += -1/(4 pi) log(1 - x.y) q, pairs with
-// x.y >= 1 - 1e-15 skipped (inverse_poisson_impl.hpp:46-49).  The logarithm
-// is log_tab (fasttab.hpp, within 1.1 ulp of the correctly rounded one) on
-// the context's table, staged in LDS.  A skipped pair (a source that coincides
-// with a target: the target's own node, or a node on a shared leaf edge) is
-// rare, so the wave tests the whole source at once (a ballot, one compare per
-// pair) and only a wave holding such a pair takes the guarded form.
-__global__ __launch_bounds__(256) void k_log64(DevTree t, const TargetTile* __restrict__ tiles, int ntiles,
-                                               const SourceSet* __restrict__ sets,
-                                               const SrcRec64* __restrict__ rec, double* __restrict__ part,
-                                               double* __restrict__ proxy, int assign) {
-  __shared__ LogTabEntry ltab[kLogTabSize];
-  for (int i = threadIdx.x; i < kLogTabSize; i += blockDim.x) ltab[i] = t.logtab[i];
+// x.y >= 1 - 1e-15 skipped (inverse_poisson_impl.hpp:46-49).  S waves share a
+// tile (pairwalk.hpp); the logarithm is log_wide (fasttab.hpp) on the context's
+// table, staged in LDS.  A pair outside its range (a source that coincides with
+// a target: the target's own node, or a node on a shared leaf edge; or one
+// closer than 4e-5 rad) is rare, so the wave tests four sources at once (one
+// ballot) and only a batch holding such a pair takes the guarded form, with
+// log_tab for the close ones.
+// Bound: FP64 vector issue, 16 instructions per pair (23 with log_tab and a
+// compare on every pair), at the 1.9 GHz the chip holds under this load: issue is
+// busy 88% of the time, the gathers from the table (9 LDS cycles each, bank
+// conflicts included) half of it.  Microseconds per launch with log_tab, one
+// wave per tile, and now: 6 x 28^2 281 -> 25, 6 x 64^2 494 -> 97, degree 10 at
+// 6 x 256^2 (theta 0.7) 1751 -> 1033, 6 x 512^2 4890 -> 3632.
+constexpr double kSkipOneMinusDot = 1.0 - (1.0 - 1e-15);
+
+// The logarithms of N values any of which may be outside log_wide's range; zero
+// at a skipped pair.
+template <int N>
+__device__ inline void log_guarded(double (&d)[N], double (&l)[N], const LogTabEntry* __restrict__ wide,
+                                   const LogTabEntry* __restrict__ tab, double c7) {
+  bool skip[N];
+  uint32_t h[N], far = 0;
+#pragma unroll
+  for (int i = 0; i < N; ++i) {
+    skip[i] = d[i] <= kSkipOneMinusDot;
+    d[i] = skip[i] ? 1.0 : d[i];
+    h[i] = log_wide_cell(d[i]);
+    far = h[i] > far ? h[i] : far;
+  }
+  if (__builtin_amdgcn_ballot_w64(far >= kLogWideSpan) != 0) {
+#pragma unroll 1
+    for (int i = 0; i < N; ++i) l[i] = log_tab(d[i], tab);
+  } else {
+#pragma unroll
+    for (int i = 0; i < N; ++i) l[i] = log_wide(d[i], h[i], wide, c7);
+  }
+#pragma unroll
+  for (int i = 0; i < N; ++i) l[i] = skip[i] ? 0.0 : l[i];
+}
+
+// Waves per tile of the log kernel, whose table (32 KB of LDS) holds a compute
+// unit to four workgroups: at 126 tiles 62 / 38 / 27 us with 4 / 8 / 16 waves, at
+// 636 122 / 105 / 112, at 2,556 316 / 280 / 346, at 40,956 4160 / 3843 / 5155.
+inline int log_waves(int ntiles) { return ntiles < 400 ? 16 : 8; }
+
+template <int S>
+__global__ __launch_bounds__(64 * S) void k_log64(DevTree t, const TargetTile* __restrict__ tiles, int ntiles,
+                                                  const SourceSet* __restrict__ sets,
+                                                  const SrcRec64* __restrict__ rec, double* __restrict__ part,
+                                                  double* __restrict__ proxy, int assign) {
+  __shared__ LogTabEntry wide[kLogWideSize];
+  for (int i = threadIdx.x; i < kLogWideSize; i += 64 * S) wide[i] = t.logwide[i];
   __syncthreads();
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int lane = threadIdx.x & 63;
-  const int tile = xcd_remap(blockIdx.x, gridDim.x) * kWavesPerBlock + wave;
-  if (tile >= ntiles) return;
-  const TargetTile T = tiles[tile];
+  const TargetTile T = tiles[xcd_remap(blockIdx.x, ntiles)];
   const int64_t u = (int64_t)T.first + (lane < T.count ? lane : T.count - 1);
   const double x = t.px[u], y = t.py[u], z = t.pz[u];
-  constexpr double kSkip = 1.0 - 1e-15;
-  const double c6 = in_vgpr(-1.0 / 6.0);
-  double acc = 0;
-  for (int e = T.src_begin; e < T.src_end; ++e) {
-    const SourceSet S = sets[e];
-    const SrcRec64* __restrict__ r = rec + S.first;
-    int k = 0;
-    for (; k + 1 < S.count; k += 2) {
-      const SrcRec64 s0 = r[k], s1 = r[k + 1];
-      const double dp0 = x * s0.x + y * s0.y + z * s0.z;
-      const double dp1 = x * s1.x + y * s1.y + z * s1.z;
-      double l0 = log_tab(1.0 - dp0, ltab, c6), l1 = log_tab(1.0 - dp1, ltab, c6);
-      const bool sk0 = dp0 >= kSkip, sk1 = dp1 >= kSkip;
-      if ((__builtin_amdgcn_ballot_w64(sk0) | __builtin_amdgcn_ballot_w64(sk1)) != 0) {
-        // a real branch (the empty asm keeps the compiler from turning it into
-        // selects on every pair); log_tab's index is masked, so the discarded
-        // values were read in bounds
-        __asm__ volatile("");
-        l0 = sk0 ? 0.0 : l0;
-        l1 = sk1 ? 0.0 : l1;
+  const double c7 = in_vgpr(1.0 / 7.0);
+  double acc[1] = {0};
+  walk_sets<S>(T, sets, wave, [&](const SourceSet& set, int a, int b) {
+    const SrcRec64* __restrict__ r = rec + set.first;
+    int k = a;
+    for (; k + 4 <= b; k += 4) {
+      double d[4];
+      uint32_t h[4], far = 0;
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        d[i] = one_minus_dot(x, y, z, r[k + i].x, r[k + i].y, r[k + i].z);
+        h[i] = log_wide_cell(d[i]);
+        far = h[i] > far ? h[i] : far;
       }
-      acc = fma(l0, s0.q, acc);
-      acc = fma(l1, s1.q, acc);
+      loaded(r[k].q, r[k + 1].q, r[k + 2].q, r[k + 3].q);
+      double l[4];
+      if (__builtin_amdgcn_ballot_w64(far >= kLogWideSpan) != 0) {
+        log_guarded(d, l, wide, t.logtab, c7);
+      } else {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) l[i] = log_wide(d[i], h[i], wide, c7);
+      }
+#pragma unroll
+      for (int i = 0; i < 4; ++i) acc[0] = fma(l[i], r[k + i].q, acc[0]);
     }
-    if (k < S.count) {
-      const SrcRec64 s0 = r[k];
-      const double dp0 = x * s0.x + y * s0.y + z * s0.z;
-      const double l0 = log_tab(1.0 - dp0, ltab, c6);
-      acc = fma(dp0 >= kSkip ? 0.0 : l0, s0.q, acc);
+    for (; k < b; ++k) {
+      const SrcRec64 s = r[k];
+      double d[1] = {one_minus_dot(x, y, z, s.x, s.y, s.z)}, l[1];
+      log_guarded(d, l, wide, t.logtab, c7);
+      acc[0] = fma(l[0], s.q, acc[0]);
     }
-  }
-  if (lane < T.count) store_s(t, u, part, proxy, acc, assign);
+  });
+  tile_sum<S>(acc, wave, lane);
+  if (wave == 0 && lane < T.count) store_s(t, u, part, proxy, acc[0], assign);
 }
 
 // Horner multipliers of the FP64 regularised-Laplacian kernel in vector registers.
@@ -1045,8 +1085,10 @@ void launch_poisson_interact64(const DevTree& t, const TargetTile* tiles, int nt
                                const SrcRec64* rec, double* out_part, double* out_proxy, hipStream_t s,
                                bool assign) {
   if (ntiles == 0) return;
-  hipLaunchKernelGGL(k_log64, dim3(blocks_for(ntiles, kWavesPerBlock)), dim3(64 * kWavesPerBlock), 0, s, t, tiles,
-                     ntiles, sets, rec, out_part, out_proxy, assign ? 1 : 0);
+  const int S = log_waves(ntiles);
+  auto kernel = S == 16 ? k_log64<16> : k_log64<8>;
+  hipLaunchKernelGGL(kernel, dim3(ntiles), dim3(64 * S), 0, s, t, tiles, ntiles, sets, rec, out_part, out_proxy,
+                     assign ? 1 : 0);
 }
 
 void launch_laplacian_interact64(const DevTree& t, const TargetTile* tiles, int ntiles, const SourceSet* sets,

@@ -58,3 +58,14 @@ def test_vortex_pairs(case, displaced):
     gp, gx = ctx.bve_vel_interactions(*up(case, [case["qp"], case["qx"]]), up(case, dp) if dp else None,
                                       up(case, dx) if dx else None, phi_part=phi_part, phi_proxy=phi_proxy)
     close(case, gp, gx, ep, ex, 0.5)
+
+
+def test_log_pairs(case):
+    """Coincident nodes (a tile's own leaf, shared leaf edges) are skipped on both sides."""
+    ctx, o = case["ctx"], case["o"]
+    ep, ex = o.poisson_fmm_interactions(case["qp"], case["qx"])
+    psi_part, psi_proxy = ctx.zeros_part(), ctx.zeros_proxy()
+    for v in (psi_part, psi_proxy):
+        v.fill_(0.5)
+    gp, gx = ctx.poisson_fmm_interactions(*up(case, [case["qp"], case["qx"]]), psi_part, psi_proxy)
+    close(case, [gp], [gx], [ep], [ex], 0.5)
