@@ -421,7 +421,7 @@ void launch_source_records_swe(const DevTree& t, int variant, const double* qz_p
                                const double* const* disp_proxy, SrcRecSwe* rec, hipStream_t s);
 void launch_swe_interact64(const DevTree& t, int variant, const TargetTile* tiles, int ntiles, const SourceSet* sets,
                            const SrcRecSwe* rec, double eps, double* const* out_part, double* const* out_proxy,
-                           hipStream_t s, bool assign = false, bool shared_tiles = false);
+                           hipStream_t s, bool assign = false, bool heaviest_first = false);
 
 // ---- adjoints (adjoint.hip: FMM transpose; remap_adjoint.hip: remap side)
 size_t adj_target_record_bytes();

@@ -232,7 +232,9 @@ __global__ __launch_bounds__(64 * S) void k_log64(DevTree t, const TargetTile* _
   __syncthreads();
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int lane = threadIdx.x & 63;
-  const TargetTile T = tiles[xcd_remap(blockIdx.x, ntiles)];
+  const int tile = strip_tile(ntiles);
+  if (tile >= ntiles) return;  // the whole workgroup
+  const TargetTile T = tiles[tile];
   const int64_t u = (int64_t)T.first + (lane < T.count ? lane : T.count - 1);
   const double x = t.px[u], y = t.py[u], z = t.pz[u];
   const double c7 = in_vgpr(1.0 / 7.0);
@@ -299,54 +301,63 @@ __device__ inline double lap_pair_slow(double dp, const LapCoef64& kp, const Lap
 // form of lapkernel.hpp (A + E B where t >= 6 eps, erf only below).  Sources
 // are displaced and projected; the records hold q' = -q/(4 pi), so the
 // coefficients arrive multiplied by -4 pi / eps^{5/2}.  Over 99% of the pair
-// work has t > 0.6, so a wave tests the whole source at once (a ballot) and
+// work has t > 0.6, so a wave tests four sources at once (a ballot) and
 // evaluates erf only when one of its pairs needs it.  The exponential is
 // exp_neg (fasttab.hpp: its argument lies in [-1/eps, 0]) on the context's
-// table, staged in LDS.
-__global__ __launch_bounds__(256) void k_lap64(DevTree t, const TargetTile* __restrict__ tiles, int ntiles,
-                                               const SourceSet* __restrict__ sets,
-                                               const SrcRec64* __restrict__ rec, LapCoef64 kp,
-                                               double* __restrict__ part, double* __restrict__ proxy, int assign) {
+// table, staged in LDS.  S waves share a tile (pairwalk.hpp).
+// Bound: FP64 vector issue, 22 instructions per pair.  Microseconds per launch
+// with one wave per tile (two sub-tiles of 18 rows in lane groups at m = 6) and
+// now: 6 x 28^2 321 -> 98, 6 x 64^2 612 -> 223, 6 x 192^2 (degree 8) 1176 -> 1028,
+// degree 10 at 6 x 256^2 2366 -> 1673.
+template <int S>
+__global__ __launch_bounds__(64 * S) void k_lap64(DevTree t, const TargetTile* __restrict__ tiles, int ntiles,
+                                                  const SourceSet* __restrict__ sets,
+                                                  const SrcRec64* __restrict__ rec, LapCoef64 kp,
+                                                  double* __restrict__ part, double* __restrict__ proxy, int assign) {
   __shared__ double etab[kExpNegTabSize];
-  for (int i = threadIdx.x; i < kExpNegTabSize; i += blockDim.x) etab[i] = t.expnegtab[i];
+  for (int i = threadIdx.x; i < kExpNegTabSize; i += 64 * S) etab[i] = t.expnegtab[i];
   __syncthreads();
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int lane = threadIdx.x & 63;
-  const int tile = xcd_remap(blockIdx.x, gridDim.x) * kWavesPerBlock + wave;
-  if (tile >= ntiles) return;
+  const int tile = strip_tile(ntiles);
+  if (tile >= ntiles) return;  // the whole workgroup
   const TargetTile T = tiles[tile];
   const int64_t u = (int64_t)T.first + (lane < T.count ? lane : T.count - 1);
   const double x = t.px[u], y = t.py[u], z = t.pz[u];
-  // every pair passes the cut when 1 - 30 eps < -1 (eps = 0.1)
-  const bool no_cut = kp.cut < -1.0;
+  // every pair passes the cut when 1 - 30 eps < -1 (eps = 0.1); else every pair takes the slow form
+  const double fast_from = kp.cut < -1.0 ? kp.t_sat : 4.0;
   const LapV64 kv{in_vgpr(kp.a1), in_vgpr(kp.b2), in_vgpr(1.0 / 24.0)};
-  double acc = 0;
-  for (int e = T.src_begin; e < T.src_end; ++e) {
-    const SourceSet S = sets[e];
-    const SrcRec64* __restrict__ r = rec + S.first;
-    int k = 0;
-    for (; k + 1 < S.count; k += 2) {
-      const SrcRec64 s0 = r[k], s1 = r[k + 1];
-      const double dp0 = x * s0.x + y * s0.y + z * s0.z;
-      const double dp1 = x * s1.x + y * s1.y + z * s1.z;
-      double K0 = lap_pair(dp0, kp, kv, etab), K1 = lap_pair(dp1, kp, kv, etab);
-      if (!no_cut || (__builtin_amdgcn_ballot_w64(dp0 < kp.t_sat) | __builtin_amdgcn_ballot_w64(dp1 < kp.t_sat)) != 0) {
-        // a real branch (the empty asm keeps the compiler from evaluating erf
-        // on every pair)
-        __asm__ volatile("");
-        K0 = lap_pair_slow(dp0, kp, kv, etab);
-        K1 = lap_pair_slow(dp1, kp, kv, etab);
+  double acc[1] = {0};
+  walk_sets<S>(T, sets, wave, [&](const SourceSet& set, int a, int b) {
+    const SrcRec64* __restrict__ r = rec + set.first;
+    int k = a;
+    for (; k + 4 <= b; k += 4) {
+      double dp[4], K[4];
+#pragma unroll
+      for (int i = 0; i < 4; ++i) dp[i] = x * r[k + i].x + y * r[k + i].y + z * r[k + i].z;
+      loaded(r[k].q, r[k + 1].q, r[k + 2].q, r[k + 3].q);
+      if (__builtin_amdgcn_ballot_w64(fmin(fmin(dp[0], dp[1]), fmin(dp[2], dp[3])) < fast_from) != 0) {
+#pragma unroll 1
+        for (int i = 0; i < 4; ++i) {
+          const SrcRec64 s = r[k + i];
+          acc[0] = fma(lap_pair_slow(x * s.x + y * s.y + z * s.z, kp, kv, etab), s.q, acc[0]);
+        }
+        continue;
       }
-      acc = fma(K0, s0.q, acc);
-      acc = fma(K1, s1.q, acc);
+#pragma unroll
+      for (int i = 0; i < 4; ++i) K[i] = lap_pair(dp[i], kp, kv, etab);
+#pragma unroll
+      for (int i = 0; i < 4; ++i) acc[0] = fma(K[i], r[k + i].q, acc[0]);
     }
-    if (k < S.count) {
-      const SrcRec64 s0 = r[k];
-      const double dp0 = x * s0.x + y * s0.y + z * s0.z;
-      acc = fma(lap_pair_slow(dp0, kp, kv, etab), s0.q, acc);
+    for (; k < b; ++k) {
+      const SrcRec64 s = r[k];
+      const double dp = x * s.x + y * s.y + z * s.z;
+      const bool slow = __builtin_amdgcn_ballot_w64(dp < fast_from) != 0;
+      acc[0] = fma(slow ? lap_pair_slow(dp, kp, kv, etab) : lap_pair(dp, kp, kv, etab), s.q, acc[0]);
     }
-  }
-  if (lane < T.count) store_s(t, u, part, proxy, acc, assign);
+  });
+  tile_sum<S>(acc, wave, lane);
+  if (wave == 0 && lane < T.count) store_s(t, u, part, proxy, acc[0], assign);
 }
 
 // Mixed-precision regularised-Laplacian pairs in the folded form of
@@ -425,55 +436,10 @@ __global__ __launch_bounds__(256) void k_lap_mixed(DevTree t, const TargetTile* 
   if (lane < T.count) store_s(t, u, part, proxy, acc, assign);
 }
 
-// k_lap64 and k_lap_mixed in lane groups (RowGroups): each 36-row tile at
-// m = 6 runs as two 18-row sub-tiles in three copies per wave, every copy
-// taking every third source of a set from records staged in LDS; one pair per
-// iteration behind the same wave-wide ballot for the erf form.
-__global__ __launch_bounds__(256) void k_lap64_gr(DevTree t, const TargetTile* __restrict__ tiles, int ntiles,
-                                                  RowGroups gs, const SourceSet* __restrict__ sets,
-                                                  const SrcRec64* __restrict__ rec, LapCoef64 kp,
-                                                  double* __restrict__ part, double* __restrict__ proxy, int assign) {
-  __shared__ double etab[kExpNegTabSize];
-  __shared__ SrcRec64 stage[kWavesPerBlock][64];
-  for (int i = threadIdx.x; i < kExpNegTabSize; i += blockDim.x) etab[i] = t.expnegtab[i];
-  __syncthreads();
-  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  int tile, row0, cg, ci;
-  if (!group_tile<true>(gs, ntiles, wave, 1, tile, row0, cg, ci)) return;
-  const TargetTile T = tiles[tile];
-  const int row = row0 + ci;
-  const int64_t u = (int64_t)T.first + (row < T.count ? row : T.count - 1);
-  const bool copy_ok = cg < gs.G;
-  const double x = t.px[u], y = t.py[u], z = t.pz[u];
-  const bool no_cut = kp.cut < -1.0;
-  const LapV64 kv{in_vgpr(kp.a1), in_vgpr(kp.b2), in_vgpr(1.0 / 24.0)};
-  double acc = 0;
-  for (int e = T.src_begin; e < T.src_end; ++e) {
-    const SourceSet S = sets[e];
-    const SrcRec64* __restrict__ r = rec + S.first;
-    for (int c0 = 0; c0 < S.count; c0 += 64) {
-      const int cn = min(64, S.count - c0);
-      stage_records(stage[wave], r + c0, cn);
-      const int trips = (cn + gs.G - 1) / gs.G;
-      for (int kk = 0; kk < trips; ++kk) {
-        const int k = kk * gs.G + cg;
-        if (!(copy_ok && k < cn)) continue;
-        const SrcRec64 s0 = stage[wave][k];
-        const double dp0 = x * s0.x + y * s0.y + z * s0.z;
-        double K0 = lap_pair(dp0, kp, kv, etab);
-        if (!no_cut || __builtin_amdgcn_ballot_w64(dp0 < kp.t_sat) != 0) {
-          // a real branch (the empty asm keeps the compiler from evaluating erf on every pair)
-          __asm__ volatile("");
-          K0 = lap_pair_slow(dp0, kp, kv, etab);
-        }
-        acc = fma(K0, s0.q, acc);
-      }
-    }
-  }
-  acc = group_sum(acc, gs, ci);
-  if (cg == 0 && row < T.count) store_s(t, u, part, proxy, acc, assign);
-}
-
+// k_lap_mixed in lane groups (RowGroups): each 36-row tile at m = 6 runs as two
+// 18-row sub-tiles in three copies per wave, every copy taking every third
+// source of a set from records staged in LDS; one pair per iteration behind the
+// same wave-wide ballot for the erf form.
 __global__ __launch_bounds__(256) void k_lap_mixed_gr(DevTree t, const TargetTile* __restrict__ tiles, int ntiles,
                                                       RowGroups gs, const SourceSet* __restrict__ sets,
                                                       const SrcRec32* __restrict__ rec, LapCoef32 kp, double c3,
@@ -1087,7 +1053,7 @@ void launch_poisson_interact64(const DevTree& t, const TargetTile* tiles, int nt
   if (ntiles == 0) return;
   const int S = log_waves(ntiles);
   auto kernel = S == 16 ? k_log64<16> : k_log64<8>;
-  hipLaunchKernelGGL(kernel, dim3(ntiles), dim3(64 * S), 0, s, t, tiles, ntiles, sets, rec, out_part, out_proxy,
+  hipLaunchKernelGGL(kernel, dim3(strip_grid(ntiles)), dim3(64 * S), 0, s, t, tiles, ntiles, sets, rec, out_part, out_proxy,
                      assign ? 1 : 0);
 }
 
@@ -1098,13 +1064,11 @@ void launch_laplacian_interact64(const DevTree& t, const TargetTile* tiles, int 
   const double eps = 0.1, pi = 3.14159265358979323846;
   // the records carry -q/(4 pi): undo it with the kernel's eps^{-5/2}
   const LapCoef64 kp = lap_coef64(eps, -4.0 * pi / std::pow(eps, 2.5));
-  const RowGroups gs = row_groups(t);
-  if (gs.G > 1)
-    hipLaunchKernelGGL(k_lap64_gr, dim3(blocks_for((int64_t)ntiles * gs.H, kWavesPerBlock)), dim3(64 * kWavesPerBlock),
-                       0, s, t, tiles, ntiles, gs, sets, rec, kp, out_part, out_proxy, assign ? 1 : 0);
-  else
-    hipLaunchKernelGGL(k_lap64, dim3(blocks_for(ntiles, kWavesPerBlock)), dim3(64 * kWavesPerBlock), 0, s, t, tiles,
-                       ntiles, sets, rec, kp, out_part, out_proxy, assign ? 1 : 0);
+  // us per launch with 4 / 8 / 16 waves: 126 tiles 181 / 116 / 98, 636 223 / 219 / 230, 10,236 1028 / 1088 / 1373
+  const int S = ntiles < 400 ? 16 : 4;
+  auto kernel = S == 16 ? k_lap64<16> : k_lap64<4>;
+  hipLaunchKernelGGL(kernel, dim3(strip_grid(ntiles)), dim3(64 * S), 0, s, t, tiles, ntiles, sets, rec, kp, out_part, out_proxy,
+                     assign ? 1 : 0);
 }
 
 void launch_laplacian_interact_mixed(const DevTree& t, const TargetTile* tiles, int ntiles, const SourceSet* sets,

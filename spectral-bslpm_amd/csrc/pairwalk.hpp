@@ -68,4 +68,23 @@ inline unsigned walk_grid(int ntiles, const PairShape& shape) {
   return (unsigned)(shape.xcd == 2 && shape.grid1 > 0 ? shape.grid1 : ntiles);
 }
 
+// Tile of this workgroup where XCD x (the hardware deals workgroup b to XCD b % 8)
+// takes strips x, x + 8, ... of neighbouring tiles: a strip's tiles share sources
+// in that XCD's L2, and 32 strips each even out the lists, whose coarse panels
+// come first and cost most.  (k_swe64 at 40,956 tiles, 64-byte records: 3.53 ms;
+// one contiguous range per XCD 3.84, workgroup b on tile b 4.21.  k_lap64, whose
+// coarse tiles evaluate erf: 1.03 ms at 10,236 tiles, one range per XCD 1.45.)
+__host__ __device__ inline int strip_length(int ntiles) {
+  const int k = ntiles / 256;
+  return k < 1 ? 1 : k < 64 ? k : 64;
+}
+__device__ inline int strip_tile(int ntiles) {
+  const int k = strip_length(ntiles), b = (int)blockIdx.x, i = b >> 3;
+  return (i / k * 8 + (b & 7)) * k + i % k;
+}
+inline unsigned strip_grid(int ntiles) {
+  const int k = 8 * strip_length(ntiles);
+  return (unsigned)((ntiles + k - 1) / k * k);
+}
+
 }  // namespace sbslpm

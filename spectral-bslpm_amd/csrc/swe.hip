@@ -14,6 +14,7 @@
 // (y' = y or y0) and forms u = x cross W + D - x S once per target, the same
 // sums regrouped.
 #include "device.hpp"
+#include "pairwalk.hpp"
 
 namespace sbslpm {
 namespace {
@@ -49,141 +50,65 @@ __global__ void k_src_swe(DevTree t, const double* __restrict__ qz_part, const d
   rec[u] = SrcRecSwe{x, y, z, kNegInv4Pi * qz, x0, y0, z0, qd_scale * qd};
 }
 
-template <int VARIANT, bool GR>
-__global__ __launch_bounds__(256) void k_swe64(DevTree t, const TargetTile* __restrict__ tiles, int ntiles,
-                                               RowGroups gs, const SourceSet* __restrict__ sets,
-                                               const SrcRecSwe* __restrict__ rec, double eps, Ptr3 part, Ptr3 proxy,
-                                               int assign) {
-  __shared__ SrcRecSwe stage[GR ? kWavesPerBlock : 1][64];
-  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  int tile, row0, cg, ci;
-  if (!group_tile<GR>(gs, ntiles, wave, 1, tile, row0, cg, ci)) return;
-  const TargetTile T = tiles[tile];
-  const int row = row0 + ci;
-  const int64_t u = (int64_t)T.first + (row < T.count ? row : T.count - 1);
-  const int ng = GR ? gs.G : 1;
-  const bool copy_ok = !GR || cg < ng;
-  const double x = t.px[u], y = t.py[u], z = t.pz[u];
-  double w0 = 0, w1 = 0, w2 = 0, d0 = 0, d1 = 0, d2 = 0, sd = 0;
-  for (int e = T.src_begin; e < T.src_end; ++e) {
-    const SourceSet S = sets[e];
-    const SrcRecSwe* __restrict__ r = rec + S.first;
-    for (int c0 = 0; c0 < S.count; c0 += GR ? 64 : S.count) {
-      const int cn = GR ? min(64, S.count - c0) : S.count;
-      if (GR) stage_records(stage[wave], r + c0, cn);
-      const int trips = GR ? (cn + ng - 1) / ng : cn;
-#pragma unroll 2
-      for (int kk = 0; kk < trips; ++kk) {
-        const int k = GR ? kk * ng + cg : kk;
-        if (GR && !(copy_ok && k < cn)) continue;
-        const SrcRecSwe s = GR ? stage[wave][k] : r[k];
-        const double dp = x * s.x + y * s.y + z * s.z;
-        const double g = rcp64_pair((1.0 - dp) + eps);
-        const double gz = g * s.qz;
-        w0 = fma(gz, s.x, w0);
-        w1 = fma(gz, s.y, w1);
-        w2 = fma(gz, s.z, w2);
-        if (VARIANT == 1) {
-          const double gd = g * s.qd;
-          d0 = fma(gd, s.x, d0);
-          d1 = fma(gd, s.y, d1);
-          d2 = fma(gd, s.z, d2);
-          sd = fma(gd, dp, sd);
-        } else {
-          const double dp0 = x * s.x0 + y * s.y0 + z * s.z0;
-          const double gd = rcp64_pair((1.0 - dp0) + eps) * s.qd;
-          d0 = fma(gd, s.x0, d0);
-          d1 = fma(gd, s.y0, d1);
-          d2 = fma(gd, s.z0, d2);
-          sd = fma(gd, dp0, sd);
-        }
-      }
-    }
-  }
-  if (GR) {
-    w0 = group_sum(w0, gs, ci); w1 = group_sum(w1, gs, ci); w2 = group_sum(w2, gs, ci);
-    d0 = group_sum(d0, gs, ci); d1 = group_sum(d1, gs, ci); d2 = group_sum(d2, gs, ci);
-    sd = group_sum(sd, gs, ci);
-  }
-  if (cg != 0 || row >= T.count) return;
-  const double a = (y * w2 - z * w1) + (d0 - x * sd);
-  const double b = (z * w0 - x * w2) + (d1 - y * sd);
-  const double c = (x * w1 - y * w0) + (d2 - z * sd);
-  double* o[3];
-  int64_t v = u;
-  if (u < t.npart) {
-    o[0] = part.p[0]; o[1] = part.p[1]; o[2] = part.p[2];
-  } else {
-    v = u - t.npart;
-    o[0] = proxy.p[0]; o[1] = proxy.p[1]; o[2] = proxy.p[2];
-  }
-  if (assign) {
-    o[0][v] = a; o[1][v] = b; o[2][v] = c;
-  } else {
-    o[0][v] += a; o[1][v] += b; o[2][v] += c;
-  }
-}
-
-// k_swe64 with the source sets of one tile shared by the workgroup's four waves
-// (wave w takes sets w, w+4, ...), the four partial sums added in wave order
-// through LDS.  For tile lists too short to fill the chip with one wave per
-// tile (the lat-lon path's irregular tree: ~2,000 tiles of long source lists),
-// this gives each SIMD four times the waves to hide the record loads behind.
-// Workgroup b takes tile b: a list sorted heaviest first is dispatched in that
-// order (longest-processing-time first), which evens the CUs' loads.
-template <int VARIANT>
-__global__ __launch_bounds__(256) void k_swe64_shared(DevTree t, const TargetTile* __restrict__ tiles, int ntiles,
-                                                      const SourceSet* __restrict__ sets,
-                                                      const SrcRecSwe* __restrict__ rec, double eps, Ptr3 part,
-                                                      Ptr3 proxy, int assign) {
+// S waves share a tile (pairwalk.hpp), sources in batches of four with one
+// shared reciprocal (two in variant 2).  S_t = sum gd (x.y') of the header is
+// x.D, formed once per target.  heaviest_first: workgroup b takes tile b, for a
+// list sorted by decreasing work (the irregular trees).
+// Bound: FP64 vector issue, 16 slots per pair (variant 1; 21 with a reciprocal
+// and the x.y' sum on every pair).  Microseconds per launch with one wave per
+// tile (in lane groups at m = 6) and now: 6 x 28^2 121 -> 25, 6 x 64^2 443 -> 85,
+// 6 x 192^2 (degree 8) 860 -> 694, 6 x 512^2 4365 -> 3525; the 1 degree lat-lon
+// tree's whole evaluation 649 -> 555.
+template <int VARIANT, int S>
+__global__ __launch_bounds__(64 * S) void k_swe64(DevTree t, const TargetTile* __restrict__ tiles, int ntiles,
+                                                  const SourceSet* __restrict__ sets,
+                                                  const SrcRecSwe* __restrict__ rec, double eps, Ptr3 part, Ptr3 proxy,
+                                                  int assign, int heaviest_first) {
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int lane = threadIdx.x & 63;
-  const int tile = blockIdx.x;
-  if (tile >= ntiles) return;  // uniform over the workgroup
+  const int tile = heaviest_first ? (int)blockIdx.x : strip_tile(ntiles);
+  if (tile >= ntiles) return;  // the whole workgroup
   const TargetTile T = tiles[tile];
   const int64_t u = (int64_t)T.first + (lane < T.count ? lane : T.count - 1);
   const double x = t.px[u], y = t.py[u], z = t.pz[u];
-  double acc[7] = {0, 0, 0, 0, 0, 0, 0};  // W (3), D (3), S
-  for (int e = T.src_begin + wave; e < T.src_end; e += kWavesPerBlock) {
-    const SourceSet S = sets[e];
-    const SrcRecSwe* __restrict__ r = rec + S.first;
-#pragma unroll 2
-    for (int k = 0; k < S.count; ++k) {
-      const SrcRecSwe s = r[k];
-      const double dp = x * s.x + y * s.y + z * s.z;
-      const double g = rcp64_pair((1.0 - dp) + eps);
-      const double gz = g * s.qz;
-      acc[0] = fma(gz, s.x, acc[0]);
-      acc[1] = fma(gz, s.y, acc[1]);
-      acc[2] = fma(gz, s.z, acc[2]);
-      if (VARIANT == 1) {
-        const double gd = g * s.qd;
-        acc[3] = fma(gd, s.x, acc[3]);
-        acc[4] = fma(gd, s.y, acc[4]);
-        acc[5] = fma(gd, s.z, acc[5]);
-        acc[6] = fma(gd, dp, acc[6]);
-      } else {
-        const double dp0 = x * s.x0 + y * s.y0 + z * s.z0;
-        const double gd = rcp64_pair((1.0 - dp0) + eps) * s.qd;
-        acc[3] = fma(gd, s.x0, acc[3]);
-        acc[4] = fma(gd, s.y0, acc[4]);
-        acc[5] = fma(gd, s.z0, acc[5]);
-        acc[6] = fma(gd, dp0, acc[6]);
+  double acc[6] = {0, 0, 0, 0, 0, 0};  // W, D
+  auto add = [&](const SrcRecSwe& s, double g, double g0) {
+    const double gz = g * s.qz, gd = g0 * s.qd;
+    acc[0] = fma(gz, s.x, acc[0]);
+    acc[1] = fma(gz, s.y, acc[1]);
+    acc[2] = fma(gz, s.z, acc[2]);
+    acc[3] = fma(gd, VARIANT == 1 ? s.x : s.x0, acc[3]);
+    acc[4] = fma(gd, VARIANT == 1 ? s.y : s.y0, acc[4]);
+    acc[5] = fma(gd, VARIANT == 1 ? s.z : s.z0, acc[5]);
+  };
+  walk_sets<S>(T, sets, wave, [&](const SourceSet& set, int a, int b) {
+    const SrcRecSwe* __restrict__ r = rec + set.first;
+    int k = a;
+    for (; k + 4 <= b; k += 4) {
+      double d[4], g[4], g0[4];
+#pragma unroll
+      for (int i = 0; i < 4; ++i) d[i] = one_minus_dot(x, y, z, r[k + i].x, r[k + i].y, r[k + i].z) + eps;
+      rcp4(d, g);
+      if (VARIANT == 2) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) d[i] = one_minus_dot(x, y, z, r[k + i].x0, r[k + i].y0, r[k + i].z0) + eps;
+        rcp4(d, g0);
       }
+#pragma unroll
+      for (int i = 0; i < 4; ++i) add(r[k + i], g[i], VARIANT == 1 ? g[i] : g0[i]);
     }
-  }
-  __shared__ double red[7][kWavesPerBlock - 1][64];
-  if (wave > 0)
-#pragma unroll
-    for (int q = 0; q < 7; ++q) red[q][wave - 1][lane] = acc[q];
-  __syncthreads();
+    for (; k < b; ++k) {
+      const SrcRecSwe s = r[k];
+      const double g = rcp64_pair(one_minus_dot(x, y, z, s.x, s.y, s.z) + eps);
+      add(s, g, VARIANT == 1 ? g : rcp64_pair(one_minus_dot(x, y, z, s.x0, s.y0, s.z0) + eps));
+    }
+  });
+  tile_sum<S>(acc, wave, lane);
   if (wave > 0 || lane >= T.count) return;
-#pragma unroll
-  for (int q = 0; q < 7; ++q)
-    for (int w = 0; w < kWavesPerBlock - 1; ++w) acc[q] += red[q][w][lane];
-  const double a = (y * acc[2] - z * acc[1]) + (acc[3] - x * acc[6]);
-  const double b = (z * acc[0] - x * acc[2]) + (acc[4] - y * acc[6]);
-  const double c = (x * acc[1] - y * acc[0]) + (acc[5] - z * acc[6]);
+  const double sd = x * acc[3] + y * acc[4] + z * acc[5];
+  const double a = (y * acc[2] - z * acc[1]) + (acc[3] - x * sd);
+  const double b = (z * acc[0] - x * acc[2]) + (acc[4] - y * sd);
+  const double c = (x * acc[1] - y * acc[0]) + (acc[5] - z * sd);
   double* o[3];
   int64_t v = u;
   if (u < t.npart) {
@@ -357,37 +282,20 @@ void launch_source_records_swe(const DevTree& t, int variant, const double* qz_p
 
 void launch_swe_interact64(const DevTree& t, int variant, const TargetTile* tiles, int ntiles, const SourceSet* sets,
                            const SrcRecSwe* rec, double eps, double* const* out_part, double* const* out_proxy,
-                           hipStream_t s, bool assign, bool shared_tiles) {
+                           hipStream_t s, bool assign, bool heaviest_first) {
   if (ntiles == 0) return;
   Ptr3 op{}, ox{};
   for (int f = 0; f < 3; ++f) {
     op.p[f] = out_part[f];
     ox.p[f] = out_proxy[f];
   }
-  if (shared_tiles) {
-    if (variant != 2)
-      hipLaunchKernelGGL(k_swe64_shared<1>, dim3(ntiles), dim3(64 * kWavesPerBlock), 0, s, t, tiles, ntiles, sets, rec,
-                         eps, op, ox, assign ? 1 : 0);
-    else
-      hipLaunchKernelGGL(k_swe64_shared<2>, dim3(ntiles), dim3(64 * kWavesPerBlock), 0, s, t, tiles, ntiles, sets, rec,
-                         eps, op, ox, assign ? 1 : 0);
-    return;
-  }
-  const RowGroups gs = row_groups(t);
-  const unsigned blocks = (unsigned)(((int64_t)ntiles * gs.H + kWavesPerBlock - 1) / kWavesPerBlock);
-  const dim3 block(64 * kWavesPerBlock);
-  const int as = assign ? 1 : 0;
-  if (variant != 2) {
-    if (gs.G > 1)
-      hipLaunchKernelGGL((k_swe64<1, true>), dim3(blocks), block, 0, s, t, tiles, ntiles, gs, sets, rec, eps, op, ox, as);
-    else
-      hipLaunchKernelGGL((k_swe64<1, false>), dim3(blocks), block, 0, s, t, tiles, ntiles, gs, sets, rec, eps, op, ox, as);
-  } else {
-    if (gs.G > 1)
-      hipLaunchKernelGGL((k_swe64<2, true>), dim3(blocks), block, 0, s, t, tiles, ntiles, gs, sets, rec, eps, op, ox, as);
-    else
-      hipLaunchKernelGGL((k_swe64<2, false>), dim3(blocks), block, 0, s, t, tiles, ntiles, gs, sets, rec, eps, op, ox, as);
-  }
+  // us per launch with 4 / 8 / 16 waves: 126 tiles 49 / 31 / 25, 636 102 / 85 / 91, 2,556 202 / 200 / 246,
+  // 10,236 694 / 710 / 903, 40,956 3525 / 3691 / 4706
+  const int S = ntiles < 400 ? 16 : ntiles < 3000 ? 8 : 4;
+  auto kernel = variant != 2 ? (S == 16 ? k_swe64<1, 16> : S == 8 ? k_swe64<1, 8> : k_swe64<1, 4>)
+                             : (S == 16 ? k_swe64<2, 16> : S == 8 ? k_swe64<2, 8> : k_swe64<2, 4>);
+  hipLaunchKernelGGL(kernel, dim3(heaviest_first ? ntiles : strip_grid(ntiles)), dim3(64 * S), 0, s, t, tiles, ntiles, sets, rec, eps, op, ox,
+                     assign ? 1 : 0, heaviest_first ? 1 : 0);
 }
 
 }  // namespace sbslpm

@@ -69,3 +69,31 @@ def test_log_pairs(case):
         v.fill_(0.5)
     gp, gx = ctx.poisson_fmm_interactions(*up(case, [case["qp"], case["qx"]]), psi_part, psi_proxy)
     close(case, [gp], [gx], [ep], [ex], 0.5)
+
+
+@pytest.mark.parametrize("variant", [1, 2])
+@pytest.mark.parametrize("displaced", [False, True])
+def test_shallow_water_pairs(case, variant, displaced):
+    ctx, o = case["ctx"], case["o"]
+    dp, dx = (case["dp"], case["dx"]) if displaced else (None, None)
+    dpart, dprox = np.roll(case["qp"], 7), np.roll(case["qx"], 7)
+    ep, ex = o.swe_vel_interactions(variant, case["qp"], case["qx"], dpart, dprox, EPS, dp, dx)
+    phi_part, phi_proxy = ctx.zeros_part(3), ctx.zeros_proxy(3)
+    for v in phi_part + phi_proxy:
+        v.fill_(0.5)
+    gp, gx = ctx.swe_vel_interactions(*up(case, [case["qp"], case["qx"], dpart, dprox]), up(case, dp) if dp else None,
+                                      up(case, dx) if dx else None, phi_part, phi_proxy, variant)
+    close(case, gp, gx, ep, ex, 0.5)
+
+
+@pytest.mark.parametrize("displaced", [False, True])
+def test_laplacian_pairs(case, displaced):
+    ctx, o = case["ctx"], case["o"]
+    dp, dx = (case["dp"], case["dx"]) if displaced else (None, None)
+    ep, ex = o.laplacian_interactions(case["qp"], case["qx"], dp, dx)
+    phi_part, phi_proxy = ctx.zeros_part(), ctx.zeros_proxy()
+    for v in (phi_part, phi_proxy):
+        v.fill_(0.5)
+    gp, gx = ctx.laplacian_interactions(*up(case, [case["qp"], case["qx"]]), up(case, dp) if dp else None,
+                                        up(case, dx) if dx else None, phi_part, phi_proxy)
+    close(case, [gp], [gx], [ep], [ex], 0.5)
