@@ -338,7 +338,8 @@ def bench_ensemble(args, torch, sb):
             if nl == 0:
                 continue
             achieved = pairs * nmem * FLOP_BS / (ms / nl / 1e3) / 1e12
-            r[name] = dict(bound="mfma", achieved=round(achieved, 3), peak=PEAK_FP32, unit="TFLOP/s",
+            r[name] = dict(bound="mfma" if kern == "bve_mrhs" else "valu", achieved=round(achieved, 3),
+                           peak=PEAK_FP32, unit="TFLOP/s",
                            frac=round(achieved / PEAK_FP32, 4), avg_launch_ms=round(ms / nl, 4), launches=nl,
                            members_per_launch=nmem, pairs_per_member=pairs, flop_per_pair=FLOP_BS)
             if kern == "bve_mrhs":
@@ -1241,15 +1242,14 @@ def main():
     roof = {}
     # executed work per pair besides the 27-flop convention (which credits a per-pair cross
     # product both kernels do once per target and source set):
-    #   FP64: x.y (5), (1 - x.y) + eps (2), rcp + one Newton step (5), g q (1), 3 fma (6) = 19;
-    #   mixed: the 16x16x4 denominator product (8 per pair), four 4x4x1 accumulation products
-    #   (8 per pair) on the matrix cores, the add of 1/2|p|^2 and the reciprocal on the vector
-    #   unit (2) = 18.
-    executed = {"bve_fp64": 19, "bve_mixed": 18}
-    limiter = {"bve_fp64": "FP64 vector FMA and reciprocal issue (78.6 TF/s vector peak)",
-               "bve_mixed": "MFMA products (64 cycles per 256 pairs) and vector work with four v_rcp_f32 "
-                            "(about 90 cycles), serialized on each SIMD (register-only probe: no vector/matrix "
-                            "co-issue; profiles/bve_mixed_issue_rates.md)"}
+    #   FP64: 1 - x.y (6), + eps (1), a quarter of a shared reciprocal with two Newton steps and
+    #   nine products (4.5), g q (1), 3 fma (6) = 18.5;
+    #   mixed: alpha + beta (1), - p.b (6), reciprocal (1), 4 fma (8) = 16.
+    executed = {"bve_fp64": 18.5, "bve_mixed": 16}
+    limiter = {"bve_fp64": "FP64 vector issue (12.25 slots of 4 cycles per pair) at the clock the chip holds under it "
+                           "(2.1 GHz)",
+               "bve_mixed": "FP32 vector issue (eight multiply-adds of 2.5 cycles and a 9-cycle v_rcp_f32 per pair) at "
+                            "the clock the chip holds under it (2.0 GHz)"}
     for ctx, name, peak in ((ctx64, "bve_fp64", PEAK_FP64), (ctxmx, "bve_mixed", PEAK_FP32)):
         ctx.enable_timing(True)
         with torch.cuda.stream(stream):
@@ -1260,7 +1260,7 @@ def main():
         ctx.enable_timing(False)
         avg = ms / nl / 1e3
         achieved = pairs * FLOP_BS / avg / 1e12
-        roof[name] = dict(bound="mfma" if name == "bve_mixed" else "valu", achieved=round(achieved, 3), peak=peak,
+        roof[name] = dict(bound="valu", achieved=round(achieved, 3), peak=peak,
                           unit="TFLOP/s", frac=round(achieved / peak, 4), traffic=None,
                           avg_launch_ms=round(ms / nl, 4), pairs_per_launch=pairs, flop_per_pair=FLOP_BS,
                           executed_flop_per_pair=executed[name],
@@ -1271,7 +1271,7 @@ def main():
     if args.config == "c3" and os.path.exists(tfile):
         with open(tfile) as fh:
             tr = json.load(fh)["kernels"]
-        for name, kern in (("bve_fp64", "k_bve64"), ("bve_mixed", "k_bve_mfma")):
+        for name, kern in (("bve_fp64", "k_bve64"), ("bve_mixed", "k_bve_lanes")):
             if tr.get(kern):
                 roof[name]["traffic"] = tr[kern]["hbm_bytes"]
                 roof[name]["traffic_kernel"] = kern

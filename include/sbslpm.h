@@ -49,8 +49,8 @@ enum { SBSLPM_RK4_REFERENCE = 0, SBSLPM_RK4_TEXTBOOK = 1 };
  * by dt/2 (swe_time_step.cpp:761).  LEAF uses the leaf's own face and displacement, the surface
  * gradient, and dt at stage 4. */
 enum { SBSLPM_SWE_RULE_REFERENCE = 0, SBSLPM_SWE_RULE_LEAF = 1 };
-/* SBSLPM_MIXED: FP32 pair arithmetic on the matrix cores (Biot-Savart) / vector unit (log), FP64
- * accumulation; SBSLPM_MIXED_VALU: the same precision with the Biot-Savart pairs on the vector unit. */
+/* SBSLPM_MIXED: FP32 pair arithmetic, FP64 accumulation per source set; SBSLPM_MIXED_VALU: the same
+ * precision with the Biot-Savart pairs in the difference form, one target per lane. */
 enum { SBSLPM_FP64 = 0, SBSLPM_MIXED = 1, SBSLPM_MIXED_VALU = 2 };
 /* SBSLPM_FLAG_GRAPH: capture steps in a hipGraph (needs a non-default stream).
  * SBSLPM_FLAG_MULTI_RHS: on a SBSLPM_MIXED context, the first RK4 stage of an ensemble step

@@ -35,7 +35,7 @@ class RunConfig:
     delta_t: float = 3600.0
     weights: str = "reference"       # reference | clenshaw_curtis | equal_area
     rk4_combine: str = "reference"   # reference | textbook
-    precision: str = "fp64"          # fp64 | mixed (matrix cores) | mixed_valu
+    precision: str = "fp64"          # fp64 | mixed (FP32 pairs, lane copies) | mixed_valu
     tracer_count: int = 0
     use_graph: bool = False
     multi_rhs: bool = False          # ensembles: first stage as one multi-RHS product (mixed only)

@@ -267,6 +267,25 @@ const HostTables& host_tables() {
 int velocity(sbslpm_ctx* c, const Work& w, int nmem, const double* area, const double* vor,
              const double* const* dpart, const double* const* dprox, double* const* vel);
 
+// Source records and pair sums of a mixed-precision context: the vector unit in
+// lane copies, or the matrix cores where bf16 M2L products are asked for.
+void mixed_records(sbslpm_ctx* c, const double* q_part, const double* q_proxy, const double* const* dpart,
+                   const double* const* dprox, SrcRecMfma* rec, int nmem = 1) {
+  if (c->dt.bf16_m2l)
+    launch_source_records_mfma(c->dt, q_part, q_proxy, dpart, dprox, rec, c->stream, nmem);
+  else
+    launch_source_records_lanes(c->dt, q_part, q_proxy, dpart, dprox, rec, c->stream, nmem);
+}
+void mixed_pairs(sbslpm_ctx* c, const SrcRecMfma* rec, double* const* out_part, double* const* out_proxy, bool assign,
+                 int nmem, PairShape shape) {
+  if (c->dt.bf16_m2l)
+    launch_bve_interact_mfma(c->dt, c->tiles, c->ntiles, c->sets, rec, c->prm.kernel_eps, out_part, out_proxy,
+                             c->stream, assign, nmem, shape);
+  else
+    launch_bve_interact_lanes(c->dt, c->tiles, c->ntiles, c->sets, rec, c->prm.kernel_eps, out_part, out_proxy,
+                              c->stream, assign, nmem, shape);
+}
+
 // Brackets one pair-kernel launch with events when timing is on.
 struct KernelTimer {
   sbslpm_ctx* c;
@@ -429,7 +448,9 @@ int sbslpm_ctx_create(const sbslpm_params* p, sbslpm_ctx** out) {
   d.expnegtab = (const double*)(b + o_entab);
   d.xcd_start = (const int*)(b + o_xcd);
   d.err = (int*)(b + o_err);
-  d.bf16_m2l = (c->prm.flags & SBSLPM_FLAG_BF16_M2L) ? 1 : 0;
+  // a list without proxy-to-proxy sets takes the FP32 kernels whatever the flag
+  d.bf16_m2l = (c->prm.flags & SBSLPM_FLAG_BF16_M2L) &&
+               std::any_of(t.srcsets.begin(), t.srcsets.end(), [](const SourceSet& q) { return q.m2l != 0; });
   d.P = t.P; d.Pl = t.Pl; d.offset = t.offset; d.n = t.n; d.dp1 = t.dp1; d.m = t.m; d.m2 = t.m2;
   d.levels = t.cfg.levels; d.npart = t.npart; d.U = t.U;
   d.m2p = t.m2p; d.np16 = t.np16; d.U16 = t.U16;
@@ -617,9 +638,9 @@ int sbslpm_bve_vel_interactions(sbslpm_ctx* c, const double* dpx, const double* 
   const double* const* dpp = dpx ? dp : nullptr;
   const double* const* dxp = dxx ? dx : nullptr;
   if (c->prm.precision == SBSLPM_MIXED) {
-    launch_source_records_mfma(c->dt, q_part, q_proxy, dpp, dxp, c->recmf, c->stream);
+    mixed_records(c, q_part, q_proxy, dpp, dxp, c->recmf);
     KernelTimer tm(c, SBSLPM_KERNEL_BVE_MIXED);
-    launch_bve_interact_mfma(c->dt, c->tiles, c->ntiles, c->sets, c->recmf, c->prm.kernel_eps, op, ox, c->stream);
+    mixed_pairs(c, c->recmf, op, ox, false, 1, {});
   } else if (c->prm.precision == SBSLPM_MIXED_VALU) {
     launch_source_records32(c->dt, q_part, q_proxy, dpp, dxp, c->rec32, c->stream);
     KernelTimer tm(c, SBSLPM_KERNEL_BVE_MIXED);
@@ -875,10 +896,9 @@ int velocity(sbslpm_ctx* c, const Work& w, int nmem, const double* area, const d
     launch_bve_interact_mrhs(c->dt, c->tiles, c->ntiles, c->sets, w.recmf, w.qcol, nmem, cb, c->prm.kernel_eps,
                              w.phipart, w.phiproxy, c->stream, true, c->mrhs_cb ? c->mrhs_shape : c->shape);
   } else if (c->prm.precision == SBSLPM_MIXED) {
-    launch_source_records_mfma(c->dt, w.qpart, w.qproxy, dpart, dprox, w.recmf, c->stream, nmem);
+    mixed_records(c, w.qpart, w.qproxy, dpart, dprox, w.recmf, nmem);
     KernelTimer tm(c, SBSLPM_KERNEL_BVE_MIXED);
-    launch_bve_interact_mfma(c->dt, c->tiles, c->ntiles, c->sets, w.recmf, c->prm.kernel_eps, w.phipart,
-                             w.phiproxy, c->stream, true, nmem, c->shape);
+    mixed_pairs(c, w.recmf, w.phipart, w.phiproxy, true, nmem, c->shape);
   } else if (c->prm.precision == SBSLPM_MIXED_VALU) {
     launch_source_records32(c->dt, w.qpart, w.qproxy, dpart, dprox, w.rec32, c->stream, nmem);
     KernelTimer tm(c, SBSLPM_KERNEL_BVE_MIXED);
@@ -1698,15 +1718,14 @@ int sbslpm_autotune(sbslpm_ctx* c, const double* area, const double* vor, double
   launch_upward_fused(c->dt, area, vor, w.qpart, w.qproxy, c->stream);
   const int prec = c->prm.precision;
   if (prec == SBSLPM_MIXED)
-    launch_source_records_mfma(c->dt, w.qpart, w.qproxy, nullptr, nullptr, w.recmf, c->stream);
+    mixed_records(c, w.qpart, w.qproxy, nullptr, nullptr, w.recmf);
   else if (prec == SBSLPM_MIXED_VALU)
     launch_source_records32(c->dt, w.qpart, w.qproxy, nullptr, nullptr, w.rec32, c->stream);
   else
     launch_source_records64(c->dt, w.qpart, w.qproxy, nullptr, nullptr, true, w.rec64, c->stream);
   auto launch = [&](PairShape sh) {
     if (prec == SBSLPM_MIXED)
-      launch_bve_interact_mfma(c->dt, c->tiles, c->ntiles, c->sets, w.recmf, c->prm.kernel_eps, w.phipart, w.phiproxy,
-                               c->stream, true, 1, sh);
+      mixed_pairs(c, w.recmf, w.phipart, w.phiproxy, true, 1, sh);
     else if (prec == SBSLPM_MIXED_VALU)
       launch_bve_interact_mixed(c->dt, c->tiles, c->ntiles, c->sets, w.rec32, c->prm.kernel_eps, w.phipart,
                                 w.phiproxy, c->stream, true, 1, sh);

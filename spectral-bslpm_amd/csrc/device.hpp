@@ -398,6 +398,16 @@ void launch_bve_interact_mfma(const DevTree& t, const TargetTile* tiles, int nti
                               const SrcRecMfma* rec, double eps, double* const* out_part, double* const* out_proxy,
                               hipStream_t s, bool assign = false, int nmem = 1, PairShape shape = {});
 
+// The mixed-precision pair kernel on the vector unit in lane copies (bve_lanes.hip);
+// rec holds 32 bytes per source in the space of the matrix-core records (members
+// U16 records apart).
+void launch_source_records_lanes(const DevTree& t, const double* q_part, const double* q_proxy,
+                                 const double* const* disp_part, const double* const* disp_proxy, void* rec,
+                                 hipStream_t s, int nmem = 1);
+void launch_bve_interact_lanes(const DevTree& t, const TargetTile* tiles, int ntiles, const SourceSet* sets,
+                               const void* rec, double eps, double* const* out_part, double* const* out_proxy,
+                               hipStream_t s, bool assign = false, int nmem = 1, PairShape shape = {});
+
 // Multi-right-hand-side MFMA pair kernel for nmem members whose sources and
 // targets share positions: one kernel matrix per wave, applied to the charge
 // columns of 4 * cb members (cb = 1 or 2 chunks of four per wave).  The columns

@@ -639,7 +639,8 @@ __global__ void k_src_mfma(DevTree t, const double* __restrict__ q_part, const d
   for (int c = 0; c < 4; ++c) tile[64 + ((i >> 2) * 4 + c) * 4 + (i & 3)] = v[4 + c];
 }
 
-// Mixed-precision Biot-Savart pair kernel on the matrix cores.
+// Mixed-precision Biot-Savart pair kernel on the matrix cores, for contexts with
+// bf16 M2L products (k_bve_lanes takes the others).
 //
 // Per wave: NTT (1..4) target tiles of 16 (up to 64 targets of one panel).
 // For every source set, coordinates are taken relative to the source-panel
@@ -658,7 +659,7 @@ __global__ void k_src_mfma(DevTree t, const double* __restrict__ q_part, const d
 // 4x4x1 form uses lanes 4 b .. 4 b + 3 (A row / B column = lane % 4, D row =
 // register).  The next source tile's operands are loaded before the current
 // tile's arithmetic (every index stays inside the set's padded records).
-template <int NTT, bool M2L>
+template <int NTT>
 __device__ inline void bve_mfma_tiles(const DevTree& t, const TargetTile& T, const SourceSet* __restrict__ sets,
                                       const float* __restrict__ rec, float eps, int lane, double (&w)[4][3]) {
   const int col = lane & 15, grp = lane >> 4;
@@ -706,7 +707,7 @@ __device__ inline void bve_mfma_tiles(const DevTree& t, const TargetTile& T, con
     const float na1 = rn[lane];
     const v4f nbq = *reinterpret_cast<const v4f*>(rn + off_b);
     v4f d[NTT];
-    kernel_products<NTT>(a1, b1, M2L && S.m2l, d);
+    kernel_products<NTT>(a1, b1, S.m2l, d);
 #pragma unroll
     for (int tt = 0; tt < NTT; ++tt)
 #pragma unroll
@@ -737,7 +738,6 @@ __device__ inline void bve_mfma_tiles(const DevTree& t, const TargetTile& T, con
   }
 }
 
-template <bool M2L>
 __global__ __launch_bounds__(256) void k_bve_mfma(DevTree t, const TargetTile* __restrict__ tiles, int ntiles,
                                                   const SourceSet* __restrict__ sets,
                                                   const float* __restrict__ rec, float eps, Ptr3 part,
@@ -755,10 +755,10 @@ __global__ __launch_bounds__(256) void k_bve_mfma(DevTree t, const TargetTile* _
 #pragma unroll
   for (int tt = 0; tt < 4; ++tt) w[tt][0] = w[tt][1] = w[tt][2] = 0.0;
   switch (ntt) {
-    case 4: bve_mfma_tiles<4, M2L>(t, T, sets, rec, eps, lane, w); break;
-    case 3: bve_mfma_tiles<3, M2L>(t, T, sets, rec, eps, lane, w); break;
-    case 2: bve_mfma_tiles<2, M2L>(t, T, sets, rec, eps, lane, w); break;
-    default: bve_mfma_tiles<1, M2L>(t, T, sets, rec, eps, lane, w); break;
+    case 4: bve_mfma_tiles<4>(t, T, sets, rec, eps, lane, w); break;
+    case 3: bve_mfma_tiles<3>(t, T, sets, rec, eps, lane, w); break;
+    case 2: bve_mfma_tiles<2>(t, T, sets, rec, eps, lane, w); break;
+    default: bve_mfma_tiles<1>(t, T, sets, rec, eps, lane, w); break;
   }
   // sum the four source quarters (lanes col, col+16, col+32, col+48)
 #pragma unroll
@@ -1010,8 +1010,7 @@ inline Ptr3 ptr3(double* const* a) {
 
 }  // namespace
 
-// The matrix-core kernels in their FP32 form or with bf16 M2L products.
-static auto mfma_kernel(const DevTree& t) { return t.bf16_m2l ? k_bve_mfma<true> : k_bve_mfma<false>; }
+// The multi-right-hand-side kernel in its FP32 form or with bf16 M2L products.
 template <int CB>
 static auto mrhs_kernel(const DevTree& t) { return t.bf16_m2l ? k_bve_mrhs<CB, true> : k_bve_mrhs<CB, false>; }
 
@@ -1108,7 +1107,7 @@ void launch_bve_interact_mfma(const DevTree& t, const TargetTile* tiles, int nti
                               hipStream_t s, bool assign, int nmem, PairShape shape) {
   if (ntiles == 0) return;
   shape = checked_shape(t, shape);
-  hipLaunchKernelGGL(mfma_kernel(t), dim3(pair_grid(ntiles, shape), nmem), dim3(64 * shape.waves), 0, s, t,
+  hipLaunchKernelGGL(k_bve_mfma, dim3(pair_grid(ntiles, shape), nmem), dim3(64 * shape.waves), 0, s, t,
                      tiles, ntiles, sets, (const float*)rec, (float)eps, ptr3(out_part), ptr3(out_proxy),
                      assign ? 1 : 0, shape.xcd);
 }

@@ -25,10 +25,10 @@ inline int tile_waves(int ntiles) { return ntiles < 1500 ? 16 : ntiles < 6000 ? 
 // f(set, a, b) for this wave's part [a, b) of each of its source sets.
 template <int S, typename F>
 __device__ inline void walk_sets(const TargetTile& T, const SourceSet* __restrict__ sets, int wave, F&& f) {
-  constexpr int SK = S / 4;  // waves per set
-  const int ws = wave & 3, wk = wave >> 2;
+  constexpr int SS = S < 4 ? S : 4, SK = S / SS;  // sets in turn, waves per set
+  const int ws = wave & (SS - 1), wk = wave / SS;
   int it = 0;
-  for (int e = T.src_begin + ws; e < T.src_end; e += 4, ++it) {
+  for (int e = T.src_begin + ws; e < T.src_end; e += SS, ++it) {
     const SourceSet set = sets[e];
     if (SK == 1) {
       f(set, 0, set.count);

@@ -97,3 +97,27 @@ def test_laplacian_pairs(case, displaced):
     gp, gx = ctx.laplacian_interactions(*up(case, [case["qp"], case["qx"]]), up(case, dp) if dp else None,
                                         up(case, dx) if dx else None, phi_part, phi_proxy)
     close(case, [gp], [gx], [ep], [ex], 0.5)
+
+
+@pytest.mark.parametrize("displaced", [False, True])
+def test_vortex_pairs_mixed(case, displaced, sb):
+    """Lane copies of 13 to 32 lanes (tiles of 25 to 64 targets), chunks and sets that they divide
+    unevenly.  In panel-centred FP32 the denominator alpha + beta - p.b is off by a few 2^-24 of
+    r^2 (r the leaf radius), which the nearest pairs (eps) magnify, on top of a few 2^-24 per pair;
+    the per-pair bound 2^-24 (8 + 2 r^2 / eps) bounds the field's relative error."""
+    ctx, o, W = case["ctx"], case["o"], case["W"]
+    cm = sb.Context(sb.RunConfig(levels=ctx.cfg.levels, interp_degree=ctx.cfg.interp_degree,
+                                 leaf_degree=ctx.cfg.leaf_degree, kernel_eps=EPS, weights="clenshaw_curtis",
+                                 precision="mixed"))
+    x, y, z, a = o.spec_points()
+    qp, qx = o.upward_pass(a, W.gaussian_vortices(x, y, z, a, seed=3))
+    dp, dx = (case["dp"], case["dx"]) if displaced else (None, None)
+    ep, ex = o.bve_vel_interactions(qp, qx, EPS, dp, dx)
+    gp, gx = cm.bve_vel_interactions(*up(case, [qp, qx]), up(case, dp) if dp else None, up(case, dx) if dx else None)
+    cm.synchronize()
+    r = np.sqrt(2) * (np.pi / 4) / 2 ** (ctx.cfg.levels - 1)
+    bound = 2.0 ** -24 * (8 + 2 * r * r / EPS)
+    assert W.vec_rel_l2([to_np(v) for v in gp], ep) < bound
+    off = o.offset
+    if np.any([np.any(np.asarray(v)[:off]) for v in ex]):
+        assert W.vec_rel_l2([to_np(v)[:off] for v in gx], [np.asarray(v)[:off] for v in ex]) < bound
