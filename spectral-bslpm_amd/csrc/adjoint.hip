@@ -18,10 +18,11 @@
 //     (dbar = (I - y y^T) ybar / |node + d|) and, for proxy sources, through
 //     the anterpolation of the charges (downward pass) and the interpolation
 //     of their displacements (scattered back to the leaf particles).
-// The pair sums run over the interaction list seen from its sources: one
-// wave per tile of at most 64 source points, each lane owning one source
-// row (assigned, no atomics), the targets' records read wave-uniformly.
-#include "device.hpp"
+// The pair sums run over the interaction list seen from its sources: a
+// workgroup per tile of at most 64 source points, every source row written once
+// (assigned, no atomics), the targets' records read wave-uniformly (FP64) or from
+// LDS in lane copies (FP32).
+#include "lanes.hpp"
 
 namespace sbslpm {
 namespace {
@@ -54,67 +55,21 @@ __global__ void k_tgt_rec(DevTree t, CPtr3 psi_part, CPtr3 psi_prox, TgtRec* __r
   rec[u] = TgtRec{x, y, z, b * z - d * y, d * x - a * z, a * y - b * x};
 }
 
-// Transposed pair sums.  POS: also the position cotangent (displaced stages).
-template <bool POS, bool GR>
-__global__ __launch_bounds__(256) void k_bve_adj64(DevTree t, const TargetTile* __restrict__ tiles, int ntiles,
-                                                   RowGroups gs, const SourceSet* __restrict__ targets,
-                                                   const TgtRec* __restrict__ trec, const SrcRec64* __restrict__ srec,
-                                                   double eps, CPtr3 dpart, CPtr3 dprox, double* __restrict__ qbar_part,
-                                                   double* __restrict__ qbar_prox, Ptr3 dbar_part, Ptr3 dbar_prox, int xcd) {
-  __shared__ TgtRec stage[GR ? kWavesPerBlock : 1][64];
-  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  int tile, row0, cg, ci;
-  if (!group_tile<GR>(gs, ntiles, wave, xcd, tile, row0, cg, ci)) return;
-  const TargetTile T = tiles[tile];
-  const int row = row0 + ci;
-  const int64_t u = (int64_t)T.first + (row < T.count ? row : T.count - 1);
-  const int ng = GR ? gs.G : 1;
-  const bool copy_ok = !GR || cg < ng;
-  const SrcRec64 S = srec[u];
-  double aq = 0, a0 = 0, a1 = 0, a2 = 0;
-  for (int e = T.src_begin; e < T.src_end; ++e) {
-    const SourceSet G = targets[e];
-    const TgtRec* __restrict__ r = trec + G.first;
-    for (int c0 = 0; c0 < G.count; c0 += GR ? 64 : G.count) {
-      const int cn = GR ? min(64, G.count - c0) : G.count;
-      if (GR) stage_records(stage[wave], r + c0, cn);
-      const int trips = GR ? (cn + ng - 1) / ng : cn;
-#pragma unroll 4
-      for (int kk = 0; kk < trips; ++kk) {
-        const int k = GR ? kk * ng + cg : kk;
-        if (GR && !(copy_ok && k < cn)) continue;
-        const TgtRec R = GR ? stage[wave][k] : r[k];
-        // the forward kernel's denominator, x = target, y = source
-        const double g = rcp64_pair((1.0 - (R.x * S.x + R.y * S.y + R.z * S.z)) + eps);
-        const double dc = S.x * R.c0 + S.y * R.c1 + S.z * R.c2;
-        aq = fma(g, dc, aq);
-        if (POS) {
-          const double h = g * dc;
-          a0 = fma(g, fma(h, R.x, R.c0), a0);
-          a1 = fma(g, fma(h, R.y, R.c1), a1);
-          a2 = fma(g, fma(h, R.z, R.c2), a2);
-        }
-      }
-    }
-  }
-  if (GR) {
-    aq = group_sum(aq, gs, ci);
-    if (POS) {
-      a0 = group_sum(a0, gs, ci);
-      a1 = group_sum(a1, gs, ci);
-      a2 = group_sum(a2, gs, ci);
-    }
-  }
-  if (cg != 0 || row >= T.count) return;
+// Source-side finish of one row: the charge cotangent and, with POS, the
+// position cotangent through the projection.
+template <bool POS>
+__device__ inline void store_row(const DevTree& t, int64_t u, const SrcRec64& S, const double* a, CPtr3 dpart,
+                                 CPtr3 dprox, double* __restrict__ qbar_part, double* __restrict__ qbar_prox,
+                                 Ptr3 dbar_part, Ptr3 dbar_prox) {
   const bool part = u < t.npart;
   const int64_t v = part ? u : u - t.npart;
-  (part ? qbar_part : qbar_prox)[v] = kNegInv4Pi * aq;
-  if (POS) {
+  (part ? qbar_part : qbar_prox)[v] = kNegInv4Pi * a[0];
+  if constexpr (POS) {
     const double w0 = t.px[u] + (part ? dpart.p[0] : dprox.p[0])[v];
     const double w1 = t.py[u] + (part ? dpart.p[1] : dprox.p[1])[v];
     const double w2 = t.pz[u] + (part ? dpart.p[2] : dprox.p[2])[v];
     const double ir = 1.0 / sqrt(w0 * w0 + w1 * w1 + w2 * w2);
-    const double yb0 = S.q * a0, yb1 = S.q * a1, yb2 = S.q * a2;
+    const double yb0 = S.q * a[1], yb1 = S.q * a[2], yb2 = S.q * a[3];
     const double yy = S.x * yb0 + S.y * yb1 + S.z * yb2;
     (part ? dbar_part.p[0] : dbar_prox.p[0])[v] = (yb0 - S.x * yy) * ir;
     (part ? dbar_part.p[1] : dbar_prox.p[1])[v] = (yb1 - S.y * yy) * ir;
@@ -122,9 +77,132 @@ __global__ __launch_bounds__(256) void k_bve_adj64(DevTree t, const TargetTile* 
   }
 }
 
-// FP32 target record: node relative to its panel centre and c = psi cross x.
+// Transposed pair sums.  POS: also the position cotangent (displaced stages).
+// S waves share a tile (pairwalk.hpp), targets in batches of four with one
+// shared reciprocal.
+// Bound: FP64 vector issue, 12 slots per pair (19 with POS).  The step adjoint (three
+// evaluations with POS and one without) before (one wave per tile, lane groups where
+// they fill more) and now: 6 x 28^2 546 -> 287 us, 6 x 64^2 1473 -> 586, 6 x 128^2
+// 2164 -> 1440, 6 x 224^2 3496 -> 2815.
+template <bool POS, int S>
+__global__ __launch_bounds__(64 * S) void k_bve_adj64(DevTree t, const TargetTile* __restrict__ tiles, int ntiles,
+                                                      const SourceSet* __restrict__ targets,
+                                                      const TgtRec* __restrict__ trec,
+                                                      const SrcRec64* __restrict__ srec, double eps, CPtr3 dpart,
+                                                      CPtr3 dprox, double* __restrict__ qbar_part,
+                                                      double* __restrict__ qbar_prox, Ptr3 dbar_part, Ptr3 dbar_prox) {
+  constexpr int K = POS ? 4 : 1;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int lane = threadIdx.x & 63;
+  const int tile = strip_tile(ntiles);
+  if (tile >= ntiles) return;  // the whole workgroup
+  const TargetTile T = tiles[tile];
+  const int64_t u = (int64_t)T.first + (lane < T.count ? lane : T.count - 1);
+  const SrcRec64 Y = srec[u];
+  double acc[K];
+#pragma unroll
+  for (int k = 0; k < K; ++k) acc[k] = 0;
+  auto add = [&](const TgtRec& R, double g) {
+    const double dc = Y.x * R.c0 + Y.y * R.c1 + Y.z * R.c2;
+    acc[0] = fma(g, dc, acc[0]);
+    if constexpr (POS) {
+      const double h = g * dc;
+      acc[K - 3] = fma(g, fma(h, R.x, R.c0), acc[K - 3]);
+      acc[K - 2] = fma(g, fma(h, R.y, R.c1), acc[K - 2]);
+      acc[K - 1] = fma(g, fma(h, R.z, R.c2), acc[K - 1]);
+    }
+  };
+  walk_sets<S>(T, targets, wave, [&](const SourceSet& set, int a, int b) {
+    const TgtRec* __restrict__ r = trec + set.first;
+    int k = a;
+    for (; k + 4 <= b; k += 4) {
+      double d[4], g[4];
+      // the forward kernel's denominator, x = target, y = source
+#pragma unroll
+      for (int i = 0; i < 4; ++i) d[i] = one_minus_dot(Y.x, Y.y, Y.z, r[k + i].x, r[k + i].y, r[k + i].z) + eps;
+      rcp4(d, g);
+#pragma unroll
+      for (int i = 0; i < 4; ++i) add(r[k + i], g[i]);
+    }
+    for (; k < b; ++k) add(r[k], rcp64_pair(one_minus_dot(Y.x, Y.y, Y.z, r[k].x, r[k].y, r[k].z) + eps));
+  });
+  tile_sum<S>(acc, wave, lane);
+  if (wave == 0 && lane < T.count)
+    store_row<POS>(t, u, Y, acc, dpart, dprox, qbar_part, qbar_prox, dbar_part, dbar_prox);
+}
+
+// The same in lane copies (lanes.hpp), two source rows per lane: for tiles of at
+// most 42 rows (lanes64), where 36 of 64 lanes held a row.  Step adjoint at
+// 6 x 192^2 (degree 8) 3.08 -> 2.71 ms, 3.21 with a row per lane.
+template <bool POS, int S>
+__global__ __launch_bounds__(64 * S) void k_bve_adj64_lanes(DevTree t, const TargetTile* __restrict__ tiles, int ntiles,
+                                                            const SourceSet* __restrict__ targets,
+                                                            const TgtRec* __restrict__ trec,
+                                                            const SrcRec64* __restrict__ srec, double eps, CPtr3 dpart,
+                                                            CPtr3 dprox, double* __restrict__ qbar_part,
+                                                            double* __restrict__ qbar_prox, Ptr3 dbar_part,
+                                                            Ptr3 dbar_prox) {
+  constexpr int NT = 2, K = POS ? 4 : 1;
+  __shared__ __align__(16) double stage[S][kLaneSlots * 6];
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int lane = threadIdx.x & 63;
+  const int tile = strip_tile(ntiles);
+  if (tile >= ntiles) return;  // the whole workgroup
+  const TargetTile T = tiles[tile];
+  const LaneTile l = lane_tile<NT>(T.count, lane);
+  double x[NT], y[NT], z[NT], w[NT][K];
+#pragma unroll
+  for (int q = 0; q < NT; ++q) {
+    const SrcRec64 Y = srec[(int64_t)T.first + min(q * l.T + l.i, T.count - 1)];
+    x[q] = Y.x; y[q] = Y.y; z[q] = Y.z;
+#pragma unroll
+    for (int k = 0; k < K; ++k) w[q][k] = 0;
+  }
+  v4f* mine = reinterpret_cast<v4f*>(stage[wave]);
+  const TgtRec pad{0, 0, 0, 0, 0, 0};  // denominator 1 + eps, no cotangent
+  lane_pads<3>(mine, 0.f, lane);
+  walk_sets<S>(T, targets, wave, [&](const SourceSet& set, int a, int b) {
+    for (int c = a; c < b; c += kLaneChunk) {
+      // an odd number of trips takes one more, of padding
+      const int cn = min(kLaneChunk, b - c), trips = (cn + l.G - 1) / l.G;
+      lane_stage<3>(mine, reinterpret_cast<const v4f*>(trec + set.first + c), cn, 0.f, lane);
+      const TgtRec* r = reinterpret_cast<const TgtRec*>(mine) + l.g;
+      for (int k = 0; k < trips; k += 2, r += 2 * l.G) {
+        const TgtRec R0 = r[0], R1 = k + 1 < trips ? r[l.G] : pad;
+        double d[4], g[4];
+#pragma unroll
+        for (int q = 0; q < NT; ++q) {
+          d[q] = one_minus_dot(x[q], y[q], z[q], R0.x, R0.y, R0.z) + eps;
+          d[2 + q] = one_minus_dot(x[q], y[q], z[q], R1.x, R1.y, R1.z) + eps;
+        }
+        rcp4(d, g);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          const int q = i & 1;
+          const TgtRec& R = i < 2 ? R0 : R1;
+          const double dc = x[q] * R.c0 + y[q] * R.c1 + z[q] * R.c2;
+          w[q][0] = fma(g[i], dc, w[q][0]);
+          if constexpr (POS) {
+            const double h = g[i] * dc;
+            w[q][K - 3] = fma(g[i], fma(h, R.x, R.c0), w[q][K - 3]);
+            w[q][K - 2] = fma(g[i], fma(h, R.y, R.c1), w[q][K - 2]);
+            w[q][K - 1] = fma(g[i], fma(h, R.z, R.c2), w[q][K - 1]);
+          }
+        }
+      }
+    }
+  });
+  double out[K];
+  lane_sum<NT, K, S>(l, w, stage, wave, lane, out);
+  if (wave > 0 || lane >= T.count) return;
+  const int64_t u = (int64_t)T.first + lane;
+  store_row<POS>(t, u, srec[u], out, dpart, dprox, qbar_part, qbar_prox, dbar_part, dbar_prox);
+}
+
+// FP32 target record: node relative to its panel centre and c = psi cross x,
+// padded to two 16-byte loads.
 struct TgtRec32 {
-  float ax, ay, az, c0, c1, c2;
+  v4f a, c;
 };
 
 __global__ void k_tgt_rec32(DevTree t, CPtr3 psi_part, CPtr3 psi_prox, TgtRec32* __restrict__ rec) {
@@ -143,90 +221,104 @@ __global__ void k_tgt_rec32(DevTree t, CPtr3 psi_part, CPtr3 psi_prox, TgtRec32*
   }
   const double x = t.px[u], y = t.py[u], z = t.pz[u];
   const DevPanel& P = t.panels[panel];
-  rec[u] = TgtRec32{(float)(x - P.cx), (float)(y - P.cy), (float)(z - P.cz), (float)(b * z - d * y),
-                    (float)(d * x - a * z), (float)(a * y - b * x)};
+  rec[u] = TgtRec32{v4f{(float)(x - P.cx), (float)(y - P.cy), (float)(z - P.cz), 0.f},
+                    v4f{(float)(b * z - d * y), (float)(d * x - a * z), (float)(a * y - b * x), 0.f}};
 }
 
 // Transposed pair sums in FP32 (mixed-precision contexts): 1 - x.y as
-// |x - y|^2 / 2 in panel-centred coordinates like the forward mixed kernel,
-// FP32 partial sums per target set flushed into FP64 accumulators, the
-// source-side finish in FP64.
-template <bool POS, bool GR>
-__global__ __launch_bounds__(256) void k_bve_adj32(DevTree t, const TargetTile* __restrict__ tiles, int ntiles,
-                                                   RowGroups gs, const SourceSet* __restrict__ targets,
-                                                   const TgtRec32* __restrict__ trec, const SrcRec64* __restrict__ srec,
-                                                   float eps, CPtr3 dpart, CPtr3 dprox, double* __restrict__ qbar_part,
-                                                   double* __restrict__ qbar_prox, Ptr3 dbar_part, Ptr3 dbar_prox, int xcd) {
-  __shared__ TgtRec32 stage[GR ? kWavesPerBlock : 1][64];
+// |x - y|^2 / 2 in panel-centred coordinates, FP32 partial sums per target set
+// flushed into FP64 accumulators, the source-side finish in FP64.  With
+// x_t = c_t + a_t the position term sum g (c + h x_t), h = g (y . c), is
+// sum g (c + h a_t) + c_t sum g h, the second sum times the panel centre once per
+// set.  Lane copies (lanes.hpp) of two source rows per lane.
+// Bound: FP32 vector issue, 11 instructions and a reciprocal per pair (19 with POS).
+// Step adjoint before (lane groups of one row per lane, bound by their LDS reads)
+// and now: 6 x 28^2 590 -> 277 us, 6 x 64^2 1341 -> 474, 6 x 96^2 994 -> 720, 6 x 192^2
+// 2251 -> 1963, degree 10 at 6 x 256^2 4804 -> 4001.
+template <bool POS, int S>
+__global__ __launch_bounds__(64 * S) void k_bve_adj32(DevTree t, const TargetTile* __restrict__ tiles, int ntiles,
+                                                      const SourceSet* __restrict__ targets,
+                                                      const TgtRec32* __restrict__ trec,
+                                                      const SrcRec64* __restrict__ srec, float eps, CPtr3 dpart,
+                                                      CPtr3 dprox, double* __restrict__ qbar_part,
+                                                      double* __restrict__ qbar_prox, Ptr3 dbar_part, Ptr3 dbar_prox) {
+  constexpr int NT = 2, K = POS ? 4 : 1;
+  __shared__ __align__(16) double stage[S][kLaneSlots * 4];
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  int tile, row0, cg, ci;
-  if (!group_tile<GR>(gs, ntiles, wave, xcd, tile, row0, cg, ci)) return;
+  const int lane = threadIdx.x & 63;
+  const int tile = strip_tile(ntiles);
+  if (tile >= ntiles) return;  // the whole workgroup
   const TargetTile T = tiles[tile];
-  const int row = row0 + ci;
-  const int64_t u = (int64_t)T.first + (row < T.count ? row : T.count - 1);
-  const int ng = GR ? gs.G : 1;
-  const bool copy_ok = !GR || cg < ng;
-  const SrcRec64 S = srec[u];
+  const LaneTile l = lane_tile<NT>(T.count, lane);
   const DevPanel& PS = t.panels[T.panel];
-  const float bx = (float)(S.x - PS.cx), by = (float)(S.y - PS.cy), bz = (float)(S.z - PS.cz);
-  const float yx = (float)S.x, yy = (float)S.y, yz = (float)S.z;
-  double aq = 0, a0 = 0, a1 = 0, a2 = 0;
-  for (int e = T.src_begin; e < T.src_end; ++e) {
-    const SourceSet G = targets[e];
-    const TgtRec32* __restrict__ r = trec + G.first;
-    // source relative to the target panel's centre
-    const float qx = bx - G.ox, qy = by - G.oy, qz = bz - G.oz;
-    float sq = 0.f, s0 = 0.f, s1 = 0.f, s2 = 0.f;
-    for (int c0 = 0; c0 < G.count; c0 += GR ? 64 : G.count) {
-      const int cn = GR ? min(64, G.count - c0) : G.count;
-      if (GR) stage_records(stage[wave], r + c0, cn);
-      const int trips = GR ? (cn + ng - 1) / ng : cn;
-#pragma unroll 4
-      for (int kk = 0; kk < trips; ++kk) {
-        const int k = GR ? kk * ng + cg : kk;
-        if (GR && !(copy_ok && k < cn)) continue;
-        const TgtRec32 R = GR ? stage[wave][k] : r[k];
-        const float d0 = R.ax - qx, d1 = R.ay - qy, d2 = R.az - qz;  // x_t - y_s
-        const float g = __builtin_amdgcn_rcpf(fmaf(0.5f, fmaf(d0, d0, fmaf(d1, d1, d2 * d2)), eps));
-        const float dc = fmaf(yx, R.c0, fmaf(yy, R.c1, yz * R.c2));
-        sq = fmaf(g, dc, sq);
-        if (POS) {
-          const float h = g * dc;
-          s0 = fmaf(g, fmaf(h, d0 + yx, R.c0), s0);
-          s1 = fmaf(g, fmaf(h, d1 + yy, R.c1), s1);
-          s2 = fmaf(g, fmaf(h, d2 + yz, R.c2), s2);
+  float bx[NT], by[NT], bz[NT], yx[NT], yy[NT], yz[NT];
+  double w[NT][K];
+#pragma unroll
+  for (int q = 0; q < NT; ++q) {
+    const SrcRec64 Y = srec[(int64_t)T.first + min(q * l.T + l.i, T.count - 1)];
+    bx[q] = (float)(Y.x - PS.cx); by[q] = (float)(Y.y - PS.cy); bz[q] = (float)(Y.z - PS.cz);
+    yx[q] = (float)Y.x; yy[q] = (float)Y.y; yz[q] = (float)Y.z;
+#pragma unroll
+    for (int k = 0; k < K; ++k) w[q][k] = 0;
+  }
+  v4f* mine = reinterpret_cast<v4f*>(stage[wave]);
+  lane_pads<2>(mine, 4.f, lane);  // padding: a target four radii away without a cotangent
+  walk_sets<S>(T, targets, wave, [&](const SourceSet& set, int a, int b) {
+    float qx[NT], qy[NT], qz[NT], sq[NT], s0[NT], s1[NT], s2[NT], sh[NT];
+#pragma unroll
+    for (int q = 0; q < NT; ++q) {  // source relative to the target panel's centre
+      qx[q] = bx[q] - set.ox; qy[q] = by[q] - set.oy; qz[q] = bz[q] - set.oz;
+      sq[q] = s0[q] = s1[q] = s2[q] = sh[q] = 0.f;
+    }
+    for (int c = a; c < b; c += kLaneChunk) {
+      const int cn = min(kLaneChunk, b - c), trips = (cn + l.G - 1) / l.G;
+      lane_stage<2>(mine, reinterpret_cast<const v4f*>(trec + set.first + c), cn, 4.f, lane);
+      const TgtRec32* r = reinterpret_cast<const TgtRec32*>(mine) + l.g;
+#pragma unroll 2
+      for (int k = 0; k < trips; ++k, r += l.G) {
+        const v4f A = r->a, C = r->c;
+#pragma unroll
+        for (int q = 0; q < NT; ++q) {
+          const float d0 = A.x - qx[q], d1 = A.y - qy[q], d2 = A.z - qz[q];  // x_t - y_s
+          const float g = __builtin_amdgcn_rcpf(fmaf(0.5f, fmaf(d0, d0, fmaf(d1, d1, d2 * d2)), eps));
+          const float dc = fmaf(yx[q], C.x, fmaf(yy[q], C.y, yz[q] * C.z));
+          if constexpr (POS) {
+            const float h = g * dc;
+            sq[q] += h;
+            sh[q] = fmaf(g, h, sh[q]);
+            s0[q] = fmaf(g, fmaf(h, A.x, C.x), s0[q]);
+            s1[q] = fmaf(g, fmaf(h, A.y, C.y), s1[q]);
+            s2[q] = fmaf(g, fmaf(h, A.z, C.z), s2[q]);
+          } else {
+            sq[q] = fmaf(g, dc, sq[q]);
+          }
         }
       }
     }
-    aq += sq;
-    if (POS) {
-      a0 += s0; a1 += s1; a2 += s2;
+    const DevPanel& PT = t.panels[set.panel];
+#pragma unroll
+    for (int q = 0; q < NT; ++q) {
+      w[q][0] += sq[q];
+      if constexpr (POS) {
+        const double hc = sh[q];
+        w[q][K - 3] += fma(hc, PT.cx, (double)s0[q]);
+        w[q][K - 2] += fma(hc, PT.cy, (double)s1[q]);
+        w[q][K - 1] += fma(hc, PT.cz, (double)s2[q]);
+      }
     }
-  }
-  if (GR) {
-    aq = group_sum(aq, gs, ci);
-    if (POS) {
-      a0 = group_sum(a0, gs, ci);
-      a1 = group_sum(a1, gs, ci);
-      a2 = group_sum(a2, gs, ci);
-    }
-  }
-  if (cg != 0 || row >= T.count) return;
-  const bool part = u < t.npart;
-  const int64_t v = part ? u : u - t.npart;
-  (part ? qbar_part : qbar_prox)[v] = kNegInv4Pi * aq;
-  if (POS) {
-    const double w0 = t.px[u] + (part ? dpart.p[0] : dprox.p[0])[v];
-    const double w1 = t.py[u] + (part ? dpart.p[1] : dprox.p[1])[v];
-    const double w2 = t.pz[u] + (part ? dpart.p[2] : dprox.p[2])[v];
-    const double ir = 1.0 / sqrt(w0 * w0 + w1 * w1 + w2 * w2);
-    const double yb0 = S.q * a0, yb1 = S.q * a1, yb2 = S.q * a2;
-    const double yy2 = S.x * yb0 + S.y * yb1 + S.z * yb2;
-    (part ? dbar_part.p[0] : dbar_prox.p[0])[v] = (yb0 - S.x * yy2) * ir;
-    (part ? dbar_part.p[1] : dbar_prox.p[1])[v] = (yb1 - S.y * yy2) * ir;
-    (part ? dbar_part.p[2] : dbar_prox.p[2])[v] = (yb2 - S.z * yy2) * ir;
-  }
+  });
+  double out[K];
+  lane_sum<NT, K, S>(l, w, stage, wave, lane, out);
+  if (wave > 0 || lane >= T.count) return;
+  const int64_t u = (int64_t)T.first + lane;
+  store_row<POS>(t, u, srec[u], out, dpart, dprox, qbar_part, qbar_prox, dbar_part, dbar_prox);
 }
+
+// Waves per tile.  Step adjoint (FP64) with 4 / 8 / 16: 126 tiles 359 / 304 / 285 us,
+// 636 626 / 591 / 627, 2,556 1469 / 1428 / 1697, 8,190 2835 / 2858 / 3531; FP32
+// 126 tiles 307 / 279 / 277, 636 482 / 475 / 526, 2,556 (36 rows) 714 / 745 / 907,
+// 10,236 1919 / 2087 / 2807.
+inline int adj_waves(int ntiles, int many) { return ntiles < 300 ? 16 : ntiles < many ? 8 : 4; }
 
 }  // namespace
 
@@ -242,11 +334,8 @@ void launch_adj_target_records32(const DevTree& t, const double* const* psi_part
 void launch_bve_adjoint32(const DevTree& t, const TargetTile* tiles, int ntiles, const SourceSet* targets,
                           const void* trec, const SrcRec64* srec, double eps, const double* const* dpart,
                           const double* const* dprox, double* qbar_part, double* qbar_prox, double* const* dbar_part,
-                          double* const* dbar_prox, hipStream_t s, PairShape shape) {
+                          double* const* dbar_prox, hipStream_t s) {
   if (ntiles == 0) return;
-  const RowGroups gs = row_groups(t);
-  const bool gr = gs.G > 1;
-  const dim3 grid((unsigned)(((int64_t)ntiles * gs.H + shape.waves - 1) / shape.waves)), block(64 * shape.waves);
   const TgtRec32* r = static_cast<const TgtRec32*>(trec);
   CPtr3 dp{}, dx{};
   Ptr3 bp{}, bx{};
@@ -256,14 +345,11 @@ void launch_bve_adjoint32(const DevTree& t, const TargetTile* tiles, int ntiles,
     bp = Ptr3{{dbar_part[0], dbar_part[1], dbar_part[2]}};
     bx = Ptr3{{dbar_prox[0], dbar_prox[1], dbar_prox[2]}};
   }
-#define SBSLPM_BVE_ADJ(P, G)                                                                                        \
-  hipLaunchKernelGGL((k_bve_adj32<P, G>), grid, block, 0, s, t, tiles, ntiles, gs, targets, r, srec, (float)eps, dp, dx,     \
-                     qbar_part, qbar_prox, bp, bx, shape.xcd)
-  if (dpart && gr) SBSLPM_BVE_ADJ(true, true);
-  else if (dpart) SBSLPM_BVE_ADJ(true, false);
-  else if (gr) SBSLPM_BVE_ADJ(false, true);
-  else SBSLPM_BVE_ADJ(false, false);
-#undef SBSLPM_BVE_ADJ
+  const int S = adj_waves(ntiles, 1500);
+  auto kernel = dpart ? (S == 16 ? k_bve_adj32<true, 16> : S == 8 ? k_bve_adj32<true, 8> : k_bve_adj32<true, 4>)
+                      : (S == 16 ? k_bve_adj32<false, 16> : S == 8 ? k_bve_adj32<false, 8> : k_bve_adj32<false, 4>);
+  hipLaunchKernelGGL(kernel, dim3(strip_grid(ntiles)), dim3(64 * S), 0, s, t, tiles, ntiles, targets, r, srec, (float)eps, dp,
+                     dx, qbar_part, qbar_prox, bp, bx);
 }
 
 void launch_adj_target_records(const DevTree& t, const double* const* psi_part, const double* const* psi_prox,
@@ -276,11 +362,8 @@ void launch_adj_target_records(const DevTree& t, const double* const* psi_part, 
 void launch_bve_adjoint64(const DevTree& t, const TargetTile* tiles, int ntiles, const SourceSet* targets,
                           const void* trec, const SrcRec64* srec, double eps, const double* const* dpart,
                           const double* const* dprox, double* qbar_part, double* qbar_prox, double* const* dbar_part,
-                          double* const* dbar_prox, hipStream_t s, PairShape shape) {
+                          double* const* dbar_prox, hipStream_t s) {
   if (ntiles == 0) return;
-  const RowGroups gs = row_groups(t);
-  const bool gr = gs.G > 1;
-  const dim3 grid((unsigned)(((int64_t)ntiles * gs.H + shape.waves - 1) / shape.waves)), block(64 * shape.waves);
   const TgtRec* r = static_cast<const TgtRec*>(trec);
   CPtr3 dp{}, dx{};
   Ptr3 bp{}, bx{};
@@ -290,14 +373,14 @@ void launch_bve_adjoint64(const DevTree& t, const TargetTile* tiles, int ntiles,
     bp = Ptr3{{dbar_part[0], dbar_part[1], dbar_part[2]}};
     bx = Ptr3{{dbar_prox[0], dbar_prox[1], dbar_prox[2]}};
   }
-#define SBSLPM_BVE_ADJ(P, G)                                                                                        \
-  hipLaunchKernelGGL((k_bve_adj64<P, G>), grid, block, 0, s, t, tiles, ntiles, gs, targets, r, srec, eps, dp, dx,     \
-                     qbar_part, qbar_prox, bp, bx, shape.xcd)
-  if (dpart && gr) SBSLPM_BVE_ADJ(true, true);
-  else if (dpart) SBSLPM_BVE_ADJ(true, false);
-  else if (gr) SBSLPM_BVE_ADJ(false, true);
-  else SBSLPM_BVE_ADJ(false, false);
-#undef SBSLPM_BVE_ADJ
+  const int S = adj_waves(ntiles, 6000);
+  auto kernel = dpart ? (S == 16 ? k_bve_adj64<true, 16> : S == 8 ? k_bve_adj64<true, 8> : k_bve_adj64<true, 4>)
+                      : (S == 16 ? k_bve_adj64<false, 16> : S == 8 ? k_bve_adj64<false, 8> : k_bve_adj64<false, 4>);
+  if (lanes64(t) && S < 16)
+    kernel = dpart ? (S == 8 ? k_bve_adj64_lanes<true, 8> : k_bve_adj64_lanes<true, 4>)
+                   : (S == 8 ? k_bve_adj64_lanes<false, 8> : k_bve_adj64_lanes<false, 4>);
+  hipLaunchKernelGGL(kernel, dim3(strip_grid(ntiles)), dim3(64 * S), 0, s, t, tiles, ntiles, targets, r, srec, eps, dp,
+                     dx, qbar_part, qbar_prox, bp, bx);
 }
 
 }  // namespace sbslpm

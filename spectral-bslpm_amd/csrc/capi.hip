@@ -2422,8 +2422,7 @@ static int fmm_adjoint(sbslpm_ctx* c, const double* area, const double* vor_eff,
   if (pos) launch_zero_rows(c->adj_zero_rows, c->adj_nzero, t.n, 3, c->adj_dbx, c->stream);
   (fp32 ? launch_bve_adjoint32 : launch_bve_adjoint64)(c->dt, c->adj_tiles, c->adj_ntiles, c->adj_targets,
                                                        c->adj_trec, c->adj_srec, c->prm.kernel_eps, dpart, dprox,
-                                                       c->adj_qbp, c->adj_qbx, c->adj_dbp, c->adj_dbx, c->stream,
-                                                       c->shape);
+                                                       c->adj_qbp, c->adj_qbx, c->adj_dbp, c->adj_dbx, c->stream);
   // charges: particle sources directly, proxy sources through P2M/M2M, whose
   // transposes are L2L/L2P
   const double* qbp[1] = {c->adj_qbp};

@@ -19,6 +19,20 @@ constexpr int kLaneChunk = 64;               // records staged at a time, one pe
 constexpr int kLanePad = 16;                 // copies at most, padding of a chunk at most kLanePad - 1
 constexpr int kLaneSlots = kLaneChunk + kLanePad;
 
+// Rows of the fullest tile of a context (a panel's points in equal tiles of at
+// most 64).  The FP64 kernels, bound by issue with scalar records at no LDS
+// cost, take lane copies where those fill more of the wave: with two rows per
+// lane three or more copies of at most 42 rows (36 rows use 54 lanes' worth
+// twice over against 36 of 64).
+inline int tile_rows(const DevTree& t) {
+  auto rows = [](int c) {
+    const int tiles = (c + 63) / 64;
+    return tiles > 0 ? (c + tiles - 1) / tiles : 0;
+  };
+  return rows(t.m2) > rows(t.n) ? rows(t.m2) : rows(t.n);
+}
+inline bool lanes64(const DevTree& t) { return tile_rows(t) <= 42; }
+
 struct LaneTile {
   int T, G, g, i;  // lanes per copy, copies, this lane's copy and lane within it
   bool active;
@@ -35,12 +49,39 @@ __device__ inline LaneTile lane_tile(int count, int lane) {
   return l;
 }
 
+// Stages N 16-byte words of each of the records [0, cn) of `src` from lane to slot,
+// and a record of zeros but for the first float, `first`, in the slots up to 64;
+// slots 64 .. 79 are filled once by lane_pads.  (Word by word: a record selected as
+// a whole is first stored as padding and then again.)
+template <int N>
+__device__ inline void lane_stage(v4f* mine, const v4f* __restrict__ src, int cn, float first, int lane) {
+  __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
+  v4f v[N];
+#pragma unroll
+  for (int i = 0; i < N; ++i) v[i] = v4f{i == 0 ? first : 0.f, 0.f, 0.f, 0.f};
+  if (lane < cn) {
+#pragma unroll
+    for (int i = 0; i < N; ++i) v[i] = src[N * lane + i];
+  }
+#pragma unroll
+  for (int i = 0; i < N; ++i) mine[N * lane + i] = v[i];
+  __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
+}
+template <int N>
+__device__ inline void lane_pads(v4f* mine, float first, int lane) {
+  if (lane < kLanePad)
+#pragma unroll
+    for (int i = 0; i < N; ++i)
+      mine[N * (kLaneChunk + lane) + i] = v4f{i == 0 ? first : 0.f, 0.f, 0.f, 0.f};
+}
+
 // Sums w[t][c] over the copies and the S waves into row t T + i of lane
 // t T + i of wave 0, valid where the lane is below the tile's count; `stage` is
-// each wave's slot of at least 192 doubles (every thread calls it).
-template <int NT, int K, int S>
-__device__ inline void lane_sum(const LaneTile& l, double (&w)[NT][K], double (*stage)[kLaneSlots * 4], int wave,
+// each wave's slot of SLOT >= 64 K doubles (every thread calls it).
+template <int NT, int K, int S, int SLOT>
+__device__ inline void lane_sum(const LaneTile& l, double (&w)[NT][K], double (*stage)[SLOT], int wave,
                                 int lane, double (&out)[K]) {
+  static_assert(SLOT >= 64 * K, "lane_sum: slot too small");
   double* mine = stage[wave];
   double v[NT][K];
 #pragma unroll

@@ -121,3 +121,22 @@ def test_vortex_pairs_mixed(case, displaced, sb):
     off = o.offset
     if np.any([np.any(np.asarray(v)[:off]) for v in ex]):
         assert W.vec_rel_l2([to_np(v)[:off] for v in gx], [np.asarray(v)[:off] for v in ex]) < bound
+
+
+@pytest.mark.parametrize("precision", ["fp64", "mixed"])
+def test_velocity_adjoint_is_the_transpose(case, precision, sb):
+    """<u, K q> = <K^T u, q>: both sides sum the same pairs, so they agree to the rounding of the
+    pair sums (FP64 as above; the FP32 bound of test_vortex_pairs_mixed) times the operands' norms."""
+    cfg = case["ctx"].cfg
+    ctx = sb.Context(sb.RunConfig(levels=cfg.levels, interp_degree=cfg.interp_degree, leaf_degree=cfg.leaf_degree,
+                                  kernel_eps=EPS, weights="clenshaw_curtis", precision=precision))
+    x, y, z, a = case["o"].spec_points()
+    rng = np.random.default_rng(4)
+    q, u = rng.normal(size=x.shape), [rng.normal(size=x.shape) for _ in range(3)]
+    ga = to_gpu(case["t"], a)
+    v = [to_np(w) for w in ctx.bve_velocity(ga, to_gpu(case["t"], q))]
+    qb = to_np(ctx.bve_velocity_adjoint(ga, up(case, u)))
+    lhs, rhs = sum(float(np.sum(p * w)) for p, w in zip(u, v)), float(np.sum(qb * q))
+    size = np.sqrt(sum(np.sum(p * p) for p in u) * sum(np.sum(w * w) for w in v))
+    r = np.sqrt(2) * (np.pi / 4) / 2 ** (cfg.levels - 1)
+    assert abs(lhs - rhs) <= (1e-12 if precision == "fp64" else 2.0 ** -24 * (8 + 2 * r * r / EPS)) * size
