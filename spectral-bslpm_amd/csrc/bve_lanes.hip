@@ -185,7 +185,7 @@ void launch_bve_interact_lanes(const DevTree& t, const TargetTile* tiles, int nt
   if (shape.xcd == 2 && (!t.xcd_start || shape.grid1 <= 0)) shape.xcd = 0;
   // us per launch with 4 / 8 waves: 126 tiles 25 / 20, 636 47 / 46, 2,556 (36 rows) 83 / 87, 10,236 267 / 302,
   // 40,956 1490 / 1562
-  const int S = ntiles < 1000 ? 8 : 4;
+  const int S = lane_waves(ntiles);
   auto kernel = S == 8 ? k_bve_lanes<8> : k_bve_lanes<4>;
   Ptr3 op{{out_part[0], out_part[1], out_part[2]}}, ox{{out_proxy[0], out_proxy[1], out_proxy[2]}};
   hipLaunchKernelGGL(kernel, dim3(walk_grid(ntiles, shape), nmem), dim3(64 * S), 0, s, t, tiles, ntiles, sets,

@@ -19,8 +19,8 @@
 #include <cmath>
 
 #include "device.hpp"
+#include "lanes.hpp"
 #include "lapkernel.hpp"
-#include "pairwalk.hpp"
 
 namespace sbslpm {
 namespace {
@@ -368,13 +368,6 @@ __global__ __launch_bounds__(64 * S) void k_lap64(DevTree t, const TargetTile* _
 // ballot finds a pair with t < 0.6 (elsewhere it is +-1 in FP32 too).  FP32
 // sums per source set; c3 (times -4 pi, undoing the record's -1/(4 pi))
 // applied per set in FP64.
-__device__ inline float lap32_K(float h2, const LapCoef32& kp, float a1v, float b2v) {
-  const float tt = fmaf(h2, -0.5f, 1.0f);
-  const float u = h2 * fmaf(h2, 0.25f * kp.k, -kp.k);
-  const float A = tt * fmaf(a1v, u, kp.a0);
-  const float B = fmaf(fmaf(b2v, u, kp.b1), u, kp.b0);
-  return fmaf(__builtin_amdgcn_exp2f(u), B, A);
-}
 __device__ inline float lap32_K_slow(float h2, const LapCoef32& kp, float a1v, float b2v) {
   const float tt = fmaf(h2, -0.5f, 1.0f);
   const float u = h2 * fmaf(h2, 0.25f * kp.k, -kp.k);
@@ -386,107 +379,81 @@ __device__ inline float lap32_K_slow(float h2, const LapCoef32& kp, float a1v, f
   return tt > kp.cut ? K : 0.0f;
 }
 
-__global__ __launch_bounds__(256) void k_lap_mixed(DevTree t, const TargetTile* __restrict__ tiles, int ntiles,
-                                                   const SourceSet* __restrict__ sets,
-                                                   const SrcRec32* __restrict__ rec, LapCoef32 kp, double c3,
-                                                   double* __restrict__ part, double* __restrict__ proxy,
-                                                   int assign) {
-  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int lane = threadIdx.x & 63;
-  const int tile = xcd_remap(blockIdx.x, gridDim.x) * kWavesPerBlock + wave;
-  if (tile >= ntiles) return;
-  const TargetTile T = tiles[tile];
-  const DevPanel& PT = t.panels[T.panel];
-  const int64_t u = (int64_t)T.first + (lane < T.count ? lane : T.count - 1);
-  const float ax = (float)(t.px[u] - PT.cx), ay = (float)(t.py[u] - PT.cy), az = (float)(t.pz[u] - PT.cz);
-  const bool no_cut = kp.cut < -1.0f;
-  // t < t_sat  <=>  h2 > h_sat
-  const float h_sat = 2.0f * (1.0f - kp.t_sat);
-  const float a1v = in_vgpr_f(kp.a1), b2v = in_vgpr_f(kp.b2);
-  double acc = 0;
-  for (int e = T.src_begin; e < T.src_end; ++e) {
-    const SourceSet S = sets[e];
-    const float px = ax + S.ox, py = ay + S.oy, pz = az + S.oz;
-    const SrcRec32* __restrict__ r = rec + S.first;
-    float v = 0.f;
-    int k = 0;
-    for (; k + 1 < S.count; k += 2) {
-      const SrcRec32 s0 = r[k], s1 = r[k + 1];
-      const float d0 = s0.x - px, d1 = s0.y - py, d2 = s0.z - pz;
-      const float g0 = s1.x - px, g1 = s1.y - py, g2 = s1.z - pz;
-      const float h0 = fmaf(d0, d0, fmaf(d1, d1, d2 * d2));
-      const float h1 = fmaf(g0, g0, fmaf(g1, g1, g2 * g2));
-      float K0 = lap32_K(h0, kp, a1v, b2v), K1 = lap32_K(h1, kp, a1v, b2v);
-      if (!no_cut || (__builtin_amdgcn_ballot_w64(h0 > h_sat) | __builtin_amdgcn_ballot_w64(h1 > h_sat)) != 0) {
-        // a real branch (the empty asm keeps the compiler from evaluating erf on every pair)
-        __asm__ volatile("");
-        K0 = lap32_K_slow(h0, kp, a1v, b2v);
-        K1 = lap32_K_slow(h1, kp, a1v, b2v);
-      }
-      v = fmaf(K0, s0.q, v);
-      v = fmaf(K1, s1.q, v);
-    }
-    if (k < S.count) {
-      const SrcRec32 s0 = r[k];
-      const float d0 = s0.x - px, d1 = s0.y - py, d2 = s0.z - pz;
-      v = fmaf(lap32_K_slow(fmaf(d0, d0, fmaf(d1, d1, d2 * d2)), kp, a1v, b2v), s0.q, v);
-    }
-    acc += c3 * (double)v;
-  }
-  if (lane < T.count) store_s(t, u, part, proxy, acc, assign);
-}
-
-// k_lap_mixed in lane groups (RowGroups): each 36-row tile at m = 6 runs as two
-// 18-row sub-tiles in three copies per wave, every copy taking every third
-// source of a set from records staged in LDS; one pair per iteration behind the
-// same wave-wide ballot for the erf form.
-__global__ __launch_bounds__(256) void k_lap_mixed_gr(DevTree t, const TargetTile* __restrict__ tiles, int ntiles,
-                                                      RowGroups gs, const SourceSet* __restrict__ sets,
+// Lane copies (lanes.hpp) of two targets.
+// Bound: FP32 vector issue, 16 instructions and a base-2 exponential per pair.
+// Microseconds per launch before and with 2 / 4 / 8 waves per tile: 126 tiles 217,
+// 162 / 88 / 56; 636 352, 153 / 97 / 90; 2,556 (36 rows) 202, 148 / 123 / 124; 10,236
+// 502, 356 / 345 / 363; 40,956 2522, 2073 / 2032 / 2068.
+template <int S>
+__global__ __launch_bounds__(64 * S) void k_lap_lanes(DevTree t, const TargetTile* __restrict__ tiles, int ntiles,
+                                                      const SourceSet* __restrict__ sets,
                                                       const SrcRec32* __restrict__ rec, LapCoef32 kp, double c3,
                                                       double* __restrict__ part, double* __restrict__ proxy,
                                                       int assign) {
-  __shared__ SrcRec32 stage[kWavesPerBlock][64];
+  constexpr int NT = 2;
+  __shared__ __align__(16) double stage[S][kLaneSlots * 2];
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  int tile, row0, cg, ci;
-  if (!group_tile<true>(gs, ntiles, wave, 1, tile, row0, cg, ci)) return;
+  const int lane = threadIdx.x & 63;
+  const int tile = strip_tile(ntiles);
+  if (tile >= ntiles) return;  // the whole workgroup
   const TargetTile T = tiles[tile];
   const DevPanel& PT = t.panels[T.panel];
-  const int row = row0 + ci;
-  const int64_t u = (int64_t)T.first + (row < T.count ? row : T.count - 1);
-  const bool copy_ok = cg < gs.G;
-  const float ax = (float)(t.px[u] - PT.cx), ay = (float)(t.py[u] - PT.cy), az = (float)(t.pz[u] - PT.cz);
-  const bool no_cut = kp.cut < -1.0f;
-  const float h_sat = 2.0f * (1.0f - kp.t_sat);
-  const float a1v = in_vgpr_f(kp.a1), b2v = in_vgpr_f(kp.b2);
-  double acc = 0;
-  for (int e = T.src_begin; e < T.src_end; ++e) {
-    const SourceSet S = sets[e];
-    const float px = ax + S.ox, py = ay + S.oy, pz = az + S.oz;
-    const SrcRec32* __restrict__ r = rec + S.first;
-    float v = 0.f;
-    for (int c0 = 0; c0 < S.count; c0 += 64) {
-      const int cn = min(64, S.count - c0);
-      stage_records(stage[wave], r + c0, cn);
-      const int trips = (cn + gs.G - 1) / gs.G;
-      for (int kk = 0; kk < trips; ++kk) {
-        const int k = kk * gs.G + cg;
-        if (!(copy_ok && k < cn)) continue;
-        const SrcRec32 s0 = stage[wave][k];
-        const float d0 = s0.x - px, d1 = s0.y - py, d2 = s0.z - pz;
-        const float h0 = fmaf(d0, d0, fmaf(d1, d1, d2 * d2));
-        float K0 = lap32_K(h0, kp, a1v, b2v);
-        if (!no_cut || __builtin_amdgcn_ballot_w64(h0 > h_sat) != 0) {
+  const LaneTile l = lane_tile<NT>(T.count, lane);
+  // t < t_sat  <=>  h2 > h_sat; every pair passes the cut when 1 - 30 eps < -1 (eps = 0.1), else every pair is slow
+  const float h_sat = kp.cut < -1.0f ? 2.0f * (1.0f - kp.t_sat) : -1.0f;
+  LapCoef32 kv = kp;  // the fast form's coefficients in vector registers
+  kv.a1 = in_vgpr_f(kp.a1); kv.a0 = in_vgpr_f(kp.a0);
+  kv.b2 = in_vgpr_f(kp.b2); kv.b1 = in_vgpr_f(kp.b1); kv.b0 = in_vgpr_f(kp.b0);
+  const float k4 = in_vgpr_f(0.25f * kp.k), km = in_vgpr_f(-kp.k);
+  float ax[NT], ay[NT], az[NT], px[NT], py[NT], pz[NT], v[NT];
+  double w[NT][1];
+#pragma unroll
+  for (int q = 0; q < NT; ++q) {
+    const int64_t u = (int64_t)T.first + min(q * l.T + l.i, T.count - 1);
+    ax[q] = (float)(t.px[u] - PT.cx);
+    ay[q] = (float)(t.py[u] - PT.cy);
+    az[q] = (float)(t.pz[u] - PT.cz);
+    w[q][0] = 0;
+  }
+  lane_walk<S, 1, 1>(
+      T, sets, reinterpret_cast<const v4f*>(rec), l, reinterpret_cast<v4f*>(stage[wave]), 0.f, wave, lane,
+      [&](const SourceSet& set) {
+#pragma unroll
+        for (int q = 0; q < NT; ++q) {
+          px[q] = ax[q] + set.ox;
+          py[q] = ay[q] + set.oy;
+          pz[q] = az[q] + set.oz;
+          v[q] = 0.f;
+        }
+      },
+      [&](const v4f* r) {
+        const v4f s = r[0];
+        float h2[NT], K[NT];
+#pragma unroll
+        for (int q = 0; q < NT; ++q) {
+          const float d0 = s.x - px[q], d1 = s.y - py[q], d2 = s.z - pz[q];
+          h2[q] = fmaf(d0, d0, fmaf(d1, d1, d2 * d2));
+          const float u = h2[q] * fmaf(h2[q], k4, km);
+          const float A = fmaf(h2[q], -0.5f, 1.0f) * fmaf(kv.a1, u, kv.a0);
+          const float B = fmaf(fmaf(kv.b2, u, kv.b1), u, kv.b0);
+          K[q] = fmaf(__builtin_amdgcn_exp2f(u), B, A);
+        }
+        if (__builtin_amdgcn_ballot_w64(fmaxf(h2[0], h2[1]) > h_sat) != 0) {
           // a real branch (the empty asm keeps the compiler from evaluating erf on every pair)
           __asm__ volatile("");
-          K0 = lap32_K_slow(h0, kp, a1v, b2v);
+#pragma unroll
+          for (int q = 0; q < NT; ++q) K[q] = lap32_K_slow(h2[q], kp, kp.a1, kp.b2);
         }
-        v = fmaf(K0, s0.q, v);
-      }
-    }
-    acc += c3 * (double)v;
-  }
-  acc = group_sum(acc, gs, ci);
-  if (cg == 0 && row < T.count) store_s(t, u, part, proxy, acc, assign);
+#pragma unroll
+        for (int q = 0; q < NT; ++q) v[q] = fmaf(K[q], s.w, v[q]);
+      },
+      [&](const SourceSet&) {
+#pragma unroll
+        for (int q = 0; q < NT; ++q) w[q][0] += c3 * (double)v[q];
+      });
+  double s[1];
+  lane_sum<NT, 1, S>(l, w, stage, wave, lane, s);
+  if (wave == 0 && lane < T.count) store_s(t, (int64_t)T.first + lane, part, proxy, s[0], assign);
 }
 
 // Mixed precision Biot-Savart: FP32 pair arithmetic in panel-centred
@@ -533,38 +500,65 @@ __global__ __launch_bounds__(256) void k_bve_mixed(DevTree t, const TargetTile* 
 // pair takes the hardware base-2 logarithm (v_log_f32; h >= 1e-15 is far from
 // the denormal range, so the library's range scaling is not needed) and the
 // factor ln 2 is applied once per source set in FP64.
-__global__ __launch_bounds__(256) void k_log_mixed(DevTree t, const TargetTile* __restrict__ tiles, int ntiles,
-                                                   const SourceSet* __restrict__ sets,
-                                                   const SrcRec32* __restrict__ rec, double* __restrict__ part,
-                                                   double* __restrict__ proxy, int assign) {
+// Lane copies (lanes.hpp) of two targets.
+// Bound: FP32 vector issue, 10 instructions and a logarithm per pair.
+// Microseconds per launch before and with 2 / 4 / 8 waves per tile: 126 tiles 125,
+// 40 / 23 / 18; 636 202, 77 / 47 / 45; 2,556 (36 rows) 203, 89 / 78 / 81; 10,236 510,
+// 258 / 258 / 270; 40,956 2039, 1537 / 1531 / 1565.
+template <int S>
+__global__ __launch_bounds__(64 * S) void k_log_lanes(DevTree t, const TargetTile* __restrict__ tiles, int ntiles,
+                                                      const SourceSet* __restrict__ sets,
+                                                      const SrcRec32* __restrict__ rec, double* __restrict__ part,
+                                                      double* __restrict__ proxy, int assign) {
+  constexpr int NT = 2;
+  __shared__ __align__(16) double stage[S][kLaneSlots * 2];
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int lane = threadIdx.x & 63;
-  const int tile = xcd_remap(blockIdx.x, gridDim.x) * kWavesPerBlock + wave;
-  if (tile >= ntiles) return;
+  const int tile = strip_tile(ntiles);
+  if (tile >= ntiles) return;  // the whole workgroup
   const TargetTile T = tiles[tile];
   const DevPanel& PT = t.panels[T.panel];
-  const int64_t u = (int64_t)T.first + (lane < T.count ? lane : T.count - 1);
-  const float ax = (float)(t.px[u] - PT.cx), ay = (float)(t.py[u] - PT.cy), az = (float)(t.pz[u] - PT.cz);
-  double acc = 0;
-  for (int e = T.src_begin; e < T.src_end; ++e) {
-    const SourceSet S = sets[e];
-    const float px = ax + S.ox, py = ay + S.oy, pz = az + S.oz;
-    const SrcRec32* __restrict__ r = rec + S.first;
-    float v = 0.f;
-#pragma unroll 4
-    for (int k = 0; k < S.count; ++k) {
-      const SrcRec32 s = r[k];
-      const float d0 = s.x - px, d1 = s.y - py, d2 = s.z - pz;
-      const float h = 0.5f * fmaf(d0, d0, fmaf(d1, d1, d2 * d2));
-      const float l2 = __builtin_amdgcn_logf(h);
-      v += (h > 1e-15f) ? l2 * s.q : 0.f;
-    }
-    acc += 0.69314718055994530942 * (double)v;
+  const LaneTile l = lane_tile<NT>(T.count, lane);
+  float ax[NT], ay[NT], az[NT], px[NT], py[NT], pz[NT], v[NT];
+  double w[NT][1];
+#pragma unroll
+  for (int q = 0; q < NT; ++q) {
+    const int64_t u = (int64_t)T.first + min(q * l.T + l.i, T.count - 1);
+    ax[q] = (float)(t.px[u] - PT.cx);
+    ay[q] = (float)(t.py[u] - PT.cy);
+    az[q] = (float)(t.pz[u] - PT.cz);
+    w[q][0] = 0;
   }
-  if (lane < T.count) store_s(t, u, part, proxy, acc, assign);
+  lane_walk<S, 1, 2>(
+      T, sets, reinterpret_cast<const v4f*>(rec), l, reinterpret_cast<v4f*>(stage[wave]), 4.f, wave, lane,
+      [&](const SourceSet& set) {
+#pragma unroll
+        for (int q = 0; q < NT; ++q) {
+          px[q] = ax[q] + set.ox;
+          py[q] = ay[q] + set.oy;
+          pz[q] = az[q] + set.oz;
+          v[q] = 0.f;
+        }
+      },
+      [&](const v4f* r) {
+        const v4f s = r[0];
+#pragma unroll
+        for (int q = 0; q < NT; ++q) {
+          const float d0 = s.x - px[q], d1 = s.y - py[q], d2 = s.z - pz[q];
+          const float h = 0.5f * fmaf(d0, d0, fmaf(d1, d1, d2 * d2));
+          const float l2 = __builtin_amdgcn_logf(h);
+          v[q] = fmaf(h > 1e-15f ? l2 : 0.f, s.w, v[q]);
+        }
+      },
+      [&](const SourceSet&) {
+#pragma unroll
+        for (int q = 0; q < NT; ++q) w[q][0] += 0.69314718055994530942 * (double)v[q];
+      });
+  double s[1];
+  lane_sum<NT, 1, S>(l, w, stage, wave, lane, s);
+  if (wave == 0 && lane < T.count) store_s(t, (int64_t)T.first + lane, part, proxy, s[0], assign);
 }
 
-typedef float v4f __attribute__((ext_vector_type(4)));
 typedef __bf16 v4bf __attribute__((ext_vector_type(4)));
 
 // The kernel products of NTT 16 x 16 tiles, D_ij = beta_i - p_j.b_i: FP32
@@ -1076,14 +1070,9 @@ void launch_laplacian_interact_mixed(const DevTree& t, const TargetTile* tiles, 
   if (ntiles == 0) return;
   const double eps = 0.1, pi = 3.14159265358979323846;
   const double c3 = -4.0 * pi / std::pow(eps, 2.5);
-  const RowGroups gs = row_groups(t);
-  if (gs.G > 1)
-    hipLaunchKernelGGL(k_lap_mixed_gr, dim3(blocks_for((int64_t)ntiles * gs.H, kWavesPerBlock)),
-                       dim3(64 * kWavesPerBlock), 0, s, t, tiles, ntiles, gs, sets, rec, lap_coef32(eps, 1.0), c3,
-                       out_part, out_proxy, assign ? 1 : 0);
-  else
-    hipLaunchKernelGGL(k_lap_mixed, dim3(blocks_for(ntiles, kWavesPerBlock)), dim3(64 * kWavesPerBlock), 0, s, t,
-                       tiles, ntiles, sets, rec, lap_coef32(eps, 1.0), c3, out_part, out_proxy, assign ? 1 : 0);
+  const int S = lane_waves(ntiles);
+  hipLaunchKernelGGL(S == 8 ? k_lap_lanes<8> : k_lap_lanes<4>, dim3(strip_grid(ntiles)), dim3(64 * S), 0, s, t, tiles, ntiles, sets, rec,
+                     lap_coef32(eps, 1.0), c3, out_part, out_proxy, assign ? 1 : 0);
 }
 
 void launch_bve_interact_mixed(const DevTree& t, const TargetTile* tiles, int ntiles, const SourceSet* sets,
@@ -1139,8 +1128,9 @@ void launch_poisson_interact_mixed(const DevTree& t, const TargetTile* tiles, in
                                    const SrcRec32* rec, double* out_part, double* out_proxy, hipStream_t s,
                                    bool assign) {
   if (ntiles == 0) return;
-  hipLaunchKernelGGL(k_log_mixed, dim3(blocks_for(ntiles, kWavesPerBlock)), dim3(64 * kWavesPerBlock), 0, s, t,
-                     tiles, ntiles, sets, rec, out_part, out_proxy, assign ? 1 : 0);
+  const int S = lane_waves(ntiles);
+  hipLaunchKernelGGL(S == 8 ? k_log_lanes<8> : k_log_lanes<4>, dim3(strip_grid(ntiles)), dim3(64 * S), 0, s, t, tiles, ntiles, sets, rec, out_part,
+                     out_proxy, assign ? 1 : 0);
 }
 
 }  // namespace sbslpm

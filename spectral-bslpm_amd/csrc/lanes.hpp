@@ -75,6 +75,30 @@ __device__ inline void lane_pads(v4f* mine, float first, int lane) {
       mine[N * (kLaneChunk + lane) + i] = v4f{i == 0 ? first : 0.f, 0.f, 0.f, 0.f};
 }
 
+// Waves per tile of the lane-copy kernels (their tables of times stand beside them).
+inline int lane_waves(int ntiles) { return ntiles < 1000 ? 8 : 4; }
+
+// Walks a wave's share of the source sets of a tile: begin(set) and flush(set)
+// around each part of a set, add(r) for each trip, r the lane's record (N 16-byte
+// words) in LDS; `first` as in lane_stage.
+template <int S, int N, int UNROLL, typename Begin, typename Add, typename Flush>
+__device__ inline void lane_walk(const TargetTile& T, const SourceSet* __restrict__ sets, const v4f* __restrict__ rec,
+                                 const LaneTile& l, v4f* mine, float first, int wave, int lane, Begin&& begin,
+                                 Add&& add, Flush&& flush) {
+  lane_pads<N>(mine, first, lane);
+  walk_sets<S>(T, sets, wave, [&](const SourceSet& set, int a, int b) {
+    begin(set);
+    for (int c = a; c < b; c += kLaneChunk) {
+      const int cn = min(kLaneChunk, b - c), trips = (cn + l.G - 1) / l.G;
+      lane_stage<N>(mine, rec + N * ((int64_t)set.first + c), cn, first, lane);
+      const v4f* r = mine + N * l.g;
+#pragma unroll UNROLL
+      for (int k = 0; k < trips; ++k, r += N * l.G) add(r);
+    }
+    flush(set);
+  });
+}
+
 // Sums w[t][c] over the copies and the S waves into row t T + i of lane
 // t T + i of wave 0, valid where the lane is below the tile's count; `stage` is
 // each wave's slot of SLOT >= 64 K doubles (every thread calls it).

@@ -14,7 +14,7 @@
 // (y' = y or y0) and forms u = x cross W + D - x S once per target, the same
 // sums regrouped.
 #include "device.hpp"
-#include "pairwalk.hpp"
+#include "lanes.hpp"
 
 namespace sbslpm {
 namespace {
@@ -154,80 +154,85 @@ __global__ void k_src_swe32(DevTree t, const double* __restrict__ qz_part, const
 
 // Mixed-precision shallow-water pairs (variants 1 and 3): with d = y - x and
 // h = |d|^2 / 2 = 1 - x.y computed in FP32 from panel-centred coordinates,
-// x cross y = x cross d and y - x (x.y) = d + x h, so
-//   u = x cross sum(g qz d) + sum(g qd d) + x sum(g qd h),   g = 1/(h + eps).
-// FP32 partial sums per source set are added into FP64; the cross product and
-// the output are FP64.
-template <bool GR>
-__global__ __launch_bounds__(256) void k_swe_mixed(DevTree t, const TargetTile* __restrict__ tiles, int ntiles,
-                                                   RowGroups gs, const SourceSet* __restrict__ sets,
-                                                   const SrcRecSwe32* __restrict__ rec, float eps, Ptr3 part,
-                                                   Ptr3 proxy, int assign) {
-  __shared__ SrcRecSwe32 stage[GR ? kWavesPerBlock : 1][64];
+// x cross y = x cross d and y - x (x.y) = d - x (x.d), so
+//   u = x cross sum(g qz d) + E - x (x.E),   E = sum(g qd d),   g = 1/(h + eps).
+// FP32 partial sums per source set are added into FP64; the cross product, the
+// projection and the output are FP64.  Lane copies (lanes.hpp) of two targets.
+// Bound: FP32 vector issue, 15 instructions and a reciprocal per pair.
+// Microseconds per launch before (one wave per tile with scalar records, or lane
+// groups of one target) and with 2 / 4 / 8 waves per tile: 126 tiles 115, 53 / 32 /
+// 25; 636 380, 106 / 67 / 65; 2,556 (36 rows) 187, 130 / 117 / 123; 10,236 543, 387 /
+// 390 / 432; 40,956 2931, 2268 / 2231 / 2318.
+template <int S>
+__global__ __launch_bounds__(64 * S) void k_swe_lanes(DevTree t, const TargetTile* __restrict__ tiles, int ntiles,
+                                                      const SourceSet* __restrict__ sets,
+                                                      const SrcRecSwe32* __restrict__ rec, float eps, Ptr3 part,
+                                                      Ptr3 proxy, int assign) {
+  constexpr int NT = 2, K = 6;
+  __shared__ __align__(16) double stage[S][64 * K];
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  int tile, row0, cg, ci;
-  if (!group_tile<GR>(gs, ntiles, wave, 1, tile, row0, cg, ci)) return;
+  const int lane = threadIdx.x & 63;
+  const int tile = strip_tile(ntiles);
+  if (tile >= ntiles) return;  // the whole workgroup
   const TargetTile T = tiles[tile];
   const DevPanel& PT = t.panels[T.panel];
-  const int row = row0 + ci;
-  const int64_t u = (int64_t)T.first + (row < T.count ? row : T.count - 1);
-  const int ng = GR ? gs.G : 1;
-  const bool copy_ok = !GR || cg < ng;
-  const double x = t.px[u], y = t.py[u], z = t.pz[u];
-  const float ax = (float)(x - PT.cx), ay = (float)(y - PT.cy), az = (float)(z - PT.cz);
-  double w0 = 0, w1 = 0, w2 = 0, d0 = 0, d1 = 0, d2 = 0, sd = 0;
-  for (int e = T.src_begin; e < T.src_end; ++e) {
-    const SourceSet S = sets[e];
-    const float px = ax + S.ox, py = ay + S.oy, pz = az + S.oz;
-    const SrcRecSwe32* __restrict__ r = rec + S.first;
-    float v0 = 0.f, v1 = 0.f, v2 = 0.f, e0 = 0.f, e1 = 0.f, e2 = 0.f, eh = 0.f;
-    for (int c0 = 0; c0 < S.count; c0 += GR ? 64 : S.count) {
-      const int cn = GR ? min(64, S.count - c0) : S.count;
-      if (GR) stage_records(stage[wave], r + c0, cn);
-      const int trips = GR ? (cn + ng - 1) / ng : cn;
-#pragma unroll 4
-      for (int kk = 0; kk < trips; ++kk) {
-        const int k = GR ? kk * ng + cg : kk;
-        if (GR && !(copy_ok && k < cn)) continue;
-        const SrcRecSwe32 s = GR ? stage[wave][k] : r[k];
-        const float c0f = s.x - px, c1f = s.y - py, c2f = s.z - pz;
-        const float h = 0.5f * fmaf(c0f, c0f, fmaf(c1f, c1f, c2f * c2f));
-        const float g = __builtin_amdgcn_rcpf(h + eps);
-        const float gz = g * s.qz, gd = g * s.qd;
-        v0 = fmaf(gz, c0f, v0);
-        v1 = fmaf(gz, c1f, v1);
-        v2 = fmaf(gz, c2f, v2);
-        e0 = fmaf(gd, c0f, e0);
-        e1 = fmaf(gd, c1f, e1);
-        e2 = fmaf(gd, c2f, e2);
-        eh = fmaf(gd, h, eh);
-      }
-    }
-    w0 += v0; w1 += v1; w2 += v2;
-    d0 += e0; d1 += e1; d2 += e2;
-    sd += eh;
+  const LaneTile l = lane_tile<NT>(T.count, lane);
+  float ax[NT], ay[NT], az[NT], px[NT], py[NT], pz[NT], v[NT][K];
+  double w[NT][K];
+#pragma unroll
+  for (int q = 0; q < NT; ++q) {
+    const int64_t u = (int64_t)T.first + min(q * l.T + l.i, T.count - 1);
+    ax[q] = (float)(t.px[u] - PT.cx);
+    ay[q] = (float)(t.py[u] - PT.cy);
+    az[q] = (float)(t.pz[u] - PT.cz);
+#pragma unroll
+    for (int k = 0; k < K; ++k) w[q][k] = 0;
   }
-  if (GR) {
-    w0 = group_sum(w0, gs, ci); w1 = group_sum(w1, gs, ci); w2 = group_sum(w2, gs, ci);
-    d0 = group_sum(d0, gs, ci); d1 = group_sum(d1, gs, ci); d2 = group_sum(d2, gs, ci);
-    sd = group_sum(sd, gs, ci);
-  }
-  if (cg != 0 || row >= T.count) return;
-  const double a = (y * w2 - z * w1) + (d0 + x * sd);
-  const double b = (z * w0 - x * w2) + (d1 + y * sd);
-  const double c = (x * w1 - y * w0) + (d2 + z * sd);
-  double* o[3];
-  int64_t v = u;
-  if (u < t.npart) {
-    o[0] = part.p[0]; o[1] = part.p[1]; o[2] = part.p[2];
-  } else {
-    v = u - t.npart;
-    o[0] = proxy.p[0]; o[1] = proxy.p[1]; o[2] = proxy.p[2];
-  }
-  if (assign) {
-    o[0][v] = a; o[1][v] = b; o[2][v] = c;
-  } else {
-    o[0][v] += a; o[1][v] += b; o[2][v] += c;
+  lane_walk<S, 2, 2>(
+      T, sets, reinterpret_cast<const v4f*>(rec), l, reinterpret_cast<v4f*>(stage[wave]), 4.f, wave, lane,
+      [&](const SourceSet& set) {
+#pragma unroll
+        for (int q = 0; q < NT; ++q) {
+          px[q] = ax[q] + set.ox;
+          py[q] = ay[q] + set.oy;
+          pz[q] = az[q] + set.oz;
+#pragma unroll
+          for (int k = 0; k < K; ++k) v[q][k] = 0.f;
+        }
+      },
+      [&](const v4f* r) {
+        const v4f s = r[0];
+        const float qd = r[1].x;
+#pragma unroll
+        for (int q = 0; q < NT; ++q) {
+          const float d0 = s.x - px[q], d1 = s.y - py[q], d2 = s.z - pz[q];
+          const float g = __builtin_amdgcn_rcpf(fmaf(0.5f, fmaf(d0, d0, fmaf(d1, d1, d2 * d2)), eps));
+          const float gz = g * s.w, gd = g * qd;
+          v[q][0] = fmaf(gz, d0, v[q][0]);
+          v[q][1] = fmaf(gz, d1, v[q][1]);
+          v[q][2] = fmaf(gz, d2, v[q][2]);
+          v[q][3] = fmaf(gd, d0, v[q][3]);
+          v[q][4] = fmaf(gd, d1, v[q][4]);
+          v[q][5] = fmaf(gd, d2, v[q][5]);
+        }
+      },
+      [&](const SourceSet&) {
+#pragma unroll
+        for (int q = 0; q < NT; ++q)
+#pragma unroll
+          for (int k = 0; k < K; ++k) w[q][k] += v[q][k];
+      });
+  double s[K];
+  lane_sum<NT, K, S>(l, w, stage, wave, lane, s);
+  if (wave > 0 || lane >= T.count) return;
+  const int64_t u = (int64_t)T.first + lane;
+  const double x = t.px[u], y = t.py[u], z = t.pz[u], sd = x * s[3] + y * s[4] + z * s[5];
+  const double o[3] = {(y * s[2] - z * s[1]) + (s[3] - x * sd), (z * s[0] - x * s[2]) + (s[4] - y * sd),
+                       (x * s[1] - y * s[0]) + (s[5] - z * sd)};
+#pragma unroll
+  for (int c = 0; c < 3; ++c) {
+    double* p = u < t.npart ? part.p[c] + u : proxy.p[c] + (u - t.npart);
+    *p = assign ? o[c] : *p + o[c];
   }
 }
 
@@ -255,15 +260,9 @@ void launch_swe_interact_mixed(const DevTree& t, const TargetTile* tiles, int nt
     op.p[f] = out_part[f];
     ox.p[f] = out_proxy[f];
   }
-  const unsigned blocks = (unsigned)((ntiles + kWavesPerBlock - 1) / kWavesPerBlock);
-  const RowGroups gs = row_groups(t);
-  if (gs.G > 1)
-    hipLaunchKernelGGL(k_swe_mixed<true>, dim3((((int64_t)ntiles * gs.H + kWavesPerBlock - 1) / kWavesPerBlock)),
-                       dim3(64 * kWavesPerBlock), 0, s, t, tiles, ntiles, gs, sets, rec, (float)eps, op, ox,
-                       assign ? 1 : 0);
-  else
-    hipLaunchKernelGGL(k_swe_mixed<false>, dim3(blocks), dim3(64 * kWavesPerBlock), 0, s, t, tiles, ntiles, gs, sets,
-                       rec, (float)eps, op, ox, assign ? 1 : 0);
+  const int S = lane_waves(ntiles);
+  hipLaunchKernelGGL(S == 8 ? k_swe_lanes<8> : k_swe_lanes<4>, dim3(strip_grid(ntiles)), dim3(64 * S), 0, s, t, tiles, ntiles, sets, rec, (float)eps, op,
+                     ox, assign ? 1 : 0);
 }
 
 void launch_source_records_swe(const DevTree& t, int variant, const double* qz_part, const double* qz_proxy,

@@ -140,3 +140,33 @@ def test_velocity_adjoint_is_the_transpose(case, precision, sb):
     size = np.sqrt(sum(np.sum(p * p) for p in u) * sum(np.sum(w * w) for w in v))
     r = np.sqrt(2) * (np.pi / 4) / 2 ** (cfg.levels - 1)
     assert abs(lhs - rhs) <= (1e-12 if precision == "fp64" else 2.0 ** -24 * (8 + 2 * r * r / EPS)) * size
+
+
+@pytest.mark.parametrize("displaced", [False, True])
+def test_other_pairs_mixed(case, displaced, sb):
+    """The FP32 shallow-water, regularised-Laplacian and log pairs in lane copies against the FP64
+    kernels (above against the oracle).  Per pair: the shallow-water bound of
+    test_vortex_pairs_mixed; the Laplacian's base-2 exponent, up to 2 / (0.1 ln 2) = 29, is off by
+    half an ulp of itself, under 64 x 2^-24 with its polynomials; the logarithm by an ulp of up to
+    -16 and 2 r^2 2^-24 over the nearest squared distance, of pairs that count as 1/N."""
+    cfg, W = case["ctx"].cfg, case["W"]
+    kw = dict(levels=cfg.levels, interp_degree=cfg.interp_degree, leaf_degree=cfg.leaf_degree, kernel_eps=EPS,
+              weights="clenshaw_curtis")
+    c64, c32 = case["ctx"], sb.Context(sb.RunConfig(precision="mixed", **kw))
+    x, y, z, a = case["o"].spec_points()
+    q = up(case, case["o"].upward_pass(a, W.gaussian_vortices(x, y, z, a, seed=3)))
+    p = up(case, case["o"].upward_pass(a, W.gaussian_vortices(x, y, z, a, seed=4)))
+    dp, dx = (up(case, case["dp"]), up(case, case["dx"])) if displaced else (None, None)
+    r = np.sqrt(2) * (np.pi / 4) / 2 ** (cfg.levels - 1)
+    off = case["o"].offset
+    calls = [(lambda c: c.swe_vel_interactions(*q, *p, dp, dx), 8 + 2 * r * r / EPS),
+             (lambda c: c.laplacian_interactions(*q, dp, dx), 64)]
+    if not displaced:
+        calls.append((lambda c: c.poisson_fmm_interactions(*q), 64))
+    for call, bound in calls:
+        (ep, ex), (gp, gx) = call(c64), call(c32)
+        flat = lambda part, proxy: np.concatenate([to_np(v).ravel() for v in (part if isinstance(part, list) else [part])]
+                                                  + [to_np(v)[:off].ravel() for v in
+                                                     (proxy if isinstance(proxy, list) else [proxy])])
+        e, g = flat(ep, ex), flat(gp, gx)
+        assert np.linalg.norm(g - e) <= 2.0 ** -24 * bound * np.linalg.norm(e)
