@@ -158,37 +158,27 @@ __global__ __launch_bounds__(64 * S) void k_bve_adj64_lanes(DevTree t, const Tar
 #pragma unroll
     for (int k = 0; k < K; ++k) w[q][k] = 0;
   }
-  v4f* mine = reinterpret_cast<v4f*>(stage[wave]);
-  const TgtRec pad{0, 0, 0, 0, 0, 0};  // denominator 1 + eps, no cotangent
-  lane_pads<3>(mine, 0.f, lane);
-  walk_sets<S>(T, targets, wave, [&](const SourceSet& set, int a, int b) {
-    for (int c = a; c < b; c += kLaneChunk) {
-      // an odd number of trips takes one more, of padding
-      const int cn = min(kLaneChunk, b - c), trips = (cn + l.G - 1) / l.G;
-      lane_stage<3>(mine, reinterpret_cast<const v4f*>(trec + set.first + c), cn, 0.f, lane);
-      const TgtRec* r = reinterpret_cast<const TgtRec*>(mine) + l.g;
-      for (int k = 0; k < trips; k += 2, r += 2 * l.G) {
-        const TgtRec R0 = r[0], R1 = k + 1 < trips ? r[l.G] : pad;
-        double d[4], g[4];
+  lane_walk2<S, 3>(T, targets, reinterpret_cast<const v4f*>(trec), l, reinterpret_cast<v4f*>(stage[wave]), wave, lane,
+                   [&](const v4f* r0, const v4f* r1) {
+    const TgtRec R[2] = {*reinterpret_cast<const TgtRec*>(r0), *reinterpret_cast<const TgtRec*>(r1)};
+    double d[4], g[4];
 #pragma unroll
-        for (int q = 0; q < NT; ++q) {
-          d[q] = one_minus_dot(x[q], y[q], z[q], R0.x, R0.y, R0.z) + eps;
-          d[2 + q] = one_minus_dot(x[q], y[q], z[q], R1.x, R1.y, R1.z) + eps;
-        }
-        rcp4(d, g);
+    for (int i = 0; i < 4; ++i) {
+      const int q = i & 1;
+      d[i] = one_minus_dot(x[q], y[q], z[q], R[i >> 1].x, R[i >> 1].y, R[i >> 1].z) + eps;
+    }
+    rcp4(d, g);
 #pragma unroll
-        for (int i = 0; i < 4; ++i) {
-          const int q = i & 1;
-          const TgtRec& R = i < 2 ? R0 : R1;
-          const double dc = x[q] * R.c0 + y[q] * R.c1 + z[q] * R.c2;
-          w[q][0] = fma(g[i], dc, w[q][0]);
-          if constexpr (POS) {
-            const double h = g[i] * dc;
-            w[q][K - 3] = fma(g[i], fma(h, R.x, R.c0), w[q][K - 3]);
-            w[q][K - 2] = fma(g[i], fma(h, R.y, R.c1), w[q][K - 2]);
-            w[q][K - 1] = fma(g[i], fma(h, R.z, R.c2), w[q][K - 1]);
-          }
-        }
+    for (int i = 0; i < 4; ++i) {
+      const int q = i & 1;
+      const TgtRec& P = R[i >> 1];
+      const double dc = x[q] * P.c0 + y[q] * P.c1 + z[q] * P.c2;
+      w[q][0] = fma(g[i], dc, w[q][0]);
+      if constexpr (POS) {
+        const double h = g[i] * dc;
+        w[q][K - 3] = fma(g[i], fma(h, P.x, P.c0), w[q][K - 3]);
+        w[q][K - 2] = fma(g[i], fma(h, P.y, P.c1), w[q][K - 2]);
+        w[q][K - 1] = fma(g[i], fma(h, P.z, P.c2), w[q][K - 1]);
       }
     }
   });

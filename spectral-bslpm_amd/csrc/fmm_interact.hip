@@ -176,6 +176,60 @@ __global__ __launch_bounds__(64 * S) void k_bve64(DevTree t, const TargetTile* _
     store_u(t, u, part, proxy, y * w[2] - z * w[1], z * w[0] - x * w[2], x * w[1] - y * w[0], assign);
 }
 
+// The same in lane copies (lanes.hpp) of two targets, for tiles of at most 42 rows
+// (lanes64), whose rows fill 36 of 64 lanes one per lane.  Microseconds per launch,
+// a row per lane and here: 6 x 96^2 (degree 8) 141 -> 132, 6 x 192^2 499 -> 415
+// (degree 5: 302 -> 250); at 16 waves per tile the short loops gain nothing.
+template <int S>
+__global__ __launch_bounds__(64 * S) void k_bve64_lanes(DevTree t, const TargetTile* __restrict__ tiles, int ntiles,
+                                                        const SourceSet* __restrict__ sets,
+                                                        const SrcRec64* __restrict__ rec, double eps, Ptr3 part,
+                                                        Ptr3 proxy, int assign, int xcd) {
+  constexpr int NT = 2;
+  __shared__ __align__(16) double stage[S][kLaneSlots * 4];
+  member_targets(t, part, proxy);
+  rec += (int64_t)blockIdx.y * t.U;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int lane = threadIdx.x & 63;
+  const int tile = walk_tile(t.xcd_start ? t.xcd_start + 9 : nullptr, xcd);
+  if (tile >= ntiles) return;  // the whole workgroup
+  const TargetTile T = tiles[tile];
+  const LaneTile l = lane_tile<NT>(T.count, lane);
+  double x[NT], y[NT], z[NT], w[NT][3];
+#pragma unroll
+  for (int q = 0; q < NT; ++q) {
+    const int64_t u = (int64_t)T.first + min(q * l.T + l.i, T.count - 1);
+    x[q] = t.px[u]; y[q] = t.py[u]; z[q] = t.pz[u];
+    w[q][0] = w[q][1] = w[q][2] = 0;
+  }
+  lane_walk2<S, 2>(T, sets, reinterpret_cast<const v4f*>(rec), l, reinterpret_cast<v4f*>(stage[wave]), wave, lane,
+                   [&](const v4f* r0, const v4f* r1) {
+    const SrcRec64 R[2] = {*reinterpret_cast<const SrcRec64*>(r0), *reinterpret_cast<const SrcRec64*>(r1)};
+    double d[4], g[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const int q = i & 1;
+      d[i] = one_minus_dot(x[q], y[q], z[q], R[i >> 1].x, R[i >> 1].y, R[i >> 1].z) + eps;
+    }
+    rcp4(d, g);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const int q = i & 1;
+      const SrcRec64& P = R[i >> 1];
+      const double gq = g[i] * P.q;
+      w[q][0] = fma(gq, P.x, w[q][0]);
+      w[q][1] = fma(gq, P.y, w[q][1]);
+      w[q][2] = fma(gq, P.z, w[q][2]);
+    }
+  });
+  double s[3];
+  lane_sum<NT, 3, S>(l, w, stage, wave, lane, s);
+  if (wave > 0 || lane >= T.count) return;
+  const int64_t u = (int64_t)T.first + lane;
+  const double X = t.px[u], Y = t.py[u], Z = t.pz[u];
+  store_u(t, u, part, proxy, Y * s[2] - Z * s[1], Z * s[0] - X * s[2], X * s[1] - Y * s[0], assign);
+}
+
 // FP64 log pair kernel: psi += -1/(4 pi) log(1 - x.y) q, pairs with
 // x.y >= 1 - 1e-15 skipped (inverse_poisson_impl.hpp:46-49).  S waves share a
 // tile (pairwalk.hpp); the logarithm is log_wide (fasttab.hpp) on the context's
@@ -273,6 +327,59 @@ __global__ __launch_bounds__(64 * S) void k_log64(DevTree t, const TargetTile* _
   if (wave == 0 && lane < T.count) store_s(t, u, part, proxy, acc[0], assign);
 }
 
+// The same in lane copies (lanes.hpp) of two targets, for tiles of at most 42 rows
+// (lanes64).  Microseconds per launch, a row per lane and here: 6 x 96^2 (degree 8)
+// 194 -> 171, 6 x 192^2 672 -> 597 (degree 5: 417 -> 393).
+template <int S>
+__global__ __launch_bounds__(64 * S) void k_log64_lanes(DevTree t, const TargetTile* __restrict__ tiles, int ntiles,
+                                                        const SourceSet* __restrict__ sets,
+                                                        const SrcRec64* __restrict__ rec, double* __restrict__ part,
+                                                        double* __restrict__ proxy, int assign) {
+  constexpr int NT = 2;
+  __shared__ LogTabEntry wide[kLogWideSize];
+  __shared__ __align__(16) double stage[S][kLaneSlots * 4];
+  for (int i = threadIdx.x; i < kLogWideSize; i += 64 * S) wide[i] = t.logwide[i];
+  __syncthreads();
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int lane = threadIdx.x & 63;
+  const int tile = strip_tile(ntiles);
+  if (tile >= ntiles) return;  // the whole workgroup
+  const TargetTile T = tiles[tile];
+  const LaneTile l = lane_tile<NT>(T.count, lane);
+  const double c7 = in_vgpr(1.0 / 7.0);
+  double x[NT], y[NT], z[NT], w[NT][1];
+#pragma unroll
+  for (int q = 0; q < NT; ++q) {
+    const int64_t u = (int64_t)T.first + min(q * l.T + l.i, T.count - 1);
+    x[q] = t.px[u]; y[q] = t.py[u]; z[q] = t.pz[u];
+    w[q][0] = 0;
+  }
+  lane_walk2<S, 2>(T, sets, reinterpret_cast<const v4f*>(rec), l, reinterpret_cast<v4f*>(stage[wave]), wave, lane,
+                   [&](const v4f* r0, const v4f* r1) {
+    const SrcRec64 R[2] = {*reinterpret_cast<const SrcRec64*>(r0), *reinterpret_cast<const SrcRec64*>(r1)};
+    double d[4], lg[4];
+    uint32_t h[4], far = 0;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const int q = i & 1;
+      d[i] = one_minus_dot(x[q], y[q], z[q], R[i >> 1].x, R[i >> 1].y, R[i >> 1].z);
+      h[i] = log_wide_cell(d[i]);
+      far = h[i] > far ? h[i] : far;
+    }
+    if (__builtin_amdgcn_ballot_w64(far >= kLogWideSpan) != 0) {
+      log_guarded(d, lg, wide, t.logtab, c7);
+    } else {
+#pragma unroll
+      for (int i = 0; i < 4; ++i) lg[i] = log_wide(d[i], h[i], wide, c7);
+    }
+#pragma unroll
+    for (int i = 0; i < 4; ++i) w[i & 1][0] = fma(lg[i], R[i >> 1].q, w[i & 1][0]);
+  });
+  double s[1];
+  lane_sum<NT, 1, S>(l, w, stage, wave, lane, s);
+  if (wave == 0 && lane < T.count) store_s(t, (int64_t)T.first + lane, part, proxy, s[0], assign);
+}
+
 // Horner multipliers of the FP64 regularised-Laplacian kernel in vector registers.
 struct LapV64 {
   double a1, b2, c24;
@@ -358,6 +465,63 @@ __global__ __launch_bounds__(64 * S) void k_lap64(DevTree t, const TargetTile* _
   });
   tile_sum<S>(acc, wave, lane);
   if (wave == 0 && lane < T.count) store_s(t, u, part, proxy, acc[0], assign);
+}
+
+// The same in lane copies (lanes.hpp) of two targets, for tiles of at most 42 rows
+// (lanes64).  Microseconds per launch in lane groups of one target, with a row per
+// lane and here: 6 x 96^2 (degree 8) 446, 355, 272; 6 x 192^2 1175, 1010, 770 (degree
+// 5: 594, 571, 453); 6 x 160^2 (degree 4) 366, 419, 339.
+template <int S>
+__global__ __launch_bounds__(64 * S) void k_lap64_lanes(DevTree t, const TargetTile* __restrict__ tiles, int ntiles,
+                                                        const SourceSet* __restrict__ sets,
+                                                        const SrcRec64* __restrict__ rec, LapCoef64 kp,
+                                                        double* __restrict__ part, double* __restrict__ proxy,
+                                                        int assign) {
+  constexpr int NT = 2;
+  __shared__ double etab[kExpNegTabSize];
+  __shared__ __align__(16) double stage[S][kLaneSlots * 4];
+  for (int i = threadIdx.x; i < kExpNegTabSize; i += 64 * S) etab[i] = t.expnegtab[i];
+  __syncthreads();
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int lane = threadIdx.x & 63;
+  const int tile = strip_tile(ntiles);
+  if (tile >= ntiles) return;  // the whole workgroup
+  const TargetTile T = tiles[tile];
+  const LaneTile l = lane_tile<NT>(T.count, lane);
+  const double fast_from = kp.cut < -1.0 ? kp.t_sat : 4.0;
+  const LapV64 kv{in_vgpr(kp.a1), in_vgpr(kp.b2), in_vgpr(1.0 / 24.0)};
+  double x[NT], y[NT], z[NT], w[NT][1];
+#pragma unroll
+  for (int q = 0; q < NT; ++q) {
+    const int64_t u = (int64_t)T.first + min(q * l.T + l.i, T.count - 1);
+    x[q] = t.px[u]; y[q] = t.py[u]; z[q] = t.pz[u];
+    w[q][0] = 0;
+  }
+  lane_walk2<S, 2, true>(T, sets, reinterpret_cast<const v4f*>(rec), l, reinterpret_cast<v4f*>(stage[wave]), wave, lane,
+                         [&](const v4f* r0, const v4f* r1) {
+    const SrcRec64 R[2] = {*reinterpret_cast<const SrcRec64*>(r0), *reinterpret_cast<const SrcRec64*>(r1)};
+    double dp[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const int q = i & 1;
+      dp[i] = x[q] * R[i >> 1].x + y[q] * R[i >> 1].y + z[q] * R[i >> 1].z;
+    }
+    if (__builtin_amdgcn_ballot_w64(fmin(fmin(dp[0], dp[1]), fmin(dp[2], dp[3])) < fast_from) != 0) {
+#pragma unroll 1
+      for (int i = 0; i < 2; ++i) {
+        const SrcRec64 s = *reinterpret_cast<const SrcRec64*>(i ? r1 : r0);
+#pragma unroll
+        for (int q = 0; q < NT; ++q)
+          w[q][0] = fma(lap_pair_slow(x[q] * s.x + y[q] * s.y + z[q] * s.z, kp, kv, etab), s.q, w[q][0]);
+      }
+    } else {
+#pragma unroll
+      for (int i = 0; i < 4; ++i) w[i & 1][0] = fma(lap_pair(dp[i], kp, kv, etab), R[i >> 1].q, w[i & 1][0]);
+    }
+  });
+  double s[1];
+  lane_sum<NT, 1, S>(l, w, stage, wave, lane, s);
+  if (wave == 0 && lane < T.count) store_s(t, (int64_t)T.first + lane, part, proxy, s[0], assign);
 }
 
 // Mixed-precision regularised-Laplacian pairs in the folded form of
@@ -1036,6 +1200,7 @@ void launch_bve_interact64(const DevTree& t, const TargetTile* tiles, int ntiles
   shape = checked_shape(t, shape);
   const int S = tile_waves(ntiles);
   auto kernel = S == 16 ? k_bve64<16> : S == 8 ? k_bve64<8> : k_bve64<4>;
+  if (lanes64(t) && S < 16) kernel = S == 8 ? k_bve64_lanes<8> : k_bve64_lanes<4>;
   hipLaunchKernelGGL(kernel, dim3(walk_grid(ntiles, shape), nmem), dim3(64 * S), 0, s, t, tiles, ntiles, sets, rec, eps,
                      ptr3(out_part), ptr3(out_proxy), assign ? 1 : 0, shape.xcd);
 }
@@ -1046,6 +1211,7 @@ void launch_poisson_interact64(const DevTree& t, const TargetTile* tiles, int nt
   if (ntiles == 0) return;
   const int S = log_waves(ntiles);
   auto kernel = S == 16 ? k_log64<16> : k_log64<8>;
+  if (lanes64(t) && S < 16) kernel = k_log64_lanes<8>;
   hipLaunchKernelGGL(kernel, dim3(strip_grid(ntiles)), dim3(64 * S), 0, s, t, tiles, ntiles, sets, rec, out_part, out_proxy,
                      assign ? 1 : 0);
 }
@@ -1060,6 +1226,7 @@ void launch_laplacian_interact64(const DevTree& t, const TargetTile* tiles, int 
   // us per launch with 4 / 8 / 16 waves: 126 tiles 181 / 116 / 98, 636 223 / 219 / 230, 10,236 1028 / 1088 / 1373
   const int S = ntiles < 400 ? 16 : 4;
   auto kernel = S == 16 ? k_lap64<16> : k_lap64<4>;
+  if (lanes64(t) && S < 16) kernel = k_lap64_lanes<4>;
   hipLaunchKernelGGL(kernel, dim3(strip_grid(ntiles)), dim3(64 * S), 0, s, t, tiles, ntiles, sets, rec, kp, out_part, out_proxy,
                      assign ? 1 : 0);
 }

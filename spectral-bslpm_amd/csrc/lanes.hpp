@@ -99,6 +99,41 @@ __device__ inline void lane_walk(const TargetTile& T, const SourceSet* __restric
   });
 }
 
+// lane_walk for the FP64 kernels: add(r0, r1) takes two trips, so that two rows of
+// two records share a reciprocal; an odd last trip is paired with a padding record
+// (slot 79, which no trip reaches).  REPEAT (N = 2, the charge in the last eight
+// bytes): padding repeats the chunk's last record without its charge, for a kernel
+// that takes another form where a pair is far away.
+template <int S, int N, bool REPEAT = false, typename Add>
+__device__ inline void lane_walk2(const TargetTile& T, const SourceSet* __restrict__ sets, const v4f* __restrict__ rec,
+                                  const LaneTile& l, v4f* mine, int wave, int lane, Add&& add) {
+  static_assert(!REPEAT || N == 2, "lane_walk2: REPEAT knows the layout of two-word records");
+  if (!REPEAT) lane_pads<N>(mine, 0.f, lane);
+  walk_sets<S>(T, sets, wave, [&](const SourceSet& set, int a, int b) {
+    for (int c = a; c < b; c += kLaneChunk) {
+      const int cn = min(kLaneChunk, b - c), trips = (cn + l.G - 1) / l.G;
+      const v4f* src = rec + N * ((int64_t)set.first + c);
+      if constexpr (REPEAT) {
+        __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
+        const int k = min(lane, cn - 1);
+        const v4f v0 = src[2 * k], v1 = src[2 * k + 1], last0 = src[2 * cn - 2], last1 = src[2 * cn - 1];
+        mine[2 * lane] = v0;
+        mine[2 * lane + 1] = lane < cn ? v1 : v4f{v1.x, v1.y, 0.f, 0.f};
+        if (lane < kLanePad) {
+          mine[2 * (kLaneChunk + lane)] = last0;
+          mine[2 * (kLaneChunk + lane) + 1] = v4f{last1.x, last1.y, 0.f, 0.f};
+        }
+        __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
+      } else {
+        lane_stage<N>(mine, src, cn, 0.f, lane);
+      }
+      const v4f* r = mine + N * l.g;
+      for (int k = 0; k < trips; k += 2, r += 2 * N * l.G)
+        add(r, k + 1 < trips ? r + N * l.G : mine + N * (kLaneSlots - 1));
+    }
+  });
+}
+
 // Sums w[t][c] over the copies and the S waves into row t T + i of lane
 // t T + i of wave 0, valid where the lane is below the tile's count; `stage` is
 // each wave's slot of SLOT >= 64 K doubles (every thread calls it).

@@ -124,6 +124,68 @@ __global__ __launch_bounds__(64 * S) void k_swe64(DevTree t, const TargetTile* _
   }
 }
 
+// Variants 1 and 3 in lane copies (lanes.hpp) of two targets, for tiles of at most
+// 42 rows (lanes64).  Microseconds per launch, a row per lane and here: 6 x 96^2
+// (degree 8) 201 -> 192, 6 x 192^2 686 -> 558 (degree 5: 423 -> 341), 6 x 160^2
+// (degree 4, 25 rows) 294 -> 253.
+template <int S>
+__global__ __launch_bounds__(64 * S) void k_swe64_lanes(DevTree t, const TargetTile* __restrict__ tiles, int ntiles,
+                                                        const SourceSet* __restrict__ sets,
+                                                        const SrcRecSwe* __restrict__ rec, double eps, Ptr3 part,
+                                                        Ptr3 proxy, int assign, int) {
+  constexpr int NT = 2, K = 6;
+  __shared__ __align__(16) double stage[S][kLaneSlots * 8];
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int lane = threadIdx.x & 63;
+  const int tile = strip_tile(ntiles);
+  if (tile >= ntiles) return;  // the whole workgroup
+  const TargetTile T = tiles[tile];
+  const LaneTile l = lane_tile<NT>(T.count, lane);
+  double x[NT], y[NT], z[NT], w[NT][K];
+#pragma unroll
+  for (int q = 0; q < NT; ++q) {
+    const int64_t u = (int64_t)T.first + min(q * l.T + l.i, T.count - 1);
+    x[q] = t.px[u]; y[q] = t.py[u]; z[q] = t.pz[u];
+#pragma unroll
+    for (int k = 0; k < K; ++k) w[q][k] = 0;
+  }
+  lane_walk2<S, 4>(T, sets, reinterpret_cast<const v4f*>(rec), l, reinterpret_cast<v4f*>(stage[wave]), wave, lane,
+                   [&](const v4f* r0, const v4f* r1) {
+    const SrcRecSwe* R[2] = {reinterpret_cast<const SrcRecSwe*>(r0), reinterpret_cast<const SrcRecSwe*>(r1)};
+    double d[4], g[4], a[2], b[2], c[2], qz[2], qd[2];
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+      a[i] = R[i]->x; b[i] = R[i]->y; c[i] = R[i]->z; qz[i] = R[i]->qz; qd[i] = R[i]->qd;
+    }
+#pragma unroll
+    for (int i = 0; i < 4; ++i) d[i] = one_minus_dot(x[i & 1], y[i & 1], z[i & 1], a[i >> 1], b[i >> 1], c[i >> 1]) + eps;
+    rcp4(d, g);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const int q = i & 1, k = i >> 1;
+      const double gz = g[i] * qz[k], gd = g[i] * qd[k];
+      w[q][0] = fma(gz, a[k], w[q][0]);
+      w[q][1] = fma(gz, b[k], w[q][1]);
+      w[q][2] = fma(gz, c[k], w[q][2]);
+      w[q][3] = fma(gd, a[k], w[q][3]);
+      w[q][4] = fma(gd, b[k], w[q][4]);
+      w[q][5] = fma(gd, c[k], w[q][5]);
+    }
+  });
+  double s[K];
+  lane_sum<NT, K, S>(l, w, stage, wave, lane, s);
+  if (wave > 0 || lane >= T.count) return;
+  const int64_t u = (int64_t)T.first + lane;
+  const double X = t.px[u], Y = t.py[u], Z = t.pz[u], sd = X * s[3] + Y * s[4] + Z * s[5];
+  const double o[3] = {(Y * s[2] - Z * s[1]) + (s[3] - X * sd), (Z * s[0] - X * s[2]) + (s[4] - Y * sd),
+                       (X * s[1] - Y * s[0]) + (s[5] - Z * sd)};
+#pragma unroll
+  for (int k = 0; k < 3; ++k) {
+    double* p = u < t.npart ? part.p[k] + u : proxy.p[k] + (u - t.npart);
+    *p = assign ? o[k] : *p + o[k];
+  }
+}
+
 // Mixed-precision records: position relative to the source panel centre (FP32)
 // and the two charges with the variant's constants, FP32.
 __global__ void k_src_swe32(DevTree t, const double* __restrict__ qz_part, const double* __restrict__ qz_proxy,
@@ -293,6 +355,7 @@ void launch_swe_interact64(const DevTree& t, int variant, const TargetTile* tile
   const int S = ntiles < 400 ? 16 : ntiles < 3000 ? 8 : 4;
   auto kernel = variant != 2 ? (S == 16 ? k_swe64<1, 16> : S == 8 ? k_swe64<1, 8> : k_swe64<1, 4>)
                              : (S == 16 ? k_swe64<2, 16> : S == 8 ? k_swe64<2, 8> : k_swe64<2, 4>);
+  if (variant != 2 && lanes64(t) && !heaviest_first && S < 16) kernel = S == 8 ? k_swe64_lanes<8> : k_swe64_lanes<4>;
   hipLaunchKernelGGL(kernel, dim3(heaviest_first ? ntiles : strip_grid(ntiles)), dim3(64 * S), 0, s, t, tiles, ntiles, sets, rec, eps, op, ox,
                      assign ? 1 : 0, heaviest_first ? 1 : 0);
 }
