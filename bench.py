@@ -851,7 +851,7 @@ def bench_c2(args, torch, sb):
     if os.path.exists(tfile):
         with open(tfile) as fh:
             tr = json.load(fh)["kernels"]
-        for name, kern in (("log_fp64", "k_log64"), ("log_mixed", "k_log_mixed")):
+        for name, kern in (("log_fp64", "k_log64"), ("log_mixed", "k_log_lanes")):
             if tr.get(kern):
                 roof[name]["traffic"] = tr[kern]["hbm_bytes"]
                 roof[name]["traffic_kernel"] = kern

@@ -58,7 +58,7 @@ struct DevTree {
 __device__ inline int64_t member_part(const DevTree& t) { return (int64_t)blockIdx.y * t.npart; }
 __device__ inline int64_t member_proxy(const DevTree& t) { return (int64_t)blockIdx.y * t.P * t.n; }
 
-// Pair kernels run one wave per target tile, four waves per workgroup.
+// Waves per workgroup of the pair kernels that run one wave per tile.
 constexpr int kWavesPerBlock = 4;
 
 // Launch shape of the Biot-Savart pair kernels, chosen by the context's

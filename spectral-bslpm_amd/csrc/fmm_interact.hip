@@ -4,18 +4,22 @@
 // and poisson_panel_interaction (inverse_poisson_impl.hpp:23-52) run one
 // thread per interaction, recompute every source node's map per pair and
 // scatter three atomics per pair.  Here:
-//   * one wave64 owns up to 64 target points of one target panel and walks
-//     that panel's source sets, so each target is accumulated in registers by
-//     one lane (no atomics, fixed summation order);
+//   * a tile of up to 64 target points of one target panel belongs to one
+//     workgroup, whose waves share that panel's source sets; a target is
+//     accumulated in registers and the waves' sums are added in order (no
+//     atomics, fixed summation order);
 //   * displaced, re-projected source positions and scaled charges are built
 //     once per evaluation into a record array (SrcRec64 / SrcRec32);
-//   * every lane of a wave reads the same source record, so the records are
-//     wave-uniform loads (scalar cache) with no LDS and no barriers;
+//   * on FP64 tiles of more than 42 rows every lane of a wave reads the same
+//     source record, a wave-uniform load through the scalar cache
+//     (pairwalk.hpp); on smaller tiles and in FP32 a wave stages the records
+//     in LDS and copies of the tile, two targets per lane, take its sources in
+//     turn (lanes.hpp);
 //   * u = sum_j g_j q_j (x cross y_j) is accumulated as x cross (sum_j g_j q_j y_j),
 //     saving the per-pair cross product (six multiplies) of the reference form.
-// Workgroups of four waves; the workgroup id is remapped so that consecutive
-// tiles (spatially adjacent target panels sharing sources) land on the same
-// XCD and its L2.
+// The workgroup id is remapped so that neighbouring tiles (adjacent target
+// panels sharing sources) land on the same XCD and its L2.  The matrix-core
+// kernels and k_bve_mixed run one wave per tile.
 #include <cmath>
 
 #include "device.hpp"

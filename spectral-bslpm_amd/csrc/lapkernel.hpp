@@ -1,6 +1,6 @@
 // lapkernel.hpp -- the regularised-Laplacian kernel of the shallow-water step
 // (lap_panel_interaction, laplacian_impl.hpp:46-66) with its constants folded
-// into short polynomials, for the forward pair kernels (k_lap64, k_lap_mixed)
+// into short polynomials, for the forward pair kernels (k_lap64, k_lap_lanes)
 // and the transposed ones (k_lap_adj64, k_lap_adj32).
 //
 // For t = x.y > 1 - 30 eps:

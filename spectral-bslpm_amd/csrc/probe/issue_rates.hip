@@ -1,5 +1,5 @@
 // issue_rates.hip -- register-only probes of the instruction mixes that bound
-// the mixed-precision Biot-Savart pair kernel (k_bve_mfma) on gfx950, for the
+// the matrix-core Biot-Savart pair kernel (k_bve_mfma) on gfx950, for the
 // per-kernel floor table of the measurement notes.  Each probe runs a fixed
 // instruction mix `iters` times on registers only (no memory traffic in the
 // loop), every wave of the grid doing the same; the host times the launch and

@@ -418,7 +418,7 @@ __global__ void k_lap_tgt32(DevTree t, const double* __restrict__ psi_part, cons
                     0.f};
 }
 
-// FP32 pairs as k_lap_mixed (lapkernel.hpp's polynomials in u, the base-2
+// FP32 pairs as k_lap_lanes (lapkernel.hpp's polynomials in u, the base-2
 // exponent of E, from the squared chord h2), erf and the e^{-s^2} term only
 // when a ballot finds a pair with t < 6 eps.
 template <bool POS>
