@@ -94,7 +94,7 @@ __global__ __launch_bounds__(64 * S) void k_bve_adj64(DevTree t, const TargetTil
   constexpr int K = POS ? 4 : 1;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int lane = threadIdx.x & 63;
-  const int tile = strip_tile(ntiles);
+  const int tile = dealt_tile(ntiles);
   if (tile >= ntiles) return;  // the whole workgroup
   const TargetTile T = tiles[tile];
   const int64_t u = (int64_t)T.first + (lane < T.count ? lane : T.count - 1);
@@ -146,7 +146,7 @@ __global__ __launch_bounds__(64 * S) void k_bve_adj64_lanes(DevTree t, const Tar
   __shared__ __align__(16) double stage[S][kLaneSlots * 6];
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int lane = threadIdx.x & 63;
-  const int tile = strip_tile(ntiles);
+  const int tile = dealt_tile(ntiles);
   if (tile >= ntiles) return;  // the whole workgroup
   const TargetTile T = tiles[tile];
   const LaneTile l = lane_tile<NT>(T.count, lane);
@@ -236,7 +236,7 @@ __global__ __launch_bounds__(64 * S) void k_bve_adj32(DevTree t, const TargetTil
   __shared__ __align__(16) double stage[S][kLaneSlots * 4];
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int lane = threadIdx.x & 63;
-  const int tile = strip_tile(ntiles);
+  const int tile = dealt_tile(ntiles);
   if (tile >= ntiles) return;  // the whole workgroup
   const TargetTile T = tiles[tile];
   const LaneTile l = lane_tile<NT>(T.count, lane);

@@ -59,7 +59,9 @@ struct sbslpm_ctx {
   SourceSet* sets = nullptr;
   int* set_start = nullptr;
   int ntiles = 0;
-  int nonleaf_tiles = 0;
+  TargetTile* bfs_tiles = nullptr;
+  TargetTile* nonleaf_tiles = nullptr;
+  int nnonleaf = 0;
 
   // workspace
   SrcRec64* rec64 = nullptr;
@@ -82,6 +84,7 @@ struct sbslpm_ctx {
   // first adjoint call
   char* adj_arena = nullptr;
   TargetTile* adj_tiles = nullptr;
+  TargetTile* adj_bfs_tiles = nullptr;
   SourceSet* adj_targets = nullptr;
   int* adj_zero_rows = nullptr;
   int adj_ntiles = 0;
@@ -375,6 +378,7 @@ int sbslpm_ctx_create(const sbslpm_params* p, sbslpm_ctx** out) {
   size_t o_po = A.take<int>(t.proxy_order.size());
   size_t o_err = A.take<int>(4), o_zr = A.take<int>(t.zero_rows.size());
   size_t o_tiles = A.take<TargetTile>(t.tiles.size()), o_sets = A.take<SourceSet>(t.srcsets.size());
+  size_t o_nlt = A.take<TargetTile>(t.nonleaf_tiles.size()), o_bfs = A.take<TargetTile>(t.bfs_tiles.size());
   size_t o_ss = A.take<int>(t.set_start.size());
   size_t o_rec64 = A.take<SrcRec64>(U), o_rec32 = A.take<SrcRec32>(U), o_recmf = A.take<SrcRecMfma>(t.U16);
   size_t o_qpart = A.take<double>(NP), o_qproxy = A.take<double>(Pn);
@@ -412,6 +416,8 @@ int sbslpm_ctx_create(const sbslpm_params* p, sbslpm_ctx** out) {
   rc |= upload(c, b + o_pxe, t.proxy_xieta.data(), t.proxy_xieta.size() * sizeof(double));
   rc |= upload(c, b + o_po, t.proxy_order.data(), t.proxy_order.size() * sizeof(int));
   rc |= upload(c, b + o_tiles, t.tiles.data(), t.tiles.size() * sizeof(TargetTile));
+  rc |= upload(c, b + o_bfs, t.bfs_tiles.data(), t.bfs_tiles.size() * sizeof(TargetTile));
+  rc |= upload(c, b + o_nlt, t.nonleaf_tiles.data(), t.nonleaf_tiles.size() * sizeof(TargetTile));
   rc |= upload(c, b + o_sets, t.srcsets.data(), t.srcsets.size() * sizeof(SourceSet));
   rc |= upload(c, b + o_zr, t.zero_rows.data(), t.zero_rows.size() * sizeof(int));
   rc |= upload(c, b + o_ss, t.set_start.data(), t.set_start.size() * sizeof(int));
@@ -457,7 +463,9 @@ int sbslpm_ctx_create(const sbslpm_params* p, sbslpm_ctx** out) {
   c->tiles = (TargetTile*)(b + o_tiles);
   c->sets = (SourceSet*)(b + o_sets);
   c->ntiles = (int)t.tiles.size();
-  c->nonleaf_tiles = t.nonleaf_tiles;
+  c->bfs_tiles = (TargetTile*)(b + o_bfs);
+  c->nonleaf_tiles = (TargetTile*)(b + o_nlt);
+  c->nnonleaf = (int)t.nonleaf_tiles.size();
   c->set_start = (int*)(b + o_ss);
   c->zero_rows = (int*)(b + o_zr);
   c->nzero_rows = (int)t.zero_rows.size();
@@ -766,7 +774,7 @@ static int swe_interactions(sbslpm_ctx* c, int variant, const double* dpx, const
                             dxx ? dx : nullptr, c->recswe, c->stream);
   {
     KernelTimer tm(c, SBSLPM_KERNEL_SWE_FP64);
-    launch_swe_interact64(c->dt, variant, c->tiles, c->ntiles, c->sets, c->recswe, c->prm.kernel_eps, op, ox,
+    launch_swe_interact64(c->dt, variant, c->bfs_tiles, c->ntiles, c->sets, c->recswe, c->prm.kernel_eps, op, ox,
                           c->stream, assign);
   }
   return launched(c);
@@ -825,10 +833,10 @@ static int eval_targets(sbslpm_ctx* c, int kind, const double* area, const doubl
   // bve_vel_impl.hpp:54-60)
   launch_source_records64(c->dt, c->qpart, c->qproxy, nullptr, nullptr, kind == 1, c->rec64, c->stream);
   if (kind == 0)
-    launch_poisson_interact64(c->dt, c->tiles, c->nonleaf_tiles, c->sets, c->rec64, c->phipart[0], c->phiproxy[0],
+    launch_poisson_interact64(c->dt, c->nonleaf_tiles, c->nnonleaf, c->sets, c->rec64, c->phipart[0], c->phiproxy[0],
                               c->stream, true);
   else
-    launch_bve_interact64(c->dt, c->tiles, c->nonleaf_tiles, c->sets, c->rec64, c->prm.kernel_eps, c->phipart,
+    launch_bve_interact64(c->dt, c->nonleaf_tiles, c->nnonleaf, c->sets, c->rec64, c->prm.kernel_eps, c->phipart,
                           c->phiproxy, c->stream, true);
   launch_l2l(c->dt, nc, c->phiproxy, c->stream, true);
   const double* far[3] = {c->phiproxy[0], c->phiproxy[1], c->phiproxy[2]};
@@ -1162,7 +1170,7 @@ static int laplacian_fmm(sbslpm_ctx* c, const double* area, const double* f, con
   } else {
     launch_source_records64(c->dt, w.qp, w.qx, dpart, dprox, true, c->rec64, c->stream);
     KernelTimer tm(c, SBSLPM_KERNEL_LAP_FP64);
-    launch_laplacian_interact64(c->dt, c->tiles, c->ntiles, c->sets, c->rec64, w.pp, w.px, c->stream, true);
+    launch_laplacian_interact64(c->dt, c->bfs_tiles, c->ntiles, c->sets, c->rec64, w.pp, w.px, c->stream, true);
   }
   const double* pp1[1] = {w.pp};
   double* out[1] = {lap};
@@ -1211,7 +1219,7 @@ int sbslpm_laplacian_interactions(sbslpm_ctx* c, const double* dpx, const double
     return launched(c);
   }
   launch_source_records64(c->dt, q_part, q_proxy, dpx ? dp : nullptr, dxx ? dx : nullptr, true, c->rec64, c->stream);
-  launch_laplacian_interact64(c->dt, c->tiles, c->ntiles, c->sets, c->rec64, phi_part, phi_proxy, c->stream, false);
+  launch_laplacian_interact64(c->dt, c->bfs_tiles, c->ntiles, c->sets, c->rec64, phi_part, phi_proxy, c->stream, false);
   return launched(c);
 }
 
@@ -1490,7 +1498,7 @@ static int swe_fmm_adjoint(sbslpm_ctx* c, const double* area_s, const double* vo
   double* qx2[2] = {a.qzx, a.qdx};
   launch_zero_rows(c->adj_zero_rows, c->adj_nzero, t.n, 2, qx2, c->stream);
   if (pos && !acc) launch_zero_rows(c->adj_zero_rows, c->adj_nzero, t.n, 3, a.dbx, c->stream);
-  launch_swe_adjoint(c->dt, fp32, c->adj_tiles, c->adj_ntiles, c->adj_targets, a.trec, c->recswe, c->prm.kernel_eps,
+  launch_swe_adjoint(c->dt, fp32, c->adj_bfs_tiles, c->adj_ntiles, c->adj_targets, a.trec, c->recswe, c->prm.kernel_eps,
                      dpart, dprox, a.qzp, a.qzx, a.qdp, a.qdx, a.dbp, a.dbx, acc, c->stream, c->shape);
   // both charge cotangents in one downward pass (two components per launch)
   const double* qp2[2] = {a.qzp, a.qdp};
@@ -1516,7 +1524,7 @@ static int lap_fmm_adjoint(sbslpm_ctx* c, const double* area_s, const double* ef
   launch_source_records64(c->dt, w.qp, w.qx, dpart, dprox, true, a.srec, c->stream);
   launch_zero_rows(c->adj_zero_rows, c->adj_nzero, t.n, 1, &a.qex, c->stream);
   if (pos) launch_zero_rows(c->adj_zero_rows, c->adj_nzero, t.n, 3, a.dbx, c->stream);
-  launch_laplacian_adjoint(c->dt, fp32, c->adj_tiles, c->adj_ntiles, c->adj_targets, a.trec, a.srec, dpart, dprox,
+  launch_laplacian_adjoint(c->dt, fp32, c->adj_bfs_tiles, c->adj_ntiles, c->adj_targets, a.trec, a.srec, dpart, dprox,
                            a.qep, a.qex, a.dbp, a.dbx, false, c->stream, c->shape);
   const double* qep[1] = {a.qep};
   launch_downward_pass(c->dt, 1, &a.qex, qep, &a.qe, c->stream, true);
@@ -2356,7 +2364,8 @@ static int ensure_adjoint(sbslpm_ctx* c) {
   build_source_major(t, sm);
   const size_t NP = (size_t)t.npart, Pn = (size_t)t.P * t.n;
   Arena A;
-  const size_t o_tiles = A.take<TargetTile>(sm.tiles.size()), o_tg = A.take<SourceSet>(sm.targets.size()),
+  const size_t o_tiles = A.take<TargetTile>(sm.tiles.size()), o_bfs = A.take<TargetTile>(sm.bfs_tiles.size()),
+               o_tg = A.take<SourceSet>(sm.targets.size()),
                o_zr = A.take<int>(sm.zero_rows.size()), o1 = A.take<double>(NP), o_pp = A.take<double>(3 * NP),
                o_px = A.take<double>(3 * Pn), o_tr = A.take<char>(t.U * adj_target_record_bytes()),
                o_sr = A.take<SrcRec64>(t.U), o_qbp = A.take<double>(NP), o_qbx = A.take<double>(Pn),
@@ -2367,6 +2376,7 @@ static int ensure_adjoint(sbslpm_ctx* c) {
   if (hipMalloc(&b, total) != hipSuccess) return fail(c, SBSLPM_E_NOMEM, "adjoint workspace: out of device memory");
   c->adj_arena = b;
   c->adj_tiles = (TargetTile*)(b + o_tiles);
+  c->adj_bfs_tiles = (TargetTile*)(b + o_bfs);
   c->adj_targets = (SourceSet*)(b + o_tg);
   c->adj_zero_rows = (int*)(b + o_zr);
   c->adj_ntiles = (int)sm.tiles.size();
@@ -2388,6 +2398,7 @@ static int ensure_adjoint(sbslpm_ctx* c) {
     c->adj_vb[i] = (double*)(b + o_vb) + i * NP;
   }
   int rc = upload(c, c->adj_tiles, sm.tiles.data(), sm.tiles.size() * sizeof(TargetTile));
+  rc |= upload(c, c->adj_bfs_tiles, sm.bfs_tiles.data(), sm.bfs_tiles.size() * sizeof(TargetTile));
   if (!rc) rc = upload(c, c->adj_targets, sm.targets.data(), sm.targets.size() * sizeof(SourceSet));
   if (!rc) rc = upload(c, c->adj_zero_rows, sm.zero_rows.data(), sm.zero_rows.size() * sizeof(int));
   if (rc) return rc;

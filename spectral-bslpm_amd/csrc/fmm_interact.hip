@@ -290,7 +290,7 @@ __global__ __launch_bounds__(64 * S) void k_log64(DevTree t, const TargetTile* _
   __syncthreads();
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int lane = threadIdx.x & 63;
-  const int tile = strip_tile(ntiles);
+  const int tile = dealt_tile(ntiles);
   if (tile >= ntiles) return;  // the whole workgroup
   const TargetTile T = tiles[tile];
   const int64_t u = (int64_t)T.first + (lane < T.count ? lane : T.count - 1);
@@ -346,7 +346,7 @@ __global__ __launch_bounds__(64 * S) void k_log64_lanes(DevTree t, const TargetT
   __syncthreads();
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int lane = threadIdx.x & 63;
-  const int tile = strip_tile(ntiles);
+  const int tile = dealt_tile(ntiles);
   if (tile >= ntiles) return;  // the whole workgroup
   const TargetTile T = tiles[tile];
   const LaneTile l = lane_tile<NT>(T.count, lane);
@@ -562,7 +562,7 @@ __global__ __launch_bounds__(64 * S) void k_lap_lanes(DevTree t, const TargetTil
   __shared__ __align__(16) double stage[S][kLaneSlots * 2];
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int lane = threadIdx.x & 63;
-  const int tile = strip_tile(ntiles);
+  const int tile = dealt_tile(ntiles);
   if (tile >= ntiles) return;  // the whole workgroup
   const TargetTile T = tiles[tile];
   const DevPanel& PT = t.panels[T.panel];
@@ -682,7 +682,7 @@ __global__ __launch_bounds__(64 * S) void k_log_lanes(DevTree t, const TargetTil
   __shared__ __align__(16) double stage[S][kLaneSlots * 2];
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int lane = threadIdx.x & 63;
-  const int tile = strip_tile(ntiles);
+  const int tile = dealt_tile(ntiles);
   if (tile >= ntiles) return;  // the whole workgroup
   const TargetTile T = tiles[tile];
   const DevPanel& PT = t.panels[T.panel];

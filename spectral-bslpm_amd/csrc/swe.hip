@@ -234,7 +234,7 @@ __global__ __launch_bounds__(64 * S) void k_swe_lanes(DevTree t, const TargetTil
   __shared__ __align__(16) double stage[S][64 * K];
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int lane = threadIdx.x & 63;
-  const int tile = strip_tile(ntiles);
+  const int tile = dealt_tile(ntiles);
   if (tile >= ntiles) return;  // the whole workgroup
   const TargetTile T = tiles[tile];
   const DevPanel& PT = t.panels[T.panel];

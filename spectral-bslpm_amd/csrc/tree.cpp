@@ -157,6 +157,24 @@ void traverse(Tree& t) {
   }
 }
 
+// Orders a list of fewer than kBalancedTiles tiles by the pairs a lane of each
+// computes (16 more per set for the per-set work), largest first, so that the
+// last workgroups to be dispatched are short ones.  Sums do not depend on it.
+void heaviest_first(std::vector<TargetTile>& tiles, const std::vector<SourceSet>& sets) {
+  if ((int)tiles.size() >= kBalancedTiles) return;
+  auto cost = [&](const TargetTile& tl) {
+    int64_t w = 0;
+    for (int e = tl.src_begin; e < tl.src_end; ++e) w += sets[e].count + 16;
+    return w;
+  };
+  std::vector<std::pair<int64_t, int>> key(tiles.size());
+  for (size_t k = 0; k < key.size(); ++k) key[k] = {-cost(tiles[k]), (int)k};
+  std::sort(key.begin(), key.end());
+  std::vector<TargetTile> out(tiles.size());
+  for (size_t k = 0; k < key.size(); ++k) out[k] = tiles[key[k].second];
+  tiles.swap(out);
+}
+
 }  // namespace
 
 double sphere_tri_area(const double* p1, const double* p2, const double* p3) { return tri_area(p1, p2, p3); }
@@ -328,12 +346,16 @@ std::string build_tree(const TreeConfig& cfg, Tree& t) {
   }
 
   t.set_start = cnt;
-  t.nonleaf_tiles = 0;
-  while (t.nonleaf_tiles < (int)t.tiles.size() && !t.pn[t.tiles[t.nonleaf_tiles].panel].is_leaf) ++t.nonleaf_tiles;
+  t.bfs_tiles = t.tiles;
+  heaviest_first(t.tiles, t.srcsets);
+  t.nonleaf_tiles.clear();
+  for (const TargetTile& tl : t.tiles)
+    if (!t.pn[tl.panel].is_leaf) t.nonleaf_tiles.push_back(tl);
+  heaviest_first(t.nonleaf_tiles, t.srcsets);
 
   // Eight contiguous ranges of the tile list with equal estimated work, one per
-  // XCD (the list is in breadth-first panel order, so a range of leaf tiles is a
-  // compact patch of the sphere and its sources stay in that XCD's L2), for two
+  // XCD (a long list is in breadth-first panel order, so a range of leaf tiles is
+  // a compact patch of the sphere and its sources stay in that XCD's L2), for two
   // work models: xcd_start[0..8] for the matrix-core kernels (a tile's 16 x 16
   // pair blocks over its source sets plus one block per set for the per-set
   // flush) and xcd_start[9..17] for the vector-unit kernels, whose wave walks
@@ -460,6 +482,8 @@ void build_source_major(const Tree& t, SourceMajor& sm) {
       sm.tiles.push_back(tl);
     }
   }
+  sm.bfs_tiles = sm.tiles;
+  heaviest_first(sm.tiles, sm.targets);
   sm.zero_rows.clear();
   for (int p = 0; p < t.P; ++p)
     if ((!t.pn[p].is_leaf && cnt[p + 1] == cnt[p]) || (t.pn[p].is_leaf && t.cfg.levels == 1)) sm.zero_rows.push_back(p);
