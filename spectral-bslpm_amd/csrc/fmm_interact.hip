@@ -1202,9 +1202,12 @@ void launch_bve_interact64(const DevTree& t, const TargetTile* tiles, int ntiles
                            hipStream_t s, bool assign, int nmem, PairShape shape) {
   if (ntiles == 0) return;
   shape = checked_shape(t, shape);
-  const int S = tile_waves(ntiles);
+  int S = tile_waves(ntiles);
   auto kernel = S == 16 ? k_bve64<16> : S == 8 ? k_bve64<8> : k_bve64<4>;
-  if (lanes64(t) && S < 16) kernel = S == 8 ? k_bve64_lanes<8> : k_bve64_lanes<4>;
+  if (lanes64(t) && S < 16) {
+    S = lane_waves(ntiles);
+    kernel = S == 8 ? k_bve64_lanes<8> : k_bve64_lanes<4>;
+  }
   hipLaunchKernelGGL(kernel, dim3(walk_grid(ntiles, shape), nmem), dim3(64 * S), 0, s, t, tiles, ntiles, sets, rec, eps,
                      ptr3(out_part), ptr3(out_proxy), assign ? 1 : 0, shape.xcd);
 }
@@ -1213,9 +1216,12 @@ void launch_poisson_interact64(const DevTree& t, const TargetTile* tiles, int nt
                                const SrcRec64* rec, double* out_part, double* out_proxy, hipStream_t s,
                                bool assign) {
   if (ntiles == 0) return;
-  const int S = log_waves(ntiles);
+  int S = log_waves(ntiles);
   auto kernel = S == 16 ? k_log64<16> : k_log64<8>;
-  if (lanes64(t) && S < 16) kernel = k_log64_lanes<8>;
+  if (lanes64(t) && S < 16) {
+    S = lane_waves(ntiles);
+    kernel = S == 8 ? k_log64_lanes<8> : k_log64_lanes<4>;
+  }
   hipLaunchKernelGGL(kernel, dim3(strip_grid(ntiles)), dim3(64 * S), 0, s, t, tiles, ntiles, sets, rec, out_part, out_proxy,
                      assign ? 1 : 0);
 }
@@ -1228,9 +1234,12 @@ void launch_laplacian_interact64(const DevTree& t, const TargetTile* tiles, int 
   // the records carry -q/(4 pi): undo it with the kernel's eps^{-5/2}
   const LapCoef64 kp = lap_coef64(eps, -4.0 * pi / std::pow(eps, 2.5));
   // us per launch with 4 / 8 / 16 waves: 126 tiles 181 / 116 / 98, 636 223 / 219 / 230, 10,236 1028 / 1088 / 1373
-  const int S = ntiles < 400 ? 16 : 4;
+  int S = ntiles < 400 ? 16 : 4;
   auto kernel = S == 16 ? k_lap64<16> : k_lap64<4>;
-  if (lanes64(t) && S < 16) kernel = k_lap64_lanes<4>;
+  if (lanes64(t) && S < 16) {
+    S = lane_waves(ntiles);
+    kernel = S == 8 ? k_lap64_lanes<8> : k_lap64_lanes<4>;
+  }
   hipLaunchKernelGGL(kernel, dim3(strip_grid(ntiles)), dim3(64 * S), 0, s, t, tiles, ntiles, sets, rec, kp, out_part, out_proxy,
                      assign ? 1 : 0);
 }

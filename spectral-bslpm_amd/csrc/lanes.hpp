@@ -75,7 +75,9 @@ __device__ inline void lane_pads(v4f* mine, float first, int lane) {
       mine[N * (kLaneChunk + lane) + i] = v4f{i == 0 ? first : 0.f, 0.f, 0.f, 0.f};
 }
 
-// Waves per tile of the lane-copy kernels (their tables of times stand beside them).
+// Waves per tile of the lane-copy kernels.  (The FP32 kernels' times stand beside them.
+// FP64 shallow-water velocity at degree 4, microseconds per call with 2 / 4 / 8 waves:
+// 510 tiles 50 / 36 / 36, 2,046 78 / 76 / 91, 8,190 211 / 209 / 282.)
 inline int lane_waves(int ntiles) { return ntiles < 1000 ? 8 : 4; }
 
 // Walks a wave's share of the source sets of a tile: begin(set) and flush(set)
@@ -99,39 +101,59 @@ __device__ inline void lane_walk(const TargetTile& T, const SourceSet* __restric
   });
 }
 
-// lane_walk for the FP64 kernels: add(r0, r1) takes two trips, so that two rows of
-// two records share a reciprocal; an odd last trip is paired with a padding record
-// (slot 79, which no trip reaches).  REPEAT (N = 2, the charge in the last eight
-// bytes): padding repeats the chunk's last record without its charge, for a kernel
-// that takes another form where a pair is far away.
+// lane_walk for the FP64 kernels, whose sums run on from set to set: a chunk is
+// filled with as many sets' records as make whole pairs of trips (up to 64), so that
+// only a wave's last chunk is padded.  (One set at a time, a set of 9 records gave 12
+// copies one trip and a padded one: the shallow-water velocity at degree 2, 24,576
+// leaves of 3 x 3, took 620 us and takes 454; at degree 4, 5 x 5, 867 and 737; the
+// vortex velocity at degree 8, 6 x 6, 411 and 408 at 6 x 192^2.)  add(r0, r1) takes two trips, so that two rows
+// of two records share a reciprocal; an odd last trip is paired with a padding record
+// (slot 79, which no trip reaches).  REPEAT (N = 2, the charge in the last eight bytes):
+// padding repeats the chunk's last record without its charge, for a kernel that takes
+// another form where a pair is far away.
 template <int S, int N, bool REPEAT = false, typename Add>
 __device__ inline void lane_walk2(const TargetTile& T, const SourceSet* __restrict__ sets, const v4f* __restrict__ rec,
                                   const LaneTile& l, v4f* mine, int wave, int lane, Add&& add) {
   static_assert(!REPEAT || N == 2, "lane_walk2: REPEAT knows the layout of two-word records");
   if (!REPEAT) lane_pads<N>(mine, 0.f, lane);
-  walk_sets<S>(T, sets, wave, [&](const SourceSet& set, int a, int b) {
-    for (int c = a; c < b; c += kLaneChunk) {
-      const int cn = min(kLaneChunk, b - c), trips = (cn + l.G - 1) / l.G;
-      const v4f* src = rec + N * ((int64_t)set.first + c);
-      if constexpr (REPEAT) {
-        __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
-        const int k = min(lane, cn - 1);
-        const v4f v0 = src[2 * k], v1 = src[2 * k + 1], last0 = src[2 * cn - 2], last1 = src[2 * cn - 1];
-        mine[2 * lane] = v0;
-        mine[2 * lane + 1] = lane < cn ? v1 : v4f{v1.x, v1.y, 0.f, 0.f};
-        if (lane < kLanePad) {
-          mine[2 * (kLaneChunk + lane)] = last0;
-          mine[2 * (kLaneChunk + lane) + 1] = v4f{last1.x, last1.y, 0.f, 0.f};
-        }
-        __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
-      } else {
-        lane_stage<N>(mine, src, cn, 0.f, lane);
-      }
-      const v4f* r = mine + N * l.g;
-      for (int k = 0; k < trips; k += 2, r += 2 * N * l.G)
-        add(r, k + 1 < trips ? r + N * l.G : mine + N * (kLaneSlots - 1));
+  const int full = kLaneChunk / (2 * l.G) * (2 * l.G);
+  SetWalk<S> part(T, sets, wave);
+  bool more = part.next();
+  while (more) {
+    int src = 0, fill = 0;  // this lane's record, records in the chunk
+    do {
+      const int n = min(full - fill, part.b - part.a), from = part.first + part.a - fill;
+      src = lane >= fill ? from + lane : src;
+      part.a += n;
+      fill += n;
+      if (part.a == part.b) more = part.next();
+    } while (more && fill < full);
+    const int trips = (fill + l.G - 1) / l.G;
+    if (REPEAT) src = lane < fill ? src : __builtin_amdgcn_readlane(src, fill - 1);
+    __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
+    v4f v[N];
+#pragma unroll
+    for (int i = 0; i < N; ++i) v[i] = v4f{0.f, 0.f, 0.f, 0.f};
+    if (REPEAT || lane < fill) {
+#pragma unroll
+      for (int i = 0; i < N; ++i) v[i] = rec[N * (int64_t)src + i];
     }
-  });
+    if constexpr (REPEAT) {
+      if (lane >= fill) v[N - 1].z = v[N - 1].w = 0.f;
+      if (lane < kLanePad) {
+        const int last = __builtin_amdgcn_readlane(src, fill - 1);
+        const v4f l0 = rec[N * (int64_t)last], l1 = rec[N * (int64_t)last + 1];
+        mine[N * (kLaneChunk + lane)] = l0;
+        mine[N * (kLaneChunk + lane) + 1] = v4f{l1.x, l1.y, 0.f, 0.f};
+      }
+    }
+#pragma unroll
+    for (int i = 0; i < N; ++i) mine[N * lane + i] = v[i];
+    __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
+    const v4f* r = mine + N * l.g;
+    for (int k = 0; k < trips; k += 2, r += 2 * N * l.G)
+      add(r, k + 1 < trips ? r + N * l.G : mine + N * (kLaneSlots - 1));
+  }
 }
 
 // Sums w[t][c] over the copies and the S waves into row t T + i of lane

@@ -22,6 +22,39 @@ namespace sbslpm {
 //   2,556 tiles  313 / 195 / 183 / 188    40,956 tiles  2538 / 2358 / 2392 / 2534
 inline int tile_waves(int ntiles) { return ntiles < 1500 ? 16 : ntiles < 6000 ? 8 : 4; }
 
+// Part [a, b) of a set of `count` records for one of SK waves that share it, `turn`
+// rotating the parts from set to set.
+template <int SK>
+__device__ inline void set_part(int count, int turn, int& a, int& b) {
+  a = 0;
+  b = count;
+  if (SK > 1) {
+    const int per = (count + 4 * SK - 1) / (4 * SK) * 4;
+    a = min(count, (turn & (SK - 1)) * per);
+    b = min(count, a + per);
+  }
+}
+
+// This wave's share of a tile's source sets, part by part: records [first + a,
+// first + b) of set e.
+template <int S>
+struct SetWalk {
+  static constexpr int SS = S < 4 ? S : 4, SK = S / SS;  // sets in turn, waves per set
+  const SourceSet* __restrict__ sets;
+  int e, end, wk, it = 0, first = 0, a = 0, b = 0;
+  __device__ SetWalk(const TargetTile& T, const SourceSet* __restrict__ s, int wave)
+      : sets(s), e(T.src_begin + (wave & (SS - 1)) - SS), end(T.src_end), wk(wave / SS) {}
+  // Moves to the next part that is not empty; false at the end.
+  __device__ bool next() {
+    while ((e += SS) < end) {
+      first = sets[e].first;
+      set_part<SK>(sets[e].count, wk + it++, a, b);
+      if (a < b) return true;
+    }
+    return false;
+  }
+};
+
 // f(set, a, b) for this wave's part [a, b) of each of its source sets.
 template <int S, typename F>
 __device__ inline void walk_sets(const TargetTile& T, const SourceSet* __restrict__ sets, int wave, F&& f) {
@@ -30,13 +63,9 @@ __device__ inline void walk_sets(const TargetTile& T, const SourceSet* __restric
   int it = 0;
   for (int e = T.src_begin + ws; e < T.src_end; e += SS, ++it) {
     const SourceSet set = sets[e];
-    if (SK == 1) {
-      f(set, 0, set.count);
-    } else {
-      const int per = (set.count + 4 * SK - 1) / (4 * SK) * 4;
-      const int a = min(set.count, ((wk + it) & (SK - 1)) * per), b = min(set.count, a + per);
-      if (a < b) f(set, a, b);
-    }
+    int a, b;
+    set_part<SK>(set.count, wk + it, a, b);
+    if (SK == 1 || a < b) f(set, a, b);
   }
 }
 

@@ -352,10 +352,13 @@ void launch_swe_interact64(const DevTree& t, int variant, const TargetTile* tile
   }
   // us per launch with 4 / 8 / 16 waves: 126 tiles 49 / 31 / 25, 636 102 / 85 / 91, 2,556 202 / 200 / 246,
   // 10,236 694 / 710 / 903, 40,956 3525 / 3691 / 4706
-  const int S = ntiles < 400 ? 16 : ntiles < 3000 ? 8 : 4;
+  int S = ntiles < 400 ? 16 : ntiles < 3000 ? 8 : 4;
   auto kernel = variant != 2 ? (S == 16 ? k_swe64<1, 16> : S == 8 ? k_swe64<1, 8> : k_swe64<1, 4>)
                              : (S == 16 ? k_swe64<2, 16> : S == 8 ? k_swe64<2, 8> : k_swe64<2, 4>);
-  if (variant != 2 && lanes64(t) && !heaviest_first && S < 16) kernel = S == 8 ? k_swe64_lanes<8> : k_swe64_lanes<4>;
+  if (variant != 2 && lanes64(t) && !heaviest_first && S < 16) {
+    S = lane_waves(ntiles);
+    kernel = S == 8 ? k_swe64_lanes<8> : k_swe64_lanes<4>;
+  }
   hipLaunchKernelGGL(kernel, dim3(heaviest_first ? ntiles : strip_grid(ntiles)), dim3(64 * S), 0, s, t, tiles, ntiles, sets, rec, eps, op, ox,
                      assign ? 1 : 0, heaviest_first ? 1 : 0);
 }
