@@ -124,11 +124,13 @@ __global__ __launch_bounds__(64 * S) void k_swe64(DevTree t, const TargetTile* _
   }
 }
 
-// Variants 1 and 3 in lane copies (lanes.hpp) of two targets, for tiles of at most
-// 42 rows (lanes64).  Microseconds per launch, a row per lane and here: 6 x 96^2
-// (degree 8) 201 -> 192, 6 x 192^2 686 -> 558 (degree 5: 423 -> 341), 6 x 160^2
-// (degree 4, 25 rows) 294 -> 253.
-template <int S>
+// The same in lane copies (lanes.hpp) of two targets, for tiles of at most 42 rows
+// (lanes64).  Microseconds per launch, a row per lane and here: 6 x 96^2 (degree 8)
+// 201 -> 192, 6 x 192^2 686 -> 558 (degree 5: 423 -> 341), 6 x 160^2 (degree 4, 25
+// rows) 294 -> 253.  Variant 2, velocity calls in lane groups, with a row per lane and
+// here: 6 x 96^2 (degree 8) 366, 258, 223; 6 x 192^2 1120, 909, 772; 6 x 160^2 (degree
+// 4) 366, 381, 278; 6 x 320^2 1201, 1396, 1013.
+template <int VARIANT, int S>
 __global__ __launch_bounds__(64 * S) void k_swe64_lanes(DevTree t, const TargetTile* __restrict__ tiles, int ntiles,
                                                         const SourceSet* __restrict__ sets,
                                                         const SrcRecSwe* __restrict__ rec, double eps, Ptr3 part,
@@ -163,10 +165,25 @@ __global__ __launch_bounds__(64 * S) void k_swe64_lanes(DevTree t, const TargetT
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
       const int q = i & 1, k = i >> 1;
-      const double gz = g[i] * qz[k], gd = g[i] * qd[k];
+      const double gz = g[i] * qz[k];
       w[q][0] = fma(gz, a[k], w[q][0]);
       w[q][1] = fma(gz, b[k], w[q][1]);
       w[q][2] = fma(gz, c[k], w[q][2]);
+    }
+    if constexpr (VARIANT == 2) {  // the divergence's pairs are at the undisplaced sources
+#pragma unroll
+      for (int i = 0; i < 2; ++i) {
+        a[i] = R[i]->x0; b[i] = R[i]->y0; c[i] = R[i]->z0;
+      }
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+        d[i] = one_minus_dot(x[i & 1], y[i & 1], z[i & 1], a[i >> 1], b[i >> 1], c[i >> 1]) + eps;
+      rcp4(d, g);
+    }
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const int q = i & 1, k = i >> 1;
+      const double gd = g[i] * qd[k];
       w[q][3] = fma(gd, a[k], w[q][3]);
       w[q][4] = fma(gd, b[k], w[q][4]);
       w[q][5] = fma(gd, c[k], w[q][5]);
@@ -355,9 +372,10 @@ void launch_swe_interact64(const DevTree& t, int variant, const TargetTile* tile
   int S = ntiles < 400 ? 16 : ntiles < 3000 ? 8 : 4;
   auto kernel = variant != 2 ? (S == 16 ? k_swe64<1, 16> : S == 8 ? k_swe64<1, 8> : k_swe64<1, 4>)
                              : (S == 16 ? k_swe64<2, 16> : S == 8 ? k_swe64<2, 8> : k_swe64<2, 4>);
-  if (variant != 2 && lanes64(t) && !heaviest_first && S < 16) {
+  if (lanes64(t) && !heaviest_first && S < 16) {
     S = lane_waves(ntiles);
-    kernel = S == 8 ? k_swe64_lanes<8> : k_swe64_lanes<4>;
+    kernel = variant != 2 ? (S == 8 ? k_swe64_lanes<1, 8> : k_swe64_lanes<1, 4>)
+                          : (S == 8 ? k_swe64_lanes<2, 8> : k_swe64_lanes<2, 4>);
   }
   hipLaunchKernelGGL(kernel, dim3(heaviest_first ? ntiles : strip_grid(ntiles)), dim3(64 * S), 0, s, t, tiles, ntiles, sets, rec, eps, op, ox,
                      assign ? 1 : 0, heaviest_first ? 1 : 0);
