@@ -367,9 +367,9 @@ void launch_bve_adjoint64(const DevTree& t, const TargetTile* tiles, int ntiles,
   auto kernel = dpart ? (S == 16 ? k_bve_adj64<true, 16> : S == 8 ? k_bve_adj64<true, 8> : k_bve_adj64<true, 4>)
                       : (S == 16 ? k_bve_adj64<false, 16> : S == 8 ? k_bve_adj64<false, 8> : k_bve_adj64<false, 4>);
   if (lanes64(t) && S < 16) {
-    S = lane_waves(ntiles);
-    kernel = dpart ? (S == 8 ? k_bve_adj64_lanes<true, 8> : k_bve_adj64_lanes<true, 4>)
-                   : (S == 8 ? k_bve_adj64_lanes<false, 8> : k_bve_adj64_lanes<false, 4>);
+    S = lane_waves64(t, ntiles);
+    kernel = dpart ? (S == 8 ? k_bve_adj64_lanes<true, 8> : S == 4 ? k_bve_adj64_lanes<true, 4> : k_bve_adj64_lanes<true, 1>)
+                   : (S == 8 ? k_bve_adj64_lanes<false, 8> : S == 4 ? k_bve_adj64_lanes<false, 4> : k_bve_adj64_lanes<false, 1>);
   }
   hipLaunchKernelGGL(kernel, dim3(strip_grid(ntiles)), dim3(64 * S), 0, s, t, tiles, ntiles, targets, r, srec, eps, dp,
                      dx, qbar_part, qbar_prox, bp, bx);

@@ -475,21 +475,23 @@ __global__ __launch_bounds__(64 * S) void k_lap64(DevTree t, const TargetTile* _
 // (lanes64).  Microseconds per launch in lane groups of one target, with a row per
 // lane and here: 6 x 96^2 (degree 8) 446, 355, 272; 6 x 192^2 1175, 1010, 770 (degree
 // 5: 594, 571, 453); 6 x 160^2 (degree 4) 366, 419, 339.
-template <int S>
-__global__ __launch_bounds__(64 * S) void k_lap64_lanes(DevTree t, const TargetTile* __restrict__ tiles, int ntiles,
+template <int S, int W>
+__global__ __launch_bounds__(64 * S * W) void k_lap64_lanes(DevTree t, const TargetTile* __restrict__ tiles, int ntiles,
                                                         const SourceSet* __restrict__ sets,
                                                         const SrcRec64* __restrict__ rec, LapCoef64 kp,
                                                         double* __restrict__ part, double* __restrict__ proxy,
                                                         int assign) {
   constexpr int NT = 2;
   __shared__ double etab[kExpNegTabSize];
-  __shared__ __align__(16) double stage[S][kLaneSlots * 4];
-  for (int i = threadIdx.x; i < kExpNegTabSize; i += 64 * S) etab[i] = t.expnegtab[i];
+  __shared__ __align__(16) double stage[W][S][kLaneSlots * 4];
+  for (int i = threadIdx.x; i < kExpNegTabSize; i += 64 * S * W) etab[i] = t.expnegtab[i];
   __syncthreads();
-  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6) % S;
+  const int sub = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6) / S;
   const int lane = threadIdx.x & 63;
-  const int tile = strip_tile(ntiles);
-  if (tile >= ntiles) return;  // the whole workgroup
+  static_assert(S == 1 || W == 1, "waves that share a tile meet at barriers: one tile per workgroup");
+  const int tile = strip_tile((ntiles + W - 1) / W) * W + sub;
+  if (tile >= ntiles) return;  // all waves of the tile
   const TargetTile T = tiles[tile];
   const LaneTile l = lane_tile<NT>(T.count, lane);
   const double fast_from = kp.cut < -1.0 ? kp.t_sat : 4.0;
@@ -501,7 +503,7 @@ __global__ __launch_bounds__(64 * S) void k_lap64_lanes(DevTree t, const TargetT
     x[q] = t.px[u]; y[q] = t.py[u]; z[q] = t.pz[u];
     w[q][0] = 0;
   }
-  lane_walk2<S, 2, true>(T, sets, reinterpret_cast<const v4f*>(rec), l, reinterpret_cast<v4f*>(stage[wave]), wave, lane,
+  lane_walk2<S, 2, true>(T, sets, reinterpret_cast<const v4f*>(rec), l, reinterpret_cast<v4f*>(stage[sub][wave]), wave, lane,
                          [&](const v4f* r0, const v4f* r1) {
     const SrcRec64 R[2] = {*reinterpret_cast<const SrcRec64*>(r0), *reinterpret_cast<const SrcRec64*>(r1)};
     double dp[4];
@@ -524,7 +526,7 @@ __global__ __launch_bounds__(64 * S) void k_lap64_lanes(DevTree t, const TargetT
     }
   });
   double s[1];
-  lane_sum<NT, 1, S>(l, w, stage, wave, lane, s);
+  lane_sum<NT, 1, S>(l, w, stage[sub], wave, lane, s);
   if (wave == 0 && lane < T.count) store_s(t, (int64_t)T.first + lane, part, proxy, s[0], assign);
 }
 
@@ -1205,8 +1207,8 @@ void launch_bve_interact64(const DevTree& t, const TargetTile* tiles, int ntiles
   int S = tile_waves(ntiles);
   auto kernel = S == 16 ? k_bve64<16> : S == 8 ? k_bve64<8> : k_bve64<4>;
   if (lanes64(t) && S < 16) {
-    S = lane_waves(ntiles);
-    kernel = S == 8 ? k_bve64_lanes<8> : k_bve64_lanes<4>;
+    S = lane_waves64(t, ntiles);
+    kernel = S == 8 ? k_bve64_lanes<8> : S == 4 ? k_bve64_lanes<4> : k_bve64_lanes<1>;
   }
   hipLaunchKernelGGL(kernel, dim3(walk_grid(ntiles, shape), nmem), dim3(64 * S), 0, s, t, tiles, ntiles, sets, rec, eps,
                      ptr3(out_part), ptr3(out_proxy), assign ? 1 : 0, shape.xcd);
@@ -1237,11 +1239,12 @@ void launch_laplacian_interact64(const DevTree& t, const TargetTile* tiles, int 
   int S = ntiles < 400 ? 16 : 4;
   auto kernel = S == 16 ? k_lap64<16> : k_lap64<4>;
   if (lanes64(t) && S < 16) {
-    S = lane_waves(ntiles);
-    kernel = S == 8 ? k_lap64_lanes<8> : k_lap64_lanes<4>;
+    S = lane_waves64(t, ntiles);
+    kernel = S == 8 ? k_lap64_lanes<8, 1> : S == 4 ? k_lap64_lanes<4, 1> : k_lap64_lanes<1, 8>;
   }
-  hipLaunchKernelGGL(kernel, dim3(strip_grid(ntiles)), dim3(64 * S), 0, s, t, tiles, ntiles, sets, rec, kp, out_part, out_proxy,
-                     assign ? 1 : 0);
+  const int per = S > 1 ? 1 : 8;  // tiles per workgroup
+  hipLaunchKernelGGL(kernel, dim3(strip_grid((ntiles + per - 1) / per)), dim3(64 * S * per), 0, s, t, tiles, ntiles,
+                     sets, rec, kp, out_part, out_proxy, assign ? 1 : 0);
 }
 
 void launch_laplacian_interact_mixed(const DevTree& t, const TargetTile* tiles, int ntiles, const SourceSet* sets,

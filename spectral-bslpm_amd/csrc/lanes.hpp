@@ -79,6 +79,14 @@ __device__ inline void lane_pads(v4f* mine, float first, int lane) {
 // FP64 shallow-water velocity at degree 4, microseconds per call with 2 / 4 / 8 waves:
 // 510 tiles 50 / 36 / 36, 2,046 78 / 76 / 91, 8,190 211 / 209 / 282.)
 inline int lane_waves(int ntiles) { return ntiles < 1000 ? 8 : 4; }
+// The FP64 kernels on long lists of tiles of at most 16 rows: one wave, whose walk of
+// short sets costs less than adding the sums of four.  (Shallow-water velocity at
+// degree 2, 3 x 3 points a leaf, with 4 waves and one: 6 x 96^2 148 and 121 us, 6 x
+// 192^2 454 and 315; at 6 x 48^2, 2,046 tiles, 66 and 67.  The Laplacian kernel puts
+// eight such tiles behind one copy of its 30 KB table: 401 and 271 us at 6 x 192^2.)
+inline int lane_waves64(const DevTree& t, int ntiles) {
+  return tile_rows(t) <= 16 && ntiles >= 6000 ? 1 : lane_waves(ntiles);
+}
 
 // Walks a wave's share of the source sets of a tile: begin(set) and flush(set)
 // around each part of a set, add(r) for each trip, r the lane's record (N 16-byte
@@ -185,7 +193,10 @@ __device__ inline void lane_sum(const LaneTile& l, double (&w)[NT][K], double (*
       if (t * l.T + lane < 64)
 #pragma unroll
         for (int c = 0; c < K; ++c) mine[c * 64 + t * l.T + lane] = v[t][c];
-  __syncthreads();
+  if constexpr (S > 1)
+    __syncthreads();
+  else
+    __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
   if (wave == 0)
 #pragma unroll
     for (int c = 0; c < K; ++c) {

@@ -373,9 +373,9 @@ void launch_swe_interact64(const DevTree& t, int variant, const TargetTile* tile
   auto kernel = variant != 2 ? (S == 16 ? k_swe64<1, 16> : S == 8 ? k_swe64<1, 8> : k_swe64<1, 4>)
                              : (S == 16 ? k_swe64<2, 16> : S == 8 ? k_swe64<2, 8> : k_swe64<2, 4>);
   if (lanes64(t) && !heaviest_first && S < 16) {
-    S = lane_waves(ntiles);
-    kernel = variant != 2 ? (S == 8 ? k_swe64_lanes<1, 8> : k_swe64_lanes<1, 4>)
-                          : (S == 8 ? k_swe64_lanes<2, 8> : k_swe64_lanes<2, 4>);
+    S = lane_waves64(t, ntiles);
+    kernel = variant != 2 ? (S == 8 ? k_swe64_lanes<1, 8> : S == 4 ? k_swe64_lanes<1, 4> : k_swe64_lanes<1, 1>)
+                          : (S == 8 ? k_swe64_lanes<2, 8> : S == 4 ? k_swe64_lanes<2, 4> : k_swe64_lanes<2, 1>);
   }
   hipLaunchKernelGGL(kernel, dim3(heaviest_first ? ntiles : strip_grid(ntiles)), dim3(64 * S), 0, s, t, tiles, ntiles, sets, rec, eps, op, ox,
                      assign ? 1 : 0, heaviest_first ? 1 : 0);
