@@ -460,6 +460,7 @@ int sbslpm_ctx_create(const sbslpm_params* p, sbslpm_ctx** out) {
   d.P = t.P; d.Pl = t.Pl; d.offset = t.offset; d.n = t.n; d.dp1 = t.dp1; d.m = t.m; d.m2 = t.m2;
   d.levels = t.cfg.levels; d.npart = t.npart; d.U = t.U;
   d.m2p = t.m2p; d.np16 = t.np16; d.U16 = t.U16;
+  d.rows = fullest_tile(t.tiles);
   c->tiles = (TargetTile*)(b + o_tiles);
   c->sets = (SourceSet*)(b + o_sets);
   c->ntiles = (int)t.tiles.size();
@@ -1941,6 +1942,7 @@ int sbslpm_irreg_create(sbslpm_ctx* c, int64_t n, const double* x, const double*
   d.P = t.P; d.Pl = (int)leaves.size(); d.offset = t.P;  // every proxy row may be an interaction source
   d.n = t.n; d.dp1 = t.dp1; d.m = 0; d.m2 = 0; d.levels = t.levels;
   d.npart = t.N; d.U = t.U; d.m2p = 0; d.np16 = 0; d.U16 = 0;
+  d.rows = mean_tile(t.tiles, t.sets);
   h->perm = (int*)(b + o_perm);
   h->leaf_first = (int*)(b + o_lf);
   h->leaf_count = (int*)(b + o_lc);

@@ -46,6 +46,7 @@ struct DevTree {
   int* err;
   int bf16_m2l;               // matrix-core kernels take bf16 kernel-product operands for M2L sets
   int P, Pl, offset, n, dp1, m, m2, levels;
+  int rows;  // per target tile (tree.hpp)
   int64_t npart, U;
   int m2p, np16;  // m2, n rounded up to 16
   int64_t U16;    // padded record count of the MFMA kernels

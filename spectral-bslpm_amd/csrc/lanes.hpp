@@ -19,19 +19,13 @@ constexpr int kLaneChunk = 64;               // records staged at a time, one pe
 constexpr int kLanePad = 16;                 // copies at most, padding of a chunk at most kLanePad - 1
 constexpr int kLaneSlots = kLaneChunk + kLanePad;
 
-// Rows of the fullest tile of a context (a panel's points in equal tiles of at
-// most 64).  The FP64 kernels, bound by issue with scalar records at no LDS
-// cost, take lane copies where those fill more of the wave: with two rows per
-// lane three or more copies of at most 42 rows (36 rows use 54 lanes' worth
-// twice over against 36 of 64).
-inline int tile_rows(const DevTree& t) {
-  auto rows = [](int c) {
-    const int tiles = (c + 63) / 64;
-    return tiles > 0 ? (c + tiles - 1) / tiles : 0;
-  };
-  return rows(t.m2) > rows(t.n) ? rows(t.m2) : rows(t.n);
-}
-inline bool lanes64(const DevTree& t) { return tile_rows(t) <= 42; }
+// The FP64 kernels, bound by issue with scalar records at no LDS cost, take lane
+// copies where those fill more of the wave: with two rows per lane three or more
+// copies of at most 42 rows (36 rows use 54 lanes' worth twice over against 36 of
+// 64).  Vortex velocity on the 1 degree lat-lon grid's tree, a row per lane and here:
+// mean 28 rows 140 and 126 us, 35 rows 157 and 147, 40 rows 358 and 317; 46 rows (degree
+// 6) 186 and 196, 48 rows 190 and 206.
+inline bool lanes64(const DevTree& t) { return t.rows <= 42; }
 
 struct LaneTile {
   int T, G, g, i;  // lanes per copy, copies, this lane's copy and lane within it
@@ -85,7 +79,7 @@ inline int lane_waves(int ntiles) { return ntiles < 1000 ? 8 : 4; }
 // 192^2 454 and 315; at 6 x 48^2, 2,046 tiles, 66 and 67.  The Laplacian kernel puts
 // eight such tiles behind one copy of its 30 KB table: 401 and 271 us at 6 x 192^2.)
 inline int lane_waves64(const DevTree& t, int ntiles) {
-  return tile_rows(t) <= 16 && ntiles >= 6000 ? 1 : lane_waves(ntiles);
+  return t.rows <= 16 && ntiles >= 6000 ? 1 : lane_waves(ntiles);
 }
 
 // Walks a wave's share of the source sets of a tile: begin(set) and flush(set)

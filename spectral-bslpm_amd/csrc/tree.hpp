@@ -66,6 +66,24 @@ struct SourceSet {
 // (pairwalk.hpp), what a long one loses without its locality at strip_length.
 constexpr int kBalancedTiles = 6000;
 
+// Rows that decide how a list's pair kernels lay out a tile: the fullest tile's of a
+// uniform tree, whose tiles differ little; of an irregular one, whose tiles hold from
+// one row to 64, the mean over the source points that the tiles' waves walk.
+inline int fullest_tile(const std::vector<TargetTile>& tiles) {
+  int rows = 0;
+  for (const TargetTile& t : tiles) rows = t.count > rows ? t.count : rows;
+  return rows;
+}
+inline int mean_tile(const std::vector<TargetTile>& tiles, const std::vector<SourceSet>& sets) {
+  int64_t rows = 0, walked = 0;
+  for (const TargetTile& t : tiles)
+    for (int e = t.src_begin; e < t.src_end; ++e) {
+      walked += sets[e].count;
+      rows += (int64_t)sets[e].count * t.count;
+    }
+  return walked > 0 ? (int)((rows + walked / 2) / walked) : 0;
+}
+
 struct Tree {
   TreeConfig cfg{};
   int P = 0, Pl = 0, offset = 0, n = 0, dp1 = 0, m = 0, m2 = 0;
