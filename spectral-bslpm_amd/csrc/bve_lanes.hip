@@ -63,9 +63,7 @@ __global__ void k_src_lanes(DevTree t, const double* __restrict__ q_part, const 
   rec[2 * u + 1] = v4f{(float)(qq * bx), (float)(qq * by), (float)(qq * bz), (float)qq};
 }
 
-constexpr int NT = 2;  // targets per lane
-
-template <int S>
+template <int S, int NT>
 __global__ __launch_bounds__(64 * S) void k_bve_lanes(DevTree t, const TargetTile* __restrict__ tiles, int ntiles,
                                                       const SourceSet* __restrict__ sets, const v4f* __restrict__ rec,
                                                       float eps, Ptr3 part, Ptr3 proxy, int assign, int xcd) {
@@ -185,8 +183,20 @@ void launch_bve_interact_lanes(const DevTree& t, const TargetTile* tiles, int nt
   if (shape.xcd == 2 && (!t.xcd_start || shape.grid1 <= 0)) shape.xcd = 0;
   // us per launch with 4 / 8 waves: 126 tiles 25 / 20, 636 47 / 46, 2,556 (36 rows) 83 / 87, 10,236 267 / 302,
   // 40,956 1490 / 1562
-  const int S = lane_waves(ntiles);
-  auto kernel = S == 8 ? k_bve_lanes<8> : k_bve_lanes<4>;
+  // (with members a short list fills the chip and 8 waves' sums cost more than they gain:
+  // 16 members at 510 tiles of 25 rows 747 us a step, 551 with 4 waves, a single step 168 and
+  // 166; at 36 rows and more 2% to 3% of a single step, so 8 stay)
+  int S = t.rows <= 32 && ntiles >= 400 ? 4 : lane_waves(ntiles);
+  auto kernel = S == 8 ? k_bve_lanes<8, 2> : k_bve_lanes<4, 2>;
+  // tiles of at most 16 rows: one target per lane halves what a set costs to centre and
+  // flush, and sets of 9 records give fewer waves enough.  Velocity at degree 2, 3 x 3
+  // points a leaf, with two targets and 4 waves, and with one and 4 / 2 / 1: 2,046 tiles
+  // 42, 38 / 42 / 54 us; 8,190 99, 86 / 86 / 91; 32,766 300, 254 / 237 / 231; a step of 16
+  // members at 2,046 tiles 1,182, 993 / 927 / 900
+  if (t.rows <= 16) {
+    S = ntiles < 1000 ? 4 : 2;
+    kernel = S == 4 ? k_bve_lanes<4, 1> : k_bve_lanes<2, 1>;
+  }
   Ptr3 op{{out_part[0], out_part[1], out_part[2]}}, ox{{out_proxy[0], out_proxy[1], out_proxy[2]}};
   hipLaunchKernelGGL(kernel, dim3(walk_grid(ntiles, shape), nmem), dim3(64 * S), 0, s, t, tiles, ntiles, sets,
                      static_cast<const v4f*>(rec), (float)eps, op, ox, assign ? 1 : 0, shape.xcd);

@@ -270,18 +270,27 @@ const HostTables& host_tables() {
 int velocity(sbslpm_ctx* c, const Work& w, int nmem, const double* area, const double* vor,
              const double* const* dpart, const double* const* dprox, double* const* vel);
 
-// Source records and pair sums of a mixed-precision context: the vector unit in
-// lane copies, or the matrix cores where bf16 M2L products are asked for.
+// Whether the vortex pairs of a mixed-precision context run on the matrix cores:
+// where bf16 M2L products are asked for, and on long lists of tiles of 13 to 16 rows,
+// which fill a 16 x 16 block per source set.  (Velocity at degree 3, 4 x 4 points a leaf,
+// 32,766 tiles, on the vector unit 268 us and here 240; a step of 16 members at 2,046
+// tiles 1,074 and 948, at 510 tiles 369 and 361, where a single step takes 157 and 181.
+// Distance from FP64 at 2,046 tiles 4.7e-8 and 5.1e-8.)
+bool matrix_pairs(const sbslpm_ctx* c) {
+  return c->dt.bf16_m2l || (c->dt.rows > 12 && c->dt.rows <= 16 && c->ntiles >= 1000);
+}
+
+// Source records and pair sums of a mixed-precision context.
 void mixed_records(sbslpm_ctx* c, const double* q_part, const double* q_proxy, const double* const* dpart,
                    const double* const* dprox, SrcRecMfma* rec, int nmem = 1) {
-  if (c->dt.bf16_m2l)
+  if (matrix_pairs(c))
     launch_source_records_mfma(c->dt, q_part, q_proxy, dpart, dprox, rec, c->stream, nmem);
   else
     launch_source_records_lanes(c->dt, q_part, q_proxy, dpart, dprox, rec, c->stream, nmem);
 }
 void mixed_pairs(sbslpm_ctx* c, const SrcRecMfma* rec, double* const* out_part, double* const* out_proxy, bool assign,
                  int nmem, PairShape shape) {
-  if (c->dt.bf16_m2l)
+  if (matrix_pairs(c))
     launch_bve_interact_mfma(c->dt, c->tiles, c->ntiles, c->sets, rec, c->prm.kernel_eps, out_part, out_proxy,
                              c->stream, assign, nmem, shape);
   else

@@ -236,18 +236,19 @@ __global__ void k_src_swe32(DevTree t, const double* __restrict__ qz_part, const
 // x cross y = x cross d and y - x (x.y) = d - x (x.d), so
 //   u = x cross sum(g qz d) + E - x (x.E),   E = sum(g qd d),   g = 1/(h + eps).
 // FP32 partial sums per source set are added into FP64; the cross product, the
-// projection and the output are FP64.  Lane copies (lanes.hpp) of two targets.
+// projection and the output are FP64.  Lane copies (lanes.hpp) of two targets, or of
+// one whose trips feed two sums in turn.
 // Bound: FP32 vector issue, 15 instructions and a reciprocal per pair.
 // Microseconds per launch before (one wave per tile with scalar records, or lane
 // groups of one target) and with 2 / 4 / 8 waves per tile: 126 tiles 115, 53 / 32 /
 // 25; 636 380, 106 / 67 / 65; 2,556 (36 rows) 187, 130 / 117 / 123; 10,236 543, 387 /
 // 390 / 432; 40,956 2931, 2268 / 2231 / 2318.
-template <int S>
+template <int S, int NT>
 __global__ __launch_bounds__(64 * S) void k_swe_lanes(DevTree t, const TargetTile* __restrict__ tiles, int ntiles,
                                                       const SourceSet* __restrict__ sets,
                                                       const SrcRecSwe32* __restrict__ rec, float eps, Ptr3 part,
                                                       Ptr3 proxy, int assign) {
-  constexpr int NT = 2, K = 6;
+  constexpr int K = 6;
   __shared__ __align__(16) double stage[S][64 * K];
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int lane = threadIdx.x & 63;
@@ -256,7 +257,7 @@ __global__ __launch_bounds__(64 * S) void k_swe_lanes(DevTree t, const TargetTil
   const TargetTile T = tiles[tile];
   const DevPanel& PT = t.panels[T.panel];
   const LaneTile l = lane_tile<NT>(T.count, lane);
-  float ax[NT], ay[NT], az[NT], px[NT], py[NT], pz[NT], v[NT][K];
+  float ax[NT], ay[NT], az[NT], px[NT], py[NT], pz[NT], v[2][K];
   double w[NT][K];
 #pragma unroll
   for (int q = 0; q < NT; ++q) {
@@ -275,9 +276,9 @@ __global__ __launch_bounds__(64 * S) void k_swe_lanes(DevTree t, const TargetTil
           px[q] = ax[q] + set.ox;
           py[q] = ay[q] + set.oy;
           pz[q] = az[q] + set.oz;
-#pragma unroll
-          for (int k = 0; k < K; ++k) v[q][k] = 0.f;
         }
+#pragma unroll
+        for (int k = 0; k < K; ++k) v[0][k] = v[1][k] = 0.f;
       },
       [&](const v4f* r) {
         const v4f s = r[0];
@@ -294,12 +295,19 @@ __global__ __launch_bounds__(64 * S) void k_swe_lanes(DevTree t, const TargetTil
           v[q][4] = fmaf(gd, d1, v[q][4]);
           v[q][5] = fmaf(gd, d2, v[q][5]);
         }
+        if constexpr (NT == 1)
+#pragma unroll
+          for (int k = 0; k < K; ++k) {
+            const float even = v[0][k];
+            v[0][k] = v[1][k];
+            v[1][k] = even;
+          }
       },
       [&](const SourceSet&) {
 #pragma unroll
-        for (int q = 0; q < NT; ++q)
+        for (int q = 0; q < 2; ++q)
 #pragma unroll
-          for (int k = 0; k < K; ++k) w[q][k] += v[q][k];
+          for (int k = 0; k < K; ++k) w[q < NT ? q : 0][k] += v[q][k];
       });
   double s[K];
   lane_sum<NT, K, S>(l, w, stage, wave, lane, s);
@@ -339,8 +347,16 @@ void launch_swe_interact_mixed(const DevTree& t, const TargetTile* tiles, int nt
     op.p[f] = out_part[f];
     ox.p[f] = out_proxy[f];
   }
-  const int S = lane_waves(ntiles);
-  hipLaunchKernelGGL(S == 8 ? k_swe_lanes<8> : k_swe_lanes<4>, dim3(strip_grid(ntiles)), dim3(64 * S), 0, s, t, tiles, ntiles, sets, rec, (float)eps, op,
+  int S = lane_waves(ntiles);
+  auto kernel = S == 8 ? k_swe_lanes<8, 2> : k_swe_lanes<4, 2>;
+  // one target per lane as in bve_lanes.hip: velocity at degree 2 with two targets and 4
+  // waves, and with one and 4 / 2 / 1: 2,046 tiles 63, 56 / 60 / 72 us; 8,190 135, 115 / 113 /
+  // 118; 32,766 409, 321 / 296 / 289
+  if (t.rows <= 16) {
+    S = ntiles < 6000 ? 4 : 2;
+    kernel = S == 4 ? k_swe_lanes<4, 1> : k_swe_lanes<2, 1>;
+  }
+  hipLaunchKernelGGL(kernel, dim3(strip_grid(ntiles)), dim3(64 * S), 0, s, t, tiles, ntiles, sets, rec, (float)eps, op,
                      ox, assign ? 1 : 0);
 }
 

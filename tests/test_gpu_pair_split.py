@@ -13,7 +13,7 @@ pytestmark = pytest.mark.gpu
 EPS = 1e-4
 # levels, proxy degree, leaf grid side: tile lists of 30 to 8,190; 9 and 16 rows, where a chunk of
 # staged records spans several sets
-TREES = [(2, 4, 5), (3, 6, 7), (3, 8, 9), (4, 10, 11), (5, 8, 6), (6, 5, 6), (4, 2, 3), (5, 3, 4)]
+TREES = [(2, 4, 5), (3, 6, 7), (3, 8, 9), (4, 10, 11), (5, 8, 6), (6, 5, 6), (4, 2, 3), (5, 3, 4), (6, 2, 3)]
 
 
 @pytest.fixture(scope="module", params=TREES, ids=lambda p: "L%d-d%d-m%d" % p)
