@@ -229,14 +229,20 @@ int upload(sbslpm_ctx* c, void* dst, const void* src, size_t bytes) {
   return SBSLPM_OK;
 }
 
+// k_bve_mixed puts four tiles on a workgroup, and four of the heaviest on each of the
+// first of a short list: breadth first, with the ranges of that order, below 2,500 tiles
+// (velocity at 636 tiles by work 265 us and breadth first 229, at 2,046 123 and 117, at
+// 2,556 of 36 rows 197 and 204, at 4,092 323 and 358).
+static bool valu_bfs(const Tree& t) { return t.tiles.size() < 2500; }
+
 // A launch shape for the context's full target-major tile list: with the
 // cost-balanced XCD mapping (xcd 2) the grid is 8 x the largest XCD range in
-// workgroups of `waves` tiles, for the ranges of the matrix-core kernels
-// (mfma) or of the vector-unit ones.
-static PairShape full_list_shape(const Tree& t, int waves, int xcd, bool mfma) {
+// workgroups of `waves` tiles, for the ranges that the precision's kernels take.
+static PairShape full_list_shape(const Tree& t, int waves, int xcd, int precision) {
   PairShape sh{waves, xcd, 0, 0};
   if (xcd == 2) {
-    const int* xs = t.xcd_start.data() + (mfma ? 0 : 9);
+    const int* xs = t.xcd_start.data() + (precision == SBSLPM_MIXED ? 0 : 9);
+    if (precision == SBSLPM_MIXED_VALU && valu_bfs(t)) xs += 18;
     int most = 0, tiles = 0;
     for (int x = 0; x < 8; ++x) {
       most = std::max(most, (xs[x + 1] - xs[x] + waves - 1) / waves);
@@ -280,6 +286,23 @@ bool matrix_pairs(const sbslpm_ctx* c) {
   return c->dt.bf16_m2l || (c->dt.rows > 12 && c->dt.rows <= 16 && c->ntiles >= 1000);
 }
 
+// The tile list of a launch: by work, but breadth first where each XCD takes an equal
+// count of neighbours (mapping 1; velocity at 6 x 128^2, degree 8, FP64: 220 us by work
+// and 198).  With equal work per XCD (mapping 2) the order by work is as good or
+// better (6 x 64^2 62 us against 69, 6 x 128^2 185 against 183).
+const TargetTile* pair_tiles(const sbslpm_ctx* c, const PairShape& shape) {
+  return shape.xcd == 1 ? c->bfs_tiles : c->tiles;
+}
+
+void valu_pairs(sbslpm_ctx* c, const SrcRec32* rec, double* const* out_part, double* const* out_proxy, bool assign,
+                int nmem, const PairShape& shape) {
+  DevTree dt = c->dt;
+  const bool bfs = valu_bfs(c->tree);
+  if (bfs) dt.xcd_start += 18;
+  launch_bve_interact_mixed(dt, bfs ? c->bfs_tiles : c->tiles, c->ntiles, c->sets, rec, c->prm.kernel_eps, out_part, out_proxy, c->stream,
+                            assign, nmem, shape);
+}
+
 // Source records and pair sums of a mixed-precision context.
 void mixed_records(sbslpm_ctx* c, const double* q_part, const double* q_proxy, const double* const* dpart,
                    const double* const* dprox, SrcRecMfma* rec, int nmem = 1) {
@@ -291,10 +314,10 @@ void mixed_records(sbslpm_ctx* c, const double* q_part, const double* q_proxy, c
 void mixed_pairs(sbslpm_ctx* c, const SrcRecMfma* rec, double* const* out_part, double* const* out_proxy, bool assign,
                  int nmem, PairShape shape) {
   if (matrix_pairs(c))
-    launch_bve_interact_mfma(c->dt, c->tiles, c->ntiles, c->sets, rec, c->prm.kernel_eps, out_part, out_proxy,
+    launch_bve_interact_mfma(c->dt, pair_tiles(c, shape), c->ntiles, c->sets, rec, c->prm.kernel_eps, out_part, out_proxy,
                              c->stream, assign, nmem, shape);
   else
-    launch_bve_interact_lanes(c->dt, c->tiles, c->ntiles, c->sets, rec, c->prm.kernel_eps, out_part, out_proxy,
+    launch_bve_interact_lanes(c->dt, pair_tiles(c, shape), c->ntiles, c->sets, rec, c->prm.kernel_eps, out_part, out_proxy,
                               c->stream, assign, nmem, shape);
 }
 
@@ -396,7 +419,7 @@ int sbslpm_ctx_create(const sbslpm_params* p, sbslpm_ctx** out) {
   size_t o_vstage = A.take<double>(9 * NP), o_newvor = A.take<double>(NP), o_dep = A.take<double>(3 * NP);
   size_t o_vnext = A.take<double>(NP), o_trnext = A.take<double>(NP * ntr);
   size_t o_ltab = A.take<LogTabEntry>(kLogTabSize), o_lwide = A.take<LogTabEntry>(kLogWideSize), o_etab = A.take<double>(kExpTabSize),
-         o_entab = A.take<double>(kExpNegTabSize), o_xcd = A.take<int>(18);
+         o_entab = A.take<double>(kExpNegTabSize), o_xcd = A.take<int>(t.xcd_start.size());
   size_t total = A.take<char>(256);
   if (hipMalloc(&c->arena, total) != hipSuccess) {
     delete c;
@@ -437,7 +460,7 @@ int sbslpm_ctx_create(const sbslpm_params* p, sbslpm_ctx** out) {
     rc |= upload(c, b + o_etab, ht.exp.data(), kExpTabSize * sizeof(double));
     rc |= upload(c, b + o_entab, ht.exp_neg.data(), kExpNegTabSize * sizeof(double));
   }
-  rc |= upload(c, b + o_xcd, t.xcd_start.data(), 18 * sizeof(int));
+  rc |= upload(c, b + o_xcd, t.xcd_start.data(), t.xcd_start.size() * sizeof(int));
   if (rc != SBSLPM_OK || hipMemset(b + o_err, 0, 4 * sizeof(int)) != hipSuccess) {
     hipFree(c->arena);
     delete c;
@@ -565,7 +588,7 @@ int sbslpm_ctx_set_precision(sbslpm_ctx* c, int precision) {
   }
   c->prm.precision = precision;
   // the balanced XCD ranges (and so the grid) differ between matrix-core and vector-unit kernels
-  c->shape = full_list_shape(c->tree, c->shape.waves, c->shape.xcd, precision == SBSLPM_MIXED);
+  c->shape = full_list_shape(c->tree, c->shape.waves, c->shape.xcd, precision);
   return SBSLPM_OK;
 }
 
@@ -662,7 +685,7 @@ int sbslpm_bve_vel_interactions(sbslpm_ctx* c, const double* dpx, const double* 
   } else if (c->prm.precision == SBSLPM_MIXED_VALU) {
     launch_source_records32(c->dt, q_part, q_proxy, dpp, dxp, c->rec32, c->stream);
     KernelTimer tm(c, SBSLPM_KERNEL_BVE_MIXED);
-    launch_bve_interact_mixed(c->dt, c->tiles, c->ntiles, c->sets, c->rec32, c->prm.kernel_eps, op, ox, c->stream);
+    valu_pairs(c, c->rec32, op, ox, false, 1, {});
   } else {
     launch_source_records64(c->dt, q_part, q_proxy, dpp, dxp, true, c->rec64, c->stream);
     KernelTimer tm(c, SBSLPM_KERNEL_BVE_FP64);
@@ -911,8 +934,9 @@ int velocity(sbslpm_ctx* c, const Work& w, int nmem, const double* area, const d
     const int cb = c->mrhs_cb ? c->mrhs_cb : mrhs_chunks_per_wave(nmem);
     launch_source_columns_mrhs(c->dt, w.qpart, w.qproxy, w.recmf, nmem, cb, w.qcol, c->stream);
     KernelTimer tm(c, SBSLPM_KERNEL_BVE_MRHS);
-    launch_bve_interact_mrhs(c->dt, c->tiles, c->ntiles, c->sets, w.recmf, w.qcol, nmem, cb, c->prm.kernel_eps,
-                             w.phipart, w.phiproxy, c->stream, true, c->mrhs_cb ? c->mrhs_shape : c->shape);
+    const PairShape& sh = c->mrhs_cb ? c->mrhs_shape : c->shape;
+    launch_bve_interact_mrhs(c->dt, pair_tiles(c, sh), c->ntiles, c->sets, w.recmf, w.qcol, nmem, cb,
+                             c->prm.kernel_eps, w.phipart, w.phiproxy, c->stream, true, sh);
   } else if (c->prm.precision == SBSLPM_MIXED) {
     mixed_records(c, w.qpart, w.qproxy, dpart, dprox, w.recmf, nmem);
     KernelTimer tm(c, SBSLPM_KERNEL_BVE_MIXED);
@@ -920,13 +944,12 @@ int velocity(sbslpm_ctx* c, const Work& w, int nmem, const double* area, const d
   } else if (c->prm.precision == SBSLPM_MIXED_VALU) {
     launch_source_records32(c->dt, w.qpart, w.qproxy, dpart, dprox, w.rec32, c->stream, nmem);
     KernelTimer tm(c, SBSLPM_KERNEL_BVE_MIXED);
-    launch_bve_interact_mixed(c->dt, c->tiles, c->ntiles, c->sets, w.rec32, c->prm.kernel_eps, w.phipart,
-                              w.phiproxy, c->stream, true, nmem, c->shape);
+    valu_pairs(c, w.rec32, w.phipart, w.phiproxy, true, nmem, c->shape);
   } else {
     launch_source_records64(c->dt, w.qpart, w.qproxy, dpart, dprox, true, w.rec64, c->stream, nmem);
     KernelTimer tm(c, SBSLPM_KERNEL_BVE_FP64);
-    launch_bve_interact64(c->dt, c->tiles, c->ntiles, c->sets, w.rec64, c->prm.kernel_eps, w.phipart, w.phiproxy,
-                          c->stream, true, nmem, c->shape);
+    launch_bve_interact64(c->dt, pair_tiles(c, c->shape), c->ntiles, c->sets, w.rec64, c->prm.kernel_eps, w.phipart,
+                          w.phiproxy, c->stream, true, nmem, c->shape);
   }
   const double* pp[3] = {w.phipart[0], w.phipart[1], w.phipart[2]};
   launch_downward_pass(c->dt, 3, w.phiproxy, pp, vel, c->stream, true, nmem);
@@ -1745,11 +1768,10 @@ int sbslpm_autotune(sbslpm_ctx* c, const double* area, const double* vor, double
     if (prec == SBSLPM_MIXED)
       mixed_pairs(c, w.recmf, w.phipart, w.phiproxy, true, 1, sh);
     else if (prec == SBSLPM_MIXED_VALU)
-      launch_bve_interact_mixed(c->dt, c->tiles, c->ntiles, c->sets, w.rec32, c->prm.kernel_eps, w.phipart,
-                                w.phiproxy, c->stream, true, 1, sh);
+      valu_pairs(c, w.rec32, w.phipart, w.phiproxy, true, 1, sh);
     else
-      launch_bve_interact64(c->dt, c->tiles, c->ntiles, c->sets, w.rec64, c->prm.kernel_eps, w.phipart, w.phiproxy,
-                            c->stream, true, 1, sh);
+      launch_bve_interact64(c->dt, pair_tiles(c, sh), c->ntiles, c->sets, w.rec64, c->prm.kernel_eps, w.phipart,
+                            w.phiproxy, c->stream, true, 1, sh);
   };
   hipEvent_t e0, e1;
   HIP_TRY(c, hipEventCreate(&e0));
@@ -1760,7 +1782,7 @@ int sbslpm_autotune(sbslpm_ctx* c, const double* area, const double* vor, double
   int k = 0;
   for (int xcd = 0; xcd < 3; ++xcd)
     for (int wi = 0; wi < 3; ++wi) {
-      const PairShape sh = full_list_shape(c->tree, waves[wi], xcd, prec == SBSLPM_MIXED);
+      const PairShape sh = full_list_shape(c->tree, waves[wi], xcd, prec);
       launch(sh);  // warm-up
       hipEventRecord(e0, c->stream);
       for (int r = 0; r < 3; ++r) launch(sh);
@@ -1806,7 +1828,7 @@ int sbslpm_set_pair_shape(sbslpm_ctx* c, int waves, int xcd) {
   if (c->capturing) return fail(c, SBSLPM_E_ARG, "set_pair_shape: not allowed during graph capture");
   if (waves != c->shape.waves || xcd != c->shape.xcd) {
     HIP_TRY(c, hipStreamSynchronize(c->stream));
-    c->shape = full_list_shape(c->tree, waves, xcd, c->prm.precision == SBSLPM_MIXED);
+    c->shape = full_list_shape(c->tree, waves, xcd, c->prm.precision);
     if (c->graph) {
       hipGraphExecDestroy(c->graph);
       c->graph = nullptr;
@@ -2714,9 +2736,9 @@ int sbslpm_autotune_ensemble(sbslpm_ctx* c, int nmem, const double* area, const 
     launch_source_columns_mrhs(c->dt, w.qpart, w.qproxy, w.recmf, nmem, cb, w.qcol, c->stream);
     for (int xcd = 0; xcd < 3; ++xcd)
       for (int wi = 0; wi < 3; ++wi) {
-        const PairShape sh = full_list_shape(c->tree, waves[wi], xcd, true);
+        const PairShape sh = full_list_shape(c->tree, waves[wi], xcd, SBSLPM_MIXED);
         auto launch = [&] {
-          launch_bve_interact_mrhs(c->dt, c->tiles, c->ntiles, c->sets, w.recmf, w.qcol, nmem, cb,
+          launch_bve_interact_mrhs(c->dt, pair_tiles(c, sh), c->ntiles, c->sets, w.recmf, w.qcol, nmem, cb,
                                    c->prm.kernel_eps, w.phipart, w.phiproxy, c->stream, true, sh);
         };
         launch();  // warm-up

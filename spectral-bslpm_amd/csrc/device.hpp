@@ -42,7 +42,7 @@ struct DevTree {
   const LogTabEntry* logwide;  // [kLogWideSize] table of log_wide
   const double* exptab;       // [kExpTabSize] table of exp_tab
   const double* expnegtab;    // [kExpNegTabSize] table of exp_neg
-  const int* xcd_start;       // [2][9] cost-balanced XCD ranges of the target-major tile list (or null)
+  const int* xcd_start;       // [4][9] cost-balanced XCD ranges of the target-major tile lists (or null)
   int* err;
   int bf16_m2l;               // matrix-core kernels take bf16 kernel-product operands for M2L sets
   int P, Pl, offset, n, dp1, m, m2, levels;
@@ -65,15 +65,17 @@ constexpr int kWavesPerBlock = 4;
 // Launch shape of the Biot-Savart pair kernels, chosen by the context's
 // autotuner: waves (tiles) per workgroup and how workgroups map to tiles:
 //   xcd 0: workgroup b takes tiles b*waves.. (the hardware deals workgroups
-//          round-robin over the XCDs, so neighbouring tiles land on different XCDs);
-//   xcd 1: each XCD takes a contiguous range of equally many tiles;
+//          round-robin over the XCDs, so consecutive tiles land on different XCDs);
+//   xcd 1: each XCD takes a contiguous range of equally many tiles, breadth first;
 //   xcd 2: each XCD takes a contiguous range of equal estimated work
 //          (DevTree::xcd_start), for the context's full target-major list
 //          only; `grid` is then the launch's workgroup count, 8 x the largest
 //          range in workgroups.
-// The default (four waves, mapping 0) needs no ranges; at 6 x 512^2 the
-// autotuner picks mapping 2.  The FP64 kernel gives a whole workgroup to each
-// tile (pairwalk.hpp): there only the mapping counts, with grid1 workgroups.
+// Lists of fewer than 6,000 tiles run by work, heaviest first, under mappings 0 and
+// 2, longer ones breadth first (neighbours share sources).  The default (four waves,
+// mapping 0) needs no ranges; at 6 x 512^2 the autotuner picks mapping 2.  The FP64
+// and the lane-copy kernels give a whole workgroup to each tile (pairwalk.hpp):
+// there only the mapping counts, with grid1 workgroups.
 struct PairShape {
   int waves = kWavesPerBlock;
   int xcd = 0;

@@ -17,9 +17,10 @@
 //     turn (lanes.hpp);
 //   * u = sum_j g_j q_j (x cross y_j) is accumulated as x cross (sum_j g_j q_j y_j),
 //     saving the per-pair cross product (six multiplies) of the reference form.
-// The workgroup id is remapped so that neighbouring tiles (adjacent target
-// panels sharing sources) land on the same XCD and its L2.  The matrix-core
-// kernels and k_bve_mixed run one wave per tile.
+// A list in breadth-first panel order is dealt in strips, so that neighbouring tiles
+// (adjacent target panels sharing sources) land on the same XCD and its L2; a short
+// one runs heaviest first (dealt_tile, PairShape).  The matrix-core kernels and
+// k_bve_mixed run one wave per tile.
 #include <cmath>
 
 #include "device.hpp"

@@ -354,27 +354,29 @@ std::string build_tree(const TreeConfig& cfg, Tree& t) {
   heaviest_first(t.nonleaf_tiles, t.srcsets);
 
   // Eight contiguous ranges of the tile list with equal estimated work, one per
-  // XCD (a long list is in breadth-first panel order, so a range of leaf tiles is
-  // a compact patch of the sphere and its sources stay in that XCD's L2), for two
-  // work models: xcd_start[0..8] for the matrix-core kernels (a tile's 16 x 16
-  // pair blocks over its source sets plus one block per set for the per-set
-  // flush) and xcd_start[9..17] for the vector-unit kernels, whose wave walks
-  // every source of a set whatever the tile's target count (the set's sources
-  // plus 16 for the per-set work).
+  // XCD (a list in breadth-first panel order gives each a compact patch of the
+  // sphere, whose sources stay in that XCD's L2), for two work models: a tile's
+  // 16 x 16 pair blocks over its source sets plus one block per set for the per-set
+  // work (the matrix-core kernels, and the lane copies of bve_lanes.hip, whose
+  // pairs follow both counts too), and the set's sources plus 16, whatever the
+  // tile's target count (a row per lane); and for two orders, `tiles` and
+  // `bfs_tiles`.
   {
     const size_t nt = t.tiles.size();
-    t.xcd_start.assign(18, (int)nt);
-    for (int model = 0; model < 2; ++model) {
+    t.xcd_start.assign(36, (int)nt);
+    for (int range = 0; range < 4; ++range) {
+      const int model = range & 1;
+      const std::vector<TargetTile>& list = range < 2 ? t.tiles : t.bfs_tiles;
       std::vector<double> pre(nt + 1, 0.0);
       for (size_t k = 0; k < nt; ++k) {
-        const TargetTile& tl = t.tiles[k];
+        const TargetTile& tl = list[k];
         const double tb = (tl.count + 15) / 16;
         double w = 0;
         for (int e = tl.src_begin; e < tl.src_end; ++e)
           w += model == 0 ? tb * ((t.srcsets[e].count + 15) / 16) + 1.0 : t.srcsets[e].count + 16.0;
         pre[k + 1] = pre[k] + w;
       }
-      int* xs = t.xcd_start.data() + 9 * model;
+      int* xs = t.xcd_start.data() + 9 * range;
       xs[0] = 0;
       size_t k = 0;
       for (int x = 1; x < 8; ++x) {

@@ -104,9 +104,9 @@ struct Tree {
   std::vector<int> set_start;           // [P+1]: source sets of target panel p are [set_start[p], set_start[p+1])
   std::vector<TargetTile> bfs_tiles;    // the same tiles in breadth-first panel order
   std::vector<TargetTile> nonleaf_tiles;  // the tiles of non-leaf target panels, in the order of `tiles`
-  std::vector<int> xcd_start;           // [2][9]: tiles [xcd_start[x], xcd_start[x+1]) of XCD x in the
-                                        // cost-balanced contiguous launch mapping (PairShape xcd 2),
-                                        // for matrix-core kernels, then for vector-unit kernels
+  std::vector<int> xcd_start;           // [4][9]: tiles [xcd_start[x], xcd_start[x+1]) of XCD x in the
+                                        // cost-balanced contiguous launch mapping (PairShape xcd 2):
+                                        // by blocks of 16, by sources; then both over bfs_tiles
   std::vector<double> px, py, pz;       // unified point coordinates [U] (targets, undisplaced sources)
   std::vector<double> m2m_hi, m2m_lo;   // [d+1][d+1]: parent basis a at child node k, A[a*(d+1)+k]
   std::vector<double> p2m;              // [d+1][m]: proxy basis a at particle node k

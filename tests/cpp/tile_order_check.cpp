@@ -3,6 +3,7 @@
 // stay in breadth-first panel order.
 #include <algorithm>
 #include <cstdio>
+#include <cmath>
 #include <cstdlib>
 
 #include "tree.hpp"
@@ -47,6 +48,27 @@ int main(int argc, char** argv) {
   SourceMajor sm;
   build_source_major(t, sm);
   if (int rc = check(sm.tiles, sm.bfs_tiles, sm.targets)) return 20 + rc;
+  // the XCD ranges cover their list and hold equal work to within a tile's
+  if (t.xcd_start.size() != 36) return 30;
+  for (int range = 0; range < 4; ++range) {
+    const std::vector<TargetTile>& list = range < 2 ? t.tiles : t.bfs_tiles;
+    const int* xs = t.xcd_start.data() + 9 * range;
+    if (xs[0] != 0 || xs[8] != (int)list.size()) return 31;
+    double all = 0, most = 0, part[8] = {};
+    for (int x = 0; x < 8; ++x)
+      for (int k = xs[x]; k < xs[x + 1]; ++k) {
+        const TargetTile& tl = list[k];
+        double w = 0;
+        for (int e = tl.src_begin; e < tl.src_end; ++e)
+          w += range & 1 ? t.srcsets[e].count + 16.0
+                         : ((tl.count + 15) / 16) * ((t.srcsets[e].count + 15) / 16) + 1.0;
+        part[x] += w;
+        all += w;
+        most = std::max(most, w);
+      }
+    for (int x = 0; x < 8; ++x)
+      if (std::abs(part[x] - all / 8) > most) return 32 + range;
+  }
   std::printf("%zu tiles, %zu non-leaf, %zu source-major\n", t.tiles.size(), nonleaf.size(), sm.tiles.size());
   return 0;
 }
