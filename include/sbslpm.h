@@ -371,11 +371,13 @@ int sbslpm_bve_departure_to_target_adjoint(sbslpm_ctx* ctx, const double* dep_x,
  * (area, vor), for every candidate of waves per workgroup (1, 2, 4) x tile-to-XCD mapping
  * (0: workgroups dealt round-robin over the XCDs by the hardware; 1: a contiguous range of
  * equally many tiles per XCD; 2: a contiguous range of equal estimated work per XCD), and
- * keeps the fastest for all later evaluations, steps and ensembles
- * and the step adjoint's transposed pair sums (captured graphs are dropped and recaptured).
- * report [ncand][3] (may be NULL) receives
- * waves, xcd, ms per launch; *ncand the number of candidates timed.  Results do not depend on
- * the shape: every target is still summed by one lane in the same order. */
+ * keeps the fastest for all later evaluations, steps and ensembles and the waves per workgroup
+ * of the shallow-water adjoint's pair sums (captured graphs are dropped and recaptured).
+ * report [ncand][3] (may be NULL) receives waves, xcd, ms per launch; *ncand the number of
+ * candidates.  A kernel that gives each tile a workgroup (SBSLPM_FP64; SBSLPM_MIXED unless its
+ * pairs run on the matrix cores) has one launch per mapping: it is timed once, reported for
+ * all three waves, and the context's waves stay.  Results do not depend on the shape: every
+ * target's sum is added in the same order. */
 int sbslpm_autotune(sbslpm_ctx* ctx, const double* area, const double* vor, double* report, int* ncand);
 /* Autotuner of the multi-right-hand-side pair kernel of ensemble steps (no reference
  * counterpart; mixed-precision context with SBSLPM_FLAG_MULTI_RHS, 2 <= nmem <= 65535): times

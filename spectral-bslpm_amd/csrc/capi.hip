@@ -1776,21 +1776,27 @@ int sbslpm_autotune(sbslpm_ctx* c, const double* area, const double* vor, double
   hipEvent_t e0, e1;
   HIP_TRY(c, hipEventCreate(&e0));
   HIP_TRY(c, hipEventCreate(&e1));
-  const int waves[3] = {1, 2, 4};
+  // A kernel that gives each tile a workgroup does not read `waves`: one launch shape
+  // per mapping is timed and stands for all three, and the context's waves, which its
+  // other kernels read, come first and stay.
+  const bool by_tile = prec == SBSLPM_FP64 || (prec == SBSLPM_MIXED && !matrix_pairs(c));
+  int waves[3] = {1, 2, 4};
+  if (by_tile) std::swap(waves[0], *std::find(waves, waves + 3, c->shape.waves));
   PairShape best = c->shape;
-  float best_ms = 1e30f;
+  float best_ms = 1e30f, ms = 0;
   int k = 0;
   for (int xcd = 0; xcd < 3; ++xcd)
     for (int wi = 0; wi < 3; ++wi) {
       const PairShape sh = full_list_shape(c->tree, waves[wi], xcd, prec);
-      launch(sh);  // warm-up
-      hipEventRecord(e0, c->stream);
-      for (int r = 0; r < 3; ++r) launch(sh);
-      hipEventRecord(e1, c->stream);
-      if (hipEventSynchronize(e1) != hipSuccess) break;
-      float ms = 0;
-      hipEventElapsedTime(&ms, e0, e1);
-      ms /= 3;
+      if (wi == 0 || !by_tile) {
+        launch(sh);  // warm-up
+        hipEventRecord(e0, c->stream);
+        for (int r = 0; r < 3; ++r) launch(sh);
+        hipEventRecord(e1, c->stream);
+        if (hipEventSynchronize(e1) != hipSuccess) break;
+        hipEventElapsedTime(&ms, e0, e1);
+        ms /= 3;
+      }
       if (report) {
         report[3 * k] = sh.waves;
         report[3 * k + 1] = sh.xcd;

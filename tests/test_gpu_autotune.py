@@ -1,7 +1,7 @@
 """The pair-kernel autotuner: it times every candidate launch shape on the
 context's own interaction list, keeps the fastest, and the results of the
-evaluation and of the (graph-captured) step do not change, since each target
-is still summed by one lane in the same order whatever the shape."""
+evaluation and of the (graph-captured) step do not change, since each target's
+sum is added in the same order whatever the shape."""
 import numpy as np
 import pytest
 
@@ -87,3 +87,26 @@ def test_autotuned_graph_step_matches_eager(sb, torch_gpu):
         ectx.bve_back_rk4_step(*g, ve, vel_e)
         ectx.synchronize()
         np.testing.assert_array_equal(to_np(vg), to_np(ve))
+
+
+# levels 5 with 16 rows a tile: mixed precision runs on the matrix cores, where waves count
+@pytest.mark.parametrize("precision,degree,leaf_degree,by_tile", [
+    ("fp64", 8, 7, True), ("mixed", 8, 7, True), ("mixed", 3, 3, False), ("mixed_valu", 8, 7, False)])
+def test_waves_are_tuned_where_they_count(sb, torch_gpu, precision, degree, leaf_degree, by_tile):
+    """A kernel with a workgroup per tile has one launch per mapping: three candidates share its
+    time, and the waves per workgroup that the context's other kernels read stay as set."""
+    t = torch_gpu
+    print(f"\n[case waves {precision} d{degree}]", flush=True)
+    ctx = sb.Context(sb.RunConfig(levels=5, interp_degree=degree, leaf_degree=leaf_degree, kernel_eps=1e-4,
+                                  weights="clenshaw_curtis", precision=precision))
+    x, y, z, a = ctx.spec_points()
+    area, vor = to_gpu(t, a), to_gpu(t, sb.workloads.gaussian_vortices(x, y, z, a, seed=5))
+    ctx.set_pair_shape(2, 0)
+    table, shape = ctx.autotune(area, vor)
+    ctx.synchronize()
+    assert sorted((int(w), int(c)) for w, c, _ in table) == sorted((w, c) for w in (1, 2, 4) for c in (0, 1, 2))
+    times = [{ms for _, c, ms in table if int(c) == xcd} for xcd in (0, 1, 2)]
+    if by_tile:
+        assert all(len(v) == 1 for v in times) and shape[0] == 2
+    else:
+        assert any(len(v) > 1 for v in times)
