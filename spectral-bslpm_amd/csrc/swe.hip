@@ -10,9 +10,8 @@
 //     u += g qz (x cross y) + g0 qd (y0 - x (x.y0)),   g0 = +1/(4 pi (1 - x.y0 + eps))
 //   variant 3 (swe_vel_panel_interaction_ll, swe_vel_impl.hpp:265-276, no displacement):
 //     u += g qz (x cross y) - g qd (y - x (x.y)),      g = -1/(4 pi (1 - x.y + eps))
-// The kernel accumulates W = sum g qz y, D = sum gd y', S = sum gd (x.y')
-// (y' = y or y0) and forms u = x cross W + D - x S once per target, the same
-// sums regrouped.
+// The kernels accumulate W = sum g qz y and D = sum gd y' (y' = y or y0) and form
+// u = x cross W + D - x (x.D) once per target, the same sums regrouped.
 #include "device.hpp"
 #include "lanes.hpp"
 
@@ -125,7 +124,7 @@ __global__ __launch_bounds__(64 * S) void k_swe64(DevTree t, const TargetTile* _
 }
 
 // The same in lane copies (lanes.hpp) of two targets, for tiles of at most 42 rows
-// (lanes64).  Microseconds per launch, a row per lane and here: 6 x 96^2 (degree 8)
+// (lanes64) and for irregular trees.  Microseconds per launch, a row per lane and here: 6 x 96^2 (degree 8)
 // 201 -> 192, 6 x 192^2 686 -> 558 (degree 5: 423 -> 341), 6 x 160^2 (degree 4, 25
 // rows) 294 -> 253.  Variant 2, velocity calls in lane groups, with a row per lane and
 // here: 6 x 96^2 (degree 8) 366, 258, 223; 6 x 192^2 1120, 909, 772; 6 x 160^2 (degree
@@ -134,12 +133,12 @@ template <int VARIANT, int S>
 __global__ __launch_bounds__(64 * S) void k_swe64_lanes(DevTree t, const TargetTile* __restrict__ tiles, int ntiles,
                                                         const SourceSet* __restrict__ sets,
                                                         const SrcRecSwe* __restrict__ rec, double eps, Ptr3 part,
-                                                        Ptr3 proxy, int assign, int) {
+                                                        Ptr3 proxy, int assign, int heaviest_first) {
   constexpr int NT = 2, K = 6;
   __shared__ __align__(16) double stage[S][kLaneSlots * 8];
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int lane = threadIdx.x & 63;
-  const int tile = strip_tile(ntiles);
+  const int tile = heaviest_first ? (int)blockIdx.x : strip_tile(ntiles);
   if (tile >= ntiles) return;  // the whole workgroup
   const TargetTile T = tiles[tile];
   const LaneTile l = lane_tile<NT>(T.count, lane);
@@ -388,7 +387,12 @@ void launch_swe_interact64(const DevTree& t, int variant, const TargetTile* tile
   int S = ntiles < 400 ? 16 : ntiles < 3000 ? 8 : 4;
   auto kernel = variant != 2 ? (S == 16 ? k_swe64<1, 16> : S == 8 ? k_swe64<1, 8> : k_swe64<1, 4>)
                              : (S == 16 ? k_swe64<2, 16> : S == 8 ? k_swe64<2, 8> : k_swe64<2, 4>);
-  if (lanes64(t) && !heaviest_first && S < 16) {
+  // An irregular tree's list (heaviest first, tiles of one row to 64, sets of a few points)
+  // takes lane copies whatever its rows.  Shallow-water velocity on the 1 degree grid, a
+  // row per lane and lane copies: 64 points a leaf at degree 4 185 and 152 us, degree 8 574
+  // and 417, degree 10 838 and 751; 324 a leaf at degree 8 278 and 249; 484 at degree 10 359
+  // and 359.
+  if ((lanes64(t) || heaviest_first) && S < 16) {
     S = lane_waves64(t, ntiles);
     kernel = variant != 2 ? (S == 8 ? k_swe64_lanes<1, 8> : S == 4 ? k_swe64_lanes<1, 4> : k_swe64_lanes<1, 1>)
                           : (S == 8 ? k_swe64_lanes<2, 8> : S == 4 ? k_swe64_lanes<2, 4> : k_swe64_lanes<2, 1>);
