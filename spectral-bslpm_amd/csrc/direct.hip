@@ -21,6 +21,8 @@ constexpr int kWaves = 8;
 struct Plan {
   int64_t tiles, chunks, chunk_len;
   int nt_lane;
+  bool shared;  // waves share a tile; else each wave takes tiles of its own
+  dim3 grid;
 };
 
 // chunks is bounded by the waves of 64 targets it takes to fill the chip (4096)
@@ -28,6 +30,12 @@ struct Plan {
 // Two targets per lane halve the source loads and the uniform work per pair:
 // taken unless the second target would idle in a list of a few 64-target rows
 // (one row of 64 against 400,000 sources: 2x the pairs for nothing).
+// A few sources for more targets than fill the chip: eight waves on a tile would each
+// start, add up and stage the log table for a few pairs, so a wave takes whole tiles
+// instead, a workgroup's waves tile after tile.  Microseconds per call, waves sharing a
+// tile and not: log sum, 2,000,000 targets x 1 / 8 / 64 sources 94 / 101 / 141 and 24 / 29 /
+// 100, velocity 115 / 122 / 149 and 39 / 40 / 82; 300,000 x 1 / 64 / 128 log 17 / 27 / 38 and
+// 12 / 28 / 48, velocity 24 / 29 / 37 and 13 / 24 / 37.
 Plan plan(int64_t nt, int64_t ns) {
   Plan p;
   const int64_t rows = (nt + 63) / 64;
@@ -39,14 +47,23 @@ Plan plan(int64_t nt, int64_t ns) {
   if (p.chunks < 1) p.chunks = 1;
   p.nt_lane = (rows & 1) && rows < 8 ? 1 : 2;
   p.tiles = (rows + p.nt_lane - 1) / p.nt_lane;
+  p.shared = p.chunk_len > 128 || p.tiles < std::max<int64_t>(1500, 25 * p.chunk_len);
+  const int64_t groups = p.shared ? p.tiles : std::min<int64_t>((p.tiles + kWaves - 1) / kWaves, 1024);
+  p.grid = dim3((unsigned)groups, (unsigned)p.chunks);
   return p;
 }
 
-// This wave's part [a, b) of the workgroup's source chunk: eighths rounded up
-// to whole batches of four.
+// This wave's part [a, b) of the workgroup's source chunk where W waves share it:
+// W-ths rounded up to whole batches of four.
+template <int W>
 __device__ inline void wave_sources(int64_t ns, int64_t chunk_len, int wave, int64_t& a, int64_t& b) {
   const int64_t j0 = (int64_t)blockIdx.y * chunk_len, j1 = std::min<int64_t>(ns, j0 + chunk_len);
-  const int64_t q = ((j1 - j0 + 4 * kWaves - 1) / (4 * kWaves)) * 4;
+  if (W == 1) {
+    a = j0;
+    b = j1;
+    return;
+  }
+  const int64_t q = ((j1 - j0 + 4 * W - 1) / (4 * W)) * 4;
   a = std::min<int64_t>(j1, j0 + wave * q);
   b = std::min<int64_t>(j1, a + q);
 }
@@ -66,6 +83,16 @@ __device__ inline void wave_sum(double (&v)[K], int wave, int lane) {
       for (int k = 0; k < K; ++k) v[k] += red[w][k][lane];
 }
 
+// The wave's tiles: the workgroup's one (W waves share it), or every 8 gridDim.x-th.
+template <int W, typename F>
+__device__ inline void for_tiles(int64_t tiles, int wave, F&& f) {
+  if constexpr (W > 1) {
+    f((int64_t)blockIdx.x);
+  } else {
+    for (int64_t tile = (int64_t)blockIdx.x * kWaves + wave; tile < tiles; tile += (int64_t)gridDim.x * kWaves) f(tile);
+  }
+}
+
 // guard 0: skip j == self_offset + i (the reference's i != j);
 // guard 1: skip x.y >= 1 - 1e-15 (the FMM kernel's coincidence guard).
 // The logarithm is log_wide (fasttab.hpp) where 1 - x.y is in its range; a batch
@@ -75,13 +102,13 @@ __device__ inline void wave_sum(double (&v)[K], int wave, int lane) {
 // Bound: FP64 vector issue, 20 instructions per pair (about 90 with the library's
 // logarithm on every pair).  24,576 x 24,576 points: 2.13 -> 0.44 ms
 // (0.57 with log_tab), vector issue busy 70% of the time.
-template <int NT>
+template <int NT, int W>
 __global__ __launch_bounds__(64 * kWaves) void k_direct_log(int64_t nt, const double* __restrict__ tx,
                                                     const double* __restrict__ ty, const double* __restrict__ tz,
                                                     int64_t ns, const double* __restrict__ sx,
                                                     const double* __restrict__ sy, const double* __restrict__ sz,
                                                     const double* __restrict__ area, const double* __restrict__ pots,
-                                                    int64_t self_offset, int guard, int64_t chunk_len,
+                                                    int64_t self_offset, int guard, int64_t chunk_len, int64_t tiles,
                                                     const LogTabEntry* __restrict__ logwide,
                                                     double* __restrict__ partials) {
   // x.y rounded exactly as written in direct_sum_impl.hpp:23 (no fused
@@ -93,69 +120,71 @@ __global__ __launch_bounds__(64 * kWaves) void k_direct_log(int64_t nt, const do
   __syncthreads();
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int lane = threadIdx.x & 63;
-  const int64_t i0 = (int64_t)blockIdx.x * (64 * NT);
-  double x[NT], y[NT], z[NT], acc[NT];
+  for_tiles<W>(tiles, wave, [&](int64_t tile) {
+    const int64_t i0 = tile * (64 * NT);
+    double x[NT], y[NT], z[NT], acc[NT];
 #pragma unroll
-  for (int t = 0; t < NT; ++t) {
-    const int64_t i = std::min<int64_t>(i0 + t * 64 + lane, nt - 1);
-    x[t] = tx[i]; y[t] = ty[i]; z[t] = tz[i];
-    acc[t] = 0;
-  }
-  int64_t a, b;
-  wave_sources(ns, chunk_len, wave, a, b);
-  const int64_t self_lo = self_offset + i0, self_hi = self_lo + 64 * NT;
-  const double c7 = in_vgpr(1.0 / 7.0);
-  auto guarded = [&](int t, int64_t j) {
-    const int64_t i = std::min<int64_t>(i0 + t * 64 + lane, nt - 1);
-    const double d = 1.0 - (x[t] * sx[j] + y[t] * sy[j] + z[t] * sz[j]);
-    const bool skip = guard ? !(d > 1.0 - (1.0 - 1e-15)) : (j == self_offset + i);
-    const double v = skip ? 1.0 : d;
-    const uint32_t h = log_wide_cell(v);
-    const bool close = h >= kLogWideSpan;
-    double l = log_wide(v, close ? 0u : h, wide, c7);
-    if (__builtin_amdgcn_ballot_w64(close) != 0) l = close ? log(fmax(v, 1e-300)) : l;
-    const double q = area[j] * pots[j];
-    acc[t] = skip ? acc[t] : fma(l, q, acc[t]);
-  };
-  int64_t j = a;
-  for (; j + 4 <= b; j += 4) {
-    double d[NT][4];
-    uint32_t h[NT][4], far = 0;
+    for (int t = 0; t < NT; ++t) {
+      const int64_t i = std::min<int64_t>(i0 + t * 64 + lane, nt - 1);
+      x[t] = tx[i]; y[t] = ty[i]; z[t] = tz[i];
+      acc[t] = 0;
+    }
+    int64_t a, b;
+    wave_sources<W>(ns, chunk_len, wave, a, b);
+    const int64_t self_lo = self_offset + i0, self_hi = self_lo + 64 * NT;
+    const double c7 = in_vgpr(1.0 / 7.0);
+    auto guarded = [&](int t, int64_t j) {
+      const int64_t i = std::min<int64_t>(i0 + t * 64 + lane, nt - 1);
+      const double d = 1.0 - (x[t] * sx[j] + y[t] * sy[j] + z[t] * sz[j]);
+      const bool skip = guard ? !(d > 1.0 - (1.0 - 1e-15)) : (j == self_offset + i);
+      const double v = skip ? 1.0 : d;
+      const uint32_t h = log_wide_cell(v);
+      const bool close = h >= kLogWideSpan;
+      double l = log_wide(v, close ? 0u : h, wide, c7);
+      if (__builtin_amdgcn_ballot_w64(close) != 0) l = close ? log(fmax(v, 1e-300)) : l;
+      const double q = area[j] * pots[j];
+      acc[t] = skip ? acc[t] : fma(l, q, acc[t]);
+    };
+    int64_t j = a;
+    for (; j + 4 <= b; j += 4) {
+      double d[NT][4];
+      uint32_t h[NT][4], far = 0;
 #pragma unroll
-    for (int k = 0; k < 4; ++k) {
-      const double s0 = sx[j + k], s1 = sy[j + k], s2 = sz[j + k];
+      for (int k = 0; k < 4; ++k) {
+        const double s0 = sx[j + k], s1 = sy[j + k], s2 = sz[j + k];
 #pragma unroll
-      for (int t = 0; t < NT; ++t) {
-        d[t][k] = 1.0 - (x[t] * s0 + y[t] * s1 + z[t] * s2);
-        h[t][k] = log_wide_cell(d[t][k]);
-        far = h[t][k] > far ? h[t][k] : far;
+        for (int t = 0; t < NT; ++t) {
+          d[t][k] = 1.0 - (x[t] * s0 + y[t] * s1 + z[t] * s2);
+          h[t][k] = log_wide_cell(d[t][k]);
+          far = h[t][k] > far ? h[t][k] : far;
+        }
+      }
+      loaded(area[j], area[j + 1], area[j + 2], area[j + 3]);
+      loaded(pots[j], pots[j + 1], pots[j + 2], pots[j + 3]);
+      const bool own = !guard && j < self_hi && j + 4 > self_lo;
+      if (own || __builtin_amdgcn_ballot_w64(far >= kLogWideSpan) != 0) {
+#pragma unroll 1
+        for (int k = 0; k < 4; ++k)
+#pragma unroll
+          for (int t = 0; t < NT; ++t) guarded(t, j + k);
+        continue;
+      }
+#pragma unroll
+      for (int k = 0; k < 4; ++k) {
+        const double q = area[j + k] * pots[j + k];
+#pragma unroll
+        for (int t = 0; t < NT; ++t) acc[t] = fma(log_wide(d[t][k], h[t][k], wide, c7), q, acc[t]);
       }
     }
-    loaded(area[j], area[j + 1], area[j + 2], area[j + 3]);
-    loaded(pots[j], pots[j + 1], pots[j + 2], pots[j + 3]);
-    const bool own = !guard && j < self_hi && j + 4 > self_lo;
-    if (own || __builtin_amdgcn_ballot_w64(far >= kLogWideSpan) != 0) {
-#pragma unroll 1
-      for (int k = 0; k < 4; ++k)
+    for (; j < b; ++j)
 #pragma unroll
-        for (int t = 0; t < NT; ++t) guarded(t, j + k);
-      continue;
-    }
+      for (int t = 0; t < NT; ++t) guarded(t, j);
+    if constexpr (W > 1) wave_sum(acc, wave, lane);
+    if (W == 1 || wave == 0)
 #pragma unroll
-    for (int k = 0; k < 4; ++k) {
-      const double q = area[j + k] * pots[j + k];
-#pragma unroll
-      for (int t = 0; t < NT; ++t) acc[t] = fma(log_wide(d[t][k], h[t][k], wide, c7), q, acc[t]);
-    }
-  }
-  for (; j < b; ++j)
-#pragma unroll
-    for (int t = 0; t < NT; ++t) guarded(t, j);
-  wave_sum(acc, wave, lane);
-  if (wave == 0)
-#pragma unroll
-    for (int t = 0; t < NT; ++t)
-      if (i0 + t * 64 + lane < nt) partials[(int64_t)blockIdx.y * nt + i0 + t * 64 + lane] = kNegInv4Pi * acc[t];
+      for (int t = 0; t < NT; ++t)
+        if (i0 + t * 64 + lane < nt) partials[(int64_t)blockIdx.y * nt + i0 + t * 64 + lane] = kNegInv4Pi * acc[t];
+  });
 }
 
 // Bound: FP64 vector issue.  The four denominators of a batch share one
@@ -164,70 +193,73 @@ __global__ __launch_bounds__(64 * kWaves) void k_direct_log(int64_t nt, const do
 // multiply-adds from 1.  4,096 targets x 393,216 sources: 4.09 -> 0.77 ms (one
 // target per lane and one source per step waited on each source's scalar loads;
 // now vector issue is busy 83% of the time, at 2.1 GHz under this load).
-template <int NT>
+template <int NT, int W>
 __global__ __launch_bounds__(64 * kWaves) void k_direct_bs(int64_t nt, const double* __restrict__ tx,
                                                    const double* __restrict__ ty, const double* __restrict__ tz,
                                                    int64_t ns, const double* __restrict__ sx,
                                                    const double* __restrict__ sy, const double* __restrict__ sz,
                                                    const double* __restrict__ area, const double* __restrict__ vor,
-                                                   double eps, int64_t chunk_len, double* __restrict__ partials) {
+                                                   double eps, int64_t chunk_len, int64_t tiles,
+                                                   double* __restrict__ partials) {
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int lane = threadIdx.x & 63;
-  const int64_t i0 = (int64_t)blockIdx.x * (64 * NT);
-  double x[NT], y[NT], z[NT], w[3 * NT];
-#pragma unroll
-  for (int t = 0; t < NT; ++t) {
-    const int64_t i = std::min<int64_t>(i0 + t * 64 + lane, nt - 1);
-    x[t] = tx[i]; y[t] = ty[i]; z[t] = tz[i];
-    w[3 * t] = w[3 * t + 1] = w[3 * t + 2] = 0;
-  }
-  int64_t a, b;
-  wave_sources(ns, chunk_len, wave, a, b);
-  int64_t j = a;
-  for (; j + 4 <= b; j += 4) {
-    double s0[4], s1[4], s2[4], q[4];
-#pragma unroll
-    for (int k = 0; k < 4; ++k) {
-      s0[k] = sx[j + k]; s1[k] = sy[j + k]; s2[k] = sz[j + k];
-      q[k] = area[j + k] * vor[j + k];
-    }
+  for_tiles<W>(tiles, wave, [&](int64_t tile) {
+    const int64_t i0 = tile * (64 * NT);
+    double x[NT], y[NT], z[NT], w[3 * NT];
 #pragma unroll
     for (int t = 0; t < NT; ++t) {
-      double d[4], g[4];
-#pragma unroll
-      for (int k = 0; k < 4; ++k) d[k] = one_minus_dot(x[t], y[t], z[t], s0[k], s1[k], s2[k]) + eps;
-      rcp4(d, g);
+      const int64_t i = std::min<int64_t>(i0 + t * 64 + lane, nt - 1);
+      x[t] = tx[i]; y[t] = ty[i]; z[t] = tz[i];
+      w[3 * t] = w[3 * t + 1] = w[3 * t + 2] = 0;
+    }
+    int64_t a, b;
+    wave_sources<W>(ns, chunk_len, wave, a, b);
+    int64_t j = a;
+    for (; j + 4 <= b; j += 4) {
+      double s0[4], s1[4], s2[4], q[4];
 #pragma unroll
       for (int k = 0; k < 4; ++k) {
-        const double gq = g[k] * q[k];
-        w[3 * t] = fma(gq, s0[k], w[3 * t]);
-        w[3 * t + 1] = fma(gq, s1[k], w[3 * t + 1]);
-        w[3 * t + 2] = fma(gq, s2[k], w[3 * t + 2]);
+        s0[k] = sx[j + k]; s1[k] = sy[j + k]; s2[k] = sz[j + k];
+        q[k] = area[j + k] * vor[j + k];
+      }
+#pragma unroll
+      for (int t = 0; t < NT; ++t) {
+        double d[4], g[4];
+#pragma unroll
+        for (int k = 0; k < 4; ++k) d[k] = one_minus_dot(x[t], y[t], z[t], s0[k], s1[k], s2[k]) + eps;
+        rcp4(d, g);
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+          const double gq = g[k] * q[k];
+          w[3 * t] = fma(gq, s0[k], w[3 * t]);
+          w[3 * t + 1] = fma(gq, s1[k], w[3 * t + 1]);
+          w[3 * t + 2] = fma(gq, s2[k], w[3 * t + 2]);
+        }
       }
     }
-  }
-  for (; j < b; ++j) {
-    const double s0 = sx[j], s1 = sy[j], s2 = sz[j], q = area[j] * vor[j];
+    for (; j < b; ++j) {
+      const double s0 = sx[j], s1 = sy[j], s2 = sz[j], q = area[j] * vor[j];
+#pragma unroll
+      for (int t = 0; t < NT; ++t) {
+        const double g = rcp64(one_minus_dot(x[t], y[t], z[t], s0, s1, s2) + eps) * q;
+        w[3 * t] = fma(g, s0, w[3 * t]);
+        w[3 * t + 1] = fma(g, s1, w[3 * t + 1]);
+        w[3 * t + 2] = fma(g, s2, w[3 * t + 2]);
+      }
+    }
+    if constexpr (W > 1) wave_sum(w, wave, lane);
+    if (W > 1 && wave > 0) return;
 #pragma unroll
     for (int t = 0; t < NT; ++t) {
-      const double g = rcp64(one_minus_dot(x[t], y[t], z[t], s0, s1, s2) + eps) * q;
-      w[3 * t] = fma(g, s0, w[3 * t]);
-      w[3 * t + 1] = fma(g, s1, w[3 * t + 1]);
-      w[3 * t + 2] = fma(g, s2, w[3 * t + 2]);
+      const int64_t i = i0 + t * 64 + lane;
+      if (i >= nt) continue;
+      const double *u = w + 3 * t;
+      double* p = partials + (int64_t)blockIdx.y * 3 * nt;
+      p[i] = kNegInv4Pi * (y[t] * u[2] - z[t] * u[1]);
+      p[nt + i] = kNegInv4Pi * (z[t] * u[0] - x[t] * u[2]);
+      p[2 * nt + i] = kNegInv4Pi * (x[t] * u[1] - y[t] * u[0]);
     }
-  }
-  wave_sum(w, wave, lane);
-  if (wave > 0) return;
-#pragma unroll
-  for (int t = 0; t < NT; ++t) {
-    const int64_t i = i0 + t * 64 + lane;
-    if (i >= nt) continue;
-    const double *u = w + 3 * t;
-    double* p = partials + (int64_t)blockIdx.y * 3 * nt;
-    p[i] = kNegInv4Pi * (y[t] * u[2] - z[t] * u[1]);
-    p[nt + i] = kNegInv4Pi * (z[t] * u[0] - x[t] * u[2]);
-    p[2 * nt + i] = kNegInv4Pi * (x[t] * u[1] - y[t] * u[0]);
-  }
+  });
 }
 
 struct Ptr3 {
@@ -235,7 +267,7 @@ struct Ptr3 {
 };
 
 // out[blockIdx.y] += the chunks' partial sums: 64 targets per workgroup, wave w
-// adds chunks w, w + 4, ..., the waves' sums are added in wave order.  (With one
+// adds chunks w, w + 8, ..., the waves' sums are added in wave order.  (With one
 // thread per target walking every chunk of three components, the 64 chunks of
 // 4,096 targets took 52 us, a chain of loads in 64 waves; now 4.9 us.)
 __global__ __launch_bounds__(64 * kWaves) void k_reduce(int64_t nt, int ncomp, int64_t chunks,
@@ -249,6 +281,26 @@ __global__ __launch_bounds__(64 * kWaves) void k_reduce(int64_t nt, int ncomp, i
   for (int64_t c = wave; c < chunks; c += kWaves) s[0] += partials[(c * ncomp + f) * nt + ic];
   wave_sum(s, wave, lane);
   if (wave == 0 && i < nt) out.p[f][i] += s[0];
+}
+
+// The same for a few chunks, a thread per target.
+__global__ __launch_bounds__(256) void k_reduce_few(int64_t nt, int ncomp, int64_t chunks,
+                                                    const double* __restrict__ partials, Ptr3 out) {
+  const int f = (int)blockIdx.y;
+  const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
+  if (i >= nt) return;
+  double s = 0;
+  for (int64_t c = 0; c < chunks; ++c) s += partials[(c * ncomp + f) * nt + i];
+  out.p[f][i] += s;
+}
+
+void launch_reduce(int64_t nt, int ncomp, int64_t chunks, const double* partials, Ptr3 out, hipStream_t s) {
+  if (chunks < 4)
+    hipLaunchKernelGGL(k_reduce_few, dim3((unsigned)((nt + 255) / 256), ncomp), dim3(256), 0, s, nt, ncomp, chunks,
+                       partials, out);
+  else
+    hipLaunchKernelGGL(k_reduce, dim3((unsigned)((nt + 63) / 64), ncomp), dim3(64 * kWaves), 0, s, nt, ncomp, chunks,
+                       partials, out);
 }
 
 // Displaced, re-projected source positions (bve_vel_impl.hpp:57-60).
@@ -306,13 +358,10 @@ void launch_direct_inv_lap(int64_t nt, const double* tx, const double* ty, const
                            const LogTabEntry* logwide, double* partials, double* soln, hipStream_t s) {
   if (nt <= 0) return;
   const Plan p = plan(nt, ns);
-  const dim3 grid((unsigned)p.tiles, (unsigned)p.chunks);
-  auto kernel = p.nt_lane == 2 ? k_direct_log<2> : k_direct_log<1>;
-  hipLaunchKernelGGL(kernel, grid, dim3(64 * kWaves), 0, s, nt, tx, ty, tz, ns, sx, sy, sz, area, pots, self_offset,
-                     guard_coincident ? 1 : 0, p.chunk_len, logwide, partials);
-  Ptr3 out{{soln, nullptr, nullptr}};
-  hipLaunchKernelGGL(k_reduce, dim3((unsigned)((nt + 63) / 64), 1), dim3(64 * kWaves), 0, s, nt, 1, p.chunks,
-                     (const double*)partials, out);
+  auto kernel = !p.shared ? k_direct_log<2, 1> : p.nt_lane == 2 ? k_direct_log<2, kWaves> : k_direct_log<1, kWaves>;
+  hipLaunchKernelGGL(kernel, p.grid, dim3(64 * kWaves), 0, s, nt, tx, ty, tz, ns, sx, sy, sz, area, pots, self_offset,
+                     guard_coincident ? 1 : 0, p.chunk_len, p.tiles, logwide, partials);
+  launch_reduce(nt, 1, p.chunks, partials, Ptr3{{soln, nullptr, nullptr}}, s);
 }
 
 void launch_direct_bve_vel(int64_t nt, const double* tx, const double* ty, const double* tz, int64_t ns,
@@ -328,13 +377,12 @@ void launch_direct_bve_vel(int64_t nt, const double* tx, const double* ty, const
                        disp[1], disp[2], moved);
     ax = moved; ay = moved + ns; az = moved + 2 * ns;
   }
-  const dim3 grid((unsigned)p.tiles, (unsigned)p.chunks);
-  auto kernel = p.nt_lane == 2 ? k_direct_bs<2> : k_direct_bs<1>;
-  hipLaunchKernelGGL(kernel, grid, dim3(64 * kWaves), 0, s, nt, tx, ty, tz, ns, ax, ay, az, area, vor, eps,
-                     p.chunk_len, partials);
-  Ptr3 out{{vel[0], vel[1], vel[2]}};
-  hipLaunchKernelGGL(k_reduce, dim3((unsigned)((nt + 63) / 64), 3), dim3(64 * kWaves), 0, s, nt, 3, p.chunks,
-                     (const double*)partials, out);
+  auto kernel = !p.shared          ? k_direct_bs<2, 1>
+                : p.nt_lane == 2 ? k_direct_bs<2, kWaves>
+                                 : k_direct_bs<1, kWaves>;
+  hipLaunchKernelGGL(kernel, p.grid, dim3(64 * kWaves), 0, s, nt, tx, ty, tz, ns, ax, ay, az, area, vor, eps,
+                     p.chunk_len, p.tiles, partials);
+  launch_reduce(nt, 3, p.chunks, partials, Ptr3{{vel[0], vel[1], vel[2]}}, s);
 }
 
 }  // namespace sbslpm

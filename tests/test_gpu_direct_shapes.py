@@ -1,4 +1,4 @@
-"""Direct sums at the edges of their tiling (64 or 128 targets per workgroup, four waves
+"""Direct sums at the edges of their tiling (64 or 128 targets per workgroup, eight waves
 sharing a source chunk, batches of four sources) against numpy in FP64, with the guarded
 pairs (a target's own source, coincident points) in first, last and inner batches."""
 import numpy as np
