@@ -155,32 +155,36 @@ __global__ __launch_bounds__(64 * S) void k_bve_adj64_lanes(DevTree t, const Tar
   for (int q = 0; q < NT; ++q) {
     const SrcRec64 Y = srec[(int64_t)T.first + min(q * l.T + l.i, T.count - 1)];
     x[q] = Y.x; y[q] = Y.y; z[q] = Y.z;
-#pragma unroll
-    for (int k = 0; k < K; ++k) w[q][k] = 0;
   }
-  lane_walk2<S, 3>(T, targets, reinterpret_cast<const v4f*>(trec), l, reinterpret_cast<v4f*>(stage[wave]), wave, lane,
-                   [&](const v4f* r0, const v4f* r1) {
-    const TgtRec R[2] = {*reinterpret_cast<const TgtRec*>(r0), *reinterpret_cast<const TgtRec*>(r1)};
-    double d[4], g[4];
+  shared_sums(w, [&](auto shared) {
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const int q = i & 1;
-      d[i] = one_minus_dot(x[q], y[q], z[q], R[i >> 1].x, R[i >> 1].y, R[i >> 1].z) + eps;
-    }
-    rcp4(d, g);
+    for (int q = 0; q < NT; ++q)
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const int q = i & 1;
-      const TgtRec& P = R[i >> 1];
-      const double dc = x[q] * P.c0 + y[q] * P.c1 + z[q] * P.c2;
-      w[q][0] = fma(g[i], dc, w[q][0]);
-      if constexpr (POS) {
-        const double h = g[i] * dc;
-        w[q][K - 3] = fma(g[i], fma(h, P.x, P.c0), w[q][K - 3]);
-        w[q][K - 2] = fma(g[i], fma(h, P.y, P.c1), w[q][K - 2]);
-        w[q][K - 1] = fma(g[i], fma(h, P.z, P.c2), w[q][K - 1]);
+      for (int k = 0; k < K; ++k) w[q][k] = 0;
+    lane_walk2<S, 3>(T, targets, reinterpret_cast<const v4f*>(trec), l, reinterpret_cast<v4f*>(stage[wave]), wave, lane,
+                     [&](const v4f* r0, const v4f* r1) {
+      const TgtRec R[2] = {*reinterpret_cast<const TgtRec*>(r0), *reinterpret_cast<const TgtRec*>(r1)};
+      double d[4], g[4];
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const int q = i & 1;
+        d[i] = one_minus_dot(x[q], y[q], z[q], R[i >> 1].x, R[i >> 1].y, R[i >> 1].z) + eps;
       }
-    }
+      rcps<decltype(shared)::value>(d, g);
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const int q = i & 1;
+        const TgtRec& P = R[i >> 1];
+        const double dc = x[q] * P.c0 + y[q] * P.c1 + z[q] * P.c2;
+        w[q][0] = fma(g[i], dc, w[q][0]);
+        if constexpr (POS) {
+          const double h = g[i] * dc;
+          w[q][K - 3] = fma(g[i], fma(h, P.x, P.c0), w[q][K - 3]);
+          w[q][K - 2] = fma(g[i], fma(h, P.y, P.c1), w[q][K - 2]);
+          w[q][K - 1] = fma(g[i], fma(h, P.z, P.c2), w[q][K - 1]);
+        }
+      }
+    });
   });
   double out[K];
   lane_sum<NT, K, S>(l, w, stage, wave, lane, out);
@@ -366,7 +370,7 @@ void launch_bve_adjoint64(const DevTree& t, const TargetTile* tiles, int ntiles,
   int S = adj_waves(ntiles, 6000);
   auto kernel = dpart ? (S == 16 ? k_bve_adj64<true, 16> : S == 8 ? k_bve_adj64<true, 8> : k_bve_adj64<true, 4>)
                       : (S == 16 ? k_bve_adj64<false, 16> : S == 8 ? k_bve_adj64<false, 8> : k_bve_adj64<false, 4>);
-  if (lanes64(t) && S < 16) {
+  if ((lanes64(t) && S < 16) || !rcp4_in_range(eps)) {
     S = lane_waves64(t, ntiles);
     kernel = dpart ? (S == 8 ? k_bve_adj64_lanes<true, 8> : S == 4 ? k_bve_adj64_lanes<true, 4> : k_bve_adj64_lanes<true, 1>)
                    : (S == 8 ? k_bve_adj64_lanes<false, 8> : S == 4 ? k_bve_adj64_lanes<false, 4> : k_bve_adj64_lanes<false, 1>);

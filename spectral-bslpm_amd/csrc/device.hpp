@@ -3,6 +3,7 @@
 #include "fasttab.hpp"
 #include <hip/hip_runtime.h>
 #include <cstdint>
+#include <type_traits>
 
 #include "geometry.hpp"
 #include "tree.hpp"
@@ -205,11 +206,12 @@ __device__ inline double rcp64_pair(double d) {
 
 // 1/d_k of four denominators from one reciprocal of their product: the
 // estimate and its two Newton steps are shared, nine multiplies hand each
-// quotient out (19 vector-issue slots for four, a quarter-rate estimate counting
-// four, against 32 with rcp64 each).  Each product adds half an ulp, about 1.5
-// ulp in all; a zero denominator makes the whole batch NaN, as it makes the
-// sum that the batch belongs to without sharing.  The product of four must stay
-// in range, which d in [1e-16, 4] does by a wide margin.
+// quotient out (17 vector-issue slots for four, a quarter-rate estimate counting
+// four, against 32 with rcp64 each).  The products' roundings enter each
+// quotient: half an ulp on average, up to about 4.  A denominator that is zero or
+// no number, or a product of four out of range, spoils all four quotients: a batch
+// of one row's pairs spoils that row, whose sum such a pair spoils anyway; lane
+// copies, whose batch holds two rows, walk again without sharing (shared_sums).
 __device__ inline void rcp4(const double (&d)[4], double (&g)[4]) {
   const double p01 = d[0] * d[1], p23 = d[2] * d[3];
   const double r = rcp64(p01 * p23);
@@ -218,6 +220,33 @@ __device__ inline void rcp4(const double (&d)[4], double (&g)[4]) {
   g[1] = r01 * d[0];
   g[2] = r23 * d[3];
   g[3] = r23 * d[2];
+}
+template <bool SHARED>
+__device__ inline void rcps(const double (&d)[4], double (&g)[4]) {
+  if constexpr (SHARED) {
+    rcp4(d, g);
+  } else {
+#pragma unroll
+    for (int i = 0; i < 4; ++i) g[i] = rcp64(d[i]);
+  }
+}
+// Whether a regularisation keeps the product of any four denominators 1 - x.y + eps in
+// range.  Outside, the kernels with a row per lane leave the pairs to the lane copies.
+inline bool rcp4_in_range(double eps) { return eps == 0 || (eps > 1e-70 && eps < 1e70); }
+
+// f(true_type) forms this wave's sums w with shared reciprocals, f(false_type) with one
+// each: the second where a lane's sum came out as no finite number, so that what one
+// pair spoils stays in its row.  (A product that leaves the range by less than a
+// factor of 4 has a reciprocal good to 2^-49, and stays.)
+template <int NT, int K, typename F>
+__device__ inline void shared_sums(double (&w)[NT][K], F&& f) {
+  f(std::true_type{});
+  double s = 0;
+#pragma unroll
+  for (int q = 0; q < NT; ++q)
+#pragma unroll
+    for (int k = 0; k < K; ++k) s += fabs(w[q][k]);
+  if (__builtin_amdgcn_ballot_w64(!(s <= 0x1.fffffffffffffp1023)) != 0) f(std::false_type{});
 }
 
 // 1 - x.y in three fused multiply-adds from 1: the partial results shrink

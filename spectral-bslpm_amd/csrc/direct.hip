@@ -193,7 +193,7 @@ __global__ __launch_bounds__(64 * kWaves) void k_direct_log(int64_t nt, const do
 // multiply-adds from 1.  4,096 targets x 393,216 sources: 4.09 -> 0.77 ms (one
 // target per lane and one source per step waited on each source's scalar loads;
 // now vector issue is busy 83% of the time, at 2.1 GHz under this load).
-template <int NT, int W>
+template <int NT, int W, bool SHARED>
 __global__ __launch_bounds__(64 * kWaves) void k_direct_bs(int64_t nt, const double* __restrict__ tx,
                                                    const double* __restrict__ ty, const double* __restrict__ tz,
                                                    int64_t ns, const double* __restrict__ sx,
@@ -227,7 +227,7 @@ __global__ __launch_bounds__(64 * kWaves) void k_direct_bs(int64_t nt, const dou
         double d[4], g[4];
 #pragma unroll
         for (int k = 0; k < 4; ++k) d[k] = one_minus_dot(x[t], y[t], z[t], s0[k], s1[k], s2[k]) + eps;
-        rcp4(d, g);
+        rcps<SHARED>(d, g);
 #pragma unroll
         for (int k = 0; k < 4; ++k) {
           const double gq = g[k] * q[k];
@@ -377,9 +377,11 @@ void launch_direct_bve_vel(int64_t nt, const double* tx, const double* ty, const
                        disp[1], disp[2], moved);
     ax = moved; ay = moved + ns; az = moved + 2 * ns;
   }
-  auto kernel = !p.shared          ? k_direct_bs<2, 1>
-                : p.nt_lane == 2 ? k_direct_bs<2, kWaves>
-                                 : k_direct_bs<1, kWaves>;
+  auto kernel = !p.shared        ? k_direct_bs<2, 1, true>
+                : p.nt_lane == 2 ? k_direct_bs<2, kWaves, true>
+                                 : k_direct_bs<1, kWaves, true>;
+  if (!rcp4_in_range(eps))
+    kernel = !p.shared ? k_direct_bs<2, 1, false> : p.nt_lane == 2 ? k_direct_bs<2, kWaves, false> : k_direct_bs<1, kWaves, false>;
   hipLaunchKernelGGL(kernel, p.grid, dim3(64 * kWaves), 0, s, nt, tx, ty, tz, ns, ax, ay, az, area, vor, eps,
                      p.chunk_len, p.tiles, partials);
   launch_reduce(nt, 3, p.chunks, partials, Ptr3{{vel[0], vel[1], vel[2]}}, s);

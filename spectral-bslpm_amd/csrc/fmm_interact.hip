@@ -205,27 +205,30 @@ __global__ __launch_bounds__(64 * S) void k_bve64_lanes(DevTree t, const TargetT
   for (int q = 0; q < NT; ++q) {
     const int64_t u = (int64_t)T.first + min(q * l.T + l.i, T.count - 1);
     x[q] = t.px[u]; y[q] = t.py[u]; z[q] = t.pz[u];
-    w[q][0] = w[q][1] = w[q][2] = 0;
   }
-  lane_walk2<S, 2>(T, sets, reinterpret_cast<const v4f*>(rec), l, reinterpret_cast<v4f*>(stage[wave]), wave, lane,
-                   [&](const v4f* r0, const v4f* r1) {
-    const SrcRec64 R[2] = {*reinterpret_cast<const SrcRec64*>(r0), *reinterpret_cast<const SrcRec64*>(r1)};
-    double d[4], g[4];
+  shared_sums(w, [&](auto shared) {
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const int q = i & 1;
-      d[i] = one_minus_dot(x[q], y[q], z[q], R[i >> 1].x, R[i >> 1].y, R[i >> 1].z) + eps;
-    }
-    rcp4(d, g);
+    for (int q = 0; q < NT; ++q) w[q][0] = w[q][1] = w[q][2] = 0;
+    lane_walk2<S, 2>(T, sets, reinterpret_cast<const v4f*>(rec), l, reinterpret_cast<v4f*>(stage[wave]), wave, lane,
+                     [&](const v4f* r0, const v4f* r1) {
+      const SrcRec64 R[2] = {*reinterpret_cast<const SrcRec64*>(r0), *reinterpret_cast<const SrcRec64*>(r1)};
+      double d[4], g[4];
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const int q = i & 1;
-      const SrcRec64& P = R[i >> 1];
-      const double gq = g[i] * P.q;
-      w[q][0] = fma(gq, P.x, w[q][0]);
-      w[q][1] = fma(gq, P.y, w[q][1]);
-      w[q][2] = fma(gq, P.z, w[q][2]);
-    }
+      for (int i = 0; i < 4; ++i) {
+        const int q = i & 1;
+        d[i] = one_minus_dot(x[q], y[q], z[q], R[i >> 1].x, R[i >> 1].y, R[i >> 1].z) + eps;
+      }
+      rcps<decltype(shared)::value>(d, g);
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const int q = i & 1;
+        const SrcRec64& P = R[i >> 1];
+        const double gq = g[i] * P.q;
+        w[q][0] = fma(gq, P.x, w[q][0]);
+        w[q][1] = fma(gq, P.y, w[q][1]);
+        w[q][2] = fma(gq, P.z, w[q][2]);
+      }
+    });
   });
   double s[3];
   lane_sum<NT, 3, S>(l, w, stage, wave, lane, s);
@@ -1208,7 +1211,7 @@ void launch_bve_interact64(const DevTree& t, const TargetTile* tiles, int ntiles
   shape = checked_shape(t, shape);
   int S = tile_waves(ntiles);
   auto kernel = S == 16 ? k_bve64<16> : S == 8 ? k_bve64<8> : k_bve64<4>;
-  if (lanes64(t) && S < 16) {
+  if ((lanes64(t) && S < 16) || !rcp4_in_range(eps)) {
     S = lane_waves64(t, ntiles);
     kernel = S == 8 ? k_bve64_lanes<8> : S == 4 ? k_bve64_lanes<4> : k_bve64_lanes<1>;
   }

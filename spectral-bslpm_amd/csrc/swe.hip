@@ -147,46 +147,50 @@ __global__ __launch_bounds__(64 * S) void k_swe64_lanes(DevTree t, const TargetT
   for (int q = 0; q < NT; ++q) {
     const int64_t u = (int64_t)T.first + min(q * l.T + l.i, T.count - 1);
     x[q] = t.px[u]; y[q] = t.py[u]; z[q] = t.pz[u];
-#pragma unroll
-    for (int k = 0; k < K; ++k) w[q][k] = 0;
   }
-  lane_walk2<S, 4>(T, sets, reinterpret_cast<const v4f*>(rec), l, reinterpret_cast<v4f*>(stage[wave]), wave, lane,
-                   [&](const v4f* r0, const v4f* r1) {
-    const SrcRecSwe* R[2] = {reinterpret_cast<const SrcRecSwe*>(r0), reinterpret_cast<const SrcRecSwe*>(r1)};
-    double d[4], g[4], a[2], b[2], c[2], qz[2], qd[2];
+  shared_sums(w, [&](auto shared) {
 #pragma unroll
-    for (int i = 0; i < 2; ++i) {
-      a[i] = R[i]->x; b[i] = R[i]->y; c[i] = R[i]->z; qz[i] = R[i]->qz; qd[i] = R[i]->qd;
-    }
+    for (int q = 0; q < NT; ++q)
 #pragma unroll
-    for (int i = 0; i < 4; ++i) d[i] = one_minus_dot(x[i & 1], y[i & 1], z[i & 1], a[i >> 1], b[i >> 1], c[i >> 1]) + eps;
-    rcp4(d, g);
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const int q = i & 1, k = i >> 1;
-      const double gz = g[i] * qz[k];
-      w[q][0] = fma(gz, a[k], w[q][0]);
-      w[q][1] = fma(gz, b[k], w[q][1]);
-      w[q][2] = fma(gz, c[k], w[q][2]);
-    }
-    if constexpr (VARIANT == 2) {  // the divergence's pairs are at the undisplaced sources
+      for (int k = 0; k < K; ++k) w[q][k] = 0;
+    lane_walk2<S, 4>(T, sets, reinterpret_cast<const v4f*>(rec), l, reinterpret_cast<v4f*>(stage[wave]), wave, lane,
+                     [&](const v4f* r0, const v4f* r1) {
+      const SrcRecSwe* R[2] = {reinterpret_cast<const SrcRecSwe*>(r0), reinterpret_cast<const SrcRecSwe*>(r1)};
+      double d[4], g[4], a[2], b[2], c[2], qz[2], qd[2];
 #pragma unroll
       for (int i = 0; i < 2; ++i) {
-        a[i] = R[i]->x0; b[i] = R[i]->y0; c[i] = R[i]->z0;
+        a[i] = R[i]->x; b[i] = R[i]->y; c[i] = R[i]->z; qz[i] = R[i]->qz; qd[i] = R[i]->qd;
       }
 #pragma unroll
-      for (int i = 0; i < 4; ++i)
-        d[i] = one_minus_dot(x[i & 1], y[i & 1], z[i & 1], a[i >> 1], b[i >> 1], c[i >> 1]) + eps;
-      rcp4(d, g);
-    }
+      for (int i = 0; i < 4; ++i) d[i] = one_minus_dot(x[i & 1], y[i & 1], z[i & 1], a[i >> 1], b[i >> 1], c[i >> 1]) + eps;
+      rcps<decltype(shared)::value>(d, g);
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const int q = i & 1, k = i >> 1;
-      const double gd = g[i] * qd[k];
-      w[q][3] = fma(gd, a[k], w[q][3]);
-      w[q][4] = fma(gd, b[k], w[q][4]);
-      w[q][5] = fma(gd, c[k], w[q][5]);
-    }
+      for (int i = 0; i < 4; ++i) {
+        const int q = i & 1, k = i >> 1;
+        const double gz = g[i] * qz[k];
+        w[q][0] = fma(gz, a[k], w[q][0]);
+        w[q][1] = fma(gz, b[k], w[q][1]);
+        w[q][2] = fma(gz, c[k], w[q][2]);
+      }
+      if constexpr (VARIANT == 2) {  // the divergence's pairs are at the undisplaced sources
+#pragma unroll
+        for (int i = 0; i < 2; ++i) {
+          a[i] = R[i]->x0; b[i] = R[i]->y0; c[i] = R[i]->z0;
+        }
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+          d[i] = one_minus_dot(x[i & 1], y[i & 1], z[i & 1], a[i >> 1], b[i >> 1], c[i >> 1]) + eps;
+        rcps<decltype(shared)::value>(d, g);
+      }
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const int q = i & 1, k = i >> 1;
+        const double gd = g[i] * qd[k];
+        w[q][3] = fma(gd, a[k], w[q][3]);
+        w[q][4] = fma(gd, b[k], w[q][4]);
+        w[q][5] = fma(gd, c[k], w[q][5]);
+      }
+    });
   });
   double s[K];
   lane_sum<NT, K, S>(l, w, stage, wave, lane, s);
@@ -392,7 +396,7 @@ void launch_swe_interact64(const DevTree& t, int variant, const TargetTile* tile
   // row per lane and lane copies: 64 points a leaf at degree 4 185 and 152 us, degree 8 574
   // and 417, degree 10 838 and 751; 324 a leaf at degree 8 278 and 249; 484 at degree 10 359
   // and 359.
-  if ((lanes64(t) || heaviest_first) && S < 16) {
+  if (((lanes64(t) || heaviest_first) && S < 16) || !rcp4_in_range(eps)) {
     S = lane_waves64(t, ntiles);
     kernel = variant != 2 ? (S == 8 ? k_swe64_lanes<1, 8> : S == 4 ? k_swe64_lanes<1, 4> : k_swe64_lanes<1, 1>)
                           : (S == 8 ? k_swe64_lanes<2, 8> : S == 4 ? k_swe64_lanes<2, 4> : k_swe64_lanes<2, 1>);
