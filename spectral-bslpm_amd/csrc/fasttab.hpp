@@ -22,8 +22,8 @@
 //   r = x c_inv - 1 (one fma, |r| < 2^-7),  log x = logc + r (1 + r p(r)),
 // p the degree-5 Taylor polynomial (first omitted term r^8/8 < 2^-59), 11
 // vector instructions against log_tab's 17.  c_inv and logc as above, without
-// the special cells at 1: the error there is below 2^-59, which is small against
-// any sum of logarithms but not in relative terms.
+// the special cells at 1: the error there is below 2^-58 (2^-58.2 found), which is
+// small against any sum of logarithms but not in relative terms.
 //
 // Exponential (general, exp_tab): n = rint(t 128/ln2), t = n ln2/128 + r with
 // |r| <= ln2/256 (Cody-Waite split of ln2/128),

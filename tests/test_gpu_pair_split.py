@@ -1,7 +1,7 @@
 """FP64 pair kernels whose workgroups share a target tile (csrc/pairwalk.hpp) against the
-oracle: 16, 8 and 4 waves per tile, source sets that batches of four and parts of a set divide
-unevenly (25, 36, 49, 81 and 121 points), one to three tiles per panel, accumulating and
-displaced.  Both sides sum the same pairs: 1e-12 leaves room for the rounding of 1 - x.y
+oracle: a row per lane at 16, 8 and 4 waves per tile, lane copies (csrc/lanes.hpp) at 8, 4 and 1,
+source sets that batches of four, parts of a set and chunks of sets divide unevenly (9, 16, 25, 36,
+49, 64, 81 and 121 points), one and two tiles per panel, accumulating and displaced.  Both sides sum the same pairs: 1e-12 leaves room for the rounding of 1 - x.y
 (a few units of 1e-16 over eps = 1e-4) at the nearest pairs."""
 import numpy as np
 import pytest
@@ -11,9 +11,10 @@ from conftest import to_gpu, to_np
 pytestmark = pytest.mark.gpu
 
 EPS = 1e-4
-# levels, proxy degree, leaf grid side: tile lists of 30 to 8,190; 9 and 16 rows, where a chunk of
-# staged records spans several sets
-TREES = [(2, 4, 5), (3, 6, 7), (3, 8, 9), (4, 10, 11), (5, 8, 6), (6, 5, 6), (4, 2, 3), (5, 3, 4), (6, 2, 3)]
+# levels, proxy degree, leaf grid side: tile lists of 30 to 8,190; tiles of 9 and 16 rows, where a
+# chunk of staged records spans several sets; more than 42 rows at 2,556 and 8,190 tiles
+TREES = [(2, 4, 5), (3, 6, 7), (3, 8, 9), (4, 10, 11), (5, 8, 6), (6, 5, 6), (4, 2, 3), (5, 3, 4), (6, 2, 3),
+         (5, 8, 8), (6, 6, 7)]
 
 
 @pytest.fixture(scope="module", params=TREES, ids=lambda p: "L%d-d%d-m%d" % p)
@@ -171,3 +172,23 @@ def test_other_pairs_mixed(case, displaced, sb):
                                                      (proxy if isinstance(proxy, list) else [proxy])])
         e, g = flat(ep, ex), flat(gp, gx)
         assert np.linalg.norm(g - e) <= 2.0 ** -24 * bound * np.linalg.norm(e)
+
+
+def test_step_adjoint_mixed_against_fp64(case, sb):
+    """The step's gradient, whose displaced stages also take the position cotangents: two sets of
+    kernels for the same sums.  A pair's g is off by the FP32 bound of test_vortex_pairs_mixed and
+    its g^2 by twice that; the rest of the step is FP64 on both sides."""
+    cfg, W = case["ctx"].cfg, case["W"]
+    x, y, z, a = case["o"].spec_points()
+    vor = W.gaussian_vortices(x, y, z, a, seed=3)
+    bar = np.random.default_rng(5).normal(size=x.shape)
+    got = []
+    for precision in ("fp64", "mixed"):
+        ctx = sb.Context(sb.RunConfig(levels=cfg.levels, interp_degree=cfg.interp_degree, leaf_degree=cfg.leaf_degree,
+                                      kernel_eps=EPS, weights="clenshaw_curtis", precision=precision, delta_t=900.0))
+        got.append(to_np(ctx.bve_back_rk4_step_adjoint(*up(case, [x, y, z, a, vor, bar]))))
+        ctx.synchronize()
+    r = np.sqrt(2) * (np.pi / 4) / 2 ** (cfg.levels - 1)
+    err = np.linalg.norm(got[1] - got[0]) / np.linalg.norm(got[0])
+    print(f"  step adjoint, mixed from fp64: {err:.2e}")
+    assert err <= 3 * 2.0 ** -24 * (8 + 2 * r * r / EPS)
