@@ -34,8 +34,8 @@ struct Plan {
 // start, add up and stage the log table for a few pairs, so a wave takes whole tiles
 // instead, a workgroup's waves tile after tile.  Microseconds per call, waves sharing a
 // tile and not: log sum, 2,000,000 targets x 1 / 8 / 64 sources 94 / 101 / 141 and 24 / 29 /
-// 100, velocity 115 / 122 / 149 and 39 / 40 / 82; 300,000 x 1 / 64 / 128 log 17 / 27 / 38 and
-// 12 / 28 / 48, velocity 24 / 29 / 37 and 13 / 24 / 37.
+// 100, velocity 115 / 122 / 149 and 39 / 40 / 82; 300,000 x 1 / 64 / 128 (two targets per
+// lane) log 17 / 27 / 38 and 12 / 28 / 48, velocity 24 / 29 / 37 and 13 / 24 / 37.
 Plan plan(int64_t nt, int64_t ns) {
   Plan p;
   const int64_t rows = (nt + 63) / 64;
@@ -48,6 +48,11 @@ Plan plan(int64_t nt, int64_t ns) {
   p.nt_lane = (rows & 1) && rows < 8 ? 1 : 2;
   p.tiles = (rows + p.nt_lane - 1) / p.nt_lane;
   p.shared = p.chunk_len > 128 || p.tiles < std::max<int64_t>(1500, 25 * p.chunk_len);
+  if (!p.shared && rows < 8192) {
+    // a target per lane, twice the waves: 300,000 x 64 log 27 -> 25 us, velocity 23 -> 22
+    p.nt_lane = 1;
+    p.tiles = rows;
+  }
   const int64_t groups = p.shared ? p.tiles : std::min<int64_t>((p.tiles + kWaves - 1) / kWaves, 1024);
   p.grid = dim3((unsigned)groups, (unsigned)p.chunks);
   return p;
@@ -358,7 +363,8 @@ void launch_direct_inv_lap(int64_t nt, const double* tx, const double* ty, const
                            const LogTabEntry* logwide, double* partials, double* soln, hipStream_t s) {
   if (nt <= 0) return;
   const Plan p = plan(nt, ns);
-  auto kernel = !p.shared ? k_direct_log<2, 1> : p.nt_lane == 2 ? k_direct_log<2, kWaves> : k_direct_log<1, kWaves>;
+  auto kernel = p.nt_lane == 2 ? (p.shared ? k_direct_log<2, kWaves> : k_direct_log<2, 1>)
+                               : (p.shared ? k_direct_log<1, kWaves> : k_direct_log<1, 1>);
   hipLaunchKernelGGL(kernel, p.grid, dim3(64 * kWaves), 0, s, nt, tx, ty, tz, ns, sx, sy, sz, area, pots, self_offset,
                      guard_coincident ? 1 : 0, p.chunk_len, p.tiles, logwide, partials);
   launch_reduce(nt, 1, p.chunks, partials, Ptr3{{soln, nullptr, nullptr}}, s);
@@ -377,11 +383,11 @@ void launch_direct_bve_vel(int64_t nt, const double* tx, const double* ty, const
                        disp[1], disp[2], moved);
     ax = moved; ay = moved + ns; az = moved + 2 * ns;
   }
-  auto kernel = !p.shared        ? k_direct_bs<2, 1, true>
-                : p.nt_lane == 2 ? k_direct_bs<2, kWaves, true>
-                                 : k_direct_bs<1, kWaves, true>;
+  auto kernel = p.nt_lane == 2 ? (p.shared ? k_direct_bs<2, kWaves, true> : k_direct_bs<2, 1, true>)
+                               : (p.shared ? k_direct_bs<1, kWaves, true> : k_direct_bs<1, 1, true>);
   if (!rcp4_in_range(eps))
-    kernel = !p.shared ? k_direct_bs<2, 1, false> : p.nt_lane == 2 ? k_direct_bs<2, kWaves, false> : k_direct_bs<1, kWaves, false>;
+    kernel = p.nt_lane == 2 ? (p.shared ? k_direct_bs<2, kWaves, false> : k_direct_bs<2, 1, false>)
+                            : (p.shared ? k_direct_bs<1, kWaves, false> : k_direct_bs<1, 1, false>);
   hipLaunchKernelGGL(kernel, p.grid, dim3(64 * kWaves), 0, s, nt, tx, ty, tz, ns, ax, ay, az, area, vor, eps,
                      p.chunk_len, p.tiles, partials);
   launch_reduce(nt, 3, p.chunks, partials, Ptr3{{vel[0], vel[1], vel[2]}}, s);
