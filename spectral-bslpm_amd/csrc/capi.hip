@@ -230,10 +230,10 @@ int upload(sbslpm_ctx* c, void* dst, const void* src, size_t bytes) {
 }
 
 // k_bve_mixed puts four tiles on a workgroup, and four of the heaviest on each of the
-// first of a short list: breadth first, with the ranges of that order, below 2,500 tiles
-// (velocity at 636 tiles by work 265 us and breadth first 229, at 2,046 123 and 117, at
-// 2,556 of 36 rows 197 and 204, at 4,092 323 and 358).
-static bool valu_bfs(const Tree& t) { return t.tiles.size() < 2500; }
+// first of a short list: breadth first, with the ranges of that order, from 400 to 2,500
+// tiles (velocity at 126 tiles by work 84 us and breadth first 89, at 636 265 and 229, at
+// 2,046 123 and 117, at 2,556 of 36 rows 197 and 204, at 4,092 323 and 358).
+static bool valu_bfs(const Tree& t) { return t.tiles.size() >= 400 && t.tiles.size() < 2500; }
 
 // A launch shape for the context's full target-major tile list: with the
 // cost-balanced XCD mapping (xcd 2) the grid is 8 x the largest XCD range in
