@@ -690,13 +690,18 @@ PROBE_MIXES = {
     7: "4 v_mfma_f32_16x16x32_bf16 (independent accumulators)",
     8: "step with a 16x16x32 bf16 first product, alpha as its accumulator, batched reciprocals",
     9: "step with a 16x16x32 bf16 first product, alpha as its accumulator, 4 reciprocals",
+    10: "16 v_fma_f32 (independent, vector-register operands)",
+    11: "16 v_fma_f32 (independent, one scalar-register operand)",
+    12: "16 v_fma_f64 (independent, vector-register operands)",
+    13: "16 v_fma_f64 (independent, one scalar-register operand)",
+    14: "16 v_rcp_f64 (independent)",
 }
 
 
 def bench_probe(args, torch):
     """Register-only issue-rate probes (spectral-bslpm_amd/csrc/probe/issue_rates.hip) behind the
-    floor table of the mixed pair kernel: shader-clock cycles per iteration of each instruction
-    mix, per wave and per SIMD, at 1 and 4 waves per SIMD (256 compute units x 4 SIMDs)."""
+    floor table of the pair kernels: shader-clock cycles per iteration of each instruction
+    mix, per wave and per SIMD, at 1, 4 and 8 waves per SIMD (256 compute units x 4 SIMDs)."""
     lib_path = os.path.join(REPO, "spectral-bslpm_amd", "libsbslpm_probe.so")
     if not os.path.exists(lib_path):
         raise SystemExit("libsbslpm_probe.so is not built: run __graft_entry__.build()")
@@ -709,7 +714,7 @@ def bench_probe(args, torch):
     out = {}
     for mix, what in PROBE_MIXES.items():
         row = {"mix": what}
-        for wps in (1, 4):
+        for wps in (1, 4, 8):
             blocks, wpb = 256 * wps, 4  # one block of 4 waves per compute unit and wps blocks per unit
             cyc, ms = ctypes.c_double(), ctypes.c_double()
             lib.sbslpm_probe_issue(mix, blocks, wpb, iters // 10, ctypes.byref(cyc), ctypes.byref(ms))  # warm-up

@@ -1,6 +1,6 @@
 // issue_rates.hip -- register-only probes of the instruction mixes that bound
-// the matrix-core Biot-Savart pair kernel (k_bve_mfma) on gfx950, for the
-// per-kernel floor table of the measurement notes.  Each probe runs a fixed
+// the matrix-core Biot-Savart pair kernel (k_bve_mfma) and the vector-unit pair
+// kernels on gfx950, for the per-kernel floor table of the measurement notes.  Each probe runs a fixed
 // instruction mix `iters` times on registers only (no memory traffic in the
 // loop), every wave of the grid doing the same; the host times the launch and
 // also reads the shader clock (s_memtime) around the loop in every wave.
@@ -20,6 +20,11 @@
 //      (operands split into three bf16 parts), alpha as its accumulator input
 //      (no adds) and the four reciprocals batched
 //   9  as 8 with four reciprocals
+//  10  16 v_fma_f32, independent, all operands in vector registers
+//  11  16 v_fma_f32, independent, the multiplier in a scalar register
+//  12  16 v_fma_f64, independent, all operands in vector registers
+//  13  16 v_fma_f64, independent, the multiplier in a scalar register
+//  14  16 v_rcp_f64, independent chains
 // C ABI: sbslpm_probe_issue(mix, blocks, waves_per_block, iters, out_cycles,
 // out_ms) launches and synchronises; out_cycles receives the mean shader clock
 // count per iteration per wave, out_ms the launch's event time.  The loops
@@ -27,6 +32,7 @@
 #include <hip/hip_runtime.h>
 
 #include <cstdint>
+#include <type_traits>
 
 namespace {
 
@@ -120,11 +126,45 @@ __global__ __launch_bounds__(1024) void k_probe(int iters, float seed, unsigned 
   if (lane == 0) atomicAdd(cycles, t1 - t0);
 }
 
+// Mixes 10 to 14.  The multiplier arrives as a kernel argument, in scalar registers (in
+// either type: a conversion would leave it in a vector register).
+template <int MIX>
+__global__ __launch_bounds__(1024) void k_probe_operands(int iters, double mul, float mulf,
+                                                         unsigned long long* cycles, float* sink) {
+  const int lane = threadIdx.x & 63;
+  typedef typename std::conditional<(MIX < 12), float, double>::type T;
+  T r[16], a = (T)mul, b = (T)1e-4;
+#pragma unroll
+  for (int i = 0; i < 16; ++i) r[i] = (T)1 + (T)0.001 * (lane + i);
+  if (MIX == 10 || MIX == 12) __asm__ volatile("" : "+v"(a));
+  __asm__ volatile("" : "+v"(b));
+  const unsigned long long t0 = __builtin_amdgcn_s_memtime();
+  for (int it = 0; it < iters; ++it) {
+#pragma unroll
+    for (int i = 0; i < 16; ++i) {
+      if constexpr (MIX == 14)
+        r[i] = __builtin_amdgcn_rcp(r[i]);
+      else if constexpr (MIX == 11)  // (left to itself the compiler copies the scalar first)
+        __asm__ volatile("v_fma_f32 %0, %0, %1, %2" : "+v"(r[i]) : "s"(mulf), "v"(b));
+      else if constexpr (MIX == 10)
+        r[i] = fmaf(r[i], a, b);
+      else
+        r[i] = fma(r[i], a, b);
+    }
+  }
+  const unsigned long long t1 = __builtin_amdgcn_s_memtime();
+  T s = 0;
+#pragma unroll
+  for (int i = 0; i < 16; ++i) s += r[i];
+  sink[blockIdx.x * blockDim.x + threadIdx.x] = (float)s;
+  if (lane == 0) atomicAdd(cycles, t1 - t0);
+}
+
 }  // namespace
 
 extern "C" int sbslpm_probe_issue(int mix, int blocks, int waves_per_block, int iters, double* out_cycles,
                                   double* out_ms) {
-  if (mix < 0 || mix > 9 || blocks < 1 || waves_per_block < 1 || waves_per_block > 16 || iters < 1) return 1;
+  if (mix < 0 || mix > 14 || blocks < 1 || waves_per_block < 1 || waves_per_block > 16 || iters < 1) return 1;
   unsigned long long* cyc = nullptr;
   float* sink = nullptr;
   const size_t nthreads = (size_t)blocks * waves_per_block * 64;
@@ -151,6 +191,11 @@ extern "C" int sbslpm_probe_issue(int mix, int blocks, int waves_per_block, int 
       case 6: hipLaunchKernelGGL(k_probe<6>, grid, block, 0, nullptr, iters, 1.0f, cyc, sink); break;
       case 7: hipLaunchKernelGGL(k_probe<7>, grid, block, 0, nullptr, iters, 1.0f, cyc, sink); break;
       case 8: hipLaunchKernelGGL(k_probe<8>, grid, block, 0, nullptr, iters, 1.0f, cyc, sink); break;
+      case 10: hipLaunchKernelGGL(k_probe_operands<10>, grid, block, 0, nullptr, iters, 0.999, 0.999f, cyc, sink); break;
+      case 11: hipLaunchKernelGGL(k_probe_operands<11>, grid, block, 0, nullptr, iters, 0.999, 0.999f, cyc, sink); break;
+      case 12: hipLaunchKernelGGL(k_probe_operands<12>, grid, block, 0, nullptr, iters, 0.999, 0.999f, cyc, sink); break;
+      case 13: hipLaunchKernelGGL(k_probe_operands<13>, grid, block, 0, nullptr, iters, 0.999, 0.999f, cyc, sink); break;
+      case 14: hipLaunchKernelGGL(k_probe_operands<14>, grid, block, 0, nullptr, iters, 0.999, 0.999f, cyc, sink); break;
       default: hipLaunchKernelGGL(k_probe<9>, grid, block, 0, nullptr, iters, 1.0f, cyc, sink); break;
     }
     (void)hipEventRecord(e1, nullptr);
