@@ -182,9 +182,11 @@ __global__ __launch_bounds__(64 * S) void k_bve64(DevTree t, const TargetTile* _
 }
 
 // The same in lane copies (lanes.hpp) of two targets, for tiles of at most 42 rows
-// (lanes64), whose rows fill 36 of 64 lanes one per lane.  Microseconds per launch,
-// a row per lane and here: 6 x 96^2 (degree 8) 141 -> 132, 6 x 192^2 499 -> 415
-// (degree 5: 302 -> 250); at 16 waves per tile the short loops gain nothing.
+// (lanes64), whose rows fill 36 of 64 lanes one per lane.  Microseconds per pair call
+// (records included), one wave per tile with a row per lane and here: 6 x 96^2 (degree
+// 8) 265 -> 117, 6 x 192^2 665 -> 400 (a row per lane and waves sharing the tile: 499 a
+// launch), degree 5 463 -> 254, 6 x 160^2 (degree 4) 324 -> 157.  At 16 waves per tile
+// the short loops gain nothing.
 template <int S>
 __global__ __launch_bounds__(64 * S) void k_bve64_lanes(DevTree t, const TargetTile* __restrict__ tiles, int ntiles,
                                                         const SourceSet* __restrict__ sets,
@@ -336,8 +338,9 @@ __global__ __launch_bounds__(64 * S) void k_log64(DevTree t, const TargetTile* _
 }
 
 // The same in lane copies (lanes.hpp) of two targets, for tiles of at most 42 rows
-// (lanes64).  Microseconds per launch, a row per lane and here: 6 x 96^2 (degree 8)
-// 194 -> 171, 6 x 192^2 672 -> 597 (degree 5: 417 -> 393).
+// (lanes64).  Microseconds per pair call, one wave per tile and here: 6 x 96^2 (degree
+// 8) 459 -> 155, 6 x 192^2 1109 -> 548 (a row per lane and waves sharing the tile: 672 a
+// launch), degree 5 725 -> 342, 6 x 160^2 (degree 4) 502 -> 232.
 template <int S>
 __global__ __launch_bounds__(64 * S) void k_log64_lanes(DevTree t, const TargetTile* __restrict__ tiles, int ntiles,
                                                         const SourceSet* __restrict__ sets,
@@ -476,9 +479,9 @@ __global__ __launch_bounds__(64 * S) void k_lap64(DevTree t, const TargetTile* _
 }
 
 // The same in lane copies (lanes.hpp) of two targets, for tiles of at most 42 rows
-// (lanes64).  Microseconds per launch in lane groups of one target, with a row per
-// lane and here: 6 x 96^2 (degree 8) 446, 355, 272; 6 x 192^2 1175, 1010, 770 (degree
-// 5: 594, 571, 453); 6 x 160^2 (degree 4) 366, 419, 339.
+// (lanes64), W tiles to a workgroup.  Microseconds per pair call in lane groups of one
+// target and here: 6 x 96^2 (degree 8) 445 -> 247, 6 x 192^2 1167 -> 762 (a row per lane:
+// 1010 a launch), degree 5 586 -> 437, 6 x 160^2 (degree 4) 360 -> 262 (419).
 template <int S, int W>
 __global__ __launch_bounds__(64 * S * W) void k_lap64_lanes(DevTree t, const TargetTile* __restrict__ tiles, int ntiles,
                                                         const SourceSet* __restrict__ sets,

@@ -1,13 +1,16 @@
-// lanes.hpp -- lane copies of a tile's targets for the FP32 pair kernels.
+// lanes.hpp -- lane copies of a tile's targets, for the FP32 pair kernels and for
+// the FP64 ones on small or uneven tiles.
 //
-// A vector instruction of FP32 operands from vector registers issues in 2.5
-// cycles per wave, one with a scalar-register operand in 4.5 (measured with
-// eight waves per SIMD), so the source records are read from LDS into vector
-// registers rather than as scalar loads.  Each lane then holds NT targets, so
-// that one record read (16 LDS cycles for 32 bytes over a wave) serves NT pairs,
-// and the tile's ceil(count / NT) lanes are repeated in as many copies as a wave
-// holds; copy g takes sources g, g + G, ... of a staged chunk.  The copies' and
-// then the waves' sums are added in order through LDS.
+// A vector instruction of FP32 operands from vector registers issues in 2.7
+// cycles per wave, one with a scalar-register operand in 4.8 (probe/issue_rates.hip,
+// mixes 10 and 11 with eight waves per SIMD at a nominal 2.4 GHz; FP64 4.8 to 5.1 with
+// either), so the source records are read from LDS into vector registers rather
+// than as scalar loads.  Each lane then holds NT targets, so that one record read
+// (16 LDS cycles for 32 bytes over a wave) serves NT pairs, and the tile's
+// ceil(count / NT) lanes are repeated in as many copies as a wave holds; copy g takes
+// sources g, g + G, ... of a staged chunk.  The copies' and then the waves' sums are
+// added in order through LDS.  In FP64 the gain is the lanes that a row per lane
+// leaves idle.
 #pragma once
 #include "pairwalk.hpp"
 

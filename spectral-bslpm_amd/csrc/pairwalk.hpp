@@ -1,12 +1,13 @@
-// pairwalk.hpp -- how the waves of an FP64 pair kernel divide a target tile's
-// source sets.
+// pairwalk.hpp -- how the waves of a pair kernel that share a target tile divide
+// its source sets: FP64 with a row per lane, and the lane copies of either
+// precision (lanes.hpp).
 //
 // A workgroup is S waves on one tile of up to 64 targets: four of them take
 // the sets in turn, and S / 4 take consecutive parts of each set, dealt round
 // so that an uneven division evens out.  The waves' sums are added in wave
 // order through LDS, so a result depends on S and on nothing else; S follows
-// from the length of the tile list alone, so members, launch shapes and graph
-// replays agree to the bit.
+// from the length of the tile list and its rows per tile alone, so members,
+// launch shapes and graph replays agree to the bit.
 //
 // One wave per tile left each SIMD with too few waves to hide the source
 // records' scalar loads behind (vector issue busy 55% at 8,190 tiles) and the

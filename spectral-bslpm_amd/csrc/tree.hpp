@@ -64,6 +64,10 @@ struct SourceSet {
 // split at 636 tiles (8% to 19% heaviest first), 8% to 16% at 2,556 (1% to 3%)
 // and 3% to 6% at 8,190; what a short list gains is measured at dealt_tile
 // (pairwalk.hpp), what a long one loses without its locality at strip_length.
+// Either side of the line, calls in breadth-first strips and heaviest first: 4,092
+// tiles (degree 8, 81 points) velocity 283 and 269 us (FP32 193 and 178), Poisson solve
+// 369 and 357, velocity adjoint 293 and 290, at degree 10 with 121 points 523 and 592;
+// 10,236 tiles (degree 8, 64 points) 642 and 616 (429 and 413), 882 and 867, 742 and 828.
 constexpr int kBalancedTiles = 6000;
 
 // Rows that decide how a list's pair kernels lay out a tile: the fullest tile's of a
@@ -103,7 +107,7 @@ struct Tree {
   std::vector<SourceSet> srcsets;       // per-tile source lists (CSR via tiles)
   std::vector<int> set_start;           // [P+1]: source sets of target panel p are [set_start[p], set_start[p+1])
   std::vector<TargetTile> bfs_tiles;    // the same tiles in breadth-first panel order
-  std::vector<TargetTile> nonleaf_tiles;  // the tiles of non-leaf target panels, in the order of `tiles`
+  std::vector<TargetTile> nonleaf_tiles;  // the tiles of non-leaf target panels, heaviest first where they are few
   std::vector<int> xcd_start;           // [4][9]: tiles [xcd_start[x], xcd_start[x+1]) of XCD x in the
                                         // cost-balanced contiguous launch mapping (PairShape xcd 2):
                                         // by blocks of 16, by sources; then both over bfs_tiles
