@@ -126,7 +126,8 @@ __global__ __launch_bounds__(64 * S) void k_swe64(DevTree t, const TargetTile* _
 // The same in lane copies (lanes.hpp) of two targets, for tiles of at most 42 rows
 // (lanes64) and for irregular trees.  Microseconds per pair call in lane groups of one
 // target and here: 6 x 96^2 (degree 8) 272 -> 150, 6 x 192^2 838 -> 530 (a row per lane:
-// 686 a launch), degree 5 478 -> 325 (423), 6 x 160^2 (degree 4, 25 rows) 267 -> 198 (294).  Variant 2, velocity calls in lane groups, with a row per lane and
+// 686 a launch), degree 5 478 -> 325 (423), 6 x 160^2 (degree 4, 25 rows) 267 -> 198
+// (294).  Variant 2, velocity calls in lane groups, with a row per lane and
 // here: 6 x 96^2 (degree 8) 366, 258, 223; 6 x 192^2 1120, 909, 772; 6 x 160^2 (degree
 // 4) 366, 381, 278; 6 x 320^2 1201, 1396, 1013.
 template <int VARIANT, int S>
