@@ -188,14 +188,19 @@ void launch_bve_interact_lanes(const DevTree& t, const TargetTile* tiles, int nt
   // 166; at 36 rows and more 2% to 3% of a single step, so 8 stay)
   int S = t.rows <= 32 && ntiles >= 400 ? 4 : lane_waves(ntiles);
   auto kernel = S == 8 ? k_bve_lanes<8, 2> : k_bve_lanes<4, 2>;
-  // tiles of at most 16 rows: one target per lane halves what a set costs to centre and
+  // tiles of at most 10 rows: one target per lane halves what a set costs to centre and
   // flush, and sets of 9 records give fewer waves enough.  Velocity at degree 2, 3 x 3
   // points a leaf, with two targets and 4 waves, and with one and 4 / 2 / 1: 2,046 tiles
   // 42, 38 / 42 / 54 us; 8,190 99, 86 / 86 / 91; 32,766 300, 254 / 237 / 231; a step of 16
-  // members at 2,046 tiles 1,182, 993 / 927 / 900
+  // members at 2,046 tiles 1,182, 993 / 927 / 900.  Their six copies or more still give each
+  // FP32 sum one record of a set; the four copies of 16 rows would give it two, and 268 us
+  // at 32,766 tiles, but 1% to 10% further from FP64: 11 to 16 rows keep two targets.
+  // With 4 / 2 / 1 waves there: 2,046 tiles 37 / 38 / 50, 8,190 104 / 104 / 116, 32,766 316 /
+  // 299 / 296; a step of 16 members at 510 tiles 411 (8 waves 636) / 408 / 443
   if (t.rows <= 16) {
-    S = ntiles < 1000 ? 4 : 2;
-    kernel = S == 4 ? k_bve_lanes<4, 1> : k_bve_lanes<2, 1>;
+    S = ntiles < (t.rows <= 10 ? 1000 : 6000) ? 4 : 2;
+    kernel = t.rows > 10 ? (S == 4 ? k_bve_lanes<4, 2> : k_bve_lanes<2, 2>)
+                         : (S == 4 ? k_bve_lanes<4, 1> : k_bve_lanes<2, 1>);
   }
   Ptr3 op{{out_part[0], out_part[1], out_part[2]}}, ox{{out_proxy[0], out_proxy[1], out_proxy[2]}};
   hipLaunchKernelGGL(kernel, dim3(walk_grid(ntiles, shape), nmem), dim3(64 * S), 0, s, t, tiles, ntiles, sets,

@@ -276,15 +276,13 @@ const HostTables& host_tables() {
 int velocity(sbslpm_ctx* c, const Work& w, int nmem, const double* area, const double* vor,
              const double* const* dpart, const double* const* dprox, double* const* vel);
 
-// Whether the vortex pairs of a mixed-precision context run on the matrix cores:
-// where bf16 M2L products are asked for, and on long lists of tiles of 13 to 16 rows,
-// which fill a 16 x 16 block per source set.  (Velocity at degree 3, 4 x 4 points a leaf,
-// 32,766 tiles, on the vector unit 268 us and here 240; a step of 16 members at 2,046
-// tiles 1,074 and 948, at 510 tiles 369 and 361, where a single step takes 157 and 181.
-// Distance from FP64 at 2,046 tiles 4.7e-8 and 5.1e-8.)
-bool matrix_pairs(const sbslpm_ctx* c) {
-  return c->dt.bf16_m2l || (c->dt.rows > 12 && c->dt.rows <= 16 && c->ntiles >= 1000);
-}
+// Whether the vortex pairs of a mixed-precision context run on the matrix cores: where
+// bf16 M2L products are asked for.  (Long lists of tiles of 13 to 16 rows, which fill a
+// 16 x 16 block per source set, would be faster there: velocity at degree 3, 4 x 4 points
+// a leaf, 32,766 tiles, 299 us on the vector unit and 240, a step of 16 members at 2,046
+// tiles 1,282 and 948.  But further from FP64: 4.14e-8 and 4.45e-8 for smooth fields,
+// 7.7e-8 and 8.4e-8 for noise, at 2,046 tiles 4.7e-8 and 5.1e-8.)
+bool matrix_pairs(const sbslpm_ctx* c) { return c->dt.bf16_m2l; }
 
 // The tile list of a launch: by work, but breadth first where each XCD takes an equal
 // count of neighbours (mapping 1; velocity at 6 x 128^2, degree 8, FP64: 220 us by work

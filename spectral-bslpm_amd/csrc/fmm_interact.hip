@@ -830,7 +830,7 @@ __global__ void k_src_mfma(DevTree t, const double* __restrict__ q_part, const d
 // 4x4x1 form uses lanes 4 b .. 4 b + 3 (A row / B column = lane % 4, D row =
 // register).  The next source tile's operands are loaded before the current
 // tile's arithmetic (every index stays inside the set's padded records).
-template <int NTT, bool M2L>
+template <int NTT>
 __device__ inline void bve_mfma_tiles(const DevTree& t, const TargetTile& T, const SourceSet* __restrict__ sets,
                                       const float* __restrict__ rec, float eps, int lane, double (&w)[4][3]) {
   const int col = lane & 15, grp = lane >> 4;
@@ -878,7 +878,7 @@ __device__ inline void bve_mfma_tiles(const DevTree& t, const TargetTile& T, con
     const float na1 = rn[lane];
     const v4f nbq = *reinterpret_cast<const v4f*>(rn + off_b);
     v4f d[NTT];
-    kernel_products<NTT>(a1, b1, M2L && S.m2l, d);
+    kernel_products<NTT>(a1, b1, S.m2l, d);
 #pragma unroll
     for (int tt = 0; tt < NTT; ++tt)
 #pragma unroll
@@ -909,7 +909,6 @@ __device__ inline void bve_mfma_tiles(const DevTree& t, const TargetTile& T, con
   }
 }
 
-template <bool M2L>
 __global__ __launch_bounds__(256) void k_bve_mfma(DevTree t, const TargetTile* __restrict__ tiles, int ntiles,
                                                   const SourceSet* __restrict__ sets,
                                                   const float* __restrict__ rec, float eps, Ptr3 part,
@@ -927,10 +926,10 @@ __global__ __launch_bounds__(256) void k_bve_mfma(DevTree t, const TargetTile* _
 #pragma unroll
   for (int tt = 0; tt < 4; ++tt) w[tt][0] = w[tt][1] = w[tt][2] = 0.0;
   switch (ntt) {
-    case 4: bve_mfma_tiles<4, M2L>(t, T, sets, rec, eps, lane, w); break;
-    case 3: bve_mfma_tiles<3, M2L>(t, T, sets, rec, eps, lane, w); break;
-    case 2: bve_mfma_tiles<2, M2L>(t, T, sets, rec, eps, lane, w); break;
-    default: bve_mfma_tiles<1, M2L>(t, T, sets, rec, eps, lane, w); break;
+    case 4: bve_mfma_tiles<4>(t, T, sets, rec, eps, lane, w); break;
+    case 3: bve_mfma_tiles<3>(t, T, sets, rec, eps, lane, w); break;
+    case 2: bve_mfma_tiles<2>(t, T, sets, rec, eps, lane, w); break;
+    default: bve_mfma_tiles<1>(t, T, sets, rec, eps, lane, w); break;
   }
   // sum the four source quarters (lanes col, col+16, col+32, col+48)
 #pragma unroll
@@ -1288,7 +1287,7 @@ void launch_bve_interact_mfma(const DevTree& t, const TargetTile* tiles, int nti
                               hipStream_t s, bool assign, int nmem, PairShape shape) {
   if (ntiles == 0) return;
   shape = checked_shape(t, shape);
-  hipLaunchKernelGGL(t.bf16_m2l ? k_bve_mfma<true> : k_bve_mfma<false>, dim3(pair_grid(ntiles, shape), nmem), dim3(64 * shape.waves), 0, s, t,
+  hipLaunchKernelGGL(k_bve_mfma, dim3(pair_grid(ntiles, shape), nmem), dim3(64 * shape.waves), 0, s, t,
                      tiles, ntiles, sets, (const float*)rec, (float)eps, ptr3(out_part), ptr3(out_proxy),
                      assign ? 1 : 0, shape.xcd);
 }

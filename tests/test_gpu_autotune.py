@@ -89,16 +89,18 @@ def test_autotuned_graph_step_matches_eager(sb, torch_gpu):
         np.testing.assert_array_equal(to_np(vg), to_np(ve))
 
 
-# levels 5 with 16 rows a tile: mixed precision runs on the matrix cores, where waves count
-@pytest.mark.parametrize("precision,degree,leaf_degree,by_tile", [
-    ("fp64", 8, 7, True), ("mixed", 8, 7, True), ("mixed", 3, 3, False), ("mixed_valu", 8, 7, False)])
-def test_waves_are_tuned_where_they_count(sb, torch_gpu, precision, degree, leaf_degree, by_tile):
+# 16 rows a tile (degree 3) stay on the vector unit, whose sums are nearer to FP64; bf16 M2L
+# products run on the matrix cores, where waves count
+@pytest.mark.parametrize("precision,degree,leaf_degree,bf16,by_tile", [
+    ("fp64", 8, 7, False, True), ("mixed", 8, 7, False, True), ("mixed", 3, 3, False, True),
+    ("mixed", 8, 7, True, False), ("mixed_valu", 8, 7, False, False)])
+def test_waves_are_tuned_where_they_count(sb, torch_gpu, precision, degree, leaf_degree, bf16, by_tile):
     """A kernel with a workgroup per tile has one launch per mapping: three candidates share its
     time, and the waves per workgroup that the context's other kernels read stay as set."""
     t = torch_gpu
-    print(f"\n[case waves {precision} d{degree}]", flush=True)
+    print(f"\n[case waves {precision} d{degree} bf16={bf16}]", flush=True)
     ctx = sb.Context(sb.RunConfig(levels=5, interp_degree=degree, leaf_degree=leaf_degree, kernel_eps=1e-4,
-                                  weights="clenshaw_curtis", precision=precision))
+                                  weights="clenshaw_curtis", precision=precision, bf16_m2l=bf16))
     x, y, z, a = ctx.spec_points()
     area, vor = to_gpu(t, a), to_gpu(t, sb.workloads.gaussian_vortices(x, y, z, a, seed=5))
     ctx.set_pair_shape(2, 0)
