@@ -88,14 +88,11 @@ __device__ inline void wave_sum(double (&v)[K], int wave, int lane) {
       for (int k = 0; k < K; ++k) v[k] += red[w][k][lane];
 }
 
-// The wave's tiles: the workgroup's one (W waves share it), or every 8 gridDim.x-th.
-template <int W, typename F>
-__device__ inline void for_tiles(int64_t tiles, int wave, F&& f) {
-  if constexpr (W > 1) {
-    f((int64_t)blockIdx.x);
-  } else {
-    for (int64_t tile = (int64_t)blockIdx.x * kWaves + wave; tile < tiles; tile += (int64_t)gridDim.x * kWaves) f(tile);
-  }
+// A wave's first tile: the workgroup's one (W waves share it), or the first of every
+// 8 gridDim.x-th.
+template <int W>
+__device__ inline int64_t first_tile(int wave) {
+  return W > 1 ? (int64_t)blockIdx.x : (int64_t)blockIdx.x * kWaves + wave;
 }
 
 // guard 0: skip j == self_offset + i (the reference's i != j);
@@ -125,7 +122,9 @@ __global__ __launch_bounds__(64 * kWaves) void k_direct_log(int64_t nt, const do
   __syncthreads();
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int lane = threadIdx.x & 63;
-  for_tiles<W>(tiles, wave, [&](int64_t tile) {
+  int64_t tile = first_tile<W>(wave);
+  if (W == 1 && tile >= tiles) return;
+  do {
     const int64_t i0 = tile * (64 * NT);
     double x[NT], y[NT], z[NT], acc[NT];
 #pragma unroll
@@ -189,7 +188,8 @@ __global__ __launch_bounds__(64 * kWaves) void k_direct_log(int64_t nt, const do
 #pragma unroll
       for (int t = 0; t < NT; ++t)
         if (i0 + t * 64 + lane < nt) partials[(int64_t)blockIdx.y * nt + i0 + t * 64 + lane] = kNegInv4Pi * acc[t];
-  });
+    tile += (int64_t)gridDim.x * kWaves;
+  } while (W == 1 && tile < tiles);
 }
 
 // Bound: FP64 vector issue.  The four denominators of a batch share one
@@ -208,7 +208,9 @@ __global__ __launch_bounds__(64 * kWaves) void k_direct_bs(int64_t nt, const dou
                                                    double* __restrict__ partials) {
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int lane = threadIdx.x & 63;
-  for_tiles<W>(tiles, wave, [&](int64_t tile) {
+  int64_t tile = first_tile<W>(wave);
+  if (W == 1 && tile >= tiles) return;
+  do {
     const int64_t i0 = tile * (64 * NT);
     double x[NT], y[NT], z[NT], w[3 * NT];
 #pragma unroll
@@ -264,7 +266,8 @@ __global__ __launch_bounds__(64 * kWaves) void k_direct_bs(int64_t nt, const dou
       p[nt + i] = kNegInv4Pi * (z[t] * u[0] - x[t] * u[2]);
       p[2 * nt + i] = kNegInv4Pi * (x[t] * u[1] - y[t] * u[0]);
     }
-  });
+    tile += (int64_t)gridDim.x * kWaves;
+  } while (W == 1 && tile < tiles);
 }
 
 struct Ptr3 {
@@ -288,15 +291,16 @@ __global__ __launch_bounds__(64 * kWaves) void k_reduce(int64_t nt, int ncomp, i
   if (wave == 0 && i < nt) out.p[f][i] += s[0];
 }
 
-// The same for a few chunks, a thread per target.
+// The same for at most three chunks, a thread per target, the chunks' loads together.
 __global__ __launch_bounds__(256) void k_reduce_few(int64_t nt, int ncomp, int64_t chunks,
                                                     const double* __restrict__ partials, Ptr3 out) {
   const int f = (int)blockIdx.y;
   const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
   if (i >= nt) return;
-  double s = 0;
-  for (int64_t c = 0; c < chunks; ++c) s += partials[(c * ncomp + f) * nt + i];
-  out.p[f][i] += s;
+  double v[3];
+#pragma unroll
+  for (int c = 0; c < 3; ++c) v[c] = c < chunks ? partials[((int64_t)c * ncomp + f) * nt + i] : 0;
+  out.p[f][i] += v[0] + v[1] + v[2];
 }
 
 void launch_reduce(int64_t nt, int ncomp, int64_t chunks, const double* partials, Ptr3 out, hipStream_t s) {
